@@ -19,7 +19,7 @@ BUILD = PKG / "_build"
 LIB = PKG / "libsphgpu.so"
 
 SOURCES = ["api.hip", "grid.hip", "solvers.hip", "iisph_df.hip", "sort.hip", "mlp.hip", "scene.cpp", "io.cpp",
-           "surface.hip", "mc_table.cpp"]
+           "surface.hip", "mc_table.cpp", "readback.hip", "xfer.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = [

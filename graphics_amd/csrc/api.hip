@@ -5,6 +5,7 @@
 #include "mlp.h"
 #include "sph_common.h"
 #include "sphgpu.h"
+#include "xfer.h"
 
 #include <algorithm>
 #include <cmath>
@@ -108,6 +109,11 @@ struct sphgpu_handle {
     double* hStats = nullptr;
     int* hLayout = nullptr;
     float* hDt = nullptr;
+    int* hRemoved = nullptr;           // written by the readback kernels
+    // readback: pinned staging, ranks of the live ids (once particles were removed)
+    HostRing ring;
+    uint32_t* idRank = nullptr;
+    long long idRankCap = 0;
     std::vector<sphgpu_stats> sceneStats;
     // learned warm start of the divergence solve
     MlpDev mlp{};
@@ -1145,6 +1151,8 @@ void sphgpu_destroy(sphgpu_handle* h) {
         for (void* m : h->allocs) hipFree(m);
         if (h->mlpLive) mlp_free(h->mlp);
         hipHostFree(h->hActive);
+        h->ring.release();
+        hipFree(h->idRank);
         if (h->snap.cs) {
             hipStreamSynchronize(h->snap.cs);
             hipEventDestroy(h->snap.copied);
@@ -1616,7 +1624,8 @@ int sphgpu_init(sphgpu_handle* h) {
         h->hStats = reinterpret_cast<double*>(c); c += 32 * (size_t)ns;
         h->hCounters = reinterpret_cast<int*>(c); c += 8 * C_COUNT;
         h->hLayout = reinterpret_cast<int*>(c); c += 16;
-        h->hDt = reinterpret_cast<float*>(c);
+        h->hDt = reinterpret_cast<float*>(c); c += 8 * (size_t)ns;
+        h->hRemoved = reinterpret_cast<int*>(c);
     }
 
     hipStream_t st = h->st;
@@ -1788,52 +1797,98 @@ int live_slots(sphgpu_handle* h, std::vector<std::pair<int, int>>& out) {
 }
 }  // namespace
 
+namespace {
+// ranks of the live ids (general readback: particles were removed); *live = their number
+int live_ranks(sphgpu_handle* h, long long* live) {
+    const long long words = h->nextId + 1;
+    if (h->idRankCap < words) {
+        hipFree(h->idRank);
+        h->idRank = nullptr;
+        h->idRankCap = 0;
+        const long long cap = words + words / 4;   // ids keep growing with appends
+        HIPCHECK(h, hipMalloc(&h->idRank, sizeof(uint32_t) * (size_t)(cap + scan_tmp_words(int(cap)))));
+        h->idRankCap = cap;
+    }
+    launch_live_ranks(h->D, h->idRank, int(h->nextId), h->idRank + h->idRankCap, h->st);
+    uint32_t n = 0;
+    HIPCHECK(h, hipMemcpyAsync(&n, h->idRank + h->nextId, sizeof(n), hipMemcpyDeviceToHost, h->st));
+    HIPCHECK(h, hipStreamSynchronize(h->st));
+    *live = n;
+    return 0;
+}
+
+// `pass(rank, removed)` queues the kernel that writes n values of `bytes`
+// each, in id order, to the device buffer `dev`; copied to `out`.  While every
+// id ever given is live (the host's count says so, and the device counts no
+// removal since) a value's place is its id; otherwise it is the rank of the id.
+int read_in_order(sphgpu_handle* h, void* out, const void* dev, size_t bytes,
+                  const std::function<void(const uint32_t*)>& pass) {
+    if (h->D.npad == 0) return 0;
+    if (h->nLive == h->nextId) {
+        pass(nullptr);
+        HIPCHECK(h, h->ring.to_host(out, dev, bytes * (size_t)h->nextId, h->st));
+        HIPCHECK(h, hipGetLastError());
+        if (*h->hRemoved == 0) return 0;
+    }
+    long long live = 0;
+    if (int rc = live_ranks(h, &live)) return rc;
+    pass(h->idRank);
+    HIPCHECK(h, h->ring.to_host(out, dev, bytes * (size_t)live, h->st));
+    HIPCHECK(h, hipGetLastError());
+    return 0;
+}
+}  // namespace
+
 int sphgpu_get_fluid(sphgpu_handle* h, int field, float* out) {
     if (!h || !out) return SPHGPU_E_ARG;
     if (!h->initialized) return fail(h, SPHGPU_E_STATE, "not initialised");
     Dev& D = h->D;
-    std::vector<std::pair<int, int>> ls;
-    int rc = live_slots(h, ls);
-    if (rc) return rc;
-    int comp = 1;
-    const void* src = nullptr;
-    bool f4 = false;
+    const bool ii = h->P.solver == SPHGPU_IISPH;
+    const float4* src4 = nullptr;
+    const float* src = nullptr;
+    int comp = 3;
     switch (field) {
-        case SPHGPU_F_POS: src = D.x; f4 = true; comp = 3; break;
-        case SPHGPU_F_VEL: src = D.v; f4 = true; comp = 3; break;
+        case SPHGPU_F_POS: src4 = D.x; break;
+        case SPHGPU_F_VEL: src4 = D.v; break;
         case SPHGPU_F_RHO: src = D.rho; break;
-        case SPHGPU_F_PRESSURE: src = (h->P.solver == SPHGPU_IISPH) ? D.kr : D.f1; break;
-        case SPHGPU_F_ACC: src = (h->P.solver == SPHGPU_IISPH) ? D.f4b : D.f4a; f4 = true; comp = 3; break;
+        case SPHGPU_F_PRESSURE: src = ii ? D.kr : D.f1; break;
+        case SPHGPU_F_ACC: src4 = ii ? D.f4b : D.f4a; break;
         case SPHGPU_F_ALPHA: src = D.alpha; break;
         case SPHGPU_F_KAPPA_SUM: src = D.ksum; break;
-        case SPHGPU_F_PHASE: src = D.x; f4 = true; comp = 1; break;
+        case SPHGPU_F_PHASE: src4 = D.x; comp = 1; break;
         case SPHGPU_F_KAPPAV_SUM: src = D.kvsum; break;
         default: return fail(h, SPHGPU_E_ARG, "unknown field %d", field);
     }
-    if (f4) {
-        std::vector<float4> buf(D.npad);
-        HIPCHECK(h, hipMemcpy(buf.data(), src, sizeof(float4) * D.npad, hipMemcpyDeviceToHost));
-        for (size_t k = 0; k < ls.size(); ++k) {
-            const float4& q = buf[ls[k].second];
-            if (field == SPHGPU_F_PHASE) out[k] = q.w;
-            else { out[3 * k] = q.x; out[3 * k + 1] = q.y; out[3 * k + 2] = q.z; }
-        }
-    } else {
-        std::vector<float> buf(D.npad);
-        HIPCHECK(h, hipMemcpy(buf.data(), src, sizeof(float) * D.npad, hipMemcpyDeviceToHost));
-        for (size_t k = 0; k < ls.size(); ++k) out[k] = buf[ls[k].second];
-    }
-    (void)comp;
-    return SPHGPU_OK;
+    // x2 is free between the passes of a step: the reorder (and the fused
+    // integration of WCSPH and IISPH) writes it before anything reads it
+    float* dev = reinterpret_cast<float*>(D.x2);
+    if (src) comp = 1;
+    return read_in_order(h, out, dev, sizeof(float) * comp, [&](const uint32_t* rank) {
+        if (src) launch_field_by_id(D, src, rank, dev, h->hRemoved, h->st);
+        else launch_field_by_id(D, src4, comp, rank, dev, h->hRemoved, h->st);
+    });
 }
 
 int sphgpu_get_fluid_ids(sphgpu_handle* h, long long* out) {
     if (!h || !out) return SPHGPU_E_ARG;
     if (!h->initialized) return fail(h, SPHGPU_E_STATE, "not initialised");
-    std::vector<std::pair<int, int>> ls;
-    int rc = live_slots(h, ls);
-    if (rc) return rc;
-    for (size_t k = 0; k < ls.size(); ++k) out[k] = ls[k].first;
+    Dev& D = h->D;
+    if (D.npad == 0) return SPHGPU_OK;
+    if (h->nLive == h->nextId) {
+        launch_ids_by_rank(D, nullptr, nullptr, h->hRemoved, h->st);
+        HIPCHECK(h, hipStreamSynchronize(h->st));
+        HIPCHECK(h, hipGetLastError());
+        if (*h->hRemoved == 0) {
+            std::iota(out, out + h->nextId, 0LL);
+            return SPHGPU_OK;
+        }
+    }
+    long long live = 0;
+    if (int rc = live_ranks(h, &live)) return rc;
+    long long* dev = reinterpret_cast<long long*>(D.x2);
+    launch_ids_by_rank(D, h->idRank, dev, h->hRemoved, h->st);
+    HIPCHECK(h, h->ring.to_host(out, dev, sizeof(long long) * (size_t)live, h->st));
+    HIPCHECK(h, hipGetLastError());
     return SPHGPU_OK;
 }
 

@@ -518,6 +518,18 @@ void launch_copy_probe(const float4* a, float4* b, size_t n, hipStream_t st);
 // dst[i] = src[i] with a kernel (graph-capturable, no copy engine)
 void launch_copy_f4(float4* dst, const float4* src, size_t n, hipStream_t st);
 
+// readback.hip: fluid fields in ascending original id.  rank[id] = place of a
+// live id among the live ids, rank[ids] their number (ids + 1 words); a field
+// is written to out[id] without a rank (every id ever given is live), to
+// out[rank[id]] with one; *removed receives the particles removed since the
+// counters were last reported.  The launches need npad > 0.
+void launch_live_ranks(const Dev& D, uint32_t* rank, int ids, uint32_t* tmp, hipStream_t st);
+void launch_field_by_id(const Dev& D, const float4* src, int comp, const uint32_t* rank, float* out, int* removed,
+                        hipStream_t st);
+void launch_field_by_id(const Dev& D, const float* src, const uint32_t* rank, float* out, int* removed,
+                        hipStream_t st);
+void launch_ids_by_rank(const Dev& D, const uint32_t* rank, long long* out, int* removed, hipStream_t st);
+
 // iisph_df.hip: the IISph class's DF_* solvers
 void launch_idf_prepare(const Dev& D, hipStream_t st);
 void launch_idf_vadv(const Dev& D, int mode, hipStream_t st);

@@ -1,0 +1,40 @@
+// Transfers between device memory and a caller's ordinary (pageable) host
+// buffer through a bounded pinned staging ring that the owning object keeps.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <cstddef>
+
+namespace sphgpu {
+
+// A copy engine writes pinned memory at 56 GB/s, while hipMemcpy to a
+// pageable buffer reaches 18 GB/s at 12 MB and 10 GB/s at 48 MB (fresh
+// destination pages), and takes 85 us for 188 KB.  The ring splits a transfer
+// into chunks: the DMA of the next chunks runs while the host copies the
+// finished ones out.  The host copy of a large transfer is bound by the
+// destination's page faults on one thread (3.4 of 3.7 ms at 48 MB), so above
+// kThreadedBytes the chunks are shared by up to four threads that end before
+// the call returns.  Measured (MI355X, fresh destination): 20 KB 16 -> 9 us,
+// 188 KB 85 -> 16 us, 1.4 MB 139 -> 78 us, 12 MB 777 -> 411 us, 48 MB 4.85 ->
+// 1.44 ms; chunks of 1 and 4 MB were 25 and 4 % slower at 48 MB, eight
+// threads no faster than four.
+struct HostRing {
+    static constexpr int kSlots = 8;
+    static constexpr size_t kChunk = size_t(2) << 20;
+    static constexpr size_t kThreadedBytes = 2 * kChunk;
+    static constexpr int kMaxThreads = 4;
+
+    char* mem = nullptr;
+    size_t cap = 0;                    // bytes pinned, at most kSlots * kChunk
+    hipEvent_t done[kSlots] = {};
+
+    // device -> host; waits for everything queued on st before it, and
+    // returns with `dst` complete
+    hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t st);
+    void release();
+
+private:
+    hipError_t reserve(size_t bytes);
+};
+
+}  // namespace sphgpu
