@@ -146,6 +146,14 @@ __global__ __launch_bounds__(256) void k_cell_build(const uint32_t* __restrict__
 // global memory directly (6 or 8 groups: LDS per block against blocks per
 // CU, chosen by the autotuner).  Both forms hold the same entries in the
 // same order.
+// Bound: on a large scene the candidate loop (about 216 candidates a
+// particle, 16 B of L1 return and fifteen VALU operations each); on a small
+// one the latency of a block's serial chain.  The loop's short form, the slot
+// bounds from the rows' end lanes only and flushing without barriers took it
+// from 887 to 740 us at 4,000,752 particles, 234 to 176 us at 1,000,000, 100
+// to 77 us at 328,233 and 54 to 41 us at 1,728 (six groups).  Not kept: the
+// next group's loads issued before this group's tests (4 % slower at 4M), the
+// nine rows in one rolled loop (25 % slower).
 template <int NB_STAGE_GROUPS>
 __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
     __shared__ int4 stage[NB_STAGE_GROUPS][256];
@@ -205,20 +213,31 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
             if (rb.y > rb.x) runB[r] = rb;
         }
     }
-    // per slot: the smallest run start and the largest run end of the tile
+    // per slot: the smallest run start and the largest run end of the tile.
+    // Along the particles of one own row the runs move up, so of each wave
+    // only the row's first and last particle with a run can hold them: two
+    // LDS atomics of at most NB16_ROWS lanes a run (from every lane they
+    // serialise on one address, 8 of the builder's 40 us on a small scene).
     if (packed && act) {
+        // lanes of this wave in the particle's own row
+        unsigned long long mine = 0;
 #pragma unroll
-        for (int r = 0; r < 9; ++r) {
-            const int slot = ord * 9 + r;
-            if (runF[r].y > runF[r].x) {
-                atomicMin(&sBase[slot], runF[r].x);
-                atomicMax(&sEnd[slot], runF[r].y);
-            }
-            if (runB[r].y > runB[r].x) {
-                atomicMin(&sBase[32 + slot], runB[r].x);
-                atomicMax(&sEnd[32 + slot], runB[r].y);
-            }
+        for (int o = 0; o < NB16_ROWS; ++o) {
+            const unsigned long long b = __ballot(ord == o);
+            if (ord == o) mine = b;
         }
+        auto bounds = [&](const int2* runs, int slot0) {
+#pragma unroll
+            for (int r = 0; r < 9; ++r) {
+                const bool has = runs[r].y > runs[r].x;
+                const unsigned long long b = __ballot(has) & mine;
+                if (!has) continue;
+                if (__ffsll((long long)b) - 1 == lane) atomicMin(&sBase[slot0 + ord * 9 + r], runs[r].x);
+                if (63 - __clzll((long long)b) == lane) atomicMax(&sEnd[slot0 + ord * 9 + r], runs[r].y);
+            }
+        };
+        bounds(runF, 0);
+        bounds(runB, 32);
     }
     __syncthreads();
     if (tid < 64 && sBase[tid] != INT_MAX && sEnd[tid] - sBase[tid] > (1 << NB16_OFF_BITS)) sOverflow = 1;
@@ -259,18 +278,16 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
             if (win && list == D.nbF16) reinterpret_cast<uint16_t*>(D.nbW16)[nb16_slot(k, i, stride)] = uint16_t(to_win(e));
         }
     };
+    // (a thread stages and flushes its own column: no barrier around either)
     auto flush = [&](int* list, int count) {
-        __syncthreads();
         const int ng = min((count + 3) >> 2, NB_STAGE_GROUPS);
         int4* out = reinterpret_cast<int4*>(list);
         for (int g = 0; g < ng; ++g) {
             const int b = (4 * g) << 8;
             out[(size_t)g * stride + i] = make_int4(st[b + tid], st[b + 256 + tid], st[b + 512 + tid], st[b + 768 + tid]);
         }
-        __syncthreads();
     };
     auto flush16 = [&](int4* out, int count) {
-        __syncthreads();
         const int ng = min((count + 7) >> 3, NB_STAGE_GROUPS);
         const bool towin = win && out == D.nbF16;
         for (int g = 0; g < ng; ++g) {
@@ -290,60 +307,84 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
                 D.nbW16[(size_t)g * stride + i] = make_int4(r[0], r[1], r[2], r[3]);
             }
         }
-        __syncthreads();
     };
     int nbn = 0, over = 0, zero = 0;
     // Candidate loop of one kind (fluid or boundary), candidates four at a
     // time (four loads in flight, tested in order).  A candidate's entry is
     // stored in LDS at the next free entry before the test decides (a miss
     // is overwritten by the next hit, or lies past the padded count that
-    // the passes read), so the common path has no branch; entries past the
-    // LDS stage go to global memory and entries past the list width are
-    // counted (both rare, in a branch of their own).  n: entries found.
-    auto candidates = [&](auto packed_c, const int2* runs, const float4* __restrict__ xs, int selfj, int cap,
+    // the passes read).  While every lane of the wave has four staged entries
+    // free, a group takes the short form: no test against the stage or the
+    // list width, the self index compared in the particle's own row only
+    // (the one row run that holds it), and coincident pairs counted only when
+    // the smallest of the four squared distances is zero.  Otherwise entries
+    // past the LDS stage go to global memory and entries past the list width
+    // are counted.  n: entries found.
+    auto candidates = [&](auto packed_c, auto fluid_c, const int2* runs, const float4* __restrict__ xs, int cap,
                           int slot0, int4* list16, int* list32, int& n) {
-        constexpr bool PK = decltype(packed_c)::value;
+        constexpr bool PK = decltype(packed_c)::value, FLUID = decltype(fluid_c)::value;
         constexpr int STAGE = PK ? NB_STAGE_GROUPS * 8 : NB_STAGE_GROUPS * 4;
 #pragma unroll
         for (int r = 0; r < 9; ++r) {
             const int2 rr = runs[r];
             const int bias = PK && rr.y > rr.x ? bias16(slot0 + ord * 9 + r) : 0;
+            const bool own = FLUID && r == 4;   // the row run that holds the particle itself
             for (int j0 = rr.x; j0 < rr.y; j0 += 4) {
                 // (up to X_TAIL records past the run are read, and not used:
                 // the position arrays are that much longer)
                 const float4* __restrict__ xg = xs + j0;
                 float4 q[4];
+                float l2[4];
+                bool hit[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) q[k] = xg[k];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    const int j = j0 + k;
-                    const float l2 = dis_square_exact(pa, q[k]);
-                    const bool hit = j < rr.y && j != selfj && l2 < D.h2;
-                    if (n < STAGE) {
-                        if (PK) st16[(n << 8) + tid] = uint16_t(j + bias);
-                        else st[(n << 8) + tid] = j;
+                    l2[k] = dis_square_exact(pa, q[k]);
+                    hit[k] = j0 + k < rr.y && l2[k] < D.h2;
+                    if (own) hit[k] = hit[k] && j0 + k != i;
+                }
+                if (__ballot(n > STAGE - 4) == 0) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (PK) st16[(n << 8) + tid] = uint16_t(j0 + k + bias);
+                        else st[(n << 8) + tid] = j0 + k;
+                        n += hit[k];
                     }
-                    if (hit && n >= STAGE) {
-                        if (n < cap) {
-                            if (PK) put16(list16, n, bias, j);
-                            else put(list32, n, j);
-                        } else {
-                            ++over;
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int j = j0 + k;
+                        if (n < STAGE) {
+                            if (PK) st16[(n << 8) + tid] = uint16_t(j + bias);
+                            else st[(n << 8) + tid] = j;
                         }
+                        if (hit[k] && n >= STAGE) {
+                            if (n < cap) {
+                                if (PK) put16(list16, n, bias, j);
+                                else put(list32, n, j);
+                            } else {
+                                ++over;
+                            }
+                        }
+                        n += hit[k];
                     }
-                    zero += (hit && l2 == 0.0f);
-                    n += hit;
+                }
+                if (own || fminf(fminf(l2[0], l2[1]), fminf(l2[2], l2[3])) == 0.0f) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) zero += (hit[k] && l2[k] == 0.0f);
                 }
             }
         }
     };
     using PackedT = std::integral_constant<bool, true>;
     using PlainT = std::integral_constant<bool, false>;
+    using FluidT = PackedT;
+    using WallT = PlainT;
     // fluid neighbours (SphBase.cpp:867-905); the particle itself is skipped
     int nf = 0;
-    if (packed) candidates(PackedT{}, runF, D.x, i, NBF_CAP, 0, D.nbF16, nullptr, nf);
-    else candidates(PlainT{}, runF, D.x, i, NBF_CAP, 0, nullptr, D.nbF, nf);
+    if (packed) candidates(PackedT{}, FluidT{}, runF, D.x, NBF_CAP, 0, D.nbF16, nullptr, nf);
+    else candidates(PlainT{}, FluidT{}, runF, D.x, NBF_CAP, 0, nullptr, D.nbF, nf);
     const int stored = min(nf, NBF_CAP);
     const int cf = act ? stored : 0;
     // pad: the particle itself
@@ -355,8 +396,8 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
     else flush(D.nbF, cf);
     // boundary neighbours (SphBase.cpp:908-930); no index is skipped
     if (act) {
-        if (packed) candidates(PackedT{}, runB, D.xb, -1, NBB_CAP, 32, D.nbB16, nullptr, nbn);
-        else candidates(PlainT{}, runB, D.xb, -1, NBB_CAP, 32, nullptr, D.nbB, nbn);
+        if (packed) candidates(PackedT{}, WallT{}, runB, D.xb, NBB_CAP, 32, D.nbB16, nullptr, nbn);
+        else candidates(PlainT{}, WallT{}, runB, D.xb, NBB_CAP, 32, nullptr, D.nbB, nbn);
     }
     const int cb = act ? min(nbn, NBB_CAP) : 0;
     // pad: the far dummy particle
