@@ -97,6 +97,7 @@ struct sphgpu_handle {
     SortScratch sort{};
     uint32_t* sk = nullptr;
     uint32_t* sv = nullptr;
+    uint32_t* order = nullptr;         // counting search: slots in cell order, by arrival
     // small device buffers
     int* layoutOut = nullptr;          // [npad_new, live]
     double* statsPart = nullptr;       // per tile 4
@@ -236,30 +237,42 @@ int run_ns(sphgpu_handle* h) {
     h->needSearch = false;
     hipStream_t st = h->st;
     int npad = D.npad;
-    {
-        ProfScope ps(h, "ns_keys", nf_live(h) * 20.0);
-        launch_fluid_keys_into(D, h->sk, h->sv, st);
+    if (D.cellRuns) {
+        {
+            ProfScope ps(h, "ns_sort", nf_live(h) * 100.0);
+            launch_search_fluid(D, h->sk, h->sv, h->order, h->layoutOut, st);
+        }
+        std::swap(D.x, D.x2);
+        std::swap(D.v, D.v2);
+        std::swap(D.id, D.id2);
+        std::swap(D.ksum, D.ksum2);
+        std::swap(D.kvsum, D.kvsum2);
+    } else {
+        {
+            ProfScope ps(h, "ns_keys", nf_live(h) * 20.0);
+            launch_fluid_keys_into(D, h->sk, h->sv, st);
+        }
+        {
+            ProfScope ps(h, "ns_sort", nf_live(h) * 16.0 * ((h->keyBits + 7) / 8));
+            radix_sort_pairs(h->sk, h->sv, npad, h->keyBits, h->sort, st);
+        }
+        launch_fill_i32(D.sceneStart, -1, D.nscenes, st);
+        launch_fill_i32(D.sceneCount, 0, D.nscenes, st);
+        launch_scene_bounds(D, h->sk, npad, st);
+        launch_scene_layout(D, h->layoutOut, st);
+        {
+            ProfScope ps(h, "ns_reorder", nf_live(h) * 64.0);
+            launch_reorder(D, h->sk, h->sv, npad, npad, st);
+        }
+        std::swap(D.x, D.x2);
+        std::swap(D.v, D.v2);
+        std::swap(D.id, D.id2);
+        std::swap(D.ksum, D.ksum2);
+        std::swap(D.kvsum, D.kvsum2);
+        std::swap(D.key, D.key2);
+        launch_cell_reset(D, D.key2, npad, D.cellF, st);
+        launch_cell_build(D, D.key, npad, D.cellF, st);
     }
-    {
-        ProfScope ps(h, "ns_sort", nf_live(h) * 16.0 * ((h->keyBits + 7) / 8));
-        radix_sort_pairs(h->sk, h->sv, npad, h->keyBits, h->sort, st);
-    }
-    launch_fill_i32(D.sceneStart, -1, D.nscenes, st);
-    launch_fill_i32(D.sceneCount, 0, D.nscenes, st);
-    launch_scene_bounds(D, h->sk, npad, st);
-    launch_scene_layout(D, h->layoutOut, st);
-    {
-        ProfScope ps(h, "ns_reorder", nf_live(h) * 64.0);
-        launch_reorder(D, h->sk, h->sv, npad, npad, st);
-    }
-    std::swap(D.x, D.x2);
-    std::swap(D.v, D.v2);
-    std::swap(D.id, D.id2);
-    std::swap(D.ksum, D.ksum2);
-    std::swap(D.kvsum, D.kvsum2);
-    std::swap(D.key, D.key2);
-    launch_cell_reset(D, D.key2, npad, D.cellF, st);
-    launch_cell_build(D, D.key, npad, D.cellF, st);
     {
         ProfScope ps(h, "ns_neighbours", nf_live(h) * 12.0);
         launch_neighbours(D, st);
@@ -692,6 +705,18 @@ int finish_step(sphgpu_handle* h, sphgpu_stats* out) {
     return 0;
 }
 
+// sk, sv: the boundary's cell keys and source indices in cell order (stable);
+// the counting search also fills its cell table
+void sort_boundary(sphgpu_handle* h, const float4* xs, const int* scene) {
+    Dev& D = h->D;
+    if (D.cellRuns) {
+        launch_search_boundary(D, xs, scene, h->sort.keys2, h->sort.vals2, h->order, h->sk, h->sv, h->st);
+    } else {
+        launch_boundary_keys_from(D, xs, scene, h->sk, h->sv, h->st);
+        radix_sort_pairs(h->sk, h->sv, D.nb, h->keyBits, h->sort, h->st);
+    }
+}
+
 // Dynamic solids, at the start of a step: new poses to the device, world
 // positions and velocities, boundary re-sort into cell order, cell ranges,
 // Akinci volumes (SphSolid::updatePaticles, SphBase::updateSolidPartWeight).
@@ -705,14 +730,15 @@ int rigid_update(sphgpu_handle* h) {
         h->posesDirty = false;
     }
     launch_rigid_pose(D, st);
-    launch_boundary_keys_from(D, D.xb, D.bscene, h->sk, h->sv, st);
-    radix_sort_pairs(h->sk, h->sv, D.nb, h->keyBits, h->sort, st);
+    sort_boundary(h, D.xb, D.bscene);
     launch_boundary_regather(D, h->sk, h->sv, st);
     std::swap(D.xb, D.xb2); std::swap(D.vb, D.vb2); std::swap(D.bloc, D.bloc2);
     std::swap(D.bid, D.bid2); std::swap(D.bsolid, D.bsolid2); std::swap(D.bscene, D.bscene2);
     std::swap(D.bkself, D.bkself2); std::swap(D.bkey, D.bkey2);
-    launch_cell_reset(D, D.bkey2, D.nb, D.cellB, st);
-    launch_cell_build(D, D.bkey, D.nb, D.cellB, st);
+    if (!D.cellRuns) {
+        launch_cell_reset(D, D.bkey2, D.nb, D.cellB, st);
+        launch_cell_build(D, D.bkey, D.nb, D.cellB, st);
+    }
     launch_boundary_volume_update(D, st);
     return 0;
 }
@@ -1115,7 +1141,7 @@ int sphgpu_create(const sphgpu_params* p, sphgpu_handle** out) {
         p->adjust_density > 1 || p->fluid_capacity < 0)
         return SPHGPU_E_ARG;
     if (!(p->spacing_r > 0) || !(p->smooth_radius_h > 0) || !(p->dt > 0)) return SPHGPU_E_ARG;
-    if (p->num_scenes < 1 || p->num_scenes > 4096) return SPHGPU_E_ARG;
+    if (p->num_scenes < 1 || p->num_scenes > MAX_SCENES) return SPHGPU_E_ARG;
     if (p->warm_start < 0 || p->warm_start > 2) return SPHGPU_E_ARG;
     if (p->warm_start == SPHGPU_WARM_LEARNED &&
         ((p->solver != SPHGPU_DFSPH && p->solver != SPHGPU_IISPH) || p->learn_steps < 0 || p->learn_iters < 0 || p->learn_batch < 16 ||
@@ -1588,6 +1614,19 @@ int sphgpu_init(sphgpu_handle* h) {
     ALLOC(h->layoutOut, 2); ALLOC(h->statsPart, 4 * (size_t)numTiles); ALLOC(h->statsOut, 4 * (size_t)ns);
     int sortItems = std::max<int>(ncap, int(nb));
     ALLOC(h->sk, sortItems); ALLOC(h->sv, sortItems);
+    // Counting search while the grid has no more cells than pay for scanning
+    // them every step (5 us a million); a sparser grid keeps the radix
+    // search, which never visits empty cells.  One WCSPH step of 15,625
+    // particles takes 96 us with 1.6 million cells, 123 with 7.8 million and
+    // 161 by radix sort; of 1,000,000 particles 386 us with 3.2 million, 455
+    // with 15.4 million and 504 by radix sort.
+    D.cellRuns = totalKeys <= (uint64_t)SEARCH_CELLS_MIN + (uint64_t)SEARCH_CELLS_PER * (uint64_t)ncap ? 1 : 0;
+    D.cellCnt = D.cellSums = nullptr;
+    D.tileLive = D.sceneShift = nullptr;
+    if (D.cellRuns) {
+        ALLOC(h->order, sortItems); ALLOC(D.tileLive, numTiles); ALLOC(D.sceneShift, ns);
+        ALLOC(D.cellCnt, totalKeys); ALLOC(D.cellSums, (totalKeys + SEARCH_KEYS - 1) / SEARCH_KEYS);
+    }
     void* sortMem;
     HIPCHECK(h, hipMalloc(&sortMem, sort_scratch_bytes(sortItems)));
     h->allocs.push_back(sortMem);
@@ -1634,6 +1673,7 @@ int sphgpu_init(sphgpu_handle* h) {
     HIPCHECK(h, hipMemcpyAsync(dkb, h->hKeyBase.data(), sizeof(uint32_t) * (ns + 1), hipMemcpyHostToDevice, st));
     HIPCHECK(h, hipMemsetAsync(D.cellF, 0, sizeof(int2) * totalKeys, st));
     HIPCHECK(h, hipMemsetAsync(D.cellB, 0, sizeof(int2) * totalKeys, st));
+    if (D.cellRuns) HIPCHECK(h, hipMemsetAsync(D.cellCnt, 0, sizeof(uint32_t) * totalKeys, st));
     HIPCHECK(h, hipMemsetAsync(D.counters, 0, sizeof(int) * C_COUNT, st));
     HIPCHECK(h, hipMemsetAsync(D.ksum, 0, sizeof(float) * ncap, st));
     HIPCHECK(h, hipMemsetAsync(D.kvsum, 0, sizeof(float) * ncap, st));
@@ -1694,10 +1734,9 @@ int sphgpu_init(sphgpu_handle* h) {
         HIPCHECK(h, hipMemcpy(tx, hb.data(), sizeof(float4) * nb, hipMemcpyHostToDevice));
         HIPCHECK(h, hipMemcpy(tsolid, h->bsolid.data(), sizeof(int) * nb, hipMemcpyHostToDevice));
         HIPCHECK(h, hipMemcpy(tscene, h->bscene.data(), sizeof(int) * nb, hipMemcpyHostToDevice));
-        launch_boundary_keys_from(D, tx, tscene, h->sk, h->sv, st);
-        radix_sort_pairs(h->sk, h->sv, int(nb), h->keyBits, h->sort, st);
+        sort_boundary(h, tx, tscene);
         launch_boundary_reorder(D, tx, tsolid, tscene, h->sk, h->sv, st);
-        launch_cell_build(D, D.bkey, int(nb), D.cellB, st);
+        if (!D.cellRuns) launch_cell_build(D, D.bkey, int(nb), D.cellB, st);
         launch_boundary_volume(D, st);
         if (D.anyDynamic) {
             // body-frame samples in sorted order, then the per-step update once.

@@ -137,6 +137,320 @@ __global__ __launch_bounds__(256) void k_cell_build(const uint32_t* __restrict__
 }
 
 
+// ---- counting search --------------------------------------------------------
+// The order of the radix search (by cell key, stable in the old slot order)
+// without its three digit passes: particles are counted per cell, the counts
+// scanned into the cell table, each particle dropped into its cell's segment
+// in arrival order, and its place in the segment found by counting the
+// segment's smaller slot indices (a cell holds about eight particles; the
+// list builder reads the particles of 27 cells per particle, so however many
+// a cell holds, this is the smaller part).  Atomics only decide the arrival
+// order, which the last step sorts out, so the result is the same every run.
+// Four launches on a small grid, six on others, for about twenty.  Bound by
+// launches and latency on a small scene, by the 104 B a particle of the reorder
+// on a large one.  Kernels of one search without the list builder, MI355X: 23
+// us for 15,625 particles (75 us by radix sort), 85 us for 1,000,000 (160),
+// 190 us for 4,000,752 (330).
+constexpr int SCAN1_THREADS = 1024;
+
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(v, off, 64);
+        if (lane >= off) v += y;
+    }
+    return v;
+}
+
+// exclusive prefix of v over a block of W waves; *total = the block's sum
+template <int W>
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* lds, uint32_t* total) {
+    const int w = threadIdx.x >> 6;
+    const uint32_t x = wave_incl_scan(v);
+    if ((threadIdx.x & 63) == 63) lds[w] = x;
+    __syncthreads();
+    uint32_t pre = 0, tot = 0;
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+        const uint32_t s = lds[k];
+        if (k < w) pre += s;
+        tot += s;
+    }
+    __syncthreads();
+    *total = tot;
+    return pre + x - v;
+}
+
+// arrival rank of each lane's particle in its cell.  Neighbouring slots mostly
+// share a cell, so one lane adds for each run of equal keys in the wave (every
+// lane of the wave calls it; key KEY_INVALID: none).
+__device__ __forceinline__ uint32_t cell_arrival(uint32_t key, uint32_t* __restrict__ cnt) {
+    const int lane = lane_id();
+    const uint32_t prev = __shfl_up(key, 1, 64);
+    const bool head = lane == 0 || prev != key;
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long upto = heads & ((2ull << lane) - 1ull), after = heads & ~((2ull << lane) - 1ull);
+    const int first = 63 - __clzll((long long)upto);
+    uint32_t base = 0;
+    if (head && key != KEY_INVALID) {
+        const int next = after ? __ffsll((long long)after) - 1 : 64;
+        base = atomicAdd(&cnt[key], (uint32_t)(next - lane));
+    }
+    return __shfl(base, first, 64) + (uint32_t)(lane - first);
+}
+
+__global__ __launch_bounds__(256) void k_count_fluid(Dev D, uint32_t* __restrict__ keys,
+                                                     uint32_t* __restrict__ arrival) {
+    const int tile = blockIdx.x, i = tile * TILE + threadIdx.x;   // npad is a multiple of TILE
+    uint32_t k = KEY_INVALID;
+    if (D.id[i] >= 0) {
+        const float4 p = D.x[i];
+        const SceneGrid G = D.grids[D.tileScene[tile]];
+        int cx, cy, cz;
+        cell_of(G, p, cx, cy, cz);
+        k = key_of(G, D.rowRank, cx, cy, cz);
+    }
+    keys[i] = k;
+    arrival[i] = cell_arrival(k, D.cellCnt);
+    const int live = __syncthreads_count(k != KEY_INVALID);
+    if (threadIdx.x == 0) D.tileLive[tile] = live;
+}
+
+__global__ __launch_bounds__(256) void k_count_boundary(Dev D, const float4* __restrict__ xs,
+                                                        const int* __restrict__ scene, uint32_t* __restrict__ keys,
+                                                        uint32_t* __restrict__ arrival) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    uint32_t k = KEY_INVALID;
+    if (i < D.nb) {
+        const SceneGrid G = D.grids[scene[i]];
+        int cx, cy, cz;
+        cell_of(G, xs[i], cx, cy, cz);
+        k = key_of(G, D.rowRank, cx, cy, cz);
+    }
+    const uint32_t a = cell_arrival(k, D.cellCnt);
+    if (i < D.nb) {
+        keys[i] = k;
+        arrival[i] = a;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_cell_sums(Dev D) {
+    __shared__ uint32_t lds[4];
+    const uint32_t k0 = blockIdx.x * (uint32_t)SEARCH_KEYS + threadIdx.x;
+    uint32_t s = 0;
+#pragma unroll
+    for (int q = 0; q < SEARCH_KEYS / 256; ++q)
+        if (k0 + q * 256 < D.totalKeys) s += D.cellCnt[k0 + q * 256];
+    uint32_t tot;
+    block_scan<4>(s, lds, &tot);
+    if (threadIdx.x == 0) D.cellSums[blockIdx.x] = tot;
+}
+
+// scene counts, padded starts and tile tables, by one block; `total` = live particles
+__device__ __forceinline__ void layout_block(const Dev& D, uint32_t total, int* __restrict__ out, uint32_t* lds) {
+    const int tid = threadIdx.x, ns = D.nscenes, tiles = D.npad / TILE, all = D.ncap / TILE;
+    __shared__ int sceneLive[MAX_SCENES];
+    if (ns == 1) {
+        // (no value read back from memory)
+        const int pad = ((int)total + TILE - 1) / TILE * TILE;
+        if (tid == 0) {
+            D.sceneCount[0] = (int)total;
+            D.sceneStart[0] = 0;
+            D.sceneShift[0] = 0;
+            D.scenePadStart[0] = 0;
+            D.scenePadStart[1] = pad;
+            out[0] = pad;
+            out[1] = (int)total;
+        }
+        for (int t = tid; t < all; t += SCAN1_THREADS) {
+            D.tileScene[t] = 0;
+            D.tileValid[t] = min(max((int)total - t * TILE, 0), TILE);
+        }
+    } else {
+        for (int s = tid; s < ns; s += SCAN1_THREADS) sceneLive[s] = 0;
+        __syncthreads();
+        // tiles of one scene lie together: one atomic per wave where they do
+        for (int t0 = 0; t0 < tiles; t0 += SCAN1_THREADS) {
+            const int t = t0 + tid;
+            const int s = t < tiles ? D.tileScene[t] : -1;
+            int c = t < tiles ? D.tileLive[t] : 0;
+            const int s0 = __builtin_amdgcn_readfirstlane(s);
+            if (__ballot(s != s0) == 0) {
+                if (s0 < 0) continue;          // past the last tile (uniform in the wave)
+                for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+                if ((tid & 63) == 0) atomicAdd(&sceneLive[s0], c);
+            } else if (s >= 0) {
+                atomicAdd(&sceneLive[s], c);
+            }
+        }
+        __syncthreads();
+        uint32_t start = 0, pad = 0;
+        for (int s0 = 0; s0 < ns; s0 += SCAN1_THREADS) {
+            const int s = s0 + tid;
+            const uint32_t c = s < ns ? (uint32_t)sceneLive[s] : 0u;
+            const uint32_t p = (c + TILE - 1) / TILE * TILE;
+            uint32_t ct, pt;
+            const uint32_t c0 = block_scan<SCAN1_THREADS / 64>(c, lds, &ct);
+            const uint32_t p0 = block_scan<SCAN1_THREADS / 64>(p, lds, &pt);
+            if (s < ns) {
+                D.sceneCount[s] = (int)c;
+                D.sceneStart[s] = (int)(start + c0);
+                D.scenePadStart[s] = (int)(pad + p0);
+                D.sceneShift[s] = (int)(pad + p0) - (int)(start + c0);
+            }
+            start += ct;
+            pad += pt;
+        }
+        if (tid == 0) {
+            D.scenePadStart[ns] = (int)pad;
+            out[0] = (int)pad;
+            out[1] = (int)total;
+        }
+        __syncthreads();
+        for (int t = tid; t < all; t += SCAN1_THREADS) {
+            const int slot = t * TILE;
+            int lo = 0, hi = ns - 1;
+            while (lo < hi) {                  // largest s with padStart[s] <= slot
+                const int mid = (lo + hi + 1) >> 1;
+                if (D.scenePadStart[mid] <= slot) lo = mid; else hi = mid - 1;
+            }
+            D.tileScene[t] = lo;
+            D.tileValid[t] = slot < (int)pad ? min(max(sceneLive[lo] - (slot - D.scenePadStart[lo]), 0), TILE) : 0;
+        }
+    }
+}
+
+// Cell table entries of the n keys from k0 on, whose counts are in LDS, by a
+// block of W waves; `first` = rank of the first key's first particle.  Each
+// thread scans `per` consecutive counts in LDS (per odd: no bank conflicts);
+// the table is written, and the counts cleared for the next search, key by
+// lane, so both stores are whole lines (eight keys a thread straight from
+// registers took 70 us for 5.3 million keys, this way 18).
+template <bool FLUID, int W>
+__device__ __forceinline__ uint32_t scan_counts(uint32_t* __restrict__ c, int n, int per, uint32_t first,
+                                                uint32_t* lds) {
+    const int t0 = (int)threadIdx.x * per, t1 = min(t0 + per, n);
+    uint32_t s = 0, tot;
+    for (int k = t0; k < t1; ++k) s += c[k];
+    uint32_t pre = first + block_scan<W>(s, lds, &tot);
+    for (int k = t0; k < t1; ++k) {
+        const uint32_t v = c[k];
+        c[k] = pre;
+        pre += v;
+    }
+    if (threadIdx.x == 0) c[n] = first + tot;
+    __syncthreads();
+    return tot;
+}
+template <bool FLUID, int W>
+__device__ __forceinline__ void write_runs(const Dev& D, uint32_t k0, const uint32_t* __restrict__ c, int n,
+                                           int2* __restrict__ table) {
+    int s = -1, shift = 0;
+    const bool scenes = FLUID && D.nscenes > 1;
+    for (int q = threadIdx.x; q < n; q += 64 * W) {
+        const uint32_t k = k0 + q;
+        if (scenes) {
+            if (s < 0) s = scene_of_key(k, D.sceneKeyBase, D.nscenes);
+            while (k >= D.sceneKeyBase[s + 1]) ++s;
+            shift = D.sceneShift[s];
+        }
+        table[k] = make_int2((int)c[q] + shift, (int)c[q + 1] + shift);
+        D.cellCnt[k] = 0;
+    }
+}
+
+// a grid of at most SEARCH_KEYS_ONE keys: scan, layout and cell table in one block
+template <bool FLUID>
+__global__ __launch_bounds__(SCAN1_THREADS) void k_search_one(Dev D, int2* __restrict__ table, int* __restrict__ out) {
+    constexpr int W = SCAN1_THREADS / 64;
+    __shared__ uint32_t lds[W];
+    __shared__ uint32_t c[SEARCH_KEYS_ONE + 1];
+    const int n = (int)D.totalKeys, per = ((n + SCAN1_THREADS - 1) / SCAN1_THREADS) | 1;
+    for (int k = threadIdx.x; k < n; k += SCAN1_THREADS) c[k] = D.cellCnt[k];
+    __syncthreads();
+    const uint32_t total = scan_counts<FLUID, W>(c, n, per, 0, lds);
+    if (FLUID) {
+        layout_block(D, total, out, lds);
+        __syncthreads();
+    }
+    write_runs<FLUID, W>(D, 0, c, n, table);
+}
+
+// larger grids: the block sums scanned (in place) by one block, which also lays out the scenes
+template <bool FLUID>
+__global__ __launch_bounds__(SCAN1_THREADS) void k_search_mid(Dev D, int blocks, int* __restrict__ out) {
+    __shared__ uint32_t lds[SCAN1_THREADS / 64];
+    uint32_t run = 0;
+    for (int b0 = 0; b0 < blocks; b0 += SCAN1_THREADS) {
+        const int b = b0 + (int)threadIdx.x;
+        const uint32_t v = b < blocks ? D.cellSums[b] : 0u;
+        uint32_t tot;
+        const uint32_t pre = block_scan<SCAN1_THREADS / 64>(v, lds, &tot);
+        if (b < blocks) D.cellSums[b] = run + pre;
+        run += tot;
+    }
+    if (FLUID) layout_block(D, run, out, lds);
+}
+
+template <bool FLUID>
+__global__ __launch_bounds__(256) void k_cell_runs(Dev D, int2* __restrict__ table) {
+    __shared__ uint32_t lds[4];
+    __shared__ uint32_t c[SEARCH_KEYS + 1];
+    const uint32_t k0 = blockIdx.x * (uint32_t)SEARCH_KEYS;
+    const int n = (int)min((uint32_t)SEARCH_KEYS, D.totalKeys - k0);
+#pragma unroll
+    for (int q = 0; q < SEARCH_KEYS / 256; ++q) {
+        const int k = q * 256 + (int)threadIdx.x;
+        if (k < n) c[k] = D.cellCnt[k0 + k];
+    }
+    __syncthreads();
+    scan_counts<FLUID, 4>(c, n, SEARCH_KEYS / 256, D.cellSums[blockIdx.x], lds);
+    write_runs<FLUID, 4>(D, k0, c, n, table);
+}
+
+__global__ __launch_bounds__(256) void k_place(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ arrival,
+                                               const int2* __restrict__ table, int n, uint32_t* __restrict__ order) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t k = keys[i];
+    if (k != KEY_INVALID) order[(uint32_t)table[k].x + arrival[i]] = (uint32_t)i;
+}
+
+// place of the particle order[t] in its cell's segment: the segment's smaller indices
+__device__ __forceinline__ int slot_in_cell(const uint32_t* __restrict__ order, uint32_t i, int2 seg) {
+    int p = seg.x;
+    for (int u = seg.x; u < seg.y; ++u) p += order[u] < i;
+    return p;
+}
+
+__global__ __launch_bounds__(256) void k_reorder_cells(Dev D, const uint32_t* __restrict__ keys,
+                                                       const uint32_t* __restrict__ order) {
+    const int tile = blockIdx.x, t = tile * TILE + threadIdx.x;
+    if ((int)threadIdx.x >= D.tileValid[tile]) {
+        D.id2[t] = -1;                         // padding
+        return;
+    }
+    const uint32_t i = order[t];
+    const int p = slot_in_cell(order, i, D.cellF[keys[i]]);
+    D.x2[p] = D.x[i];
+    D.v2[p] = D.v[i];
+    D.id2[p] = D.id[i];
+    D.ksum2[p] = D.ksum[i];
+    D.kvsum2[p] = D.kvsum[i];
+}
+
+__global__ __launch_bounds__(256) void k_order_boundary(Dev D, const uint32_t* __restrict__ keys,
+                                                        const uint32_t* __restrict__ order, uint32_t* __restrict__ sk,
+                                                        uint32_t* __restrict__ sv) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= D.nb) return;
+    const uint32_t i = order[t], k = keys[i];
+    const int p = slot_in_cell(order, i, D.cellB[k]);
+    sk[p] = k;
+    sv[p] = i;
+}
+
 // Lists are built in LDS, one column per thread, and written out group by
 // group (16 bytes per particle), so each store instruction of a wave writes
 // whole cache lines.  A tile whose particles span at most NB16_ROWS own rows,
@@ -200,17 +514,38 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
     // the nine fluid and boundary row runs (rows y+dy, z+dz, r = 3 (dz+1) +
     // (dy+1)), looked up once and kept in registers; empty: (0, 0)
     int2 runF[9], runB[9];
+    if (D.cellRuns) {
+        // without branches, so that the loads of all nine rows are in flight
+        // together (three round trips instead of one after another per row)
+        int rk[9];
 #pragma unroll
-    for (int r = 0; r < 9; ++r) {
-        runF[r] = make_int2(0, 0);
-        runB[r] = make_int2(0, 0);
-        const int z = cz + r / 3 - 1, y = cy + r % 3 - 1;
-        if (act && z >= 0 && z < G.nz && y >= 0 && y < G.ny) {
-            const uint32_t k0 = key_of(G, D.rowRank, cx, y, z);
-            const int2 rf = run3(D.cellF, k0, cx, G.nx);
-            const int2 rb = run3(D.cellB, k0, cx, G.nx);
-            if (rf.y > rf.x) runF[r] = rf;
-            if (rb.y > rb.x) runB[r] = rb;
+        for (int r = 0; r < 9; ++r) {
+            const int z = min(max(cz + r / 3 - 1, 0), max(G.nz - 1, 0)), y = min(max(cy + r % 3 - 1, 0), max(G.ny - 1, 0));
+            rk[r] = act ? D.rowRank[G.rowBase + z * G.ny + y] : 0;
+        }
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            const int z = cz + r / 3 - 1, y = cy + r % 3 - 1;
+            const bool in = act && z >= 0 && z < G.nz && y >= 0 && y < G.ny;
+            const uint32_t k0 = act ? G.keyBase + (uint32_t)rk[r] * (uint32_t)G.nx + (uint32_t)cx : 0u;
+            const int2 rf = run3(D.cellF, k0, act ? cx : 0, G.nx, 1);
+            const int2 rb = run3(D.cellB, k0, act ? cx : 0, G.nx, 1);
+            runF[r] = in && rf.y > rf.x ? rf : make_int2(0, 0);
+            runB[r] = in && rb.y > rb.x ? rb : make_int2(0, 0);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            runF[r] = make_int2(0, 0);
+            runB[r] = make_int2(0, 0);
+            const int z = cz + r / 3 - 1, y = cy + r % 3 - 1;
+            if (act && z >= 0 && z < G.nz && y >= 0 && y < G.ny) {
+                const uint32_t k0 = key_of(G, D.rowRank, cx, y, z);
+                const int2 rf = run3(D.cellF, k0, cx, G.nx, 0);
+                const int2 rb = run3(D.cellB, k0, cx, G.nx, 0);
+                if (rf.y > rf.x) runF[r] = rf;
+                if (rb.y > rb.x) runB[r] = rb;
+            }
         }
     }
     // per slot: the smallest run start and the largest run end of the tile.
@@ -477,7 +812,7 @@ __global__ __launch_bounds__(256) void k_boundary_volume(Dev D) {
             int y = cy + dy;
             if (y < 0 || y >= G.ny) continue;
             uint32_t k0 = key_of(G, D.rowRank, cx, y, z);
-            int2 rb = run3(D.cellB, k0, cx, G.nx);
+            int2 rb = run3(D.cellB, k0, cx, G.nx, D.cellRuns);
             for (int j = rb.x; j < rb.y; ++j) {
                 if (j == i) continue;
                 float4 pb = D.xb[j];
@@ -560,7 +895,7 @@ __global__ __launch_bounds__(256) void k_boundary_volume_update(Dev D) {
         for (int dy = -1; dy <= 1; ++dy) {
             int y = cy + dy;
             if (y < 0 || y >= G.ny) continue;
-            int2 rb = run3(D.cellB, key_of(G, D.rowRank, cx, y, z), cx, G.nx);
+            int2 rb = run3(D.cellB, key_of(G, D.rowRank, cx, y, z), cx, G.nx, D.cellRuns);
             for (int j = rb.x; j < rb.y; ++j) {
                 if (j == i || D.bsolid[j] == sa) continue;
                 float l2 = dis_square_exact(pa, D.xb[j]);
@@ -605,7 +940,7 @@ __global__ __launch_bounds__(256) void k_rigid_reaction(Dev D, int mode) {
         for (int dy = -1; dy <= 1; ++dy) {
             int y = cy + dy;
             if (y < 0 || y >= G.ny) continue;
-            int2 rf = run3(D.cellF, key_of(G, D.rowRank, cx, y, z), cx, G.nx);
+            int2 rf = run3(D.cellF, key_of(G, D.rowRank, cx, y, z), cx, G.nx, D.cellRuns);
             for (int j = rf.x; j < rf.y; ++j) {
                 const float4 pb = D.x[j];
                 const float l2 = dis_square_exact(pa, pb);
@@ -717,7 +1052,43 @@ __global__ __launch_bounds__(256) void k_neighbour_dump(Dev D, int cap, int* cou
 
 inline int blocks_for(int n) { return (n + 255) / 256; }
 
+// counts -> cell table (and, for the fluid, the scene layout)
+template <bool FLUID>
+void scan_cells(const Dev& D, int2* table, int* layoutOut, hipStream_t st) {
+    if (D.totalKeys <= (uint32_t)SEARCH_KEYS_ONE) {
+        hipLaunchKernelGGL(k_search_one<FLUID>, dim3(1), dim3(SCAN1_THREADS), 0, st, D, table, layoutOut);
+        return;
+    }
+    const int blocks = int((D.totalKeys + SEARCH_KEYS - 1) / SEARCH_KEYS);
+    hipLaunchKernelGGL(k_cell_sums, dim3(blocks), dim3(256), 0, st, D);
+    hipLaunchKernelGGL(k_search_mid<FLUID>, dim3(1), dim3(SCAN1_THREADS), 0, st, D, blocks, layoutOut);
+    hipLaunchKernelGGL(k_cell_runs<FLUID>, dim3(blocks), dim3(256), 0, st, D, table);
+}
+
 }  // namespace
+
+void launch_search_fluid(const Dev& D, uint32_t* keys, uint32_t* arrival, uint32_t* order, int* layoutOut,
+                         hipStream_t st) {
+    const int tiles = D.npad / TILE;
+    if (tiles > 0) hipLaunchKernelGGL(k_count_fluid, dim3(tiles), dim3(256), 0, st, D, keys, arrival);
+    scan_cells<true>(D, D.cellF, layoutOut, st);
+    if (tiles == 0) return;
+    hipLaunchKernelGGL(k_place, dim3(tiles), dim3(256), 0, st, (const uint32_t*)keys, (const uint32_t*)arrival,
+                       (const int2*)D.cellF, D.npad, order);
+    hipLaunchKernelGGL(k_reorder_cells, dim3(tiles), dim3(256), 0, st, D, (const uint32_t*)keys,
+                       (const uint32_t*)order);
+}
+
+void launch_search_boundary(const Dev& D, const float4* xs, const int* scene, uint32_t* keys, uint32_t* arrival,
+                            uint32_t* order, uint32_t* sk, uint32_t* sv, hipStream_t st) {
+    const dim3 g(blocks_for(D.nb)), b(256);
+    if (D.nb > 0) hipLaunchKernelGGL(k_count_boundary, g, b, 0, st, D, xs, scene, keys, arrival);
+    scan_cells<false>(D, D.cellB, nullptr, st);
+    if (D.nb <= 0) return;
+    hipLaunchKernelGGL(k_place, g, b, 0, st, (const uint32_t*)keys, (const uint32_t*)arrival, (const int2*)D.cellB,
+                       D.nb, order);
+    hipLaunchKernelGGL(k_order_boundary, g, b, 0, st, D, (const uint32_t*)keys, (const uint32_t*)order, sk, sv);
+}
 
 void launch_fluid_keys_into(const Dev& D, uint32_t* keys, uint32_t* vals, hipStream_t st) {
     hipLaunchKernelGGL(k_fluid_keys, dim3(blocks_for(D.npad)), dim3(256), 0, st, D, keys, vals);

@@ -170,12 +170,12 @@ __device__ __forceinline__ void boundary_stencil(const Dev& D, int b, float4 pa,
             const int y = cy + dy;
             if (y < 0 || y >= G.ny) continue;
             const uint32_t k0 = key_of(G, D.rowRank, cx, y, z);
-            const int2 rf = run3(D.cellF, k0, cx, G.nx);
+            const int2 rf = run3(D.cellF, k0, cx, G.nx, D.cellRuns);
             for (int j = rf.x; j < rf.y; ++j) {
                 const float4 pb = D.x[j];
                 if (dis_square_exact(pa, pb) < D.h2) fluid(j, pair_of(D, pa, pb));
             }
-            const int2 rb = run3(D.cellB, k0, cx, G.nx);
+            const int2 rb = run3(D.cellB, k0, cx, G.nx, D.cellRuns);
             for (int j = rb.x; j < rb.y; ++j) {
                 if (j == b || D.bsolid[j] == sa) continue;
                 const float4 pb = D.xb[j];

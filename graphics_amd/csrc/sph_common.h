@@ -16,6 +16,7 @@ constexpr int WIN_ALL = 31;
 constexpr int NBB_CAP = 48;          // boundary neighbours kept per particle
 constexpr int REF_NEIGHBOUR_CAP = 48;  // NeigbStr::maxNeigbNum (SphBase.h:630)
 constexpr int MAX_PHASES = 8;
+constexpr int MAX_SCENES = 4096;
 constexpr uint32_t KEY_INVALID = 0xFFFFFFFFu;
 constexpr int SOLVER_IISPH_DF = 4;   // SPHGPU_IISPH_DF: the IISph class's DF_* solvers
 
@@ -175,6 +176,12 @@ struct Dev {
     int2* cellF;       // [start, end) of fluid slots per key
     int2* cellB;       // [start, end) of boundary particles per key
     uint32_t totalKeys;
+    int cellRuns;      // 1 (counting search): every key's entry is set, an empty cell's as
+                       // (s, s) at its place; 0 (radix search): empty cells hold (0, 0)
+    uint32_t* cellCnt;   // counting search: particles per key, zero between searches
+    uint32_t* cellSums;  // per SEARCH_KEYS keys
+    int* tileLive;       // live particles of each tile before the search
+    int* sceneShift;     // padded slot minus sorted rank of each scene
 
     // ---- scene layout
     int* sceneStart;     // first sorted rank of each scene (unpadded)
@@ -231,8 +238,12 @@ __device__ __forceinline__ uint32_t key_of(const SceneGrid& G, const int* rowRan
     return G.keyBase + (uint32_t)row * (uint32_t)G.nx + (uint32_t)cx;
 }
 
-// union of the [start,end) ranges of three consecutive keys (empty = start >= end)
-__device__ __forceinline__ int2 run3(const int2* __restrict__ table, uint32_t k0, int cx, int nx) {
+// union of the [start,end) ranges of three consecutive keys (empty = start >= end).
+// filled (Dev::cellRuns): entries of empty cells lie in place too, so the run
+// is [start of the first, end of the last): two loads and no branch.
+__device__ __forceinline__ int2 run3(const int2* __restrict__ table, uint32_t k0, int cx, int nx, int filled) {
+    if (filled)
+        return make_int2(table[k0 - (cx > 0 ? 1 : 0)].x, table[k0 + (cx + 1 < nx ? 1 : 0)].y);
     int s = 0x7fffffff, e = 0;
     for (int dx = -1; dx <= 1; ++dx) {
         int c = cx + dx;
@@ -450,6 +461,18 @@ int scan_tmp_words(int n);
 void exclusive_scan_u32(uint32_t* data, int n, uint32_t* tmp, hipStream_t st);
 
 // grid.hip
+// Counting search (Dev::cellRuns): particles counted per cell key, the counts
+// scanned into the cell table, and each cell's particles put in slot order.
+constexpr int SEARCH_KEYS = 9 * 256;       // keys per block of the scan (nine a thread: odd)
+constexpr int SEARCH_KEYS_ONE = 32768;     // grids up to this are scanned by one block
+constexpr int SEARCH_CELLS_MIN = 12000000; // largest grid: SEARCH_CELLS_MIN cells and
+constexpr int SEARCH_CELLS_PER = 8;        // SEARCH_CELLS_PER per particle slot
+void launch_search_fluid(const Dev& D, uint32_t* keys, uint32_t* arrival, uint32_t* order, int* layoutOut,
+                         hipStream_t st);
+// sorted keys and source indices of the boundary (sk, sv) and its cell table
+void launch_search_boundary(const Dev& D, const float4* xs, const int* scene, uint32_t* keys, uint32_t* arrival,
+                            uint32_t* order, uint32_t* sk, uint32_t* sv, hipStream_t st);
+// radix search
 void launch_fluid_keys_into(const Dev& D, uint32_t* keys, uint32_t* vals, hipStream_t st);
 void launch_scene_bounds(const Dev& D, const uint32_t* sortedKeys, int n, hipStream_t st);
 void launch_scene_layout(const Dev& D, int* hostOut, hipStream_t st);
