@@ -101,7 +101,6 @@ struct sphgpu_handle {
     // small device buffers
     int* layoutOut = nullptr;          // [npad_new, live]
     double* statsPart = nullptr;       // per tile 4
-    double* statsOut = nullptr;        // per scene 4
     // pinned host mirrors
     int* hActive = nullptr;
     int* hIters = nullptr;
@@ -128,6 +127,7 @@ struct sphgpu_handle {
     float* btgt = nullptr;
     int learned = 0;                   // training steps done
     int lastIters[2] = {0, 0};         // iterations of the previous solve (density, divergence)
+    int prevIters[2] = {0, 0};         // and of the one before
     int curIter = -1;                  // iteration being launched (profiling)
     // captured step segments (use_graph)
     std::vector<GraphEntry> graphs;
@@ -280,19 +280,25 @@ int run_ns(sphgpu_handle* h) {
     return 0;
 }
 
-// `odd`: the flags to read are those of an odd iteration (the second buffer
-// of the DFSPH loops)
-int sync_active(sphgpu_handle* h, bool* any, bool odd = false) {
-    Dev& D = h->D;
-    int ns = D.nscenes;
-    // flags, iteration counts and errors: one block, same layout on both sides
-    HIPCHECK(h, hipMemcpyAsync(h->hActive, D.active, 24 * (size_t)ns, hipMemcpyDeviceToHost, h->st));
+// Waits for the loop's queued iterations and reads the flags of iteration
+// parity `odd` (every test writes its results to the pinned copy).
+int sync_active(sphgpu_handle* h, bool* any, bool odd) {
+    const int ns = h->D.nscenes;
     HIPCHECK(h, hipStreamSynchronize(h->st));
+    HIPCHECK(h, hipGetLastError());
     const int* flags = odd ? h->hActive + ns : h->hActive;
     bool a = false;
     for (int s = 0; s < ns; ++s) a = a || flags[s] != 0;
     *any = a;
     return 0;
+}
+
+// largest iteration count of a loop (it ends there whatever its error)
+int loop_cap(const sphgpu_handle* h, int which) {
+    const sphgpu_params& P = h->P;
+    if (P.solver == SPHGPU_DFSPH) return which == 0 ? P.max_iter_density : P.max_iter_div + 1;
+    if (P.solver == SPHGPU_IISPH_DF) return (which == 0 ? P.max_iter_density : P.max_iter_div) + 1;
+    return P.max_iter_density;
 }
 
 // one solver loop; records per-scene iterations/errors into field `which`
@@ -303,79 +309,90 @@ int sync_active(sphgpu_handle* h, bool* any, bool odd = false) {
 // past convergence cost only their launches.  The host reads the flags
 // after a first batch sized from the previous step's count, then after
 // every second iteration.
-void launch_iteration(sphgpu_handle* h, int which, int it) {
-    Dev& D = h->D;
+//
+// Iteration `it` runs under flag buffer it & 1, and the test on its partial
+// sums writes the other buffer: inside the same iteration's second pass
+// (DFSPH, PCISPH), in the next iteration's first pass (IISPH, whose partial
+// sums come from its second; the last iteration of a batch is tested by a
+// kernel of its own), or in a kernel after the iteration (IISPH_DF).  A
+// separate test costs 4.7 us an iteration, 6 % of one at 300,000 particles.
+void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bool lastOfBatch) {
     const sphgpu_params& P = h->P;
     h->curIter = it;
-    {
-        if (P.solver == SPHGPU_DFSPH) {
-            // iteration `it` gates on flag buffer it & 1; the velocity pass
-            // tests convergence on the partials pass A left and writes the
-            // other buffer for the next iteration (a separate reduction
-            // kernel when a scene has no tile to host its test)
-            Dev Dq = D;
-            Dq.active = (it & 1) ? D.active1 : D.active;
-            const bool fused = D.npad / TILE >= D.nscenes;
-            Dq.activeNext = (it & 1) ? D.active : D.active1;
-            if (fused) {
-                Dq.redMode = which == 0 ? 0 : 1;
-                Dq.redTol = which == 0 ? P.density_tol : P.divergence_tol;
-                Dq.redMinIt = which == 0 ? P.min_iter_density : P.min_iter_div;
-                Dq.redCap = which == 0 ? P.max_iter_density : P.max_iter_div + 1;
-            }
-            if (which == 0) {
-                ProfScope ps(h, "df_pass_density", nf_live(h) * 36.0);
-                launch_df_pass_density(Dq, h->st);
-            } else {
-                ProfScope ps(h, "df_pass_divergence", nf_live(h) * 36.0);
-                launch_df_pass_divergence(Dq, P.warm_start != SPHGPU_WARM_NONE && it == 0, h->st);
-            }
-            {
-                ProfScope ps(h, "df_pass_velocity", nf_live(h) * 44.0);
-                launch_df_pass_velocity(Dq, h->st);
-            }
-            if (!fused)
-                launch_scene_reduce(Dq, which == 0 ? 0 : 1, which == 0 ? P.density_tol : P.divergence_tol,
-                                    which == 0 ? P.min_iter_density : P.min_iter_div,
-                                    which == 0 ? P.max_iter_density : P.max_iter_div + 1, h->st);
-        } else if (P.solver == SPHGPU_IISPH_DF) {
-            // IISph.cpp:840-1004 (which 0) and 1062-1207 (which 1): the loops
-            // break when the iteration count exceeds the maximum
-            {
-                ProfScope ps(h, which == 0 ? "idf_kappa_density" : "idf_kappa_divergence", nf_live(h) * 36.0);
-                launch_idf_kappa(D, which == 0 ? 0 : 1, h->st);
-            }
-            {
-                ProfScope ps(h, "idf_velocity", nf_live(h) * 44.0);
-                launch_idf_velocity(D, h->st);
-            }
-            if (which == 0)
-                launch_scene_reduce(D, 1, P.density_tol, P.min_iter_density, P.max_iter_density + 1, h->st);
-            else
-                launch_scene_reduce(D, 1, P.divergence_tol, P.min_iter_div, P.max_iter_div + 1, h->st);
-        } else if (P.solver == SPHGPU_PCISPH) {
-            {
-                ProfScope ps(h, "pci_density", nf_live(h) * 44.0);
-                launch_pci_density(D, h->st);
-            }
-            {
-                ProfScope ps(h, "pci_pressure", nf_live(h) * 64.0);
-                launch_pci_pressure(D, h->st);
-            }
-            launch_scene_reduce(D, 2, P.density_tol, P.min_iter_density,
-                                P.max_iter_density, h->st);
-        } else {  // IISPH
-            {
-                ProfScope ps(h, "ii_sumdij", nf_live(h) * 32.0);
-                launch_ii_sumdij(D, h->st);
-            }
-            {
-                ProfScope ps(h, "ii_pressure", nf_live(h) * 56.0);
-                launch_ii_pressure(D, h->st);
-            }
-            launch_scene_reduce(D, 1, P.density_tol, P.min_iter_density,
-                                P.max_iter_density, h->st);
+    int* const buf[2] = {h->D.active, h->D.active1};
+    Dev D = h->D;
+    D.active = buf[it & 1];
+    D.activeNext = buf[(it + 1) & 1];
+    // the test: mode 0 DFSPH density, 1 mean of the partial sums, 2 PCISPH
+    const bool div = which == 1;
+    const int mode = P.solver == SPHGPU_DFSPH && !div ? 0 : P.solver == SPHGPU_PCISPH ? 2 : 1;
+    const float tol = div ? P.divergence_tol : P.density_tol;
+    const int minIt = div ? P.min_iter_div : P.min_iter_density, cap = loop_cap(h, which);
+    auto with_test = [&](Dev q) {
+        q.redMode = mode;
+        q.redTol = tol;
+        q.redMinIt = minIt;
+        q.redCap = cap;
+        return q;
+    };
+    if (P.solver == SPHGPU_DFSPH) {
+        // (a separate reduction kernel when a scene has no tile to host its test)
+        const bool fused = D.npad / TILE >= D.nscenes;
+        if (!div) {
+            ProfScope ps(h, "df_pass_density", nf_live(h) * 36.0);
+            launch_df_pass_density(D, h->st);
+        } else {
+            ProfScope ps(h, "df_pass_divergence", nf_live(h) * 36.0);
+            launch_df_pass_divergence(D, P.warm_start != SPHGPU_WARM_NONE && it == 0, h->st);
         }
+        {
+            ProfScope ps(h, "df_pass_velocity", nf_live(h) * 44.0);
+            launch_df_pass_velocity(fused ? with_test(D) : D, h->st);
+        }
+        if (!fused) launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
+    } else if (P.solver == SPHGPU_IISPH_DF) {
+        // IISph.cpp:840-1004 (which 0) and 1062-1207 (which 1): the loops
+        // break when the iteration count exceeds the maximum
+        {
+            ProfScope ps(h, !div ? "idf_kappa_density" : "idf_kappa_divergence", nf_live(h) * 36.0);
+            launch_idf_kappa(D, which, h->st);
+        }
+        {
+            ProfScope ps(h, "idf_velocity", nf_live(h) * 44.0);
+            launch_idf_velocity(D, h->st);
+        }
+        launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
+    } else if (P.solver == SPHGPU_PCISPH) {
+        const bool fused = D.npad / TILE >= D.nscenes;
+        {
+            ProfScope ps(h, "pci_density", nf_live(h) * 44.0);
+            launch_pci_density(D, h->st);
+        }
+        {
+            ProfScope ps(h, "pci_pressure", nf_live(h) * 64.0);
+            launch_pci_pressure(fused ? with_test(D) : D, h->st);
+        }
+        if (!fused) launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
+    } else {  // IISPH
+        {
+            // after the first iteration of a batch the pass runs under the
+            // flag of the iteration before, whose test it holds: one pass
+            // too many for a scene that has just converged, whose result
+            // (f4b) nothing reads
+            Dev q = D;
+            if (!firstOfBatch) {
+                q = with_test(D);
+                q.active = buf[(it + 1) & 1];
+                q.activeNext = buf[it & 1];
+            }
+            ProfScope ps(h, "ii_sumdij", nf_live(h) * 32.0);
+            launch_ii_sumdij(q, h->st);
+        }
+        {
+            ProfScope ps(h, "ii_pressure", nf_live(h) * 56.0);
+            launch_ii_pressure(D, h->st);
+        }
+        if (lastOfBatch) launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
     }
 }
 
@@ -384,13 +401,19 @@ void launch_iteration(sphgpu_handle* h, int which, int it) {
 int first_batch(const sphgpu_handle* h, int which) {
     const bool divLoop = which == 1 && (h->P.solver == SPHGPU_DFSPH || h->P.solver == SPHGPU_IISPH_DF);
     const int minIt = divLoop ? h->P.min_iter_div : h->P.min_iter_density;
-    return std::max({1, minIt, h->lastIters[which] - 1});
+    // a count that came up twice running is launched whole: one wait a loop;
+    // otherwise one iteration fewer, since one too many costs its launches
+    const int last = h->lastIters[which];
+    return std::max({1, minIt, last == h->prevIters[which] ? last : last - 1});
+}
+
+void launch_batch(sphgpu_handle* h, int which, int first, int n) {
+    for (int q = 0; q < n; ++q) launch_iteration(h, which, first + q, q == 0, q == n - 1);
 }
 
 void solver_loop_start(sphgpu_handle* h, int which, int batch) {
-    Dev& D = h->D;
-    launch_loop_start(D, h->st);
-    for (int q = 0; q < batch; ++q) launch_iteration(h, which, q);
+    launch_loop_start(h->D, h->st);
+    launch_batch(h, which, 0, batch);
 }
 
 // rest of a solver loop whose first `launched` iterations are queued:
@@ -402,14 +425,17 @@ int solver_loop_finish(sphgpu_handle* h, int which, int launched, size_t profSta
     if (extra) *extra = 0;
     for (;;) {
         bool any = false;
-        // the DFSPH loops keep the flag of iteration k in buffer k & 1
-        int rc = sync_active(h, &any, h->P.solver == SPHGPU_DFSPH && (launched & 1));
+        int rc = sync_active(h, &any, (launched & 1) != 0);
         if (rc) return rc;
         if (!any) break;
-        for (int q = 0; q < 2; ++q) launch_iteration(h, which, launched++);
-        if (extra) *extra += 2;
+        // (an active scene has not reached the cap, so at least one is left)
+        const int n = std::max(1, std::min(2, loop_cap(h, which) - launched));
+        launch_batch(h, which, launched, n);
+        launched += n;
+        if (extra) *extra += n;
     }
     for (int s = 0; s < ns; ++s) maxIt = std::max(maxIt, h->hIters[s]);
+    h->prevIters[which] = h->lastIters[which];
     h->lastIters[which] = maxIt;
     h->curIter = -1;
     // launches past the last iteration of every scene processed nothing
@@ -657,11 +683,7 @@ int finish_step(sphgpu_handle* h, sphgpu_stats* out) {
         ++h->frame;
         return 0;
     }
-    launch_stats(D, h->statsPart, h->statsOut, h->st);
-    HIPCHECK(h, hipMemcpyAsync(h->hStats, h->statsOut, sizeof(double) * 4 * ns, hipMemcpyDeviceToHost, h->st));
-    HIPCHECK(h, hipMemcpyAsync(h->hCounters, D.counters, sizeof(int) * C_COUNT, hipMemcpyDeviceToHost, h->st));
-    HIPCHECK(h, hipMemcpyAsync(h->hLayout, h->layoutOut, sizeof(int) * 2, hipMemcpyDeviceToHost, h->st));
-    HIPCHECK(h, hipMemcpyAsync(h->hDt, D.dt, sizeof(float) * ns, hipMemcpyDeviceToHost, h->st));
+    launch_stats(D, h->statsPart, h->layoutOut, StatsHost{h->hStats, h->hCounters, h->hLayout, h->hDt}, h->st);
     HIPCHECK(h, hipStreamSynchronize(h->st));
     HIPCHECK(h, hipGetLastError());
     // shrink the slot bound to the new padded layout
@@ -698,7 +720,6 @@ int finish_step(sphgpu_handle* h, sphgpu_stats* out) {
     agg.max_iter_hit = h->hCounters[C_COUNT - 1];
     h->nLive = (long long)nsum;
     agg.num_fluid = h->nLive;
-    launch_fill_i32(D.counters, 0, C_COUNT, h->st);
     if (out) *out = agg;
     ++h->frame;
     if (agg.nan_count > 0) return fail(h, SPHGPU_E_DIVERGED, "%d non-finite fluid particles", agg.nan_count);
@@ -935,7 +956,11 @@ int step_iisph(sphgpu_handle* h, sphgpu_stats* st) {
             launch_ii_warm_apply(D, h->ypred, h->feat, h->st);
         }
         solver_loop_start(h, 0, batch);
-        if (graph) launch_ii_force_integrate(h->D, 1, h->st);
+        if (graph) {
+            Dev q = h->D;
+            if (batch & 1) q.active = q.active1;   // the flags after the batch
+            launch_ii_force_integrate(q, 1, h->st);
+        }
     };
     if (h->D.anyDynamic && (rc = rigid_update(h))) return rc;
     if (graph) {
@@ -1611,7 +1636,7 @@ int sphgpu_init(sphgpu_handle* h) {
         D.redTol = 0.0f;
     }
     ALLOC(D.partial, 2 * (size_t)numTiles); ALLOC(D.counters, C_COUNT); ALLOC(D.vmaxPartial, numTiles);
-    ALLOC(h->layoutOut, 2); ALLOC(h->statsPart, 4 * (size_t)numTiles); ALLOC(h->statsOut, 4 * (size_t)ns);
+    ALLOC(h->layoutOut, 2); ALLOC(h->statsPart, 4 * (size_t)numTiles);
     int sortItems = std::max<int>(ncap, int(nb));
     ALLOC(h->sk, sortItems); ALLOC(h->sv, sortItems);
     // Counting search while the grid has no more cells than pay for scanning
@@ -1660,6 +1685,8 @@ int sphgpu_init(sphgpu_handle* h) {
         h->hActive = reinterpret_cast<int*>(c); c += 8 * (size_t)ns;
         h->hIters = reinterpret_cast<int*>(c); c += 8 * (size_t)ns;
         h->hErr = reinterpret_cast<double*>(c); c += 8 * (size_t)ns;
+        D.loopDev = reinterpret_cast<const char*>(D.active);
+        D.loopHost = reinterpret_cast<char*>(h->hActive);
         h->hStats = reinterpret_cast<double*>(c); c += 32 * (size_t)ns;
         h->hCounters = reinterpret_cast<int*>(c); c += 8 * C_COUNT;
         h->hLayout = reinterpret_cast<int*>(c); c += 16;

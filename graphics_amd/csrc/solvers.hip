@@ -429,16 +429,19 @@ __global__ __launch_bounds__(256) void k_cfl_reduce(Dev D, float cfl, float spac
     m = block_max_256(m, lds);
     if (threadIdx.x == 0) {
         float dt = dtMax;
-        if (cfl > 0.0f) {
-            float vmax = sqrtf(m);
-            if (vmax > 0.0f) dt = fminf(dtMax, cfl * spacing / vmax);
-            dt = fmaxf(dt, dtMin);
-        }
-        D.dt[sc] = dt;
+        float vmax = sqrtf(m);
+        if (vmax > 0.0f) dt = fminf(dtMax, cfl * spacing / vmax);
+        D.dt[sc] = fmaxf(dt, dtMin);
     }
 }
 
 // ------------------------------------------------------- scene reduce ----
+// the copy in pinned host memory of a word of the loop-state block
+template <class T>
+__device__ __forceinline__ T* on_host(const Dev& D, const T* p) {
+    return reinterpret_cast<T*>(D.loopHost + (reinterpret_cast<const char*>(p) - D.loopDev));
+}
+
 // mode 0: DFSPH density  err = sum(rho*/rho0)/n - 1          (DFSPH.cpp:696)
 // mode 1: DFSPH divergence / IISPH error   err = sum/n      (DFSPH.cpp:896, IISph_M.cpp:353)
 // mode 2: PCISPH  err = max error/rho0 (second partial)     (PciSph.cpp:344-350)
@@ -451,7 +454,10 @@ __device__ __forceinline__ void scene_reduce_block(const Dev& D, int sc, int mod
                                                    int* out) {
     __shared__ double lds[4];
     if (!D.active[sc]) {   // uniform per block
-        if (threadIdx.x == 0 && out != D.active) out[sc] = 0;
+        if (threadIdx.x == 0 && out != D.active) {
+            out[sc] = 0;
+            *on_host(D, out + sc) = 0;
+        }
         return;
     }
     int t0 = D.scenePadStart[sc] / TILE, t1 = D.scenePadStart[sc + 1] / TILE;
@@ -491,7 +497,17 @@ __device__ __forceinline__ void scene_reduce_block(const Dev& D, int sc, int mod
             D.counters[C_COUNT - 1] = 1;  // max-iteration flag
         }
         out[sc] = cont ? 1 : 0;
+        *on_host(D, out + sc) = cont ? 1 : 0;
+        *on_host(D, D.iters + sc) = it;
+        *on_host(D, D.sceneErr + sc) = err;
     }
+}
+
+// the loop's convergence test in front of a pass (scene b on blocks b, b + gridDim, ...)
+__device__ __forceinline__ void loop_test(const Dev& D) {
+    if (D.redMode >= 0)
+        for (int sc = blockIdx.x; sc < D.nscenes; sc += gridDim.x)
+            scene_reduce_block(D, sc, D.redMode, D.redTol, D.redMinIt, D.redCap, D.activeNext);
 }
 
 __global__ __launch_bounds__(256) void k_scene_reduce(Dev D, int mode, float tol, int minIt, int cap) {
@@ -530,8 +546,11 @@ __global__ __launch_bounds__(256) void k_stats_partial(Dev D, double* part) {
     }
 }
 
-// per scene: [mean(rho/rho0-1), max(rho/rho0-1), kinetic energy, count]
-__global__ __launch_bounds__(256) void k_stats_reduce(Dev D, const double* part, double* out) {
+// per scene: [mean(rho/rho0-1), max(rho/rho0-1), kinetic energy, count], to
+// pinned host memory with what else the host reads at the end of a step (one
+// wait, no transfers: five small copies and a fill took 30 us of a 1,728-
+// particle step)
+__global__ __launch_bounds__(256) void k_stats_reduce(Dev D, const double* part, const int* layout, StatsHost out) {
     __shared__ double lds[4];
     __shared__ float ldf[4];
     int sc = blockIdx.x;
@@ -549,11 +568,17 @@ __global__ __launch_bounds__(256) void k_stats_reduce(Dev D, const double* part,
     sn = block_sum_256(sn, lds);
     mx = block_max_256(mx, ldf);
     if (threadIdx.x == 0) {
-        out[4 * sc] = sn > 0 ? se / sn : 0.0;
-        out[4 * sc + 1] = sn > 0 ? (double)mx : 0.0;
-        out[4 * sc + 2] = sk;
-        out[4 * sc + 3] = sn;
+        out.stats[4 * sc] = sn > 0 ? se / sn : 0.0;
+        out.stats[4 * sc + 1] = sn > 0 ? (double)mx : 0.0;
+        out.stats[4 * sc + 2] = sk;
+        out.stats[4 * sc + 3] = sn;
+        out.dt[sc] = D.dt[sc];
     }
+    if (sc == 0 && threadIdx.x < C_COUNT) {
+        out.counters[threadIdx.x] = D.counters[threadIdx.x];
+        D.counters[threadIdx.x] = 0;
+    }
+    if (sc == 0 && threadIdx.x < 2) out.layout[threadIdx.x] = layout[threadIdx.x];
 }
 
 // ------------------------------------------------------ shared passes ----
@@ -1112,11 +1137,7 @@ __device__ __forceinline__ void velocity_particle(const Dev& D, const Slot& s, c
 
 template <bool WIN>
 __global__ __launch_bounds__(256, WIN ? 2 : 1) void k_df_pass_velocity(Dev D) {
-    // the loop's convergence test on pass A's partial sums (scene b on
-    // blocks b, b + gridDim, ...)
-    if (D.redMode >= 0)
-        for (int sc = blockIdx.x; sc < D.nscenes; sc += gridDim.x)
-            scene_reduce_block(D, sc, D.redMode, D.redTol, D.redMinIt, D.redCap, D.activeNext);
+    loop_test(D);   // on pass A's partial sums
     if constexpr (WIN) {
         __shared__ float4 s_wxk[WIN_MAX];   // window records: xk of each neighbour
         window_pair<WIN_VELOCITY, false>(
@@ -1372,6 +1393,7 @@ __device__ __forceinline__ void sumdij_particle(const Dev& D, const Slot& s, con
 
 template <bool WIN>
 __global__ __launch_bounds__(256, WIN ? 2 : 1) void k_ii_sumdij(Dev D) {
+    loop_test(D);   // of the iteration before, on its pressure pass's partial sums
     if constexpr (WIN) {
         __shared__ float4 s_wxk[WIN_MAX];   // window records: xk of each neighbour
         window_pair<WIN_SUMDIJ, false>(
@@ -1680,6 +1702,7 @@ __global__ __launch_bounds__(256) void k_pci_density(Dev D) {
 // 2 p_a/rho_a^2 when p_a > 0.  Then the next prediction x* = x + (v + (a +
 // a_p) dt) dt.
 __global__ __launch_bounds__(256) void k_pci_pressure(Dev D) {
+    loop_test(D);   // on the density pass's partial sums
     Slot s = slot_nb(D, true);
     if (!s.live) return;
     const int i = s.i;
@@ -1781,6 +1804,7 @@ void launch_copy_probe(const float4* a, float4* b, size_t n, hipStream_t st) {
 void launch_copy_f4(float4* dst, const float4* src, size_t n, hipStream_t st) { launch_copy_probe(src, dst, n, st); }
 
 void launch_cfl(const Dev& D, float cfl, float spacing, float dtMax, float dtMin, hipStream_t st) {
+    if (!(cfl > 0.0f)) return;   // a fixed step: D.dt holds dtMax from the start
     if (tiles_of(D) > 0) hipLaunchKernelGGL(k_cfl_partial, dim3(tiles_of(D)), dim3(256), 0, st, D);
     hipLaunchKernelGGL(k_cfl_reduce, dim3(D.nscenes), dim3(256), 0, st, D, cfl, spacing, dtMax, dtMin);
 }
@@ -1790,9 +1814,9 @@ void launch_loop_start(const Dev& D, hipStream_t st) {
 void launch_scene_reduce(const Dev& D, int mode, float tol, int minIt, int cap, hipStream_t st) {
     hipLaunchKernelGGL(k_scene_reduce, dim3(D.nscenes), dim3(256), 0, st, D, mode, tol, minIt, cap);
 }
-void launch_stats(const Dev& D, double* part, double* out, hipStream_t st) {
+void launch_stats(const Dev& D, double* part, const int* layout, const StatsHost& out, hipStream_t st) {
     if (tiles_of(D) > 0) hipLaunchKernelGGL(k_stats_partial, dim3(tiles_of(D)), dim3(256), 0, st, D, part);
-    hipLaunchKernelGGL(k_stats_reduce, dim3(D.nscenes), dim3(256), 0, st, D, (const double*)part, out);
+    hipLaunchKernelGGL(k_stats_reduce, dim3(D.nscenes), dim3(256), 0, st, D, (const double*)part, layout, out);
 }
 void launch_fill_i32(int* p, int v, int n, hipStream_t st) {
     if (n > 0) hipLaunchKernelGGL(k_fill_i32, dim3((n + 255) / 256), dim3(256), 0, st, p, v, n);

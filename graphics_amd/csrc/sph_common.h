@@ -194,19 +194,25 @@ struct Dev {
     // ---- per-scene solver scalars
     float* dt;           // per scene
     int* active;         // per scene: 1 while its solver loop runs
-    int* active1;        // the DFSPH loops' second flag buffer (odd iterations)
+    int* active1;        // the loops' second flag buffer (odd iterations)
     int* iters;          // per scene: iterations of the current loop
     int* integ;          // per scene: 1 once a captured IISPH step integrated it
     double* sceneErr;    // per scene
     double* partial;     // per tile partial sums (2 per tile)
-    // The DFSPH loops run their convergence test inside the velocity pass
-    // (pass B): its first nscenes blocks reduce the partial sums pass A left
-    // and write the flag of the next iteration to activeNext, while every
-    // block gates on `active`, the flag pass A ran under (the launcher swaps
-    // the two buffers by iteration parity).  redMode < 0: no test.
+    // The loops run their convergence test inside a pass that follows the one
+    // that leaves the partial sums: the DFSPH velocity pass, the PCISPH
+    // pressure pass, the IISPH sum d_ij p_j pass of the next iteration.  Its
+    // first nscenes blocks reduce the sums and write the next flag to
+    // activeNext, while every block gates on `active`, the flag the sums were
+    // formed under (the launcher swaps the two buffers).  redMode < 0: no test.
     int* activeNext;
     int redMode, redMinIt, redCap;
     float redTol;
+    // the flags, counts and errors above lie in one device block from loopDev
+    // on; every test also writes them to its copy in pinned host memory, so
+    // that the host reads them after a wait, without a transfer
+    const char* loopDev;
+    char* loopHost;
     int* counters;       // Counter
     float* vmaxPartial;  // per tile
 };
@@ -535,7 +541,15 @@ void launch_pci_integrate(const Dev& D, hipStream_t st);
 void launch_scene_reduce(const Dev& D, int mode, float tol, int minIt, int cap, hipStream_t st);
 // start of a solver loop: every scene active, iteration counts zero
 void launch_loop_start(const Dev& D, hipStream_t st);
-void launch_stats(const Dev& D, double* part, double* out, hipStream_t st);
+// per-scene statistics, the counters (then cleared), the layout and the time
+// steps, written to pinned host memory
+struct StatsHost {
+    double* stats;     // [4 * nscenes]
+    int* counters;     // [C_COUNT]
+    int* layout;       // [2]
+    float* dt;         // [nscenes]
+};
+void launch_stats(const Dev& D, double* part, const int* layout, const StatsHost& out, hipStream_t st);
 void launch_fill_i32(int* p, int v, int n, hipStream_t st);
 void launch_copy_probe(const float4* a, float4* b, size_t n, hipStream_t st);
 // dst[i] = src[i] with a kernel (graph-capturable, no copy engine)
