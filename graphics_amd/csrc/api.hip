@@ -312,10 +312,10 @@ int loop_cap(const sphgpu_handle* h, int which) {
 //
 // Iteration `it` runs under flag buffer it & 1, and the test on its partial
 // sums writes the other buffer: inside the same iteration's second pass
-// (DFSPH, PCISPH), in the next iteration's first pass (IISPH, whose partial
-// sums come from its second; the last iteration of a batch is tested by a
-// kernel of its own), or in a kernel after the iteration (IISPH_DF).  A
-// separate test costs 4.7 us an iteration, 6 % of one at 300,000 particles.
+// (DFSPH, PCISPH, IISPH_DF) or in the next iteration's first pass (IISPH,
+// whose partial sums come from its second; the last iteration of a batch is
+// tested by a kernel of its own).  A separate test costs 4.7 us an
+// iteration, 6 % of one at 300,000 particles.
 void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bool lastOfBatch) {
     const sphgpu_params& P = h->P;
     h->curIter = it;
@@ -357,11 +357,12 @@ void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bo
             ProfScope ps(h, !div ? "idf_kappa_density" : "idf_kappa_divergence", nf_live(h) * 36.0);
             launch_idf_kappa(D, which, h->st);
         }
+        const bool fused = D.npad / TILE >= D.nscenes;
         {
             ProfScope ps(h, "idf_velocity", nf_live(h) * 44.0);
-            launch_idf_velocity(D, h->st);
+            launch_idf_velocity(fused ? with_test(D) : D, h->st);
         }
-        launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
+        if (!fused) launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
     } else if (P.solver == SPHGPU_PCISPH) {
         const bool fused = D.npad / TILE >= D.nscenes;
         {
@@ -1659,6 +1660,7 @@ int sphgpu_init(sphgpu_handle* h) {
     if (P.solver == SPHGPU_IISPH_DF) {
         ALLOC(D.pm, ncap);
         ALLOC(D.brho, nb + 1); ALLOC(D.balpha, nb + 1); ALLOC(D.bk, nb + 1);
+        ALLOC(D.bnF, (size_t)BNF_CAP * nb); ALLOC(D.bnB, (size_t)BNB_CAP * nb); ALLOC(D.bnCnt, nb);
         HIPCHECK(h, hipMemset(D.bk, 0, sizeof(float) * (nb + 1)));   // the list-padding dummy stays 0
         HIPCHECK(h, hipMemset(D.pm, 0, sizeof(float) * ncap));
     }

@@ -16,76 +16,23 @@
 //   - the divergence-free solve runs first, at the same positions, then the
 //     constant-density solve, then updateFluids (the order of the commented
 //     calls at IISph.cpp:59-60).
-// Boundary particles find their neighbours by scanning the 27 cells around
-// them (fluid through cellF, boundary through cellB, the reference's
-// predicate, no pair with a particle of the same solid: every solid is
-// rigid); fluid particles use their neighbour lists.
-#include "sph_common.h"
+// Boundary particles find their neighbours once a step by scanning the 27
+// cells around them (fluid through cellF, boundary through cellB, the
+// reference's predicate, no pair with a particle of the same solid: every
+// solid is rigid) and keep them in lists of their own; fluid particles use
+// their neighbour lists.
+//
+// Bound: the latency of the neighbours' loads.  The lists are read in batches
+// of gathers (each_fluid_lu, each_boundary_lu), one launch takes the fluid
+// tiles and the boundary particles of a stiffness pass, and the convergence
+// test runs in the velocity pass.  An iteration on 87,075 fluid and 33,312
+// wall particles takes 33 us (114 us with one load at a time and every wall
+// particle scanning its cells in every iteration).
+#include "passes.h"
 
 namespace sphgpu {
 
 namespace {
-
-__shared__ int g_idftab[NB16_TAB];
-
-struct SlotI {
-    int i, tile, scene;
-    bool live, packed;
-};
-
-__device__ __forceinline__ SlotI slot_idf(const Dev& D, bool gated) {
-    SlotI s;
-    s.tile = tile_of_block(D.tileMap);
-    s.i = s.tile * TILE + threadIdx.x;
-    s.scene = D.tileScene[s.tile];
-    s.live = (int)threadIdx.x < D.tileValid[s.tile];
-    if (gated) s.live = s.live && D.active[s.scene] != 0;
-    if (threadIdx.x < NB16_TAB) g_idftab[threadIdx.x] = D.nbTab[(size_t)s.tile * NB16_TAB + threadIdx.x];
-    __syncthreads();
-    s.packed = __builtin_amdgcn_readfirstlane(g_idftab[NB16_FLAG]) != 0;
-    return s;
-}
-
-__device__ __forceinline__ int nf_cnt(int c) { return c & 0xff; }
-__device__ __forceinline__ int nb_cnt(int c) { return (c >> 16) & 0xff; }
-
-// every listed fluid neighbour j of slot s (padding entries, the particle
-// itself, included: they contribute nothing to gradient sums and are skipped
-// by index in density sums)
-template <class F>
-__device__ __forceinline__ void fluid_list(const Dev& D, const SlotI& s, int n, F&& f) {
-    if (s.packed) {
-        const int4* col = D.nbF16 + s.i;
-        const int n4 = (n + 3) & ~3;
-        for (int k = 0; k < n4; ++k) {
-            const int4 g = col[(size_t)(k >> 3) * D.ncap];
-            const int w = (k & 7) >> 1;
-            const unsigned word = (unsigned)(w == 0 ? g.x : w == 1 ? g.y : w == 2 ? g.z : g.w);
-            const unsigned e = (word >> (16 * (k & 1))) & 0xffffu;
-            f(g_idftab[e >> NB16_OFF_BITS] + (int)e);
-        }
-    } else {
-        const int* col = D.nbF;
-        const int n4 = (n + 3) & ~3;
-        for (int k = 0; k < n4; ++k) f(col[nb_slot(k, s.i, D.ncap)]);
-    }
-}
-
-template <class F>
-__device__ __forceinline__ void boundary_list(const Dev& D, const SlotI& s, int n, F&& f) {
-    if (s.packed) {
-        const int4* col = D.nbB16 + s.i;
-        for (int k = 0; k < n; ++k) {
-            const int4 g = col[(size_t)(k >> 3) * D.ncap];
-            const int w = (k & 7) >> 1;
-            const unsigned word = (unsigned)(w == 0 ? g.x : w == 1 ? g.y : w == 2 ? g.z : g.w);
-            const unsigned e = (word >> (16 * (k & 1))) & 0xffffu;
-            f(g_idftab[32 + (e >> NB16_OFF_BITS)] + (int)e);
-        }
-    } else {
-        for (int k = 0; k < n; ++k) f(D.nbB[nb_slot(k, s.i, D.ncap)]);
-    }
-}
 
 __device__ __forceinline__ float rest_of(const Dev& D, int i, int ph) { return D.rho0[ph] * D.ksum[i]; }
 
@@ -103,6 +50,12 @@ __device__ __forceinline__ Pair pair_of(const Dev& D, float4 a, float4 b) {
     return p;
 }
 
+// a gather record and one scalar of the same neighbour (mass, stiffness)
+struct RecM {
+    float4 x;
+    float m;
+};
+
 // ---------------------------------------------------------------- masses ----
 // m = rho0 beta v0 of every live slot (IISph.cpp:110-115)
 __global__ __launch_bounds__(256) void k_idf_mass(Dev D) {
@@ -116,33 +69,35 @@ __global__ __launch_bounds__(256) void k_idf_mass(Dev D) {
 // fluid density and alpha (IISph.cpp:143-200); publishes rho in v.w for the
 // non-pressure acceleration pass
 __global__ __launch_bounds__(256) void k_idf_prepare_fluid(Dev D) {
-    const SlotI s = slot_idf(D, false);
+    const Slot s = slot_nb(D, false);
     if (!s.live) return;
     const int i = s.i;
     const float4 pa = D.x[i];
-    const int ph = (int)pa.w;
+    const int ph = phase_of(pa);
     const float ma = D.pm[i], resta = rest_of(D, i, ph);
     const int c = D.cnt[i];
     Kahan rho;
     rho.init(ma * D.W0);
     float a1x = 0.f, a1y = 0.f, a1z = 0.f, a2 = 0.f;
-    fluid_list(D, s, nf_cnt(c), [&](int j) {
+    // (padding entries, the particle itself and the far dummy, are skipped:
+    // adding a zero would change a compensated sum)
+    each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return RecM{D.x[j], D.pm[j]}; }, [&](int j, RecM rec) {
         if (j == i) return;
-        const Pair p = pair_of(D, pa, D.x[j]);
-        const float mb = D.pm[j];
+        const Pair p = pair_of(D, pa, rec.x);
+        const float mb = rec.m;
         rho.add((D.adjustDensity ? ma : mb) * kernel_W(p.r, D));     // IISph.cpp:163-164
         const float gm = p.g * mb;
         a1x += p.dx * gm; a1y += p.dy * gm; a1z += p.dz * gm;
         const float gs = gm * p.r;                                   // |dW/dr| m_b
         a2 += gs * gs;
     });
-    boundary_list(D, s, nb_cnt(c), [&](int j) {
-        const float4 pb = D.xb[j];
+    each_boundary_lu<8>(D, s, nb_of(c), [&](int j) { return D.xb[j]; }, [&](int j, float4 pb) {
+        if (j == D.nb) return;
         const Pair p = pair_of(D, pa, pb);
         rho.add(resta * pb.w * kernel_W(p.r, D));                     // IISph.cpp:187
         const float gm = p.g * D.boundaryDensity * pb.w;             // IISph.cpp:192
         a1x += p.dx * gm; a1y += p.dy * gm; a1z += p.dz * gm;
-        if (D.anyDynamic && j < D.nb && D.solids[D.bsolid[j]].dynamic) {   // IISph.cpp:193-195
+        if (D.anyDynamic && D.solids[D.bsolid[j]].dynamic) {          // IISph.cpp:193-195
             const float gs = gm * p.r;
             a2 += gs * gs;
         }
@@ -156,7 +111,8 @@ __global__ __launch_bounds__(256) void k_idf_prepare_fluid(Dev D) {
 }
 
 // every fluid and boundary neighbour of boundary particle b, from the 27
-// cells around it: fluid(j, pair), boundary(j, pair, V_j)
+// cells around it: fluid(j, pair), boundary(j, pair, V_j).  Candidates come
+// four at a time (up to X_TAIL records past a run are read, and not used).
 template <class FF, class FB>
 __device__ __forceinline__ void boundary_stencil(const Dev& D, int b, float4 pa, FF&& fluid, FB&& bound) {
     const SceneGrid G = D.grids[D.bscene[b]];
@@ -171,10 +127,15 @@ __device__ __forceinline__ void boundary_stencil(const Dev& D, int b, float4 pa,
             if (y < 0 || y >= G.ny) continue;
             const uint32_t k0 = key_of(G, D.rowRank, cx, y, z);
             const int2 rf = run3(D.cellF, k0, cx, G.nx, D.cellRuns);
-            for (int j = rf.x; j < rf.y; ++j) {
-                const float4 pb = D.x[j];
-                if (dis_square_exact(pa, pb) < D.h2) fluid(j, pair_of(D, pa, pb));
+            for (int j0 = rf.x; j0 < rf.y; j0 += 4) {
+                float4 q[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) q[k] = D.x[j0 + k];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (j0 + k < rf.y && dis_square_exact(pa, q[k]) < D.h2) fluid(j0 + k, pair_of(D, pa, q[k]));
             }
+            if (D.nsolids < 2) continue;          // its own solid's particles only
             const int2 rb = run3(D.cellB, k0, cx, G.nx, D.cellRuns);
             for (int j = rb.x; j < rb.y; ++j) {
                 if (j == b || D.bsolid[j] == sa) continue;
@@ -185,8 +146,39 @@ __device__ __forceinline__ void boundary_stencil(const Dev& D, int b, float4 pa,
     }
 }
 
+// the same neighbours in the same order from the lists k_idf_prepare_boundary
+// keeps: fluid(j, pair, v*_j), boundary(j, pair, V_j, v_j)
+template <class FF, class FB>
+__device__ __forceinline__ void boundary_neighbours(const Dev& D, int b, float4 pa, FF&& fluid, FB&& bound) {
+    const int c = D.bnCnt[b];
+    if (c < 0) {
+        boundary_stencil(D, b, pa, [&](int j, const Pair& p) { fluid(j, p, D.vs[j]); },
+                         [&](int j, const Pair& p, float vol) { bound(j, p, vol, D.vb[j]); });
+        return;
+    }
+    const int nf = c & 0xff, nb = c >> 8;
+    const int4* lf = reinterpret_cast<const int4*>(D.bnF) + b;
+    for (int g = 0; 4 * g < nf; ++g) {
+        const int4 e = lf[(size_t)g * D.nb];
+        // entries past the count are left from earlier steps: the first stands in
+        const int j[4] = {e.x, 4 * g + 1 < nf ? e.y : e.x, 4 * g + 2 < nf ? e.z : e.x, 4 * g + 3 < nf ? e.w : e.x};
+        Rec2 r[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) r[k] = Rec2{D.x[j[k]], D.vs[j[k]]};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (4 * g + k < nf) fluid(j[k], pair_of(D, pa, r[k].a), r[k].b);
+    }
+    for (int k = 0; k < nb; ++k) {
+        const int j = D.bnB[nb_slot(k, b, D.nb)];
+        const float4 pb = D.xb[j];
+        bound(j, pair_of(D, pa, pb), pb.w, D.vb[j]);
+    }
+}
+
 // boundary density and alpha (IISph.cpp:234-287); the mass of a boundary
-// particle is boundaryDensity V_b (IISph.cpp:130)
+// particle is boundaryDensity V_b (IISph.cpp:130).  Also keeps its neighbours
+// in lists for the passes of the step's loops.
 __global__ __launch_bounds__(256) void k_idf_prepare_boundary(Dev D) {
     const int b = blockIdx.x * 256 + threadIdx.x;
     if (b >= D.nb) return;
@@ -195,14 +187,22 @@ __global__ __launch_bounds__(256) void k_idf_prepare_boundary(Dev D) {
     Kahan rho;
     rho.init(ma * D.W0);
     float a2 = 0.0f;
+    int nf = 0, nb = 0;
     boundary_stencil(D, b, pa,
         [&](int j, const Pair& p) {
+            if (nf < BNF_CAP) D.bnF[nb_slot(nf, b, D.nb)] = j;
+            ++nf;
             const float mf = D.pm[j];
             rho.add((D.adjustDensity ? ma : mf) * kernel_W(p.r, D));
             const float gs = p.g * p.r * mf;
             a2 += gs * gs;
         },
-        [&](int, const Pair& p, float vol) { rho.add(D.boundaryDensity * vol * kernel_W(p.r, D)); });
+        [&](int j, const Pair& p, float vol) {
+            if (nb < BNB_CAP) D.bnB[nb_slot(nb, b, D.nb)] = j;
+            ++nb;
+            rho.add(D.boundaryDensity * vol * kernel_W(p.r, D));
+        });
+    D.bnCnt[b] = nf <= BNF_CAP && nb <= BNB_CAP ? nf | nb << 8 : -1;
     const float density = rho.s;
     D.brho[b] = density;
     D.balpha[b] = density / (a2 < 1.0e-6f ? 1.0e-6f : a2);
@@ -229,8 +229,7 @@ __global__ __launch_bounds__(256) void k_idf_vadv(Dev D, int mode) {
 
 // boundary particles' own stiffness, kappa/rho into bk:
 // mode 0 density (IISph.cpp:849-904), mode 1 divergence (1069-1115)
-__global__ __launch_bounds__(256) void k_idf_kappa_boundary(Dev D, int mode) {
-    const int b = blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void kappa_boundary(const Dev& D, int b, int mode) {
     if (b >= D.nb) return;
     const int sc = D.bscene[b];
     if (!D.active[sc]) return;
@@ -238,13 +237,11 @@ __global__ __launch_bounds__(256) void k_idf_kappa_boundary(Dev D, int mode) {
     const float ma = D.boundaryDensity * pa.w, rest = D.boundaryDensity;
     const bool adjust = mode == 0 && D.adjustDensity;
     float sf = 0.0f, sb = 0.0f;
-    boundary_stencil(D, b, pa,
-        [&](int j, const Pair& p) {
-            const float4 u = D.vs[j];
+    boundary_neighbours(D, b, pa,
+        [&](int j, const Pair& p, float4 u) {
             sf += (adjust ? ma : u.w) * p.g * dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz);
         },
-        [&](int j, const Pair& p, float vol) {
-            const float4 u = D.vb[j];
+        [&](int j, const Pair& p, float vol, float4 u) {
             sb += vol * p.g * dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz);
         });
     const float dt = D.dt[sc], rho = D.brho[b];
@@ -263,26 +260,36 @@ __global__ __launch_bounds__(256) void k_idf_kappa_boundary(Dev D, int mode) {
 
 // fluid stiffness (mode 0 density, IISph.cpp:910-965; mode 1 divergence,
 // 1120-1165) -> xk = (x, kappa/rho); partial sums of the loop's error:
-// (rho_adv - rest)/rest (IISph.cpp:956-957), or Drho/Dt dt (1204-1207)
-__global__ __launch_bounds__(256) void k_idf_kappa_fluid(Dev D, int mode) {
+// (rho_adv - rest)/rest (IISph.cpp:956-957), or Drho/Dt dt (1204-1207).
+// Blocks past the tiles take the boundary particles (neither reads what the
+// other writes).
+__global__ __launch_bounds__(256) void k_idf_kappa(Dev D, int mode, int tiles) {
+    if ((int)blockIdx.x >= tiles) {
+        kappa_boundary(D, ((int)blockIdx.x - tiles) * 256 + threadIdx.x, mode);
+        return;
+    }
     __shared__ double lds[4];
-    const SlotI s = slot_idf(D, true);
+    const Slot s = slot_nb(D, true, tiles);
+    if (!D.active[s.scene]) {   // uniform: a converged scene's tiles contribute nothing
+        if (threadIdx.x == 0) D.partial[2 * s.tile] = 0.0;
+        return;
+    }
     double contrib = 0.0;
     if (s.live) {
         const int i = s.i;
         const float4 pa = D.x[i], va = D.vs[i];
-        const int ph = (int)pa.w;
+        const int ph = phase_of(pa);
         const float ma = va.w, rest = rest_of(D, i, ph);
         const int c = D.cnt[i];
         const bool adjust = mode == 0 && D.adjustDensity;
         float sf = 0.0f, sb = 0.0f;
-        fluid_list(D, s, nf_cnt(c), [&](int j) {
-            const float4 u = D.vs[j];
-            const Pair p = pair_of(D, pa, D.x[j]);
+        each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.vs[j]}; }, [&](int, Rec2 rec) {
+            const float4 u = rec.b;
+            const Pair p = pair_of(D, pa, rec.a);
             sf += (adjust ? ma : u.w) * p.g * dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz);
         });
-        boundary_list(D, s, nb_cnt(c), [&](int j) {
-            const float4 pb = D.xb[j], u = D.vb[j];
+        each_boundary_lu<4>(D, s, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; }, [&](int, Rec2 rec) {
+            const float4 pb = rec.a, u = rec.b;
             const Pair p = pair_of(D, pa, pb);
             sb += pb.w * p.g * dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz);
         });
@@ -301,31 +308,29 @@ __global__ __launch_bounds__(256) void k_idf_kappa_fluid(Dev D, int mode) {
         }
         D.xk[i] = make_float4(pa.x, pa.y, pa.z, kr);
     }
-    const double t = block_sum_256(contrib, lds);
-    if (threadIdx.x == 0) D.partial[2 * s.tile] = t;
+    write_partial(D, s.tile, 0, contrib, lds);
 }
 
 // velocity pass of both loops (IISph.cpp:966-1001, 1166-1206):
 // v_adv -= dt (sum_f m_b (k_a/rho_a + k_b/rho_b) gradW
 //              + sum_b boundaryDensity V_b (k_a/rho_a + k_b/rho_b) gradW)
 __global__ __launch_bounds__(256) void k_idf_velocity(Dev D) {
-    const SlotI s = slot_idf(D, true);
+    loop_test(D);   // on the stiffness pass's partial sums
+    const Slot s = slot_nb(D, true);
     if (!s.live) return;
     const int i = s.i;
     const float4 pa = D.xk[i];
     const float ka = pa.w;
     const int c = D.cnt[i];
     float fx = 0.f, fy = 0.f, fz = 0.f, bx = 0.f, by = 0.f, bz = 0.f;
-    fluid_list(D, s, nf_cnt(c), [&](int j) {
-        const float4 pb = D.xk[j];
-        const Pair p = pair_of(D, pa, pb);
-        const float w = p.g * D.pm[j] * (ka + pb.w);
+    each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return RecM{D.xk[j], D.pm[j]}; }, [&](int, RecM rec) {
+        const Pair p = pair_of(D, pa, rec.x);
+        const float w = p.g * rec.m * (ka + rec.x.w);
         fx += p.dx * w; fy += p.dy * w; fz += p.dz * w;
     });
-    boundary_list(D, s, nb_cnt(c), [&](int j) {
-        const float4 pb = D.xb[j];
-        const Pair p = pair_of(D, pa, pb);
-        const float w = p.g * pb.w * (ka + D.bk[j]);
+    each_boundary_lu<4>(D, s, nb_of(c), [&](int j) { return RecM{D.xb[j], D.bk[j]}; }, [&](int, RecM rec) {
+        const Pair p = pair_of(D, pa, rec.x);
+        const float w = p.g * rec.x.w * (ka + rec.m);
         bx += p.dx * w; by += p.dy * w; bz += p.dz * w;
     });
     const float dt = D.dt[s.scene], cb = dt * D.boundaryDensity;
@@ -355,8 +360,8 @@ void launch_idf_vadv(const Dev& D, int mode, hipStream_t st) {
 }
 
 void launch_idf_kappa(const Dev& D, int mode, hipStream_t st) {
-    if (D.nb > 0) hipLaunchKernelGGL(k_idf_kappa_boundary, dim3(bblocks(D)), dim3(256), 0, st, D, mode);
-    if (tiles_of(D) > 0) hipLaunchKernelGGL(k_idf_kappa_fluid, dim3(tiles_of(D)), dim3(256), 0, st, D, mode);
+    const int t = tiles_of(D), g = t + bblocks(D);
+    if (g > 0) hipLaunchKernelGGL(k_idf_kappa, dim3(g), dim3(256), 0, st, D, mode, t);
 }
 
 void launch_idf_velocity(const Dev& D, hipStream_t st) {

@@ -6,166 +6,11 @@
 // each neighbour costs one or two gathers.  Sums that decide convergence are
 // reduced in FP64: a fixed-order block tree per tile (deterministic), then a
 // fixed-order per-scene reduction.
-#include "sph_common.h"
+#include "passes.h"
 
 namespace sphgpu {
 
 namespace {
-
-struct Slot {
-    int i, tile, scene;
-    bool live;
-    bool packed;   // the tile's neighbour lists are in the packed 16-bit form
-};
-
-__device__ __forceinline__ Slot slot_of(const Dev& D, bool gated) {
-    Slot s;
-    s.tile = tile_of_block(D.tileMap);
-    s.i = s.tile * TILE + threadIdx.x;
-    s.scene = D.tileScene[s.tile];
-    s.live = (int)threadIdx.x < D.tileValid[s.tile];
-    if (gated) s.live = s.live && D.active[s.scene] != 0;
-    s.packed = false;
-    return s;
-}
-
-// The tile's list table (fluid slots 0..31, boundary 32..63) and the window
-// offset of each fluid slot ([31]: the window size), staged in LDS by the
-// kernels that read neighbour lists.
-__shared__ int g_nbtab[NB16_TAB];
-__shared__ int g_winoff[32];
-
-// slot_of for kernels that read neighbour lists: every thread of the block
-// calls it before any returns (it stages the tile's tables in LDS, both with
-// one round trip).  A gated block whose scene has converged loads nothing
-// (its particles are not live): solver iterations launched past convergence
-// return at once.
-__device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated) {
-    Slot s = slot_of(D, gated);
-    if (gated && !D.active[s.scene]) return s;   // uniform per block
-    if (threadIdx.x < NB16_TAB) g_nbtab[threadIdx.x] = D.nbTab[(size_t)s.tile * NB16_TAB + threadIdx.x];
-    else if (threadIdx.x < NB16_TAB + 32)
-        g_winoff[threadIdx.x - NB16_TAB] = D.nbWin[(size_t)s.tile * 32 + threadIdx.x - NB16_TAB];
-    __syncthreads();
-    s.packed = __builtin_amdgcn_readfirstlane(g_nbtab[NB16_FLAG]) != 0;
-    return s;
-}
-
-// A list group is read once per pass.  Where the lists and records together
-// fit the last-level cache the plain load lets the next pass find the list
-// there; on larger scenes a streaming load keeps the list from pushing the
-// gathered records out (Dev::listNT, chosen by the autotuner).
-typedef int v4i_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ int4 ld_group(const int4* p, bool nt) {
-    if (nt) {
-        const v4i_t v = __builtin_nontemporal_load(reinterpret_cast<const v4i_t*>(p));
-        return make_int4(v.x, v.y, v.z, v.w);
-    }
-    return *p;
-}
-
-// Neighbour loops in split form: load(j) issues the gather(s) of neighbour j
-// and returns the record(s), use(j, r) consumes them.  A batch of neighbours is gathered first, then the next list group is
-// requested, then the batch is used: a wave waits for its memory returns in
-// issue order, so a list load issued ahead of the gathers would hold up every
-// batch.  W = 8: one batch of eight per packed group (single-record passes);
-// W = 4: two batches of four (two-record passes: eight gathers in flight
-// either way).  Entries past the padded count still gather (from the padding
-// index) but are not used, so every pass sums exactly the listed entries.
-template <int W, int TOFF, class LD, class US>
-__device__ __forceinline__ void each_in_list16_lu(const int4* __restrict__ list, int ncap, int i, int n, int padj,
-                                                  bool nt, LD&& load, US&& use) {
-    static_assert(W == 4 || W == 8, "batch of four or eight");
-    const int4* __restrict__ col = list + i;
-    const int ng = (n + 7) >> 3;
-    if (ng <= 0) return;
-    const int n4 = (n + 3) & ~3;
-    int4 cur = ld_group(&col[0], nt);
-    for (int g = 0; g < ng; ++g) {
-        const unsigned w[4] = {(unsigned)cur.x, (unsigned)cur.y, (unsigned)cur.z, (unsigned)cur.w};
-        const bool second = 8 * g + 4 < n4;   // entries 8g+4..8g+7 are listed
-        int j[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const unsigned e = (w[k >> 1] >> (16 * (k & 1))) & 0xffffu;
-            const int jj = g_nbtab[TOFF + (e >> NB16_OFF_BITS)] + (int)e;
-            j[k] = (k < 4 || second) ? jj : padj;
-        }
-        int4 nxt = cur;
-        if (W == 8) {
-            decltype(load(0)) r[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) r[k] = load(j[k]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (g + 1 < ng) nxt = ld_group(&col[(size_t)(g + 1) * ncap], nt);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) use(j[k], r[k]);
-            if (second) {
-#pragma unroll
-                for (int k = 4; k < 8; ++k) use(j[k], r[k]);
-            }
-        } else {
-            decltype(load(0)) r[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) r[k] = load(j[k]);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) use(j[k], r[k]);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) r[k] = load(j[4 + k]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (g + 1 < ng) nxt = ld_group(&col[(size_t)(g + 1) * ncap], nt);
-            __builtin_amdgcn_sched_barrier(0);
-            if (second) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) use(j[4 + k], r[k]);
-            }
-        }
-        cur = nxt;
-    }
-}
-
-// the same for 32-bit lists (groups of four, all listed or padding)
-template <class LD, class US>
-__device__ __forceinline__ void each_in_list_lu(const int* __restrict__ list, int ncap, int i, int n, bool nt,
-                                                LD&& load, US&& use) {
-    const int4* __restrict__ col = reinterpret_cast<const int4*>(list) + i;
-    const int ng = (n + 3) >> 2;
-    if (ng <= 0) return;
-    int4 cur = ld_group(&col[0], nt);
-    for (int g = 0; g < ng; ++g) {
-        const int j[4] = {cur.x, cur.y, cur.z, cur.w};
-        decltype(load(0)) r[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) r[k] = load(j[k]);
-        int4 nxt = cur;
-        __builtin_amdgcn_sched_barrier(0);
-        if (g + 1 < ng) nxt = ld_group(&col[(size_t)(g + 1) * ncap], nt);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) use(j[k], r[k]);
-        cur = nxt;
-    }
-}
-
-template <int W, class LD, class US>
-__device__ __forceinline__ void each_fluid_lu(const Dev& D, const Slot& s, int nf, LD&& load, US&& use) {
-    const bool nt = __builtin_amdgcn_readfirstlane(D.listNT) != 0;
-    if (s.packed) each_in_list16_lu<W, 0>(D.nbF16, D.ncap, s.i, nf, s.i, nt, load, use);
-    else each_in_list_lu(D.nbF, D.ncap, s.i, nf, nt, load, use);
-}
-
-template <int W, class LD, class US>
-__device__ __forceinline__ void each_boundary_lu(const Dev& D, const Slot& s, int nb, LD&& load, US&& use) {
-    const bool nt = __builtin_amdgcn_readfirstlane(D.listNT) != 0;
-    if (s.packed) each_in_list16_lu<W, 32>(D.nbB16, D.ncap, s.i, nb, D.nb, nt, load, use);
-    else each_in_list_lu(D.nbB, D.ncap, s.i, nb, nt, load, use);
-}
-
-// two gather records of one neighbour
-struct Rec2 {
-    float4 a, b;
-};
 
 // ---- LDS windows --------------------------------------------------------
 // The fluid neighbours of a packed tile all lie in its slot runs (one
@@ -266,21 +111,6 @@ __device__ __forceinline__ void each_in_win16(const List16& L, int n, LD&& load,
         }
     }
 }
-
-__device__ __forceinline__ int phase_of(float4 x) { return (int)x.w; }
-
-__device__ __forceinline__ void write_partial(const Dev& D, int tile, int q, double v, double* lds) {
-    double t = block_sum_256(v, lds);
-    if (threadIdx.x == 0) D.partial[2 * tile + q] = t;
-}
-
-// packed counts: stored fluid entries | fluid neighbours found (the stored
-// ones plus any beyond the list capacity, up to 255) << 8 | boundary << 16 |
-// the particle's phase << 24
-__device__ __forceinline__ int nf_of(int c) { return c & 0xff; }
-__device__ __forceinline__ int nf_real(int c) { return (c >> 8) & 0xff; }
-__device__ __forceinline__ int nb_of(int c) { return (c >> 16) & 0xff; }
-__device__ __forceinline__ int phase_of_cnt(int c) { return c >> 24; }
 
 // The window-index list of a live particle of a tile that may stage a
 // window for the pass `bit` (packed, the pass's window on); the window itself
@@ -433,81 +263,6 @@ __global__ __launch_bounds__(256) void k_cfl_reduce(Dev D, float cfl, float spac
         if (vmax > 0.0f) dt = fminf(dtMax, cfl * spacing / vmax);
         D.dt[sc] = fmaxf(dt, dtMin);
     }
-}
-
-// ------------------------------------------------------- scene reduce ----
-// the copy in pinned host memory of a word of the loop-state block
-template <class T>
-__device__ __forceinline__ T* on_host(const Dev& D, const T* p) {
-    return reinterpret_cast<T*>(D.loopHost + (reinterpret_cast<const char*>(p) - D.loopDev));
-}
-
-// mode 0: DFSPH density  err = sum(rho*/rho0)/n - 1          (DFSPH.cpp:696)
-// mode 1: DFSPH divergence / IISPH error   err = sum/n      (DFSPH.cpp:896, IISph_M.cpp:353)
-// mode 2: PCISPH  err = max error/rho0 (second partial)     (PciSph.cpp:344-350)
-// Loop continuation (while err > tol || it < minIt; PCISPH err >= tol,
-// PciSph.cpp:116), stopping at `cap`.
-// Writes the scene's continuation flag to out (the active array itself, or
-// the next iteration's buffer of the DFSPH loops; a scene already done stays
-// done).  Every thread of the block calls it.
-__device__ __forceinline__ void scene_reduce_block(const Dev& D, int sc, int mode, float tol, int minIt, int cap,
-                                                   int* out) {
-    __shared__ double lds[4];
-    if (!D.active[sc]) {   // uniform per block
-        if (threadIdx.x == 0 && out != D.active) {
-            out[sc] = 0;
-            *on_host(D, out + sc) = 0;
-        }
-        return;
-    }
-    int t0 = D.scenePadStart[sc] / TILE, t1 = D.scenePadStart[sc + 1] / TILE;
-    __shared__ float ldsf[4];
-    double s = 0.0;
-    float mx = 0.0f;
-    // each thread sums tiles t0 + tid, + 256, + 512, ... in that order; the
-    // loads of eight of them are issued together
-    for (int t = t0 + threadIdx.x; t < t1; t += 256 * 8) {
-        double v[8];
-        float w[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int tt = t + 256 * k;
-            v[k] = tt < t1 ? D.partial[2 * tt] : 0.0;
-            w[k] = (mode == 2 && tt < t1) ? (float)D.partial[2 * tt + 1] : 0.0f;
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (t + 256 * k < t1) s += v[k];
-            mx = fmaxf(mx, w[k]);
-        }
-    }
-    s = block_sum_256(s, lds);
-    mx = block_max_256(mx, ldsf);
-    if (threadIdx.x == 0) {
-        int n = D.sceneCount[sc];
-        double err = n > 0 ? s / n : 0.0;
-        if (mode == 0) err = n > 0 ? err - 1.0 : 0.0;
-        if (mode == 2) err = (double)mx;
-        int it = D.iters[sc] + 1;
-        D.iters[sc] = it;
-        D.sceneErr[sc] = err;
-        bool cont = (mode == 2 ? err >= (double)tol : err > (double)tol) || (it < minIt);
-        if (cont && it >= cap) {
-            cont = false;
-            D.counters[C_COUNT - 1] = 1;  // max-iteration flag
-        }
-        out[sc] = cont ? 1 : 0;
-        *on_host(D, out + sc) = cont ? 1 : 0;
-        *on_host(D, D.iters + sc) = it;
-        *on_host(D, D.sceneErr + sc) = err;
-    }
-}
-
-// the loop's convergence test in front of a pass (scene b on blocks b, b + gridDim, ...)
-__device__ __forceinline__ void loop_test(const Dev& D) {
-    if (D.redMode >= 0)
-        for (int sc = blockIdx.x; sc < D.nscenes; sc += gridDim.x)
-            scene_reduce_block(D, sc, D.redMode, D.redTol, D.redMinIt, D.redCap, D.activeNext);
 }
 
 __global__ __launch_bounds__(256) void k_scene_reduce(Dev D, int mode, float tol, int minIt, int cap) {

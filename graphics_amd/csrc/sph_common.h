@@ -14,6 +14,7 @@ constexpr int NBF_CAP = 64;          // fluid neighbours kept per particle (ELL 
 constexpr int WIN_DENSITY = 1, WIN_DIVERGENCE = 2, WIN_VELOCITY = 4, WIN_SUMDIJ = 8, WIN_PRESSURE = 16;
 constexpr int WIN_ALL = 31;
 constexpr int NBB_CAP = 48;          // boundary neighbours kept per particle
+constexpr int BNF_CAP = 64, BNB_CAP = 16;   // IISph DF_*: neighbours kept per boundary particle
 constexpr int REF_NEIGHBOUR_CAP = 48;  // NeigbStr::maxNeigbNum (SphBase.h:630)
 constexpr int MAX_PHASES = 8;
 constexpr int MAX_SCENES = 4096;
@@ -129,6 +130,13 @@ struct Dev {
     float* brho;       // IISph DF_*: boundary particles' density, alpha, kappa/rho
     float* balpha;
     float* bk;
+    // the neighbours of each boundary particle, found once a step: fluid slots
+    // and other solids' boundary particles, four a group as in nbF with the
+    // boundary particles in place of the slots; bnCnt: fluid | boundary << 8,
+    // -1: more than the lists hold (that particle scans its cells)
+    int* bnF;
+    int* bnB;
+    int* bnCnt;
 
     // ---- neighbour lists.  Packed form: 16-bit entries, eight per int4,
     // group g of particle i at g*ncap + i, decoded through the tile's base
@@ -281,10 +289,12 @@ __device__ __forceinline__ int xcd_block(int b, int n) {
     return x * q + min(x, r) + b / NUM_XCD;
 }
 
-// tile of a workgroup under the mapping the autotuner chose (Dev::tileMap)
-__device__ __forceinline__ int tile_of_block(int map) {
-    return map ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+// tile of a workgroup under the mapping the autotuner chose (Dev::tileMap);
+// blocks: the workgroups that take tiles (the first ones of the grid)
+__device__ __forceinline__ int tile_of_block(int map, int blocks) {
+    return map ? xcd_block(blockIdx.x, blocks) : (int)blockIdx.x;
 }
+__device__ __forceinline__ int tile_of_block(int map) { return tile_of_block(map, gridDim.x); }
 
 __device__ __forceinline__ uint32_t morton2(uint32_t a, uint32_t b) {
     auto spread = [](uint32_t v) {
@@ -568,7 +578,7 @@ void launch_field_by_id(const Dev& D, const float* src, const uint32_t* rank, fl
 void launch_ids_by_rank(const Dev& D, const uint32_t* rank, long long* out, int* removed, hipStream_t st);
 
 // iisph_df.hip: the IISph class's DF_* solvers
-void launch_idf_prepare(const Dev& D, hipStream_t st);
+void launch_idf_prepare(const Dev& D, hipStream_t st);   // also the boundary particles' lists
 void launch_idf_vadv(const Dev& D, int mode, hipStream_t st);
 void launch_idf_kappa(const Dev& D, int mode, hipStream_t st);
 void launch_idf_velocity(const Dev& D, hipStream_t st);
