@@ -886,7 +886,7 @@ int step_dfsph(sphgpu_handle* h, sphgpu_stats* st) {
         if (mode == 2) {
             ProfScope ps(h, "mlp_forward", nf_live(h) * 36.0);
             // (the warm start reads the prediction only where Drho/Dt > 0)
-            mlp_forward(h->mlp, h->feat, h->ypred, D.npad, nullptr, h->st, true);
+            mlp_forward(h->mlp, h->feat, h->ypred, D.npad, h->st, true);
         }
         launch_df_warm_apply(D, h->ypred, h->feat, mode, h->st);
         if (mode != 0) {
@@ -953,7 +953,7 @@ int step_iisph(sphgpu_handle* h, sphgpu_stats* st) {
         }
         if (predict) {
             ProfScope ps(h, "mlp_forward", nf_live(h) * 36.0);
-            mlp_forward(h->mlp, h->feat, h->ypred, D.npad, nullptr, h->st);
+            mlp_forward(h->mlp, h->feat, h->ypred, D.npad, h->st);
             launch_ii_warm_apply(D, h->ypred, h->feat, h->st);
         }
         solver_loop_start(h, 0, batch);

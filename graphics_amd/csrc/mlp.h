@@ -9,9 +9,17 @@ constexpr int MLP_IN = 8;
 constexpr int MLP_PARAMS = 64 * 8 + 64 + 64 * 64 + 64 + 64 * 64 + 64 + 64 + 1;   // 8961
 constexpr int MLP_FWD_FRAGS = 22;    // BF16 A fragments of the forward pass
 constexpr int MLP_BWD_FRAGS = 20;    // BF16 A fragments of the backward pass
-constexpr int MLP_STORE = 196;       // per-sample row: z1 z2 z3 (3 x 64), y at 192
 constexpr int MLP_WGRAD_TILES = 53;  // 40 weight tiles + 13 bias tiles
-constexpr int MLP_WGRAD_SLICE = 128; // samples per weight-gradient block
+constexpr int MLP_SLICES = 512;      // blocks of a gradient at most: two on each CU
+// Samples of a gradient block for n samples: 64, the least a block's four
+// waves take, until that gives MLP_SLICES blocks; from there on a block takes
+// several of its chunks and the partial gradients (54 KB a block) stay as many.
+constexpr int mlp_slice_samples(long long n) { return int(64 * ((n + 64LL * MLP_SLICES - 1) / (64LL * MLP_SLICES))); }
+constexpr int mlp_slices(long long n) { return int((n + mlp_slice_samples(n) - 1) / mlp_slice_samples(n)); }
+// the most slices of any 1 <= n <= cap
+constexpr int mlp_max_slices(long long cap) { return int((cap + 63) / 64 < MLP_SLICES ? (cap + 63) / 64 : MLP_SLICES); }
+
+constexpr size_t MLP_LOSS_OFFSET = (sizeof(float) * MLP_PARAMS + 255) / 256 * 256;   // of lossPart behind grad
 
 struct MlpDev {
     float* params = nullptr;    // FP32 master parameters (W1 b1 W2 b2 W3 b3 W4 b4)
@@ -20,11 +28,7 @@ struct MlpDev {
     float* grad = nullptr;
     void* fwd = nullptr;        // MLP_FWD_FRAGS x 64 lanes x 8 BF16
     void* bwd = nullptr;        // MLP_BWD_FRAGS x 64 lanes x 8 BF16
-    float* store = nullptr;     // cap x MLP_STORE: pre-activations / output
-    float* dz = nullptr;        // cap x MLP_STORE: gradients w.r.t. pre-activations
-    float* dy = nullptr;        // cap
-    float* scratchY = nullptr;  // cap
-    double* lossPart = nullptr; // cap / 256 + 1
+    double* lossPart = nullptr; // mlp_max_slices(cap), behind grad in one block
     float* gradPart = nullptr;  // slices x MLP_WGRAD_TILES x 256 partial gradient tiles
     float overWeight = 1.0f;    // loss weight where the prediction exceeds the target
     int cap = 0;                // samples per gradient evaluation
@@ -32,11 +36,9 @@ struct MlpDev {
 };
 
 void mlp_pack(MlpDev& m, hipStream_t st);
-// y[i] = MLP(feat[8 i .. 8 i + 7]); store (cap x MLP_STORE) receives activations when non-null
-// gate1 (inference only): tiles of 16 particles whose feature 1 is negative
-// for all 16 are skipped, their outputs left as they were
-void mlp_forward(const MlpDev& m, const float* feat, float* y, int n, float* store, hipStream_t st,
-                 bool gate1 = false);
+// y[i] = MLP(feat[8 i .. 8 i + 7]); gate1: tiles of 16 particles whose feature
+// 1 is negative for all 16 are skipped, their outputs left as they were
+void mlp_forward(const MlpDev& m, const float* feat, float* y, int n, hipStream_t st, bool gate1 = false);
 // gradient of mean((MLP(feat) - target)^2) into m.grad (n <= m.cap); loss parts in m.lossPart
 void mlp_grad(MlpDev& m, const float* feat, const float* target, int n, hipStream_t st);
 void mlp_adam(MlpDev& m, float lr, hipStream_t st);
@@ -48,5 +50,8 @@ namespace sphgpu {
 void mlp_init_params(std::vector<float>& p, unsigned long long seed);
 int mlp_alloc(MlpDev& m, int cap);
 void mlp_free(MlpDev& m);
-double mlp_loss_host(const MlpDev& m, int n, hipStream_t st);
+// bytes from MlpDev::grad on: the gradient, then room for the loss partial sums of up to n samples
+inline size_t mlp_result_bytes(long long n) { return MLP_LOSS_OFFSET + sizeof(double) * (size_t)mlp_max_slices(n); }
+// mean loss of n samples from the partial sums, in order
+double mlp_loss_sum(const double* part, int n);
 }  // namespace sphgpu

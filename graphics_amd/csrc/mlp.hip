@@ -12,16 +12,17 @@
 // not depend on the hardware's own K order.
 //
 // Kernels: fragment packing (FP32 master weights -> BF16 A fragments),
-// forward (inference; in training also stores pre/post activations),
-// backward through the activations (dh = W^T dz, same chaining with the
-// transposed fragments), weight/bias gradients (MFMA with K = particles),
-// and Adam.
+// inference, the gradient of a slice of samples (forward, loss, backward
+// through the activations, weight and bias gradients with K = samples), the
+// sum of the slices, and Adam.
 #include "sph_common.h"
 #include "mlp.h"
 #include "sphgpu.h"
+#include "xfer.h"
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -47,10 +48,9 @@ __device__ __forceinline__ float gelu_sigma(float x) {
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
 }
 __device__ __forceinline__ float gelu(float x) { return x * gelu_sigma(x); }
-// d/dx x sigma(2u) = sigma + 2 x sigma (1 - sigma) c (1 + 3 * 0.044715 x^2)
-__device__ __forceinline__ float gelu_grad(float x) {
+// d/dx x sigma(2u) = sigma + 2 x sigma (1 - sigma) c (1 + 3 * 0.044715 x^2), sg = sigma(2u)
+__device__ __forceinline__ float gelu_grad(float x, float sg) {
     const float c = 0.7978845608028654f;
-    const float sg = gelu_sigma(x);
     return sg + 2.0f * x * sg * (1.0f - sg) * c * (1.0f + 3.0f * 0.044715f * x * x);
 }
 
@@ -121,86 +121,9 @@ __device__ __forceinline__ bf16x8 chain(const float (&h)[4][4], int s) {
     return b;
 }
 
-// forward of 16 particles [p0, p0+16); optionally stores z/h rows for training
-struct FwdOut {
-    float z[3][4][4];   // pre-activations (layer, tile, j)
-    float y;
-};
-
-__device__ __forceinline__ void forward_tile(const bf16x8* __restrict__ F, const float* __restrict__ P,
-                                             const float* __restrict__ feat, int p0, int n, FwdOut& o,
-                                             float* __restrict__ store) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    const int p = p0 + c;
-    bf16x8 x;
-    for (int j = 0; j < 8; ++j) x[j] = to_bf16(0.0f);
-    if (g < 2 && p < n) {
-        const float4 f = reinterpret_cast<const float4*>(feat)[p * 2 + g];
-        x[0] = to_bf16(f.x); x[1] = to_bf16(f.y); x[2] = to_bf16(f.z); x[3] = to_bf16(f.w);
-    }
-    float h[4][4];
-    // layer 1
-    for (int t = 0; t < 4; ++t) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma(F[(0 + t) * 64 + lane], x, acc);
-        for (int j = 0; j < 4; ++j) {
-            int u = 16 * t + 4 * g + j;
-            float z = acc[j] + P[OFF_B1 + u];
-            o.z[0][t][j] = z;
-            h[t][j] = gelu(z);
-        }
-    }
-    // layers 2, 3
-    const int fbase[2] = {4, 12}, boff[2] = {OFF_B2, OFF_B3};
-    for (int L = 0; L < 2; ++L) {
-        bf16x8 b0 = chain(h, 0), b1 = chain(h, 1);
-        for (int t = 0; t < 4; ++t) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = mfma(F[(fbase[L] + 2 * t) * 64 + lane], b0, acc);
-            acc = mfma(F[(fbase[L] + 2 * t + 1) * 64 + lane], b1, acc);
-            for (int j = 0; j < 4; ++j) {
-                int u = 16 * t + 4 * g + j;
-                float z = acc[j] + P[boff[L] + u];
-                o.z[L + 1][t][j] = z;
-                h[t][j] = gelu(z);
-            }
-        }
-    }
-    // layer 4 (1 output row)
-    {
-        bf16x8 b0 = chain(h, 0), b1 = chain(h, 1);
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma(F[20 * 64 + lane], b0, acc);
-        acc = mfma(F[21 * 64 + lane], b1, acc);
-        o.y = acc[0] + P[OFF_B4];       // row 0: lanes g == 0, j == 0
-    }
-    if (store && p < n) {
-        // rows [p][layer*64 + unit]: z1 z2 z3, then y at 192
-        for (int L = 0; L < 3; ++L)
-            for (int t = 0; t < 4; ++t)
-                for (int j = 0; j < 4; ++j) store[(size_t)p * MLP_STORE + L * 64 + 16 * t + 4 * g + j] = o.z[L][t][j];
-        if (g == 0) store[(size_t)p * MLP_STORE + 192] = o.y;
-    }
-}
-
-__global__ __launch_bounds__(256) void k_mlp_forward(const bf16x8* __restrict__ F, const float* __restrict__ P,
-                                                   const float* __restrict__ feat, float* __restrict__ y, int n,
-                                                   float* __restrict__ store) {
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int nw = (gridDim.x * blockDim.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    const int ntile = (n + 15) / 16;
-    for (int tile = wave; tile < ntile; tile += nw) {
-        FwdOut o;
-        forward_tile(F, P, feat, tile * 16, n, o, store);
-        int p = tile * 16 + (lane & 15);
-        if ((lane >> 4) == 0 && p < n) y[p] = o.y;
-    }
-}
-
 // Inference only: the 22 weight fragments stay in registers and the biases
 // in LDS for all the tiles of 16 particles a wave processes (the training
-// forward above re-reads them per tile).  gate1: a tile whose 16 particles
+// pass re-reads them per tile).  gate1: a tile whose 16 particles
 // all have feature 1 below zero is skipped and its outputs are not written
 // (the DFSPH warm start reads the output only where Drho/Dt > 0, and feature
 // 1 is asinh of a positive multiple of Drho/Dt, negative only where it is).
@@ -261,57 +184,6 @@ __global__ __launch_bounds__(256, 3) void k_mlp_infer(const bf16x8* __restrict__
     }
 }
 
-// backward through the activations for 16 particles: dL/dy -> dz3, dz2, dz1,
-// stored as rows [p][layer*64 + unit] in dz (FP32).  Pre-activations come
-// from the forward store.
-__global__ __launch_bounds__(256) void k_mlp_backward(const bf16x8* __restrict__ B, const float* __restrict__ store,
-                                                    const float* __restrict__ dy, float* __restrict__ dz, int n) {
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int nw = (gridDim.x * blockDim.x) >> 6;
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    const int ntile = (n + 15) / 16;
-    for (int tile = wave; tile < ntile; tile += nw) {
-        const int p = tile * 16 + c;
-        const bool ok = p < n;
-        // B operand: dz4 (1 x P) in K slot (0, 0)
-        bf16x8 b;
-        for (int j = 0; j < 8; ++j) b[j] = to_bf16(0.0f);
-        if (g == 0 && ok) b[0] = to_bf16(dy[p]);
-        float d[4][4];
-        // dh3 = W4^T dz4 ; dz3 = dh3 * gelu'(z3)
-        for (int t = 0; t < 4; ++t) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = mfma(B[(0 + t) * 64 + lane], b, acc);
-            for (int j = 0; j < 4; ++j) {
-                int u = 16 * t + 4 * g + j;
-                float z = ok ? store[(size_t)p * MLP_STORE + 2 * 64 + u] : 0.0f;
-                d[t][j] = acc[j] * gelu_grad(z);
-                if (ok) dz[(size_t)p * MLP_STORE + 2 * 64 + u] = d[t][j];
-            }
-        }
-        // dh2 = W3^T dz3 -> dz2 ; dh1 = W2^T dz2 -> dz1
-        const int fb[2] = {4, 12}, zl[2] = {1, 0};
-        for (int L = 0; L < 2; ++L) {
-            bf16x8 b0 = chain(d, 0), b1 = chain(d, 1);
-            float e[4][4];
-            for (int t = 0; t < 4; ++t) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                acc = mfma(B[(fb[L] + 2 * t) * 64 + lane], b0, acc);
-                acc = mfma(B[(fb[L] + 2 * t + 1) * 64 + lane], b1, acc);
-                for (int j = 0; j < 4; ++j) {
-                    int u = 16 * t + 4 * g + j;
-                    float z = ok ? store[(size_t)p * MLP_STORE + zl[L] * 64 + u] : 0.0f;
-                    e[t][j] = acc[j] * gelu_grad(z);
-                    if (ok) dz[(size_t)p * MLP_STORE + zl[L] * 64 + u] = e[t][j];
-                }
-            }
-            for (int t = 0; t < 4; ++t)
-                for (int j = 0; j < 4; ++j) d[t][j] = e[t][j];
-        }
-        if (g == 0 && ok) dz[(size_t)p * MLP_STORE + 192] = dy[p];
-    }
-}
-
 // Tile t of the weight/bias gradient: 16x16 blocks of dW (out x in) per
 // layer, then bias blocks.  L1 4x1, L2 4x4, L3 4x4, L4 1x4 (W), then bias
 // tiles 4+4+4+1.
@@ -335,23 +207,28 @@ __device__ __forceinline__ GradTile grad_tile(int t) {
     return r;
 }
 
-// Weight and bias gradients, K = samples split into slices of
-// MLP_WGRAD_SLICE: one block per slice.  For each chunk of 32 samples the
-// block stages in LDS, once, the chunk's pre-activation gradients dz (the A
-// operand: output unit x sample) and its layer inputs h = features,
-// GELU(z1), GELU(z2), GELU(z3) (the B operand: sample x input unit), both as
-// BF16 and unit-major so that a fragment's eight samples are two 8-byte LDS
-// reads: thread t loads column t of the chunk's rows (coalesced across the
-// wave), applies GELU once and writes its unit's 32 samples with 8-byte
-// stores.  The next chunk's loads are issued before this chunk's tiles run;
-// the four waves accumulate the 53 tiles (each wave every fourth) on the
-// matrix cores.  k_mlp_wgrad_reduce sums the slices in a fixed order
-// (deterministic).
-constexpr int WG_CHUNK = 32;
-constexpr int WG_ROW = WG_CHUNK + 4;     // LDS row pitch in BF16 (8-byte aligned, staggered banks)
-constexpr int WG_DZ = 193;               // dz rows: z1 z2 z3 (192) and y
-constexpr int WG_H = 200;                // input rows: features (8), h1, h2, h3
-constexpr int WG_TILES_PER_WAVE = (MLP_WGRAD_TILES + 3) / 4;
+// Gradient of one slice of samples (mlp_slice_samples) a block, in chunks of
+// 64: each wave takes 16 samples forward and backward, dh = W^T dz chained on
+// the matrix cores like the forward pass, with loss = w e^2, e = y - target,
+// w = over where e > 0 else 1 (dL/dy = 2 w e / n).  What the weight gradients
+// contract over the samples, the layer inputs (features, GELU(z1..3)) and the
+// output gradients (dz1..3, dL/dy), goes to LDS as BF16, unit-major, so that a
+// fragment's eight samples are two 8-byte reads; after the chunk's four waves
+// are done each of them accumulates every fourth of the 53 tiles
+// (k_mlp_wgrad_reduce sums the slices in a fixed order: deterministic).  One
+// FP64 loss partial a block.  sigma is evaluated once for GELU and its
+// derivative, which stays in registers until the way back.
+// Bound by the wave's chain of layers and the weights' loads at one block a CU.
+// Measured (MI355X, one training iteration): 4,096 samples 18.2 us, 16,384
+// 24.9 (this kernel 15.6), 60,000 35.8, 262,144 81; as separate passes that
+// kept z and dz in memory 43.8, 54.5 (48.8), 98.6 and 501.  The weights staged in
+// LDS (one block a CU): 20.9, 27.7, 47.6, 115; held in registers over the
+// chunks: 19.6, 26.0, 46.2, 114.
+constexpr int TR_CHUNK = 64;
+constexpr int TR_ROW = TR_CHUNK + 4;     // LDS row pitch in BF16 (8-byte aligned, staggered banks)
+constexpr int TR_DZ = 193;               // rows of output gradients: dz1 dz2 dz3 (192) and dL/dy
+constexpr int TR_H = 200;                // rows of inputs: features (8), h1, h2, h3
+constexpr int TR_TILES_PER_WAVE = (MLP_WGRAD_TILES + 3) / 4;
 
 __device__ __forceinline__ bf16x8 lds_frag(const __bf16* row, int g) {
     // samples kmap(g, 0..3) = 4g..4g+3 and kmap(g, 4..7) = 16+4g..16+4g+3
@@ -363,94 +240,134 @@ __device__ __forceinline__ bf16x8 lds_frag(const __bf16* row, int g) {
     return v;
 }
 
-// One chunk's operands in registers: thread t holds column t of the chunk's
-// 32 store rows (z1 z2 z3) and 32 dz rows, and feature (t & 7) of sample
-// t >> 3.  Each load instruction reads 64 consecutive floats of one row.
-struct WgCols {
-    float z[WG_CHUNK];
-    float d[WG_CHUNK];
-    float f;
-};
-
-__device__ __forceinline__ void wg_load(const float* __restrict__ feat, const float* __restrict__ store,
-                                        const float* __restrict__ dz, int q, int p1, int tid, WgCols& C) {
+__global__ __launch_bounds__(256, 2) void k_mlp_train(const bf16x8* __restrict__ F, const bf16x8* __restrict__ B,
+                                                    const float* __restrict__ P, const float* __restrict__ feat,
+                                                    const float* __restrict__ target, float* __restrict__ part,
+                                                    double* __restrict__ lossPart, int n, int per, float over) {
+    __shared__ __attribute__((aligned(16))) __bf16 sA[TR_DZ * TR_ROW];
+    __shared__ __attribute__((aligned(16))) __bf16 sB[(TR_H + 1) * TR_ROW];   // last row: bias input 1 / 0
+    __shared__ double sLoss[4];
+    const int slice = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int col = 16 * wave + c;           // the sample's column
+    f32x4 acc[TR_TILES_PER_WAVE];
 #pragma unroll
-    for (int s = 0; s < WG_CHUNK; ++s) {
-        const size_t row = (size_t)(q + s) * MLP_STORE + tid;
-        const bool ok = q + s < p1;
-        C.z[s] = ok && tid < 192 ? store[row] : 0.0f;
-        C.d[s] = ok && tid < WG_DZ ? dz[row] : 0.0f;
-    }
-    const int p = q + (tid >> 3);
-    C.f = p < p1 ? feat[(size_t)p * 8 + (tid & 7)] : 0.0f;
-}
-
-// four BF16 of a unit-major LDS row (one 8-byte store)
-__device__ __forceinline__ void st_bf16x4(__bf16* dst, float a, float b, float c, float d) {
-    const __bf16 v[4] = {to_bf16(a), to_bf16(b), to_bf16(c), to_bf16(d)};
-    uint2 u;
-    __builtin_memcpy(&u, v, 8);
-    *reinterpret_cast<uint2*>(dst) = u;
-}
-
-__device__ __forceinline__ void wg_store(const WgCols& C, int q, int p1, int tid, __bf16* sA, __bf16* sB) {
-    if (tid < 192) {
-        __bf16* row = sB + (8 + tid) * WG_ROW;
+    for (int k = 0; k < TR_TILES_PER_WAVE; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    double loss = 0.0;
+    const long long p1 = min((long long)n, (long long)(slice + 1) * per);
+    for (long long q = (long long)slice * per; q < p1; q += TR_CHUNK) {
+        const long long p = q + col;
+        const bool ok = p < p1;
+        // keeps the weights' loads in the loop: the compiler would hold the 42
+        // fragments in registers over all chunks and spill for it
+        int again = 0;
+        asm volatile("" : "+s"(again));
+        const bf16x8 *const Fc = F + again, *const Bc = B + again;
+        const float* const Pc = P + again;
+        float h[4][4], gp[3][4][4];
+        {
+            bf16x8 x = bf16x8{};
+            if (g < 2) {
+                if (ok) {
+                    const float4 f = reinterpret_cast<const float4*>(feat)[p * 2 + g];
+                    x[0] = to_bf16(f.x); x[1] = to_bf16(f.y); x[2] = to_bf16(f.z); x[3] = to_bf16(f.w);
+                }
 #pragma unroll
-        for (int s = 0; s < WG_CHUNK; s += 4)
-            st_bf16x4(row + s, gelu(C.z[s]), gelu(C.z[s + 1]), gelu(C.z[s + 2]), gelu(C.z[s + 3]));
-    }
-    if (tid < WG_DZ) {
-        __bf16* row = sA + tid * WG_ROW;
+                for (int j = 0; j < 4; ++j) sB[(4 * g + j) * TR_ROW + col] = x[j];
+            }
+            if (g == 2) sB[TR_H * TR_ROW + col] = to_bf16(ok ? 1.0f : 0.0f);
 #pragma unroll
-        for (int s = 0; s < WG_CHUNK; s += 4) st_bf16x4(row + s, C.d[s], C.d[s + 1], C.d[s + 2], C.d[s + 3]);
-    }
-    sB[(tid & 7) * WG_ROW + (tid >> 3)] = to_bf16(C.f);
-    if (tid < WG_CHUNK) sB[WG_H * WG_ROW + tid] = to_bf16(q + tid < p1 ? 1.0f : 0.0f);
-}
-
-__global__ __launch_bounds__(256) void k_mlp_wgrad(const float* __restrict__ feat, const float* __restrict__ store,
-                                                 const float* __restrict__ dz, float* __restrict__ part, int n) {
-    __shared__ __attribute__((aligned(16))) __bf16 sA[WG_DZ * WG_ROW];
-    __shared__ __attribute__((aligned(16))) __bf16 sB[(WG_H + 1) * WG_ROW];   // last row: bias input 1 / 0
-    const int slice = blockIdx.x, tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
-    f32x4 acc[WG_TILES_PER_WAVE];
+            for (int L = 0; L < 3; ++L) {
+                const bf16x8 b0 = L ? chain(h, 0) : x, b1 = L ? chain(h, 1) : x;
 #pragma unroll
-    for (int k = 0; k < WG_TILES_PER_WAVE; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int p0 = slice * MLP_WGRAD_SLICE, p1 = min(n, p0 + MLP_WGRAD_SLICE);
-    WgCols C;
-    wg_load(feat, store, dz, p0, p1, tid, C);
-    for (int q = p0; q < p1; q += WG_CHUNK) {
-        __syncthreads();   // the previous chunk's fragments are read
-        wg_store(C, q, p1, tid, sA, sB);
-        __syncthreads();
-        // the next chunk's loads are in flight while this one's tiles run
-        if (q + WG_CHUNK < p1) wg_load(feat, store, dz, q + WG_CHUNK, p1, tid, C);
+                for (int t = 0; t < 4; ++t) {
+                    f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                    if (L == 0) {
+                        z = mfma(Fc[t * 64 + lane], b0, z);
+                    } else {
+                        z = mfma(Fc[(8 * L - 4 + 2 * t) * 64 + lane], b0, z);
+                        z = mfma(Fc[(8 * L - 4 + 2 * t + 1) * 64 + lane], b1, z);
+                    }
 #pragma unroll
-        for (int k = 0; k < WG_TILES_PER_WAVE; ++k) {
+                    for (int j = 0; j < 4; ++j) {
+                        const int u = 16 * t + 4 * g + j;
+                        const float v = z[j] + Pc[(L == 0 ? OFF_B1 : L == 1 ? OFF_B2 : OFF_B3) + u];
+                        const float sg = gelu_sigma(v);
+                        h[t][j] = v * sg;
+                        gp[L][t][j] = gelu_grad(v, sg);
+                        sB[(8 + 64 * L + u) * TR_ROW + col] = to_bf16(ok ? h[t][j] : 0.0f);
+                    }
+                }
+            }
+        }
+        // B operand of the way back: dz4 (1 x P) in K slot (0, 0); y is row 0 of
+        // the last layer's product: lanes g == 0, j == 0
+        bf16x8 b = bf16x8{};
+        {
+            f32x4 y = {0.f, 0.f, 0.f, 0.f};
+            y = mfma(Fc[20 * 64 + lane], chain(h, 0), y);
+            y = mfma(Fc[21 * 64 + lane], chain(h, 1), y);
+            if (g == 0) {
+                if (ok) {
+                    const float e = y[0] + Pc[OFF_B4] - target[p];
+                    const float w = e > 0.0f ? over : 1.0f;
+                    loss += (double)w * (double)e * (double)e;
+                    b[0] = to_bf16(2.0f * w * e / (float)n);
+                }
+                sA[192 * TR_ROW + col] = b[0];
+            }
+        }
+        // dh3 = W4^T dz4, dh2 = W3^T dz3, dh1 = W2^T dz2; dz = dh * gelu'(z)
+        float d[4][4];
+#pragma unroll
+        for (int L = 2; L >= 0; --L) {
+            const bf16x8 b0 = L == 2 ? b : chain(d, 0), b1 = L == 2 ? b : chain(d, 1);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                f32x4 dh = {0.f, 0.f, 0.f, 0.f};
+                if (L == 2) {
+                    dh = mfma(Bc[t * 64 + lane], b0, dh);
+                } else {
+                    dh = mfma(Bc[(12 - 8 * L + 2 * t) * 64 + lane], b0, dh);
+                    dh = mfma(Bc[(12 - 8 * L + 2 * t + 1) * 64 + lane], b1, dh);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    d[t][j] = dh[j] * gp[L][t][j];
+                    sA[(64 * L + 16 * t + 4 * g + j) * TR_ROW + col] = to_bf16(ok ? d[t][j] : 0.0f);
+                }
+            }
+        }
+        __syncthreads();   // the chunk's columns are written
+#pragma unroll
+        for (int k = 0; k < TR_TILES_PER_WAVE; ++k) {
             const int t = wave + 4 * k;
             if (t >= MLP_WGRAD_TILES) break;
             const GradTile T = grad_tile(t);
             const int nin = (T.L == 0) ? 8 : 64, nout = (T.L == 3) ? 1 : 64;
-            const int zoff = (T.L < 3) ? T.L * 64 : 192;            // dz rows of layer L's output
+            const int zoff = (T.L < 3) ? T.L * 64 : 192;            // rows of layer L's output gradient
             const int hoff = (T.L == 0) ? 0 : 8 + (T.L - 1) * 64;   // rows of layer L's input
             const int orow = 16 * T.to + c, icol = 16 * T.ti + c;
-            const bf16x8 zero = bf16x8{};
-            const bf16x8 a = orow < nout ? lds_frag(sA + (zoff + orow) * WG_ROW, g) : zero;
-            const bf16x8 b = T.bias ? lds_frag(sB + WG_H * WG_ROW, g)
-                                    : (icol < nin ? lds_frag(sB + (hoff + icol) * WG_ROW, g) : zero);
-            acc[k] = mfma(a, b, acc[k]);
+#pragma unroll
+            for (int s = 0; s < TR_CHUNK; s += 32) {
+                const bf16x8 zero = bf16x8{};
+                const bf16x8 a = orow < nout ? lds_frag(sA + (zoff + orow) * TR_ROW + s, g) : zero;
+                const bf16x8 v = T.bias ? lds_frag(sB + TR_H * TR_ROW + s, g)
+                                        : (icol < nin ? lds_frag(sB + (hoff + icol) * TR_ROW + s, g) : zero);
+                acc[k] = mfma(a, v, acc[k]);
+            }
         }
+        __syncthreads();   // the fragments are read: the next chunk may overwrite them
     }
     // D[4g+j][c] of each tile
 #pragma unroll
-    for (int k = 0; k < WG_TILES_PER_WAVE; ++k) {
+    for (int k = 0; k < TR_TILES_PER_WAVE; ++k) {
         const int t = wave + 4 * k;
         if (t >= MLP_WGRAD_TILES) break;
         float* out = part + ((size_t)slice * MLP_WGRAD_TILES + t) * 256;
         for (int j = 0; j < 4; ++j) out[(4 * g + j) * 16 + c] = acc[k][j];
     }
+    const double s = block_sum_256(loss, sLoss);
+    if (threadIdx.x == 0) lossPart[slice] = s;
 }
 
 // Sum of the slices' partial tiles: eight threads per gradient element,
@@ -481,24 +398,6 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad_reduce(const float* __restric
     else grad[woff[T.L] + out * nin + in] = s * scale;
 }
 
-// MSE loss gradient dL/dy = 2 (y - t) / n (times `scale` for normalised targets)
-// loss = mean(w e^2), e = y - target, w = over where e > 0 else 1
-__global__ void k_mlp_loss(const float* __restrict__ store, const float* __restrict__ target,
-                           float* __restrict__ dy, double* __restrict__ lossPart, int n, float over) {
-    __shared__ double lds[4];
-    int i = blockIdx.x * 256 + threadIdx.x;
-    double l = 0.0;
-    if (i < n) {
-        float y = store[(size_t)i * MLP_STORE + 192];
-        float e = y - target[i];
-        float w = e > 0.0f ? over : 1.0f;
-        dy[i] = 2.0f * w * e / (float)n;
-        l = (double)w * (double)e * (double)e;
-    }
-    double s = block_sum_256(l, lds);
-    if (threadIdx.x == 0) lossPart[blockIdx.x] = s;
-}
-
 __global__ void k_mlp_adam(float* __restrict__ P, float* __restrict__ M, float* __restrict__ V,
                            const float* __restrict__ grad, float lr, float b1, float b2, float eps, float c1,
                            float c2) {
@@ -520,33 +419,20 @@ void mlp_pack(MlpDev& m, hipStream_t st) {
                        (bf16x8*)m.fwd, (bf16x8*)m.bwd);
 }
 
-void mlp_forward(const MlpDev& m, const float* feat, float* y, int n, float* store, hipStream_t st, bool gate1) {
+void mlp_forward(const MlpDev& m, const float* feat, float* y, int n, hipStream_t st, bool gate1) {
     if (n <= 0) return;
-    int waves = (n + 15) / 16;
-    if (!store) {
-        // about three waves per SIMD, each looping over tiles
-        const int blocks = std::min((waves + 3) / 4, 768);
-        hipLaunchKernelGGL(k_mlp_infer, dim3(blocks), dim3(256), 0, st, (const bf16x8*)m.fwd, (const float*)m.params,
-                           feat, y, n, gate1 ? 1 : 0);
-        return;
-    }
-    int blocks = std::min((waves + 3) / 4, 8192);
-    hipLaunchKernelGGL(k_mlp_forward, dim3(blocks), dim3(256), 0, st, (const bf16x8*)m.fwd,
-                       (const float*)m.params, feat, y, n, store);
+    const int waves = (n + 15) / 16;
+    // about three waves per SIMD, each looping over tiles
+    const int blocks = std::min((waves + 3) / 4, 768);
+    hipLaunchKernelGGL(k_mlp_infer, dim3(blocks), dim3(256), 0, st, (const bf16x8*)m.fwd, (const float*)m.params,
+                       feat, y, n, gate1 ? 1 : 0);
 }
 
 void mlp_grad(MlpDev& m, const float* feat, const float* target, int n, hipStream_t st) {
-    mlp_forward(m, feat, m.scratchY, n, m.store, st);
-    int lb = (n + 255) / 256;
-    hipLaunchKernelGGL(k_mlp_loss, dim3(lb), dim3(256), 0, st, (const float*)m.store, target, m.dy, m.lossPart, n,
+    const int slices = mlp_slices(n);
+    hipLaunchKernelGGL(k_mlp_train, dim3(slices), dim3(256), 0, st, (const bf16x8*)m.fwd, (const bf16x8*)m.bwd,
+                       (const float*)m.params, feat, target, m.gradPart, m.lossPart, n, mlp_slice_samples(n),
                        m.overWeight);
-    int waves = (n + 15) / 16;
-    int blocks = std::min((waves + 3) / 4, 8192);
-    hipLaunchKernelGGL(k_mlp_backward, dim3(blocks), dim3(256), 0, st, (const bf16x8*)m.bwd,
-                       (const float*)m.store, (const float*)m.dy, m.dz, n);
-    const int slices = (n + MLP_WGRAD_SLICE - 1) / MLP_WGRAD_SLICE;
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3(slices), dim3(256), 0, st, feat, (const float*)m.store,
-                       (const float*)m.dz, m.gradPart, n);
     hipLaunchKernelGGL(k_mlp_wgrad_reduce, dim3(8 * MLP_WGRAD_TILES), dim3(256), 0, st, (const float*)m.gradPart,
                        m.grad, slices, 1.0f);
 }
@@ -579,37 +465,27 @@ int mlp_alloc(MlpDev& m, int cap) {
     m.cap = std::max(cap, 16);
     auto al = [](void** p, size_t b) { return hipMalloc(p, std::max<size_t>(b, 256)) == hipSuccess; };
     bool ok = al((void**)&m.params, sizeof(float) * MLP_PARAMS) && al((void**)&m.adamM, sizeof(float) * MLP_PARAMS) &&
-              al((void**)&m.adamV, sizeof(float) * MLP_PARAMS) && al((void**)&m.grad, sizeof(float) * MLP_PARAMS) &&
+              al((void**)&m.adamV, sizeof(float) * MLP_PARAMS) && al((void**)&m.grad, mlp_result_bytes(m.cap)) &&
               al(&m.fwd, 16 * 64 * MLP_FWD_FRAGS) && al(&m.bwd, 16 * 64 * MLP_BWD_FRAGS) &&
-              al((void**)&m.store, sizeof(float) * MLP_STORE * (size_t)m.cap) &&
-              al((void**)&m.dz, sizeof(float) * MLP_STORE * (size_t)m.cap) &&
-              al((void**)&m.dy, sizeof(float) * m.cap) && al((void**)&m.scratchY, sizeof(float) * m.cap) &&
-              al((void**)&m.lossPart, sizeof(double) * (m.cap / 256 + 2)) &&
-              al((void**)&m.gradPart, sizeof(float) * 256 * MLP_WGRAD_TILES *
-                                          (size_t)((m.cap + MLP_WGRAD_SLICE - 1) / MLP_WGRAD_SLICE));
+              al((void**)&m.gradPart, sizeof(float) * 256 * MLP_WGRAD_TILES * (size_t)mlp_max_slices(m.cap));
+    m.lossPart = reinterpret_cast<double*>(reinterpret_cast<char*>(m.grad) + MLP_LOSS_OFFSET);
     if (!ok) return -1;
     hipMemset(m.adamM, 0, sizeof(float) * MLP_PARAMS);
     hipMemset(m.adamV, 0, sizeof(float) * MLP_PARAMS);
-    hipMemset(m.dz, 0, sizeof(float) * MLP_STORE * (size_t)m.cap);
     m.adamStep = 0;
     return 0;
 }
 
 void mlp_free(MlpDev& m) {
-    void* ps[] = {m.params, m.adamM, m.adamV, m.grad, m.fwd, m.bwd, m.store, m.dz, m.dy, m.scratchY, m.lossPart,
-                  m.gradPart};
+    void* ps[] = {m.params, m.adamM, m.adamV, m.grad, m.fwd, m.bwd, m.gradPart};
     for (void* p : ps)
         if (p) hipFree(p);
     m = MlpDev{};
 }
 
-double mlp_loss_host(const MlpDev& m, int n, hipStream_t st) {
-    int lb = (n + 255) / 256;
-    std::vector<double> part(lb);
-    hipMemcpyAsync(part.data(), m.lossPart, sizeof(double) * lb, hipMemcpyDeviceToHost, st);
-    hipStreamSynchronize(st);
+double mlp_loss_sum(const double* part, int n) {
     double s = 0.0;
-    for (double v : part) s += v;
+    for (int k = 0; k < mlp_slices(n); ++k) s += part[k];
     return n > 0 ? s / n : 0.0;
 }
 
@@ -623,20 +499,15 @@ constexpr int MLP_DEV_MAX = SPHGPU_MLP_DEVICE_MAX;
 constexpr size_t al256(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr size_t SCR_FWD = 0;
 constexpr size_t SCR_BWD = SCR_FWD + al256(16 * 64 * MLP_FWD_FRAGS);
-constexpr size_t SCR_STORE = SCR_BWD + al256(16 * 64 * MLP_BWD_FRAGS);
-constexpr size_t SCR_DZ = SCR_STORE + al256(sizeof(float) * MLP_STORE * (size_t)MLP_DEV_MAX);
-constexpr size_t SCR_DY = SCR_DZ + al256(sizeof(float) * MLP_STORE * (size_t)MLP_DEV_MAX);
-constexpr size_t SCR_Y = SCR_DY + al256(sizeof(float) * MLP_DEV_MAX);
-constexpr size_t SCR_LOSS = SCR_Y + al256(sizeof(float) * MLP_DEV_MAX);
-constexpr size_t SCR_GPART = SCR_LOSS + al256(sizeof(double) * (MLP_DEV_MAX / 256 + 2));
-constexpr size_t SCR_BYTES =
-    SCR_GPART + al256(sizeof(float) * 256 * MLP_WGRAD_TILES * ((MLP_DEV_MAX + MLP_WGRAD_SLICE - 1) / MLP_WGRAD_SLICE));
+constexpr size_t SCR_LOSS = SCR_BWD + al256(16 * 64 * MLP_BWD_FRAGS);
+constexpr size_t SCR_GPART = SCR_LOSS + al256(sizeof(double) * mlp_max_slices(MLP_DEV_MAX));
+constexpr size_t SCR_BYTES = SCR_GPART + al256(sizeof(float) * 256 * MLP_WGRAD_TILES * (size_t)mlp_max_slices(MLP_DEV_MAX));
 
 static __device__ __align__(256) unsigned char scratch[SCR_BYTES];
 
 namespace {
 // mean loss: the block partials summed in order by one thread (the order
-// mlp_loss_host sums them in), divided by n
+// mlp_loss_sum sums them in), divided by n
 __global__ void k_mlp_loss_final(const double* __restrict__ part, int parts, int n, double* __restrict__ out) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     double s = 0.0;
@@ -670,6 +541,8 @@ struct sphgpu_mlp {
     float* feat = nullptr;
     float* target = nullptr;
     float* y = nullptr;
+    sphgpu::HostRing ring;
+    std::vector<unsigned char> result;   // gradient and loss partial sums as read back
 };
 
 extern "C" int sphgpu_mlp_create(int capacity, unsigned long long seed, sphgpu_mlp** out) {
@@ -696,6 +569,7 @@ extern "C" void sphgpu_mlp_destroy(sphgpu_mlp* h) {
     if (h->feat) hipFree(h->feat);
     if (h->target) hipFree(h->target);
     if (h->y) hipFree(h->y);
+    h->ring.release();
     if (h->st) hipStreamDestroy(h->st);
     delete h;
 }
@@ -724,40 +598,52 @@ extern "C" int sphgpu_mlp_forward(sphgpu_mlp* h, long long n, const float* feat,
     if (!h || n < 0 || (n > 0 && (!feat || !out))) return SPHGPU_E_ARG;
     for (long long o = 0; o < n; o += h->m.cap) {
         int k = int(std::min<long long>(h->m.cap, n - o));
-        hipMemcpyAsync(h->feat, feat + 8 * o, sizeof(float) * 8 * k, hipMemcpyHostToDevice, h->st);
-        sphgpu::mlp_forward(h->m, h->feat, h->y, k, nullptr, h->st);
-        hipMemcpyAsync(out + o, h->y, sizeof(float) * k, hipMemcpyDeviceToHost, h->st);
+        if (h->ring.to_device(h->feat, feat + 8 * o, sizeof(float) * 8 * k, h->st) != hipSuccess) return SPHGPU_E_DEVICE;
+        sphgpu::mlp_forward(h->m, h->feat, h->y, k, h->st);
+        if (h->ring.to_host(out + o, h->y, sizeof(float) * k, h->st) != hipSuccess) return SPHGPU_E_DEVICE;
     }
     return hipStreamSynchronize(h->st) == hipSuccess && hipGetLastError() == hipSuccess ? SPHGPU_OK : SPHGPU_E_DEVICE;
+}
+
+// uploads a batch
+static int batch_to_device(sphgpu_mlp* h, int k, const float* feat, const float* target) {
+    return h->ring.to_device(h->feat, feat, sizeof(float) * 8 * k, h->st) == hipSuccess &&
+                   h->ring.to_device(h->target, target, sizeof(float) * k, h->st) == hipSuccess
+               ? SPHGPU_OK
+               : SPHGPU_E_DEVICE;
+}
+
+// gradient (where wanted) and loss of the last mlp_grad of k samples, with one transfer
+static int results_to_host(sphgpu_mlp* h, int k, float* grad, double* loss) {
+    const size_t bytes = sphgpu::mlp_result_bytes(k);
+    h->result.resize(bytes);
+    if (h->ring.to_host(h->result.data(), h->m.grad, bytes, h->st) != hipSuccess) return SPHGPU_E_DEVICE;
+    if (grad) std::memcpy(grad, h->result.data(), sizeof(float) * sphgpu::MLP_PARAMS);
+    if (loss)
+        *loss = sphgpu::mlp_loss_sum(reinterpret_cast<const double*>(h->result.data() + sphgpu::MLP_LOSS_OFFSET), k);
+    return hipGetLastError() == hipSuccess ? SPHGPU_OK : SPHGPU_E_DEVICE;
 }
 
 extern "C" int sphgpu_mlp_gradient(sphgpu_mlp* h, long long n, const float* feat, const float* target, float* grad,
                                    double* loss) {
     if (!h || n <= 0 || n > h->m.cap || !feat || !target || !grad) return SPHGPU_E_ARG;
-    int k = int(n);
-    hipMemcpyAsync(h->feat, feat, sizeof(float) * 8 * k, hipMemcpyHostToDevice, h->st);
-    hipMemcpyAsync(h->target, target, sizeof(float) * k, hipMemcpyHostToDevice, h->st);
+    const int k = int(n);
+    if (int rc = batch_to_device(h, k, feat, target)) return rc;
     sphgpu::mlp_grad(h->m, h->feat, h->target, k, h->st);
-    hipMemcpyAsync(grad, h->m.grad, sizeof(float) * sphgpu::MLP_PARAMS, hipMemcpyDeviceToHost, h->st);
-    double l = sphgpu::mlp_loss_host(h->m, k, h->st);
-    if (loss) *loss = l;
-    return hipGetLastError() == hipSuccess ? SPHGPU_OK : SPHGPU_E_DEVICE;
+    return results_to_host(h, k, grad, loss);
 }
 
 extern "C" int sphgpu_mlp_train(sphgpu_mlp* h, long long n, const float* feat, const float* target, int iters, float lr,
                                 double* loss) {
     if (!h || n <= 0 || n > h->m.cap || !feat || !target || iters < 0) return SPHGPU_E_ARG;
-    int k = int(n);
-    hipMemcpyAsync(h->feat, feat, sizeof(float) * 8 * k, hipMemcpyHostToDevice, h->st);
-    hipMemcpyAsync(h->target, target, sizeof(float) * k, hipMemcpyHostToDevice, h->st);
+    const int k = int(n);
+    if (int rc = batch_to_device(h, k, feat, target)) return rc;
     for (int it = 0; it < iters; ++it) {
         sphgpu::mlp_grad(h->m, h->feat, h->target, k, h->st);
         sphgpu::mlp_adam(h->m, lr, h->st);
     }
     sphgpu::mlp_grad(h->m, h->feat, h->target, k, h->st);
-    double l = sphgpu::mlp_loss_host(h->m, k, h->st);
-    if (loss) *loss = l;
-    return hipGetLastError() == hipSuccess ? SPHGPU_OK : SPHGPU_E_DEVICE;
+    return results_to_host(h, k, nullptr, loss);
 }
 
 extern "C" int sphgpu_mlp_gradient_device(const float* params, long long n, const float* feat, const float* target,
@@ -775,10 +661,6 @@ extern "C" int sphgpu_mlp_gradient_device(const float* params, long long n, cons
     m.grad = grad;
     m.fwd = base + SCR_FWD;
     m.bwd = base + SCR_BWD;
-    m.store = reinterpret_cast<float*>(base + SCR_STORE);
-    m.dz = reinterpret_cast<float*>(base + SCR_DZ);
-    m.dy = reinterpret_cast<float*>(base + SCR_DY);
-    m.scratchY = reinterpret_cast<float*>(base + SCR_Y);
     m.lossPart = reinterpret_cast<double*>(base + SCR_LOSS);
     m.gradPart = reinterpret_cast<float*>(base + SCR_GPART);
     m.overWeight = over_weight;
@@ -789,7 +671,7 @@ extern "C" int sphgpu_mlp_gradient_device(const float* params, long long n, cons
     // partials per block, gradient partials per slice
     mlp_pack(m, st);
     mlp_grad(m, feat, target, k, st);
-    hipLaunchKernelGGL(k_mlp_loss_final, dim3(1), dim3(64), 0, st, (const double*)m.lossPart, (k + 255) / 256, k,
+    hipLaunchKernelGGL(k_mlp_loss_final, dim3(1), dim3(64), 0, st, (const double*)m.lossPart, mlp_slices(k), k,
                        loss);
     return hipGetLastError() == hipSuccess ? SPHGPU_OK : SPHGPU_E_DEVICE;
 }

@@ -18,11 +18,16 @@ namespace sphgpu {
 // 188 KB 85 -> 16 us, 1.4 MB 139 -> 78 us, 12 MB 777 -> 411 us, 48 MB 4.85 ->
 // 1.44 ms; chunks of 1 and 4 MB were 25 and 4 % slower at 48 MB, eight
 // threads no faster than four.
+// To the device: hipMemcpy from a pageable buffer took 33 us for 64 KB, 47 to
+// 210 for 512 KB and 1.29 ms for 38 MB; through the ring 10, 21 and 0.97 (two
+// threads; one 1.30).
 struct HostRing {
     static constexpr int kSlots = 8;
     static constexpr size_t kChunk = size_t(2) << 20;
     static constexpr size_t kThreadedBytes = 2 * kChunk;
     static constexpr int kMaxThreads = 4;
+    static constexpr size_t kUpThreadedBytes = 4 * kChunk;
+    static constexpr int kUpThreads = 2;
 
     char* mem = nullptr;
     size_t cap = 0;                    // bytes pinned, at most kSlots * kChunk
@@ -31,10 +36,15 @@ struct HostRing {
     // device -> host; waits for everything queued on st before it, and
     // returns with `dst` complete
     hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t st);
+    // host -> device, queued on st; `src` may be changed once it returns.
+    // Every transfer of a ring goes through one stream.
+    hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t st);
     void release();
 
 private:
-    hipError_t reserve(size_t bytes);
+    size_t used = 0;                   // bytes from `mem` on that queued transfers to the device may still read
+    hipError_t reserve(size_t bytes, hipStream_t st);
+    hipError_t drain(hipStream_t st);  // waits for them
 };
 
 }  // namespace sphgpu
