@@ -70,22 +70,25 @@ __device__ __forceinline__ int cell_axis(float v, float mn, float inv, int n) {
     return min(max(c, 0), n - 1);
 }
 
-__global__ __launch_bounds__(256) void k_sf_keys(SurfParams S, const float4* __restrict__ x, int n,
+// x: the caller's positions, three floats a particle
+__global__ __launch_bounds__(256) void k_sf_keys(SurfParams S, const float* __restrict__ x, int n,
                                                  uint32_t* keys, uint32_t* vals) {
     int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    float4 p = x[i];
-    int cx = cell_axis(p.x, S.gmin[0], S.ginv, S.gnum[0]);
-    int cy = cell_axis(p.y, S.gmin[1], S.ginv, S.gnum[1]);
-    int cz = cell_axis(p.z, S.gmin[2], S.ginv, S.gnum[2]);
+    const size_t q = 3 * (size_t)i;
+    int cx = cell_axis(x[q], S.gmin[0], S.ginv, S.gnum[0]);
+    int cy = cell_axis(x[q + 1], S.gmin[1], S.ginv, S.gnum[1]);
+    int cz = cell_axis(x[q + 2], S.gmin[2], S.ginv, S.gnum[2]);
     keys[i] = (uint32_t)((cz * S.gnum[1] + cy) * S.gnum[0] + cx);
     vals[i] = (uint32_t)i;
 }
 
-__global__ __launch_bounds__(256) void k_sf_gather(const float4* __restrict__ x, const uint32_t* __restrict__ vals,
+__global__ __launch_bounds__(256) void k_sf_gather(const float* __restrict__ x, const uint32_t* __restrict__ vals,
                                                    int n, float4* xs) {
     int r = blockIdx.x * 256 + threadIdx.x;
-    if (r < n) xs[r] = x[vals[r]];
+    if (r >= n) return;
+    const size_t q = 3 * (size_t)vals[r];
+    xs[r] = make_float4(x[q], x[q + 1], x[q + 2], 0.0f);
 }
 
 __global__ __launch_bounds__(256) void k_sf_fill_i2(int2* p, int n) {
@@ -471,67 +474,171 @@ struct McTable {
 };
 __constant__ McTable c_mc;
 
-__device__ __forceinline__ int mc_case(const float* __restrict__ f, const int N[3], int ix, int iy, int iz, float iso,
-                                       float v[8]) {
-    const size_t sy = N[0], sz = (size_t)N[0] * N[1];
-    const size_t base = (size_t)iz * sz + (size_t)iy * sy + ix;
-    const int off[8][3] = {{0, 0, 0}, {0, 0, 1}, {0, 1, 1}, {0, 1, 0}, {1, 0, 0}, {1, 0, 1}, {1, 1, 1}, {1, 1, 0}};
-    int ci = 0;
-    for (int k = 0; k < 8; ++k) {
-        v[k] = f[base + off[k][0] + off[k][1] * sy + off[k][2] * sz];
-        if (v[k] < iso) ci |= 1 << k;
+// Marching cubes.  Cubes are numbered by their lowest node, n = ix + nx (iy +
+// ny iz) (the nodes of the upper faces have none), triangles lie in that
+// order.  A wave takes MC_UNIT nodes in chunks of 64: it loads the four node
+// rows of its cubes and ballots "below iso", so a cube's case is eight bits of
+// four masks and a chunk the surface does not cross is skipped after four
+// loads and compares.  One pass counts the triangles of each unit, the units
+// are scanned, and the second pass writes those of the units that have any, a
+// lane a vertex, so that the stores are contiguous.
+// Bound by the field's transfer to the device; of the kernels by reading the
+// field.  9.5 million nodes, 0.2 million triangles (MI355X): a case and a
+// count for each cube, a scan over all cubes and a thread a cube took 34 + 73
+// + 59 us.
+constexpr int MC_CHUNKS = 8;
+constexpr int MC_UNIT = 64 * MC_CHUNKS;
+
+struct McGrid {
+    int nx, ny, nz;
+    size_t nodes;
+    float iso, mn[3], cell;
+};
+
+struct McMasks {          // "below iso" of the nodes n.. of a chunk and of those one further
+    uint64_t lo[4], hi[4];   // rows (0, 0), (+y), (+z), (+y +z)
+};
+
+__device__ __forceinline__ size_t mc_row(const McGrid& G, int r) {
+    return (r & 1 ? (size_t)G.nx : 0) + (r & 2 ? (size_t)G.nx * G.ny : 0);
+}
+// node n + the offset of row r; beyond the grid, where no cube is, its last node
+__device__ __forceinline__ float mc_load(const McGrid& G, const float* __restrict__ f, size_t n, int r) {
+    const size_t k = n + mc_row(G, r);
+    return f[k < G.nodes ? k : G.nodes - 1];
+}
+
+// the masks of chunk k from all of a unit's loads
+__device__ __forceinline__ void mc_unit(const McGrid& G, const float* __restrict__ f, size_t base, int lane,
+                                        uint64_t (&m)[MC_CHUNKS][4], uint32_t& last) {
+    float v[MC_CHUNKS][4];
+#pragma unroll
+    for (int k = 0; k < MC_CHUNKS; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[k][r] = mc_load(G, f, base + 64 * k + lane, r);
+    // the node after the unit in each row: lanes 0..3
+    const float e = mc_load(G, f, base + MC_UNIT, lane & 3);
+#pragma unroll
+    for (int k = 0; k < MC_CHUNKS; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m[k][r] = __ballot(v[k][r] < G.iso);
+    last = (uint32_t)__ballot(e < G.iso) & 15u;
+}
+__device__ __forceinline__ bool mc_masks(const uint64_t (&m)[MC_CHUNKS][4], uint32_t last, int k, McMasks& M) {
+    uint64_t any = 0, all = ~0ull;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint64_t next = k + 1 < MC_CHUNKS ? m[k + 1 < MC_CHUNKS ? k + 1 : k][r] & 1ull : (last >> r) & 1u;
+        M.lo[r] = m[k][r];
+        M.hi[r] = (m[k][r] >> 1) | (next << 63);
+        any |= M.lo[r] | M.hi[r];
+        all &= M.lo[r] & M.hi[r];
     }
+    return any != 0 && all != ~0ull;
+}
+// The cube's case: bit k for corner k; the corners' (x, y, z) offsets in order
+// are (0,0,0) (0,0,1) (0,1,1) (0,1,0) (1,0,0) (1,0,1) (1,1,1) (1,1,0)
+__device__ __forceinline__ int mc_case(const McMasks& M, int lane) {
+    const int row[4] = {0, 2, 3, 1};
+    int ci = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ci |= (int((M.lo[row[k]] >> lane) & 1) << k) | (int((M.hi[row[k]] >> lane) & 1) << (4 + k));
     return ci;
 }
-
-__global__ __launch_bounds__(256) void k_mc_count(const float* __restrict__ f, int nx, int ny, int nz, float iso,
-                                                  uint32_t* __restrict__ count) {
-    const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t cubes = (size_t)(nx - 1) * (ny - 1) * (nz - 1);
-    if (c >= cubes) return;
-    const int ix = int(c % (nx - 1)), iy = int((c / (nx - 1)) % (ny - 1)), iz = int(c / ((size_t)(nx - 1) * (ny - 1)));
-    const int N[3] = {nx, ny, nz};
-    float v[8];
-    count[c] = c_mc.ntris[mc_case(f, N, ix, iy, iz, iso, v)];
+struct McNode {
+    int ix, iy, iz;
+};
+// position of node base + d (d < 2 MC_UNIT); base's own is wave-uniform
+__device__ __forceinline__ McNode mc_node(const McGrid& G, size_t base, uint32_t d) {
+    const uint64_t row = base / (uint32_t)G.nx;
+    const uint32_t x = uint32_t(base - row * (uint32_t)G.nx) + d, up = x / (uint32_t)G.nx;
+    const uint32_t y = uint32_t(row % (uint32_t)G.ny) + up, uz = y / (uint32_t)G.ny;
+    return McNode{int(x - up * (uint32_t)G.nx), int(y - uz * (uint32_t)G.ny), int(uint32_t(row / (uint32_t)G.ny) + uz)};
+}
+__device__ __forceinline__ bool mc_cube(const McGrid& G, const McNode& p) {
+    return p.ix < G.nx - 1 && p.iy < G.ny - 1 && p.iz < G.nz - 1;
 }
 
-__global__ __launch_bounds__(256) void k_mc_emit(const float* __restrict__ f, int nx, int ny, int nz, float iso,
-                                                 float mnx, float mny, float mnz, float cell,
+__global__ __launch_bounds__(256) void k_mc_count(McGrid G, const float* __restrict__ f, int units,
+                                                  uint32_t* __restrict__ count) {
+    const int u = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    if (u >= units) return;
+    const size_t base = (size_t)u * MC_UNIT;
+    uint64_t m[MC_CHUNKS][4];
+    uint32_t last, nt = 0;
+    mc_unit(G, f, base, lane, m, last);
+#pragma unroll
+    for (int k = 0; k < MC_CHUNKS; ++k) {
+        McMasks M;
+        if (!mc_masks(m, last, k, M)) continue;
+        const int ci = mc_case(M, lane);
+        if (ci != 0 && ci != 255 && mc_cube(G, mc_node(G, base, 64 * k + lane))) nt += c_mc.ntris[ci];
+    }
+    for (int o = 32; o > 0; o >>= 1) nt += __shfl_xor(nt, o, 64);
+    if (lane == 0) {
+        count[u] = nt;
+        if (u == units - 1) count[units] = 0;   // the total after the scan
+    }
+}
+
+__global__ __launch_bounds__(256) void k_mc_emit(McGrid G, const float* __restrict__ f, int units,
                                                  const uint32_t* __restrict__ offset, float* __restrict__ out,
                                                  long long cap) {
-    const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t cubes = (size_t)(nx - 1) * (ny - 1) * (nz - 1);
-    if (c >= cubes) return;
-    const int ix = int(c % (nx - 1)), iy = int((c / (nx - 1)) % (ny - 1)), iz = int(c / ((size_t)(nx - 1) * (ny - 1)));
-    const int N[3] = {nx, ny, nz};
-    float v[8];
-    const int ci = mc_case(f, N, ix, iy, iz, iso, v);
-    const int nt = c_mc.ntris[ci];
-    if (nt == 0) return;
+    __shared__ uint16_t sTri[4][64 * 5];   // a chunk's triangles: lane * 8 + number in the cube
+    __shared__ uint8_t sCase[4][64];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int u = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + w);
+    if (u >= units) return;
+    long long first = offset[u];
+    if (offset[u + 1] == (uint32_t)first) return;
+    const size_t base = (size_t)u * MC_UNIT;
+    uint64_t m[MC_CHUNKS][4];
+    uint32_t last;
+    mc_unit(G, f, base, lane, m, last);
     const int off[8][3] = {{0, 0, 0}, {0, 0, 1}, {0, 1, 1}, {0, 1, 0}, {1, 0, 0}, {1, 0, 1}, {1, 1, 1}, {1, 1, 0}};
-    const int E[12][2] = {{0, 1}, {1, 2}, {2, 3}, {3, 0}, {4, 5}, {5, 6}, {6, 7}, {7, 4}, {0, 4}, {1, 5}, {2, 6}, {3, 7}};
-    const long long first = offset[c];
-    for (int t = 0; t < nt; ++t) {
-        if (first + t >= cap) return;
-        for (int m = 0; m < 3; ++m) {
-            const int e = c_mc.tris[ci][3 * t + m];
-            int a = E[e][0], b = E[e][1];
-            // VertexInterp (marching_cubes.cpp:40-41) from the grid edge's
-            // lower node, with node positions from integer indices: the
-            // cubes on either side of an edge compute the same vertex
-            if (off[a][0] + off[a][1] + off[a][2] > off[b][0] + off[b][1] + off[b][2]) {
-                const int tmp = a; a = b; b = tmp;
-            }
-            const float mu = (iso - v[a]) / (v[b] - v[a]);
-            const float ax = mnx + float(ix + off[a][0]) * cell, ay = mny + float(iy + off[a][1]) * cell,
-                        az = mnz + float(iz + off[a][2]) * cell;
-            const float bx = mnx + float(ix + off[b][0]) * cell, by = mny + float(iy + off[b][1]) * cell,
-                        bz = mnz + float(iz + off[b][2]) * cell;
-            float* o = out + 9 * (first + t) + 3 * m;
+    // an edge's corners, the one with the lower node first
+    const int E[12][2] = {{0, 1}, {1, 2}, {3, 2}, {0, 3}, {4, 5}, {5, 6}, {7, 6}, {4, 7}, {0, 4}, {1, 5}, {2, 6}, {3, 7}};
+#pragma unroll
+    for (int k = 0; k < MC_CHUNKS; ++k) {
+        McMasks M;
+        if (!mc_masks(m, last, k, M)) continue;
+        const int ci = mc_case(M, lane);
+        int nt = 0;
+        if (ci != 0 && ci != 255 && mc_cube(G, mc_node(G, base, 64 * k + lane))) nt = c_mc.ntris[ci];
+        int incl = nt;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
+        }
+        const int total = __shfl(incl, 63, 64);
+        sCase[w][lane] = (uint8_t)ci;
+        for (int t = 0; t < nt; ++t) sTri[w][incl - nt + t] = uint16_t(lane * 8 + t);
+        wave_order();
+        for (int q = lane; q < 3 * total; q += 64) {
+            const int tri = q / 3, at = q - 3 * tri;
+            if (first + tri >= cap) break;
+            const int code = sTri[w][tri], owner = code >> 3;
+            const int e = c_mc.tris[sCase[w][owner]][3 * (code & 7) + at];
+            const McNode p = mc_node(G, base, 64 * k + owner);
+            // The edge's vertex by linear interpolation from its lower node,
+            // with node positions from integer indices: the cubes around an
+            // edge compute the same vertex (marching_cubes.cpp:40-41)
+            const int a = E[e][0], b = E[e][1];
+            const size_t n = base + 64 * k + owner, sy = G.nx, sz = (size_t)G.nx * G.ny;
+            const float va = f[n + off[a][0] + off[a][1] * sy + off[a][2] * sz];
+            const float vb = f[n + off[b][0] + off[b][1] * sy + off[b][2] * sz];
+            const float mu = (G.iso - va) / (vb - va);
+            const float ax = G.mn[0] + float(p.ix + off[a][0]) * G.cell, ay = G.mn[1] + float(p.iy + off[a][1]) * G.cell,
+                        az = G.mn[2] + float(p.iz + off[a][2]) * G.cell;
+            const float bx = G.mn[0] + float(p.ix + off[b][0]) * G.cell, by = G.mn[1] + float(p.iy + off[b][1]) * G.cell,
+                        bz = G.mn[2] + float(p.iz + off[b][2]) * G.cell;
+            float* o = out + 9 * (first + tri) + 3 * at;
             o[0] = ax + mu * (bx - ax);
             o[1] = ay + mu * (by - ay);
             o[2] = az + mu * (bz - az);
         }
+        wave_order();
+        first += total;
     }
 }
 
@@ -545,19 +652,21 @@ struct sphgpu_surfacer {
     hipStream_t st = nullptr;
     float* field = nullptr;
     int cap = 0;
-    float4 *x = nullptr, *xs = nullptr;
+    float* x = nullptr;            // positions as given
+    float4* xs = nullptr;          // by cell
     uint32_t *keys = nullptr, *vals = nullptr;
     int2* ranges = nullptr;
     SurfRec* rec = nullptr;
     SurfBox* box = nullptr;
     int* far = nullptr;            // far particles' indices, then their number at [cap]
-    HostRing ring;                 // readback staging
+    HostRing ring;                 // staging of transfers
     void* sortMem = nullptr;
     SortScratch sort{};
     int keyBits = 1;
     uint32_t* mcCount = nullptr;
     uint32_t* mcTmp = nullptr;
-    size_t mcCap = 0;
+    float* mcOut = nullptr;        // triangles
+    long long mcOutCap = 0;
     int nrec = 0;
     std::string err;
 };
@@ -586,9 +695,9 @@ int ensure_particles(sphgpu_surfacer* s, int n) {
     (void)hipFree(s->rec); (void)hipFree(s->box); (void)hipFree(s->far); (void)hipFree(s->sortMem);
     s->cap = 0;
     s->box = nullptr; s->far = nullptr;
-    s->x = s->xs = nullptr; s->keys = s->vals = nullptr; s->rec = nullptr; s->sortMem = nullptr;
+    s->x = nullptr; s->xs = nullptr; s->keys = s->vals = nullptr; s->rec = nullptr; s->sortMem = nullptr;
     const int cap = std::max(n, 1024);
-    SCHECK(s, hipMalloc(&s->x, sizeof(float4) * cap));
+    SCHECK(s, hipMalloc(&s->x, 3 * sizeof(float) * cap));
     SCHECK(s, hipMalloc(&s->xs, sizeof(float4) * cap));
     SCHECK(s, hipMalloc(&s->keys, sizeof(uint32_t) * cap));
     SCHECK(s, hipMalloc(&s->vals, sizeof(uint32_t) * cap));
@@ -629,22 +738,25 @@ int field_of(sphgpu_surfacer* s, long long n, const float* xyz, bool aniso) {
     if (n < 0 || (n > 0 && !xyz)) return sfail(s, SPHGPU_E_ARG, "bad particle array");
     if (n > (1 << 30)) return sfail(s, SPHGPU_E_CAPACITY, "too many particles");
     if (int rc = ensure_particles(s, int(n))) return rc;
-    std::vector<float4> h(static_cast<size_t>(n));
-    for (long long i = 0; i < n; ++i) {
-        h[i] = make_float4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], 0.0f);
-        if (!std::isfinite(h[i].x) || !std::isfinite(h[i].y) || !std::isfinite(h[i].z))
-            return sfail(s, SPHGPU_E_ARG, "non-finite position %lld", i);
+    for (long long i = 0; i < n;) {   // blocks of particles, without a branch for each
+        const long long end = std::min(n, i + 1024);
+        bool ok = true;
+        for (long long k = 3 * i; k < 3 * end; ++k) ok &= std::isfinite(xyz[k]);
+        for (; !ok && i < end; ++i)
+            if (!std::isfinite(xyz[3 * i]) || !std::isfinite(xyz[3 * i + 1]) || !std::isfinite(xyz[3 * i + 2]))
+                return sfail(s, SPHGPU_E_ARG, "non-finite position %lld", i);
+        i = end;
     }
-    SCHECK(s, hipMemcpyAsync(s->x, h.data(), sizeof(float4) * n, hipMemcpyHostToDevice, s->st));
+    SCHECK(s, s->ring.to_device(s->x, xyz, 3 * sizeof(float) * size_t(n), s->st));
     s->nrec = int(n);
     const int blocks = int((n + 255) / 256);
     int* const nfar = s->far + s->cap;
     SCHECK(s, hipMemsetAsync(nfar, 0, sizeof(int), s->st));
     if (n > 0) {
-        hipLaunchKernelGGL(k_sf_keys, dim3(blocks), dim3(256), 0, s->st, s->S, (const float4*)s->x, int(n), s->keys,
+        hipLaunchKernelGGL(k_sf_keys, dim3(blocks), dim3(256), 0, s->st, s->S, (const float*)s->x, int(n), s->keys,
                            s->vals);
         radix_sort_pairs(s->keys, s->vals, int(n), s->keyBits, s->sort, s->st);
-        hipLaunchKernelGGL(k_sf_gather, dim3(blocks), dim3(256), 0, s->st, (const float4*)s->x,
+        hipLaunchKernelGGL(k_sf_gather, dim3(blocks), dim3(256), 0, s->st, (const float*)s->x,
                            (const uint32_t*)s->vals, int(n), s->xs);
     }
     hipLaunchKernelGGL(k_sf_fill_i2, dim3(int((s->ncells + 255) / 256)), dim3(256), 0, s->st, s->ranges, int(s->ncells));
@@ -770,7 +882,7 @@ void sphgpu_surfacer_destroy(sphgpu_surfacer* s) {
     (void)hipFree(s->field); (void)hipFree(s->ranges); (void)hipFree(s->x); (void)hipFree(s->xs);
     (void)hipFree(s->keys); (void)hipFree(s->vals); (void)hipFree(s->rec); (void)hipFree(s->box); (void)hipFree(s->far); (void)hipFree(s->sortMem);
     s->ring.release();
-    (void)hipFree(s->mcCount); (void)hipFree(s->mcTmp);
+    (void)hipFree(s->mcCount); (void)hipFree(s->mcTmp); (void)hipFree(s->mcOut);
     if (s->st) (void)hipStreamDestroy(s->st);
     delete s;
 }
@@ -834,7 +946,7 @@ int sphgpu_surfacer_get_field(sphgpu_surfacer* s, float* out) {
 int sphgpu_surfacer_set_field(sphgpu_surfacer* s, const float* in) {
     if (!s || !in) return SPHGPU_E_ARG;
     if (!s->st) return sfail(s, SPHGPU_E_DEVICE, "no gfx9 HIP device available");
-    SCHECK(s, hipMemcpyAsync(s->field, in, sizeof(float) * s->nfield, hipMemcpyHostToDevice, s->st));
+    SCHECK(s, s->ring.to_device(s->field, in, sizeof(float) * s->nfield, s->st));
     SCHECK(s, hipStreamSynchronize(s->st));
     return SPHGPU_OK;
 }
@@ -848,33 +960,42 @@ int sphgpu_surfacer_marching_cubes(sphgpu_surfacer* s, float iso, float* tris, l
     if (nx < 2 || ny < 2 || nz < 2) return SPHGPU_OK;
     const size_t cubes = size_t(nx - 1) * (ny - 1) * (nz - 1);
     if (cubes >= (size_t(1) << 31)) return sfail(s, SPHGPU_E_CAPACITY, "too many cubes");
-    if (s->mcCap < cubes) {
-        (void)hipFree(s->mcCount); (void)hipFree(s->mcTmp);
-        s->mcCount = s->mcTmp = nullptr;
-        SCHECK(s, hipMalloc(&s->mcCount, sizeof(uint32_t) * (cubes + 1)));
-        SCHECK(s, hipMalloc(&s->mcTmp, sizeof(uint32_t) * (size_t)scan_tmp_words(int(cubes + 1))));
-        s->mcCap = cubes;
+    const size_t nodes = size_t(nx) * ny * nz;
+    // (units: fewer than 2^31, there being at most 8 nodes to a cube)
+    const int units = int((nodes + MC_UNIT - 1) / MC_UNIT);
+    if (!s->mcTmp) {   // the grid is the object's: its size does not change
+        if (!s->mcCount) SCHECK(s, hipMalloc(&s->mcCount, sizeof(uint32_t) * (size_t(units) + 1)));
+        SCHECK(s, hipMalloc(&s->mcTmp, sizeof(uint32_t) * (size_t)scan_tmp_words(units + 1)));
     }
-    const unsigned blocks = unsigned((cubes + 255) / 256);
-    hipLaunchKernelGGL(k_mc_count, dim3(blocks), dim3(256), 0, s->st, (const float*)s->field, nx, ny, nz, iso,
-                       s->mcCount);
-    SCHECK(s, hipMemsetAsync(s->mcCount + cubes, 0, sizeof(uint32_t), s->st));
-    exclusive_scan_u32(s->mcCount, int(cubes + 1), s->mcTmp, s->st);
+    McGrid G{nx, ny, nz, nodes, iso, {float(s->fmin[0]), float(s->fmin[1]), float(s->fmin[2])}, float(s->cell)};
+    const unsigned blocks = unsigned((units + 3) / 4);
+    hipLaunchKernelGGL(k_mc_count, dim3(blocks), dim3(256), 0, s->st, G, (const float*)s->field, units, s->mcCount);
+    exclusive_scan_u32(s->mcCount, units + 1, s->mcTmp, s->st);
     uint32_t total = 0;
-    SCHECK(s, hipMemcpyAsync(&total, s->mcCount + cubes, sizeof(uint32_t), hipMemcpyDeviceToHost, s->st));
-    SCHECK(s, hipStreamSynchronize(s->st));
+    SCHECK(s, s->ring.to_host(&total, s->mcCount + units, sizeof(uint32_t), s->st));
     *ntris = total;
     if (!tris || total == 0) return SPHGPU_OK;
     const long long keep = std::min<long long>(cap, total);
-    float* dout = nullptr;
-    SCHECK(s, hipMalloc(&dout, sizeof(float) * 9 * std::max<long long>(keep, 1)));
-    hipLaunchKernelGGL(k_mc_emit, dim3(blocks), dim3(256), 0, s->st, (const float*)s->field, nx, ny, nz, iso,
-                       float(s->fmin[0]), float(s->fmin[1]), float(s->fmin[2]), float(s->cell),
-                       (const uint32_t*)s->mcCount, dout, keep);
-    hipError_t e1 = hipMemcpyAsync(tris, dout, sizeof(float) * 9 * keep, hipMemcpyDeviceToHost, s->st);
-    hipError_t e2 = hipStreamSynchronize(s->st);
-    (void)hipFree(dout);
-    if (e1 != hipSuccess || e2 != hipSuccess) return sfail(s, SPHGPU_E_DEVICE, "marching cubes readback failed");
+    if (keep > 0) {
+        if (s->mcOutCap < keep) {
+            (void)hipFree(s->mcOut);
+            s->mcOut = nullptr;
+            s->mcOutCap = 0;
+            long long room = keep + keep / 4;   // for a surface that grows from call to call
+            if (hipMalloc(&s->mcOut, sizeof(float) * 9 * room) != hipSuccess) {
+                (void)hipGetLastError();
+                s->mcOut = nullptr;
+                room = keep;
+                SCHECK(s, hipMalloc(&s->mcOut, sizeof(float) * 9 * room));
+            }
+            s->mcOutCap = room;
+        }
+        hipLaunchKernelGGL(k_mc_emit, dim3(blocks), dim3(256), 0, s->st, G, (const float*)s->field, units,
+                           (const uint32_t*)s->mcCount, s->mcOut, keep);
+        if (s->ring.to_host(tris, s->mcOut, sizeof(float) * 9 * keep, s->st) != hipSuccess ||
+            hipGetLastError() != hipSuccess)
+            return sfail(s, SPHGPU_E_DEVICE, "marching cubes readback failed");
+    }
     if (keep < (long long)total) return sfail(s, SPHGPU_E_CAPACITY, "%u triangles, room for %lld", total, cap);
     return SPHGPU_OK;
 }
