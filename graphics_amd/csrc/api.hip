@@ -493,7 +493,7 @@ float time_launches(sphgpu_handle* h, const std::function<void()>& f, const std:
 }
 
 // Per solver-loop pass: stage the tile's neighbour window in LDS (fewer
-// cache-line lookups, but 48-72 KB of LDS per block: two or three blocks per
+// cache-line lookups, but 48-76 KB of LDS per block: two or three blocks per
 // CU) or gather each neighbour per lane (five waves per SIMD).  Each pass is
 // timed both ways on the scene's lists (best of two single launches: six
 // forms, twelve launches a pass, about 4 ms per pass at 4M particles, so the

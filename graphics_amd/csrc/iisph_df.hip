@@ -69,13 +69,13 @@ __global__ __launch_bounds__(256) void k_idf_mass(Dev D) {
 // fluid density and alpha (IISph.cpp:143-200); publishes rho in v.w for the
 // non-pressure acceleration pass
 __global__ __launch_bounds__(256) void k_idf_prepare_fluid(Dev D) {
-    const Slot s = slot_nb(D, false);
+    float4 pa;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i]; });
     if (!s.live) return;
     const int i = s.i;
-    const float4 pa = D.x[i];
     const int ph = phase_of(pa);
     const float ma = D.pm[i], resta = rest_of(D, i, ph);
-    const int c = D.cnt[i];
+    const int c = s.c;
     Kahan rho;
     rho.init(ma * D.W0);
     float a1x = 0.f, a1y = 0.f, a1z = 0.f, a2 = 0.f;
@@ -269,7 +269,8 @@ __global__ __launch_bounds__(256) void k_idf_kappa(Dev D, int mode, int tiles) {
         return;
     }
     __shared__ double lds[4];
-    const Slot s = slot_nb(D, true, tiles);
+    float4 pa, va;
+    const Slot s = slot_nb<1>(D, true, [&](int i) { pa = D.x[i], va = D.vs[i]; }, tiles);
     if (!D.active[s.scene]) {   // uniform: a converged scene's tiles contribute nothing
         if (threadIdx.x == 0) D.partial[2 * s.tile] = 0.0;
         return;
@@ -277,10 +278,9 @@ __global__ __launch_bounds__(256) void k_idf_kappa(Dev D, int mode, int tiles) {
     double contrib = 0.0;
     if (s.live) {
         const int i = s.i;
-        const float4 pa = D.x[i], va = D.vs[i];
         const int ph = phase_of(pa);
         const float ma = va.w, rest = rest_of(D, i, ph);
-        const int c = D.cnt[i];
+        const int c = s.c;
         const bool adjust = mode == 0 && D.adjustDensity;
         float sf = 0.0f, sb = 0.0f;
         each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.vs[j]}; }, [&](int, Rec2 rec) {
@@ -316,12 +316,12 @@ __global__ __launch_bounds__(256) void k_idf_kappa(Dev D, int mode, int tiles) {
 //              + sum_b boundaryDensity V_b (k_a/rho_a + k_b/rho_b) gradW)
 __global__ __launch_bounds__(256) void k_idf_velocity(Dev D) {
     loop_test(D);   // on the stiffness pass's partial sums
-    const Slot s = slot_nb(D, true);
+    float4 pa;
+    const Slot s = slot_nb<1>(D, true, [&](int i) { pa = D.xk[i]; });
     if (!s.live) return;
     const int i = s.i;
-    const float4 pa = D.xk[i];
     const float ka = pa.w;
-    const int c = D.cnt[i];
+    const int c = s.c;
     float fx = 0.f, fy = 0.f, fz = 0.f, bx = 0.f, by = 0.f, bz = 0.f;
     each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return RecM{D.xk[j], D.pm[j]}; }, [&](int, RecM rec) {
         const Pair p = pair_of(D, pa, rec.x);

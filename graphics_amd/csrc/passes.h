@@ -12,17 +12,20 @@ struct Slot {
     int i, tile, scene;
     bool live;
     bool packed;   // the tile's neighbour lists are in the packed 16-bit form
+    int c;         // the particle's count word (slot_nb; 0: not live)
 };
 
-// blocks: the workgroups that take tiles (0: the whole grid)
+// blocks: the workgroups that take tiles (0: the whole grid); K: lanes a particle
+template <int K = 1>
 __device__ __forceinline__ Slot slot_of(const Dev& D, bool gated, int blocks = 0) {
     Slot s;
     s.tile = tile_of_block(D.tileMap, blocks ? blocks : (int)gridDim.x);
-    s.i = s.tile * TILE + threadIdx.x;
+    s.i = s.tile * TILE + (int)threadIdx.x / K;
     s.scene = D.tileScene[s.tile];
-    s.live = (int)threadIdx.x < D.tileValid[s.tile];
+    s.live = (int)threadIdx.x / K < D.tileValid[s.tile];
     if (gated) s.live = s.live && D.active[s.scene] != 0;
     s.packed = false;
+    s.c = 0;
     return s;
 }
 
@@ -33,20 +36,44 @@ __shared__ int g_nbtab[NB16_TAB];
 __shared__ int g_winoff[32];
 
 // slot_of for kernels that read neighbour lists: every thread of the block
-// calls it before any returns (it stages the tile's tables in LDS, both with
-// one round trip).  A gated block whose scene has converged loads nothing
-// (its particles are not live): solver iterations launched past convergence
-// return at once.
-__device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated, int blocks = 0) {
-    Slot s = slot_of(D, gated, blocks);
-    if (gated && !D.active[s.scene]) return s;   // uniform per block
-    if (threadIdx.x < NB16_TAB) g_nbtab[threadIdx.x] = D.nbTab[(size_t)s.tile * NB16_TAB + threadIdx.x];
-    else if (threadIdx.x < NB16_TAB + 32)
-        g_winoff[threadIdx.x - NB16_TAB] = D.nbWin[(size_t)s.tile * 32 + threadIdx.x - NB16_TAB];
+// calls it before any returns (it stages the tile's tables in LDS).  What
+// depends on the tile or the slot alone (the tables, the count word and what
+// `own`(i) loads) is requested before the scene's state is known, so that a
+// pass starts with two dependent round trips to memory instead of five.  A
+// gated block whose scene has converged has no live particles and returns at
+// once: solver iterations launched past convergence cost little.
+template <int K = 1, class OWN>
+__device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated, OWN&& own, int blocks = 0) {
+    Slot s;
+    s.tile = tile_of_block(D.tileMap, blocks ? blocks : (int)gridDim.x);
+    s.i = s.tile * TILE + (int)threadIdx.x / K;
+    const int t = threadIdx.x;
+    int tab = D.nbTab[(size_t)s.tile * NB16_TAB + (t & (NB16_TAB - 1))];
+    int win = D.nbWin[(size_t)s.tile * 32 + (t & 31)];
+    const int c = D.cnt[s.i];
+    own(s.i);
+    s.scene = D.tileScene[s.tile];
+    const int valid = D.tileValid[s.tile];
+    const bool on = !gated || D.active[s.scene] != 0;
+    s.live = on && (int)threadIdx.x / K < valid;
+    s.packed = false;
+    s.c = s.live ? c : 0;
+    asm volatile("" : "+v"(tab), "+v"(win));   // (else the loads are moved behind the branch)
+    if (!on) return s;   // uniform per block
+    if (t < NB16_TAB) g_nbtab[t] = tab;
+    else if (t < NB16_TAB + 32) g_winoff[t - NB16_TAB] = win;
     __syncthreads();
     s.packed = __builtin_amdgcn_readfirstlane(g_nbtab[NB16_FLAG]) != 0;
     return s;
 }
+__device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated, int blocks = 0) {
+    return slot_nb<1>(D, gated, [](int) {}, blocks);
+}
+
+// mass, rest density and viscosity of a phase; one phase: no load that waits for it
+__device__ __forceinline__ float mass_of(const Dev& D, int ph) { return D.nphases > 1 ? D.mass[ph] : D.mass[0]; }
+__device__ __forceinline__ float visc_of(const Dev& D, int ph) { return D.nphases > 1 ? D.visc[ph] : D.visc[0]; }
+__device__ __forceinline__ float rho0_of(const Dev& D, int ph) { return D.nphases > 1 ? D.rho0[ph] : D.rho0[0]; }
 
 // A list group is read once per pass.  Where the lists and records together
 // fit the last-level cache the plain load lets the next pass find the list
@@ -159,12 +186,180 @@ __device__ __forceinline__ void each_boundary_lu(const Dev& D, const Slot& s, in
     else each_in_list_lu(D.nbB, D.ncap, s.i, nb, nt, load, use);
 }
 
+// ---- K lanes a particle ---------------------------------------------------
+// K = 2 or 4 neighbouring lanes of a wave share a particle: of every eight
+// list entries lane h gathers and evaluates entries h * 8/K .. + 8/K - 1 (term),
+// then lane 0 adds the terms of the eight in list order (add), taking the
+// others' with a DPP quad permute, so its sums, the particle's, have the same
+// bits as those of one lane a particle (the other lanes' sums are not used).
+template <int K>
+struct Lanes {
+    static_assert(K == 2 || K == 4, "two or four lanes a particle");
+    static constexpr int E = 8 / K;   // entries of a group a lane owns
+};
+// v of lane O of the particle's K
+template <int K, int O, class T>
+__device__ __forceinline__ T lane_term(const T& v) {
+    if constexpr (O == 0) {
+        return v;   // (lane 0's sum is the particle's)
+    } else {
+        constexpr int ctrl = K == 2 ? 0xF5 : O * 0x55;
+        constexpr int N = sizeof(T) / 4;
+        int w[N];
+        __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+        for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_mov_dpp(w[k], ctrl, 0xf, 0xf, true);
+        T r;
+        __builtin_memcpy(&r, w, sizeof(T));
+        return r;
+    }
+}
+// adds a group's terms in order: entries 0..3, and 4..7 where they are listed
+template <int K, class T, class AD>
+__device__ __forceinline__ void add_group(const T (&t)[Lanes<K>::E], bool second, AD&& add) {
+    constexpr int E = Lanes<K>::E;
+    add(lane_term<K, 0 / E>(t[0 % E]));
+    add(lane_term<K, 1 / E>(t[1 % E]));
+    add(lane_term<K, 2 / E>(t[2 % E]));
+    add(lane_term<K, 3 / E>(t[3 % E]));
+    if (second) {
+        add(lane_term<K, 4 / E>(t[4 % E]));
+        add(lane_term<K, 5 / E>(t[5 % E]));
+        add(lane_term<K, 6 / E>(t[6 % E]));
+        add(lane_term<K, 7 / E>(t[7 % E]));
+    }
+}
+
+// a lane's 8/K packed entries of a group: 4/K words
+template <int K>
+struct Words {
+    unsigned w[4 / K];
+};
+template <int K>
+__device__ __forceinline__ Words<K> ld_words(const int4* group, int h, bool nt) {
+    Words<K> r;
+    const unsigned* p = reinterpret_cast<const unsigned*>(group) + h * (4 / K);
+    if constexpr (K == 2) {
+        typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
+        const v2u_t* q = reinterpret_cast<const v2u_t*>(p);
+        const v2u_t v = nt ? __builtin_nontemporal_load(q) : *q;
+        r.w[0] = v.x;
+        r.w[1] = v.y;
+    } else {
+        r.w[0] = nt ? __builtin_nontemporal_load(p) : *p;
+    }
+    return r;
+}
+// entry e of the words
+template <int K>
+__device__ __forceinline__ unsigned word_entry(const Words<K>& w, int e) {
+    return (w.w[e >> 1] >> (16 * (e & 1))) & 0xffffu;
+}
+
+// each_in_list16_lu with K lanes a particle
+template <int K, int TOFF, class LD, class TM, class AD>
+__device__ __forceinline__ void each_in_list16_lanes(const int4* __restrict__ list, int ncap, int i, int h, int n,
+                                                     int padj, bool nt, LD&& load, TM&& term, AD&& add) {
+    constexpr int E = Lanes<K>::E;
+    const int4* __restrict__ col = list + i;
+    const int ng = (n + 7) >> 3;
+    if (ng <= 0) return;
+    const int n4 = (n + 3) & ~3;
+    Words<K> cur = ld_words<K>(&col[0], h, nt);
+    for (int g = 0; g < ng; ++g) {
+        const bool second = 8 * g + 4 < n4;
+        int j[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            const unsigned e = word_entry<K>(cur, k);
+            const int jj = g_nbtab[TOFF + (e >> NB16_OFF_BITS)] + (int)e;
+            j[k] = (second || h * E + k < 4) ? jj : padj;
+        }
+        decltype(load(0)) r[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) r[k] = load(j[k]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (g + 1 < ng) cur = ld_words<K>(&col[(size_t)(g + 1) * ncap], h, nt);
+        __builtin_amdgcn_sched_barrier(0);
+        decltype(term(0, r[0])) t[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) t[k] = term(j[k], r[k]);
+        add_group<K>(t, second, add);
+    }
+}
+
+// the same for 32-bit lists (groups of four, all listed or padding): lane h
+// owns entries h * 4/K .. of each group
+template <int K, class LD, class TM, class AD>
+__device__ __forceinline__ void each_in_list_lanes(const int* __restrict__ list, int ncap, int i, int h, int n,
+                                                   bool nt, LD&& load, TM&& term, AD&& add) {
+    constexpr int E = Lanes<K>::E;
+    const int4* __restrict__ col = reinterpret_cast<const int4*>(list) + i;
+    const int ng = (n + 3) >> 2;
+    // eight entries a turn: two groups, the lane's entries all in one of them
+    for (int g = 0; g < ng; g += 2) {
+        const bool second = g + 1 < ng;
+        const bool mine = second || h * E < 4;
+        const int4 v = ld_group(&col[(size_t)(mine ? g + (h * E) / 4 : g) * ncap], nt);
+        const int w[4] = {v.x, v.y, v.z, v.w};
+        decltype(load(0)) r[E];
+        int j[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            j[k] = K == 2 ? w[k] : ((h & 1) ? w[2 + k] : w[k]);
+            r[k] = load(j[k]);
+        }
+        decltype(term(0, r[0])) t[E];
+#pragma unroll
+        for (int k = 0; k < E; ++k) t[k] = term(j[k], r[k]);
+        add_group<K>(t, second, add);
+    }
+}
+
+// The neighbour loops of a particle: load(j) gathers the record of neighbour
+// j, term(j, r) is the pair's term, add(t) adds it.  K = 1: one lane a
+// particle, W records a batch.
+template <int K, int W, class LD, class TM, class AD>
+__device__ __forceinline__ void each_fluid(const Dev& D, const Slot& s, int h, int nf, LD&& load, TM&& term, AD&& add) {
+    if constexpr (K == 1) {
+        each_fluid_lu<W>(D, s, nf, load, [&](int j, const decltype(load(0))& r) { add(term(j, r)); });
+    } else {
+        const bool nt = __builtin_amdgcn_readfirstlane(D.listNT) != 0;
+        if (s.packed) each_in_list16_lanes<K, 0>(D.nbF16, D.ncap, s.i, h, nf, s.i, nt, load, term, add);
+        else each_in_list_lanes<K>(D.nbF, D.ncap, s.i, h, nf, nt, load, term, add);
+    }
+}
+template <int K, int W, class LD, class TM, class AD>
+__device__ __forceinline__ void each_boundary(const Dev& D, const Slot& s, int h, int nb, LD&& load, TM&& term,
+                                              AD&& add) {
+    if constexpr (K == 1) {
+        each_boundary_lu<W>(D, s, nb, load, [&](int j, const decltype(load(0))& r) { add(term(j, r)); });
+    } else {
+        const bool nt = __builtin_amdgcn_readfirstlane(D.listNT) != 0;
+        if (s.packed) each_in_list16_lanes<K, 32>(D.nbB16, D.ncap, s.i, h, nb, D.nb, nt, load, term, add);
+        else each_in_list_lanes<K>(D.nbB, D.ncap, s.i, h, nb, nt, load, term, add);
+    }
+}
+
 // two gather records of one neighbour
 struct Rec2 {
     float4 a, b;
 };
 
 __device__ __forceinline__ int phase_of(float4 x) { return (int)x.w; }
+
+// the tile's sum of v, each of its particles' K lanes holding the particle's
+// own: in the order of one lane a particle
+template <int K>
+__device__ __forceinline__ double tile_sum(double v, double* part, double* lds) {
+    const int t = threadIdx.x;
+    if constexpr (K > 1) {
+        if (t % K == 0) part[t / K] = v;
+        __syncthreads();
+        v = t < TILE ? part[t] : 0.0;
+    }
+    return block_sum_256(v, lds);
+}
 
 __device__ __forceinline__ void write_partial(const Dev& D, int tile, int q, double v, double* lds) {
     double t = block_sum_256(v, lds);
@@ -196,7 +391,7 @@ __device__ __forceinline__ T* on_host(const Dev& D, const T* p) {
 // done).  Every thread of the block calls it.
 __device__ __forceinline__ void scene_reduce_block(const Dev& D, int sc, int mode, float tol, int minIt, int cap,
                                                    int* out) {
-    __shared__ double lds[4];
+    __shared__ double lds[16];
     if (!D.active[sc]) {   // uniform per block
         if (threadIdx.x == 0 && out != D.active) {
             out[sc] = 0;
@@ -205,12 +400,13 @@ __device__ __forceinline__ void scene_reduce_block(const Dev& D, int sc, int mod
         return;
     }
     int t0 = D.scenePadStart[sc] / TILE, t1 = D.scenePadStart[sc + 1] / TILE;
-    __shared__ float ldsf[4];
+    __shared__ float ldsf[16];
     double s = 0.0;
     float mx = 0.0f;
     // each thread sums tiles t0 + tid, + 256, + 512, ... in that order; the
-    // loads of eight of them are issued together
-    for (int t = t0 + threadIdx.x; t < t1; t += 256 * 8) {
+    // loads of eight of them are issued together (a larger block's further
+    // threads have no part)
+    for (int t = threadIdx.x < 256 ? t0 + (int)threadIdx.x : t1; t < t1; t += 256 * 8) {
         double v[8];
         float w[8];
 #pragma unroll

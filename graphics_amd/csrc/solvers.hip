@@ -34,81 +34,87 @@ __device__ __forceinline__ int win_layout(const Dev& D, const Slot& s, int bit) 
     return n <= WIN_MAX ? n : 0;
 }
 
-// sorted particle index of window record k (0 <= k < window size): the slot
-// holding k is the largest s with g_winoff[s] <= k (empty slots share their
-// offset with the next one)
-__device__ __forceinline__ int win_particle(int k) {
-    int s = 0;
-#pragma unroll
-    for (int b = 16; b > 0; b >>= 1)
-        if (g_winoff[s + b] <= k) s += b;
-    return g_nbtab[s] + (s << NB16_OFF_BITS) + (k - g_winoff[s]);
-}
+// Lanes a particle of the window builds.
+constexpr int WIN_LANES = 2;
 
 // Stages the window: load(j) reads what a record needs from particle j,
-// store(k, r) writes it to window record k.  A window holds at most
-// WIN_MAX = 12 x 256 records, so each thread requests all of its records
-// before it stores the first.
-template <class LD, class ST>
-__device__ __forceinline__ void win_stage(int n, LD&& load, ST&& store) {
-    constexpr int DEPTH = WIN_MAX / 256;
+// store(k, r) writes it to window record k.  A wave copies chunks of up to 64
+// consecutive records of one slot run; each lane holds one slot, so the slot of
+// a chunk is a ballot and its run three lane reads, and a record costs one
+// addition (a search of the slot for each record took a third of the pass's
+// instructions and two fifths of its LDS reads).  All of a wave's chunks are
+// requested before the first is stored.
+// A window of WIN_MAX records in up to 9 * NB16_ROWS runs has at most WIN_MAX /
+// 64 chunks and one partial one a run.
+constexpr int WIN_CHUNKS = WIN_MAX / 64 + 9 * NB16_ROWS;
+template <int WAVES, class LD, class ST>
+__device__ __forceinline__ void win_stage(LD&& load, ST&& store) {
+    constexpr int DEPTH = (WIN_CHUNKS + WAVES - 1) / WAVES;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int off = g_winoff[lane & 31], len = lane < 31 ? g_winoff[(lane + 1) & 31] - off : 0;
+    const int src = g_nbtab[lane & 31] + ((lane & 31) << NB16_OFF_BITS);
+    int end = (len + 63) >> 6;   // chunks up to and with this slot
+    for (int o = 1; o < 32; o <<= 1) {
+        const int y = __shfl_up(end, o, 64);
+        if (lane >= o) end += y;
+    }
+    const int chunks = __builtin_amdgcn_readlane(end, 31);
+    const int first = end - ((len + 63) >> 6);
     decltype(load(0)) r[DEPTH];
+    int at[DEPTH];
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) {
-        const int k = threadIdx.x + 256 * u;
-        if (k < n) r[u] = load(win_particle(k));
+        const int q = wave + WAVES * u;
+        at[u] = -1;
+        if (q < chunks) {   // uniform
+            const int s = __popcll(__ballot(lane < 31 && end <= q));
+            const int p = 64 * (q - __builtin_amdgcn_readlane(first, s)) + lane;
+            if (p < __builtin_amdgcn_readlane(len, s)) {
+                r[u] = load(__builtin_amdgcn_readlane(src, s) + p);
+                at[u] = __builtin_amdgcn_readlane(off, s) + p;
+            }
+        }
     }
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u) {
-        const int k = threadIdx.x + 256 * u;
-        if (k < n) store(k, r[u]);
-    }
+    for (int u = 0; u < DEPTH; ++u)
+        if (at[u] >= 0) store(at[u], r[u]);
     __syncthreads();
 }
 
-// The packed fluid list of one particle in registers: every group is
-// requested at once, before the pass stages its window, so the list loads
-// overlap the staging instead of waiting one group at a time.
+// The packed fluid list of one particle (lane h's words of every group) in
+// registers: all groups are requested at once, before the pass stages its
+// window, so the list loads overlap the staging.
 constexpr int NB16_GROUPS = NBF_CAP / 8;
-struct List16 {
-    int4 g[NB16_GROUPS];
+template <int K>
+struct ListWords {
+    Words<K> g[NB16_GROUPS];
 };
-__device__ __forceinline__ void list16_load(const int4* __restrict__ list, int ncap, int i, int n, bool nt,
-                                            List16& L) {
-    const int ng = (n + 7) >> 3;
-#pragma unroll
-    for (int g = 0; g < NB16_GROUPS; ++g)
-        L.g[g] = g < ng ? ld_group(&list[(size_t)g * ncap + i], nt) : make_int4(0, 0, 0, 0);
-}
 
 // Neighbour loop over a window-index list (in registers) whose records are
-// in the LDS window: load(k) reads window record k, use(k, r) consumes it.
-// Entries past the padded count are read from record 0 and not used.
-template <class LD, class US>
-__device__ __forceinline__ void each_in_win16(const List16& L, int n, LD&& load, US&& use) {
+// in the LDS window: load(k) reads window record k, term(k, r) is the pair's
+// term, add(t) adds it.  Entries past the padded count are read from record 0
+// and not used.
+template <int K, class LD, class TM, class AD>
+__device__ __forceinline__ void each_in_win(const ListWords<K>& L, int h, int n, LD&& load, TM&& term, AD&& add) {
+    constexpr int E = Lanes<K>::E;
     const int ng = (n + 7) >> 3;
     const int n4 = (n + 3) & ~3;
 #pragma unroll
     for (int g = 0; g < NB16_GROUPS; ++g) {
         if (g >= ng) break;
-        const int4 cur = L.g[g];
-        const unsigned w[4] = {(unsigned)cur.x, (unsigned)cur.y, (unsigned)cur.z, (unsigned)cur.w};
         const bool second = 8 * g + 4 < n4;
-        int k[8];
+        decltype(load(0)) r[E];
+        int k[E];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int kq = (int)((w[q >> 1] >> (16 * (q & 1))) & 0xffffu);
-            k[q] = (q < 4 || second) ? kq : 0;
+        for (int q = 0; q < E; ++q) {
+            const int kq = (int)word_entry<K>(L.g[g], q);
+            k[q] = (second || h * E + q < 4) ? kq : 0;
+            r[q] = load(k[q]);
         }
-        decltype(load(0)) r[8];
+        decltype(term(0, r[0])) t[E];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) r[q] = load(k[q]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) use(k[q], r[q]);
-        if (second) {
-#pragma unroll
-            for (int q = 4; q < 8; ++q) use(k[q], r[q]);
-        }
+        for (int q = 0; q < E; ++q) t[q] = term(k[q], r[q]);
+        add_group<K>(t, second, add);
     }
 }
 
@@ -116,118 +122,55 @@ __device__ __forceinline__ void each_in_win16(const List16& L, int n, LD&& load,
 // window for the pass `bit` (packed, the pass's window on); the window itself
 // is decided by win_layout (the list builder writes this list for exactly the
 // tiles whose window it accepts).
-__device__ __forceinline__ void list16_prefetch(const Dev& D, const Slot& s, int c, List16& L, int bit) {
-    if (s.live && s.packed && (D.winMask & bit)) {
-        const bool nt = __builtin_amdgcn_readfirstlane(D.listNT) != 0;
-        list16_load(D.nbW16, D.ncap, s.i, nf_of(c), nt, L);
-    }
+template <int K>
+__device__ __forceinline__ void list_prefetch(const Dev& D, const Slot& s, int h, int c, ListWords<K>& L, int bit) {
+    const bool on = s.live && s.packed && (D.winMask & bit);
+    const int ng = on ? (nf_of(c) + 7) >> 3 : 0;
+    const bool nt = __builtin_amdgcn_readfirstlane(D.listNT) != 0;
+#pragma unroll
+    for (int g = 0; g < NB16_GROUPS; ++g)
+        L.g[g] = g < ng ? ld_words<K>(&D.nbW16[(size_t)g * D.ncap + s.i], h, nt) : Words<K>{};
 }
 
-// ---- two tiles per block ------------------------------------------------
-// The LDS-window builds take two consecutive tiles per block: the second
-// tile's window records are requested into registers before the first
-// tile's neighbour loops run, so their latency is spent on the first tile's
-// work instead of in a second staging phase.  Each particle's own values are
-// loaded before them (a wait for a later load waits for every earlier one).
 struct Rec3x2 {
     float3 a, b;
 };
-__device__ __forceinline__ Slot slot_tile(const Dev& D, int tile) {
-    Slot s;
-    s.tile = tile;
-    s.i = tile * TILE + threadIdx.x;
-    s.scene = D.tileScene[tile];
-    s.live = (int)threadIdx.x < D.tileValid[tile] && D.active[s.scene] != 0;
-    s.packed = false;
-    return s;
-}
-// win_particle with the tables in `tab` (list table, then window offsets)
-__device__ __forceinline__ int win_particle_tab(const int* tab, int k) {
-    const int* off = tab + NB16_TAB;
-    int s = 0;
-#pragma unroll
-    for (int b = 16; b > 0; b >>= 1)
-        if (off[s + b] <= k) s += b;
-    return tab[s] + (s << NB16_OFF_BITS) + (k - off[s]);
-}
 
-// The LDS-window build of a solver-loop pass: two consecutive tiles per
-// block.  own(s, c) loads what a particle reads of itself, load(j) a window
-// record of particle j, store(k, r) writes window record k, body(s, c, nw,
-// L, own) runs the tile's particles (nw > 0: their fluid neighbours are in
-// the window) and returns the particle's part of the tile's partial sum,
-// which PARTIAL blocks write.  The second tile's records are requested
-// before the first tile's body runs and stored after it.
-template <int BIT, bool PARTIAL, class OwnF, class LoadF, class StoreF, class BodyF>
-__device__ __forceinline__ void window_pair(const Dev& D, OwnF&& own, LoadF&& load, StoreF&& store, BodyF&& body) {
-    __shared__ double lds[4];
-    __shared__ int tabB[NB16_TAB + 32];   // the second tile's list table and window offsets
-    const int tA = 2 * tile_of_block(D.tileMap), tB = tA + 1;
-    const bool hasB = tB < D.npad / TILE;
-    Slot sA = slot_tile(D, tA);
-    Slot sB = slot_tile(D, hasB ? tB : tA);
-    const bool actA = D.active[sA.scene] != 0;
-    const bool actB = hasB && D.active[sB.scene] != 0;
-    if (!hasB) sB.live = false;
-    const int t = threadIdx.x;
-    // both tiles' tables with one round trip
-    if (actA) {
-        if (t < NB16_TAB) g_nbtab[t] = D.nbTab[(size_t)tA * NB16_TAB + t];
-        else if (t < NB16_TAB + 32) g_winoff[t - NB16_TAB] = D.nbWin[(size_t)tA * 32 + t - NB16_TAB];
+// The LDS-window build of a solver-loop pass: one tile a block, K lanes a
+// particle.  own(i) loads what particle i reads of itself, load(j) a window
+// record of particle j, store(k, r) writes window record k, body(s, h, c, nw,
+// L, own) runs lane h of the tile's particles (nw > 0: their fluid neighbours
+// are in the window) and returns the particle's part of the tile's partial sum,
+// which PARTIAL blocks write.
+// A window of the size a tile needs (2,400 records on a dam) leaves room for
+// two blocks a CU (pass A), so the passes wait on memory unless each block
+// holds many waves: with two lanes a particle there are 16 on a CU, and the
+// arithmetic takes two thirds of the time.  Two tiles a block with one lane a
+// particle, the second tile's window requested during the first's loops (8
+// waves a CU), took 290 / 292 us for the divergence / density pass of 4M
+// particles, 80 / 84 of 1M and 21 / 21 of 117k; two lanes take 248 / 256,
+// 67 / 71 and 15 / 15 (gathers: 302 / 301, 74 / 77 and 18 / 18; four lanes
+// 300 / 311, 81 / 85 and 17 / 18: more instructions).  Passes of one record
+// (velocity, sum d_ij p_j) are faster as gathers (41 against 59 us at 1M).
+template <int K, int BIT, bool PARTIAL, class OwnF, class LoadF, class StoreF, class BodyF>
+__device__ __forceinline__ void window_tile(const Dev& D, OwnF&& own, LoadF&& load, StoreF&& store, BodyF&& body) {
+    decltype(own(0)) o;
+    const Slot s = slot_nb<K>(D, true, [&](int i) { o = own(i); });
+    if (!D.active[s.scene]) {   // uniform: a converged scene's tiles contribute nothing
+        if (PARTIAL && threadIdx.x == 0) D.partial[2 * s.tile] = 0.0;
+        return;
     }
-    if (actB) {
-        if (t >= 128 && t < 128 + NB16_TAB) tabB[t - 128] = D.nbTab[(size_t)tB * NB16_TAB + t - 128];
-        else if (t >= 128 + NB16_TAB && t < 128 + NB16_TAB + 32)
-            tabB[t - 128] = D.nbWin[(size_t)tB * 32 + t - 128 - NB16_TAB];
-    }
-    __syncthreads();
-    sA.packed = actA && __builtin_amdgcn_readfirstlane(g_nbtab[NB16_FLAG]) != 0;
-    sB.packed = actB && __builtin_amdgcn_readfirstlane(tabB[NB16_FLAG]) != 0;
-    // the first tile: list and own values, then its window
-    const int cA = sA.live ? D.cnt[sA.i] : 0;
-    List16 LA;
-    list16_prefetch(D, sA, cA, LA, BIT);
-    const auto oA = own(sA, cA);
-    const int nwA = win_layout(D, sA, BIT);
-    if (nwA) win_stage(nwA, load, store);
-    // the second tile's window records, in flight during the first tile's body
-    int nwB = 0;
-    if (sB.packed && (D.winMask & BIT)) {
-        nwB = __builtin_amdgcn_readfirstlane(tabB[NB16_TAB + 31]);
-        if (nwB > WIN_MAX) nwB = 0;
-    }
-    constexpr int DEPTH = WIN_MAX / 256;
-    decltype(load(0)) rB[DEPTH];
-#pragma unroll
-    for (int u = 0; u < DEPTH; ++u) {
-        const int k = t + 256 * u;
-        if (k < nwB) rB[u] = load(win_particle_tab(tabB, k));
-    }
-    const double sumA = body(sA, cA, nwA, LA, oA);
-    if (PARTIAL) {
-        if (actA) write_partial(D, tA, 0, sumA, lds);
-        else if (t == 0) D.partial[2 * tA] = 0.0;
-    }
-    if (!hasB) return;   // uniform
-    __syncthreads();     // every lane is done with the first tile's window and tables
-    if (actB) {
-        if (t < NB16_TAB) g_nbtab[t] = tabB[t];
-        else if (t < NB16_TAB + 32) g_winoff[t - NB16_TAB] = tabB[t];
-    }
-#pragma unroll
-    for (int u = 0; u < DEPTH; ++u) {
-        const int k = t + 256 * u;
-        if (k < nwB) store(k, rB[u]);
-    }
-    __syncthreads();
-    const int cB = sB.live ? D.cnt[sB.i] : 0;
-    List16 LB;
-    list16_prefetch(D, sB, cB, LB, BIT);
-    const auto oB = own(sB, cB);
-    const double sumB = body(sB, cB, nwB, LB, oB);
-    if (PARTIAL) {
-        if (actB) write_partial(D, tB, 0, sumB, lds);
-        else if (t == 0) D.partial[2 * tB] = 0.0;
+    const int h = threadIdx.x % K;
+    const int c = s.c;
+    ListWords<K> L;
+    list_prefetch(D, s, h, c, L, BIT);
+    const int nw = win_layout(D, s, BIT);
+    if (nw) win_stage<4 * K>(load, store);
+    const double v = body(s, h, c, nw, L, o);
+    if constexpr (PARTIAL) {
+        __shared__ double part[TILE], lds[4 * K];
+        const double sum = tile_sum<K>(v, part, lds);
+        if (threadIdx.x == 0) D.partial[2 * s.tile] = sum;
     }
 }
 
@@ -281,11 +224,11 @@ __global__ __launch_bounds__(256) void k_stats_partial(Dev D, double* part) {
         float4 x = D.x[s.i], v = D.v[s.i];
         int ph = phase_of(x);
         float r = D.rho[s.i];
-        float ee = r / D.rho0[ph] - 1.0f;
+        float ee = r / rho0_of(D, ph) - 1.0f;
         e = (double)ee;
         emax = ee;
         n = 1.0;
-        ke = 0.5 * (double)D.mass[ph] * (double)(v.x * v.x + v.y * v.y + v.z * v.z);
+        ke = 0.5 * (double)mass_of(D, ph) * (double)(v.x * v.x + v.y * v.y + v.z * v.z);
         if (!isfinite(x.x + x.y + x.z + v.x + v.y + v.z)) nan = 1;
     }
     double se = block_sum_256(e, lds);
@@ -356,32 +299,45 @@ __device__ __forceinline__ float density_sum(const Dev& D, const Slot& s, float4
     return rho.s;
 }
 
-// one pair's term g(r) (v*_a - v*_b).x_ab of the density change rate
-__device__ __forceinline__ float dchange_term(const Dev& D, float4 pa, float4 va, float bx, float by, float bz,
-                                              float ux, float uy, float uz) {
+// one pair's term of the density change rate: g(r) and (v*_a - v*_b).x_ab
+__device__ __forceinline__ float2 dchange_pair(const Dev& D, float4 pa, float4 va, float bx, float by, float bz,
+                                               float ux, float uy, float uz) {
     const float dx = pa.x - bx, dy = pa.y - by, dz = pa.z - bz;
     const float g = kernel_gradfac_sq(dot3f(dx, dy, dz, dx, dy, dz), D);
-    return g * dot3f(va.x - ux, va.y - uy, va.z - uz, dx, dy, dz);
+    return make_float2(g, dot3f(va.x - ux, va.y - uy, va.z - uz, dx, dy, dz));
+}
+__device__ __forceinline__ float dchange_term(const Dev& D, float4 pa, float4 va, float bx, float by, float bz,
+                                              float ux, float uy, float uz) {
+    const float2 t = dchange_pair(D, pa, va, bx, by, bz, ux, uy, uz);
+    return t.x * t.y;
 }
 
 // sum_b V_b gradW.(v*_a - v_b) over the boundary neighbours
-__device__ __forceinline__ float dchange_boundary(const Dev& D, const Slot& s, float4 pa, float4 va, int c) {
+template <int K = 1>
+__device__ __forceinline__ float dchange_boundary(const Dev& D, const Slot& s, int h, float4 pa, float4 va, int c) {
     float sb = 0.0f;
-    each_boundary_lu<4>(D, s, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; }, [&](int j, Rec2 rec) {
-        sb += rec.a.w * dchange_term(D, pa, va, rec.a.x, rec.a.y, rec.a.z, rec.b.x, rec.b.y, rec.b.z);
-    });
+    each_boundary<K, 4>(
+        D, s, h, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; },
+        [&](int, const Rec2& r) {
+            return make_float2(r.a.w, dchange_term(D, pa, va, r.a.x, r.a.y, r.a.z, r.b.x, r.b.y, r.b.z));
+        },
+        [&](float2 t) { sb += t.x * t.y; });
     return sb;
 }
 
 // sum_f m gradW.(v*_a - v*_b) + sum_b rho0 V_b gradW.(v*_a - v_b): the
 // predicted density change rate (DFSPH.cpp:589-617, 795-825)
-__device__ __forceinline__ float density_change(const Dev& D, const Slot& s, float4 pa, float4 va, float m,
+template <int K = 1>
+__device__ __forceinline__ float density_change(const Dev& D, const Slot& s, int h, float4 pa, float4 va, float m,
                                                 float rho0, int c) {
-    float sf = 0.0f, sb = 0.0f;
-    each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.vs[j]}; }, [&](int j, Rec2 rec) {
-        sf += dchange_term(D, pa, va, rec.a.x, rec.a.y, rec.a.z, rec.b.x, rec.b.y, rec.b.z);
-    });
-    sb = dchange_boundary(D, s, pa, va, c);
+    float sf = 0.0f;
+    each_fluid<K, 4>(
+        D, s, h, nf_of(c), [&](int j) { return Rec2{D.x[j], D.vs[j]}; },
+        [&](int, const Rec2& r) {
+            return dchange_pair(D, pa, va, r.a.x, r.a.y, r.a.z, r.b.x, r.b.y, r.b.z);
+        },
+        [&](float2 t) { sf += t.x * t.y; });
+    const float sb = dchange_boundary<K>(D, s, h, pa, va, c);
     return m * sf + rho0 * sb;
 }
 
@@ -389,13 +345,13 @@ __device__ __forceinline__ float density_change(const Dev& D, const Slot& s, flo
 // WcSph::wc_computePressure (WcSph.cpp:99-153): rho (Kahan), Tait p >= 0.
 // Publishes the force pass's gather records: xk = (x, p/rho^2), v.w = rho.
 __global__ __launch_bounds__(256) void k_wc_pressure(Dev D) {
-    Slot s = slot_nb(D, false);
+    float4 pa;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], rho0 = D.rho0[ph];
-    float density = density_sum(D, s, pa, m, rho0, D.cnt[i]);
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph);
+    float density = density_sum(D, s, pa, m, rho0, s.c);
     float p = D.tait_B[ph] * (powf(density / rho0, D.gamma) - 1.0f);
     p = p < 0.0f ? 0.0f : p;
     D.rho[i] = density;
@@ -408,18 +364,18 @@ __global__ __launch_bounds__(256) void k_wc_pressure(Dev D) {
 // Euler-Cromer update and domain removal of SphBase::updateFluids
 // (SphBase.cpp:377-402): writes x2/v2, the caller swaps buffers.
 __global__ __launch_bounds__(256) void k_wc_force(Dev D) {
-    Slot s = slot_nb(D, false);
+    float4 pa, va;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i], va = D.v[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], rho0 = D.rho0[ph], alpha = D.visc[ph];
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph), alpha = visc_of(D, ph);
     float rhoa = va.w, pra = D.f1[i];
     float pa_r2 = pra / (rhoa * rhoa);
     const float Hcs2 = 2.0f * D.Hs * D.cs;
     const bool multi = D.nphases > 1;
     float ax = D.gx, ay = D.gy, az = D.gz;
-    int c = D.cnt[i];
+    const int c = s.c;
     each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.xk[j], D.v[j]}; }, [&](int j, Rec2 rec) {
         const float4 pb = rec.a, vb = rec.b;   // (x, p/rho^2), (v, rho)
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
@@ -470,16 +426,16 @@ __global__ __launch_bounds__(256) void k_wc_force(Dev D) {
 // DFSPH::DF_constantDensitySolverFirst (DFSPH.cpp:84-193): rho (Kahan) and alpha.
 template <bool WARM>
 __global__ __launch_bounds__(256) void k_df_density_alpha(Dev D, float* __restrict__ feat) {
-    Slot s = slot_nb(D, false);
+    float4 pa;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], rho0 = D.rho0[ph];
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph);
     Kahan rho;
     rho.init(m * D.W0);
     float a1x = 0.f, a1y = 0.f, a1z = 0.f, a2 = 0.f;
-    int c = D.cnt[i];
+    const int c = s.c;
     // WARM: also Drho/Dt with v* = v (density_change) and the nearest
     // boundary distance, for the warm start of the divergence loop
     const float4 va = WARM ? D.v[i] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -546,18 +502,18 @@ __global__ __launch_bounds__(256) void k_df_density_alpha(Dev D, float* __restri
 // kappa: it only pushes (rho* >= rho0, DFSPH.cpp:620-623), so a warm guess
 // that overshoots would never be taken back.
 __global__ __launch_bounds__(256) void k_df_aadv(Dev D) {
-    Slot s = slot_nb(D, false);
+    float4 pa, va;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i], va = D.v[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], rho0 = D.rho0[ph], alpha = D.visc[ph];
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph), alpha = visc_of(D, ph);
     float rhoa = va.w;
     const float nu10 = 10.0f * D.nu;
     const float Hcs2 = 2.0f * D.Hs * D.cs;
     const bool multi = D.nphases > 1;
     float ax = D.gx, ay = D.gy, az = D.gz;
-    int c = D.cnt[i];
+    const int c = s.c;
     each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.v[j]}; }, [&](int j, Rec2 rec) {
         const float4 pb = rec.a, vb = rec.b;   // vb = (v, rho)
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
@@ -636,14 +592,14 @@ __global__ __launch_bounds__(256) void k_df_warm_apply(Dev D, const float* __res
     float dt = D.dt[s.scene];
     float kv = 0.0f, d = D.f2[i];
     // only where the solve itself would apply stiffness (DFSPH.cpp:829-832)
-    if (d > 0.0f && !(D.rho[i] + d * dt < D.rho0[ph])) {
+    if (d > 0.0f && !(D.rho[i] + d * dt < rho0_of(D, ph))) {
         const float kprev = D.kvsum[i];
         if (mode == 1) {
             kv = D.warm_scale * kprev;
         } else {
             const float alpha = D.alpha[i];
             float u = feat[8 * (size_t)i + 3] + y[i];
-            float kp = expm1f(fminf(fmaxf(u, 0.0f), 12.0f)) * 1.0e-3f * alpha * D.rho0[ph] / dt;
+            float kp = expm1f(fminf(fmaxf(u, 0.0f), 12.0f)) * 1.0e-3f * alpha * rho0_of(D, ph) / dt;
             kv = D.learn_scale * fminf(kp, fmaxf(kprev, d * alpha));
         }
     }
@@ -658,7 +614,7 @@ __global__ __launch_bounds__(256) void k_df_targets(Dev D, const float* __restri
     if (!s.live) return;
     const int i = s.i;
     int ph = phase_of(D.x[i]);
-    tgt[i] = log1pf(fmaxf(D.kvsum[i] * D.dt[s.scene] / (D.alpha[i] * D.rho0[ph]) * 1000.0f, 0.0f)) -
+    tgt[i] = log1pf(fmaxf(D.kvsum[i] * D.dt[s.scene] / (D.alpha[i] * rho0_of(D, ph)) * 1000.0f, 0.0f)) -
              feat[8 * (size_t)i + 3];
 }
 
@@ -713,21 +669,18 @@ __device__ __forceinline__ void store_xyz2(WinXV w, int k, const Rec3x2& r) {
     w.zv[k] = make_float4(r.a.z, r.b.x, r.b.y, r.b.z);
 }
 
-__device__ __forceinline__ void stage_xv(const Dev& D, int n, WinXV w) {
-    win_stage(n, [&](int j) { return Rec2{D.x[j], D.vs[j]}; }, [&](int k, Rec2 r) {
-        w.xy[k] = make_float2(r.a.x, r.a.y);
-        w.zv[k] = make_float4(r.a.z, r.b.x, r.b.y, r.b.z);
-    });
-}
-
 // density_change with the fluid records read from the LDS window
-__device__ __forceinline__ float density_change_win(const Dev& D, const Slot& s, float4 pa, float4 va, float m,
-                                                    float rho0, int c, WinXV w, const List16& L) {
+template <int K>
+__device__ __forceinline__ float density_change_win(const Dev& D, const Slot& s, int h, float4 pa, float4 va, float m,
+                                                    float rho0, int c, WinXV w, const ListWords<K>& L) {
     float sf = 0.0f;
-    each_in_win16(L, nf_of(c), [&](int k) { return RecW{w.xy[k], w.zv[k]}; }, [&](int, RecW rec) {
-        sf += dchange_term(D, pa, va, rec.a.x, rec.a.y, rec.b.x, rec.b.y, rec.b.z, rec.b.w);
-    });
-    const float sb = dchange_boundary(D, s, pa, va, c);
+    each_in_win<K>(
+        L, h, nf_of(c), [&](int k) { return RecW{w.xy[k], w.zv[k]}; },
+        [&](int, const RecW& r) {
+            return dchange_pair(D, pa, va, r.a.x, r.a.y, r.b.x, r.b.y, r.b.z, r.b.w);
+        },
+        [&](float2 t) { sf += t.x * t.y; });
+    const float sb = dchange_boundary<K>(D, s, h, pa, va, c);
     return m * sf + rho0 * sb;
 }
 
@@ -752,45 +705,38 @@ __device__ __forceinline__ float density_change_win(const Dev& D, const Slot& s,
 // what a particle of pass A reads of itself
 struct OwnAB {
     float4 pa, va;
-    float m, rho0, dt, alpha, acc;
+    float alpha, acc;
 };
 template <int MODE>
-__device__ __forceinline__ OwnAB own_ab(const Dev& D, const Slot& s) {
-    OwnAB o{};
-    if (!s.live) return o;
-    o.pa = D.x[s.i];
-    o.va = D.vs[s.i];   // v* carries rho in w (as v does), one array fewer to stream
-    o.dt = D.dt[s.scene];
-    o.alpha = D.alpha[s.i];
-    o.acc = MODE == 0 ? D.ksum[s.i] : D.kvsum[s.i];
-    const int ph = phase_of(o.pa);
-    o.m = D.mass[ph];
-    o.rho0 = D.rho0[ph];
-    return o;
+__device__ __forceinline__ OwnAB own_ab(const Dev& D, int i) {
+    // v* carries rho in w (as v does), one array fewer to stream
+    return OwnAB{D.x[i], D.vs[i], D.alpha[i], MODE == 0 ? D.ksum[i] : D.kvsum[i]};
 }
 
-// one particle of pass A; nw > 0: its fluid neighbours are in the LDS window
+// one particle of pass A with its rate dd; h: the lane of the particle (0 writes)
 template <int MODE>
-__device__ __forceinline__ double pass_ab_particle(const Dev& D, const Slot& s, const OwnAB& o, int c, int nw,
-                                                   WinXV win, const List16& L, int projected) {
-    if (!s.live) return 0.0;
+__device__ __forceinline__ double pass_ab_particle(const Dev& D, const Slot& s, int h, const OwnAB& o, float dd,
+                                                   int projected) {
     const int i = s.i;
     const float4 pa = o.pa, va = o.va;
-    const float m = o.m, rho0 = o.rho0, dt = o.dt, rhoa = va.w;
-    float dd = nw ? density_change_win(D, s, pa, va, m, rho0, c, win, L) : density_change(D, s, pa, va, m, rho0, c);
+    const float rho0 = rho0_of(D, phase_of(pa)), dt = D.dt[s.scene], rhoa = va.w;
     if (MODE == 0) {
         float rs = rhoa + dt * dd;
         if (rs < rho0) rs = rho0;
         const float dev = (rs - rho0) * o.alpha;   // kappa * dt^2
-        D.xk[i] = make_float4(pa.x, pa.y, pa.z, dev / (dt * dt) / rhoa);
-        D.ksum[i] = o.acc + dev;
+        if (h == 0) {
+            D.xk[i] = make_float4(pa.x, pa.y, pa.z, dev / (dt * dt) / rhoa);
+            D.ksum[i] = o.acc + dev;
+        }
         return (double)rs / (double)rho0;
     }
     if (!projected) {
         if (dd < 0.0f || (rhoa + dd * dt) < rho0) dd = 0.0f;
         const float kv = dd * o.alpha / dt;
-        D.xk[i] = make_float4(pa.x, pa.y, pa.z, kv / rhoa);
-        D.kvsum[i] = o.acc + kv * dt;
+        if (h == 0) {
+            D.xk[i] = make_float4(pa.x, pa.y, pa.z, kv / rhoa);
+            D.kvsum[i] = o.acc + kv * dt;
+        }
         return (double)dd;
     }
     // below rest density the solve applies no stiffness: the whole guess is
@@ -799,8 +745,10 @@ __device__ __forceinline__ double pass_ab_particle(const Dev& D, const Slot& s, 
     float inc = dd * alpha;
     if ((rhoa + dd * dt) < rho0 || inc < -K) inc = -K;
     const float kv = inc / dt;
-    D.xk[i] = make_float4(pa.x, pa.y, pa.z, kv / rhoa);
-    D.kvsum[i] = K + inc;
+    if (h == 0) {
+        D.xk[i] = make_float4(pa.x, pa.y, pa.z, kv / rhoa);
+        D.kvsum[i] = K + inc;
+    }
     return (double)(fabsf(inc) / alpha);
 }
 
@@ -808,38 +756,48 @@ __device__ __forceinline__ double pass_ab_particle(const Dev& D, const Slot& s, 
 template <int MODE>
 __device__ __forceinline__ void pass_ab_gather(const Dev& D, int projected) {
     __shared__ double lds[4];
-    Slot s = slot_nb(D, true);
+    OwnAB o;
+    const Slot s = slot_nb<1>(D, true, [&](int i) { o = own_ab<MODE>(D, i); });
     if (!D.active[s.scene]) {   // uniform: a converged scene's tiles contribute nothing
         if (threadIdx.x == 0) D.partial[2 * s.tile] = 0.0;
         return;
     }
-    const int c = s.live ? D.cnt[s.i] : 0;
-    const OwnAB o = own_ab<MODE>(D, s);
-    const List16 L{};
-    write_partial(D, s.tile, 0, pass_ab_particle<MODE>(D, s, o, c, 0, WinXV{nullptr, nullptr}, L, projected), lds);
+    double v = 0.0;
+    if (s.live) {
+        const int ph = phase_of(o.pa);
+        const float dd = density_change(D, s, 0, o.pa, o.va, mass_of(D, ph), rho0_of(D, ph), s.c);
+        v = pass_ab_particle<MODE>(D, s, 0, o, dd, projected);
+    }
+    write_partial(D, s.tile, 0, v, lds);
 }
 
-// LDS-window build: two tiles per block (window_pair)
-template <int MODE>
-__device__ __forceinline__ void pass_ab_window_pair(const Dev& D, int projected) {
+// LDS-window build
+template <int MODE, int K>
+__device__ __forceinline__ void pass_ab_window(const Dev& D, int projected) {
     WIN_XV_DECL(WIN_MAX)
-    window_pair<MODE == 0 ? WIN_DENSITY : WIN_DIVERGENCE, true>(
-        D, [&](const Slot& s, int) { return own_ab<MODE>(D, s); }, [&](int j) { return load_xyz2(D.x, D.vs, j); },
+    window_tile<K, MODE == 0 ? WIN_DENSITY : WIN_DIVERGENCE, true>(
+        D, [&](int i) { return own_ab<MODE>(D, i); }, [&](int j) { return load_xyz2(D.x, D.vs, j); },
         [&](int k, const Rec3x2& r) { store_xyz2(win, k, r); },
-        [&](const Slot& s, int c, int nw, const List16& L, const OwnAB& o) {
-            return pass_ab_particle<MODE>(D, s, o, c, nw, win, L, projected);
+        [&](const Slot& s, int h, int c, int nw, const ListWords<K>& L, const OwnAB& o) {
+            if (!s.live) return 0.0;
+            const int ph = phase_of(o.pa);
+            const float m = mass_of(D, ph), rho0 = rho0_of(D, ph);
+            const float dd = nw ? density_change_win<K>(D, s, h, o.pa, o.va, m, rho0, c, win, L)
+                                : density_change<K>(D, s, h, o.pa, o.va, m, rho0, c);
+            return pass_ab_particle<MODE>(D, s, h, o, dd, projected);
         });
 }
 
 template <bool WIN>
-__global__ __launch_bounds__(256, WIN ? 2 : 1) void k_df_pass_density(Dev D) {
-    if constexpr (WIN) pass_ab_window_pair<0>(D, 0);
+__global__ __launch_bounds__(WIN ? 256 * WIN_LANES : 256, WIN ? 2 * WIN_LANES : 1) void k_df_pass_density(Dev D) {
+    if constexpr (WIN) pass_ab_window<0, WIN_LANES>(D, 0);
     else pass_ab_gather<0>(D, 0);
 }
 
 template <bool WIN>
-__global__ __launch_bounds__(256, WIN ? 2 : 1) void k_df_pass_divergence(Dev D, int projected) {
-    if constexpr (WIN) pass_ab_window_pair<1>(D, projected);
+__global__ __launch_bounds__(WIN ? 256 * WIN_LANES : 256, WIN ? 2 * WIN_LANES : 1) void k_df_pass_divergence(
+    Dev D, int projected) {
+    if constexpr (WIN) pass_ab_window<1, WIN_LANES>(D, projected);
     else pass_ab_gather<1>(D, projected);
 }
 
@@ -847,42 +805,42 @@ __global__ __launch_bounds__(256, WIN ? 2 : 1) void k_df_pass_divergence(Dev D, 
 // v* -= dt (m sum (kr_a + kr_b) gradW + rho0 sum V_b kr_a gradW), kr = xk.w
 struct OwnV {
     float4 pa, v;
-    float m, rho0, dt;
 };
-__device__ __forceinline__ OwnV own_v(const Dev& D, const Slot& s, int c) {
-    OwnV o{};
-    if (!s.live) return o;
-    o.pa = D.xk[s.i];
-    o.v = D.vs[s.i];
-    o.dt = D.dt[s.scene];
-    const int ph = phase_of_cnt(c);   // (the phase from the count word: no read of x)
-    o.m = D.mass[ph];
-    o.rho0 = D.rho0[ph];
-    return o;
-}
-// one particle of pass B; nw > 0: its fluid neighbours are in the window wxk
-__device__ __forceinline__ void velocity_particle(const Dev& D, const Slot& s, const OwnV& o, int c, int nw,
-                                                  const float4* wxk, const List16& L) {
+__device__ __forceinline__ OwnV own_v(const Dev& D, int i) { return OwnV{D.xk[i], D.vs[i]}; }
+// lane h of one particle of pass B; nw > 0: its fluid neighbours are in the window wxk
+template <int K>
+__device__ __forceinline__ void velocity_particle(const Dev& D, const Slot& s, int h, const OwnV& o, int c, int nw,
+                                                  const float4* wxk, const ListWords<K>* L) {
     if (!s.live) return;
     const float4 pa = o.pa;
     const float ka = pa.w;
     float fx = 0.f, fy = 0.f, fz = 0.f, bx = 0.f, by = 0.f, bz = 0.f;
+    // (x_ab, g): the pair's term is x_ab g
     auto fluid = [&](int, float4 pb) {
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
         float g = kernel_gradfac_sq(dot3f(dx, dy, dz, dx, dy, dz), D) * (ka + pb.w);
-        fx += dx * g; fy += dy * g; fz += dz * g;
+        return make_float4(dx, dy, dz, g);
     };
-    if (nw) {
-        each_in_win16(L, nf_of(c), [&](int k) { return wxk[k]; }, fluid);
-    } else {
-        each_fluid_lu<8>(D, s, nf_of(c), [&](int j) { return D.xk[j]; }, fluid);
+    auto add = [&](float4 t) { fx += t.x * t.w; fy += t.y * t.w; fz += t.z * t.w; };
+    bool win = false;
+    if constexpr (K > 1) {
+        win = nw != 0;
+        if (win) each_in_win<K>(*L, h, nf_of(c), [&](int k) { return wxk[k]; }, fluid, add);
     }
-    each_boundary_lu<8>(D, s, nb_of(c), [&](int j) { return D.xb[j]; }, [&](int j, float4 pb) {
-        float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-        float g = kernel_gradfac_sq(dx * dx + dy * dy + dz * dz, D) * pb.w;
-        bx += dx * g; by += dy * g; bz += dz * g;
-    });
-    const float cf = o.dt * o.m, cb = o.dt * o.rho0 * ka;
+    if (!win) each_fluid<K, 8>(D, s, h, nf_of(c), [&](int j) { return D.xk[j]; }, fluid, add);
+    each_boundary<K, 8>(
+        D, s, h, nb_of(c), [&](int j) { return D.xb[j]; },
+        [&](int, float4 pb) {
+            float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
+            float g = kernel_gradfac_sq(dx * dx + dy * dy + dz * dz, D) * pb.w;
+            return make_float4(dx, dy, dz, g);
+        },
+        [&](float4 t) { bx += t.x * t.w; by += t.y * t.w; bz += t.z * t.w; });
+    if (h != 0) return;
+    // (the phase from the count word: no read of x)
+    const int ph = phase_of_cnt(c);
+    const float dt = D.dt[s.scene], rho0 = rho0_of(D, ph);
+    const float cf = dt * mass_of(D, ph), cb = dt * rho0 * ka;
     float4 v = o.v;
     v.x -= cf * fx + cb * bx;
     v.y -= cf * fy + cb * by;
@@ -891,24 +849,22 @@ __device__ __forceinline__ void velocity_particle(const Dev& D, const Slot& s, c
 }
 
 template <bool WIN>
-__global__ __launch_bounds__(256, WIN ? 2 : 1) void k_df_pass_velocity(Dev D) {
+__global__ __launch_bounds__(WIN ? 256 * WIN_LANES : 256, WIN ? 2 * WIN_LANES : 1) void k_df_pass_velocity(Dev D) {
     loop_test(D);   // on pass A's partial sums
     if constexpr (WIN) {
         __shared__ float4 s_wxk[WIN_MAX];   // window records: xk of each neighbour
-        window_pair<WIN_VELOCITY, false>(
-            D, [&](const Slot& s, int c) { return own_v(D, s, c); }, [&](int j) { return D.xk[j]; },
+        window_tile<WIN_LANES, WIN_VELOCITY, false>(
+            D, [&](int i) { return own_v(D, i); }, [&](int j) { return D.xk[j]; },
             [&](int k, const float4& r) { s_wxk[k] = r; },
-            [&](const Slot& s, int c, int nw, const List16& L, const OwnV& o) {
-                velocity_particle(D, s, o, c, nw, s_wxk, L);
+            [&](const Slot& s, int h, int c, int nw, const ListWords<WIN_LANES>& L, const OwnV& o) {
+                velocity_particle<WIN_LANES>(D, s, h, o, c, nw, s_wxk, &L);
                 return 0.0;
             });
     } else {
-        Slot s = slot_nb(D, true);
+        OwnV o;
+        const Slot s = slot_nb<1>(D, true, [&](int i) { o = own_v(D, i); });
         if (!D.active[s.scene]) return;   // uniform per block
-        const int c = s.live ? D.cnt[s.i] : 0;
-        const OwnV o = own_v(D, s, c);
-        const List16 L{};
-        velocity_particle(D, s, o, c, 0, nullptr, L);
+        velocity_particle<1>(D, s, 0, o, s.c, 0, nullptr, nullptr);
     }
 }
 
@@ -933,30 +889,30 @@ __global__ __launch_bounds__(256) void k_df_integrate(Dev D) {
 // density (IISph_M.cpp:101-112), computed before a_adv so that a_adv reads
 // this step's densities; published as v.w for the a_adv gathers.
 __global__ __launch_bounds__(256) void k_ii_density(Dev D) {
-    Slot s = slot_nb(D, false);
+    float4 pa;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i];
     int ph = phase_of(pa);
-    float density = density_sum(D, s, pa, D.mass[ph], D.rho0[ph], D.cnt[i]);
+    float density = density_sum(D, s, pa, mass_of(D, ph), rho0_of(D, ph), s.c);
     D.rho[i] = density;
     D.v[i].w = density;
 }
 
 // a_adv (IISph_M.cpp:364-476), d_ii (114-130) and v_adv (135)
 __global__ __launch_bounds__(256) void k_ii_aadv_dii(Dev D) {
-    Slot s = slot_nb(D, false);
+    float4 pa, va;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i], va = D.v[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], rho0 = D.rho0[ph], alpha = D.visc[ph];
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph), alpha = visc_of(D, ph);
     float rhoa = va.w;
     const float nu10 = 10.0f * D.nu, Hcs2 = 2.0f * D.Hs * D.cs;
     const bool multi = D.nphases > 1;
     float ax = D.gx, ay = D.gy, az = D.gz;
     float dfx = 0.f, dfy = 0.f, dfz = 0.f, dbx = 0.f, dby = 0.f, dbz = 0.f;
-    int c = D.cnt[i];
+    const int c = s.c;
     each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.v[j]}; }, [&](int j, Rec2 rec) {
         const float4 pb = rec.a, vb = rec.b;   // vb = (v, rho)
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
@@ -1006,19 +962,19 @@ __global__ __launch_bounds__(256) void k_ii_aadv_dii(Dev D) {
 //   7 dt / dt_max
 template <bool WARM>
 __global__ __launch_bounds__(256) void k_ii_aii(Dev D, float* __restrict__ feat) {
-    Slot s = slot_nb(D, false);
+    float4 pa, va, dii;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i], va = D.vs[i], dii = D.f4a[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i], va = D.vs[i], dii = D.f4a[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], rho0 = D.rho0[ph];
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph);
     float rhoa = D.rho[i];
     float dt = D.dt[s.scene];
     float cji = m * dt * dt / (rhoa * rhoa);
     float t1f = 0.f, t1b = 0.f, t2f = 0.f, t2b = 0.f, cself = 0.f;
     const float sp = D.spacing;
     float bmin2 = 4.0f * sp * sp;
-    int c = D.cnt[i];
+    const int c = s.c;
     const bool cons = D.mpCons && D.nphases > 1;
     each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.vs[j]}; }, [&](int j, Rec2 rec) {
         const float4 pb = rec.a, vb = rec.b;
@@ -1081,7 +1037,7 @@ __global__ __launch_bounds__(256) void k_ii_warm_apply(Dev D, const float* __res
     const int i = s.i;
     const float4 pa = D.x[i];
     const int ph = phase_of(pa);
-    const float rho0 = D.rho0[ph], aii = D.alpha[i], rhoa = D.rho[i];
+    const float rho0 = rho0_of(D, ph), aii = D.alpha[i], rhoa = D.rho[i];
     const float u = feat[8 * (size_t)i + 3] + y[i];
     float pl = 0.0f;
     if (aii < 0.0f) {
@@ -1090,7 +1046,7 @@ __global__ __launch_bounds__(256) void k_ii_warm_apply(Dev D, const float* __res
         pl = fminf(pm, fmaxf(D.ksum[i], pj));
     }
     D.kr[i] = pl;
-    const float m = D.mass[ph];
+    const float m = mass_of(D, ph);
     D.xk[i].w = (D.mpCons && D.nphases > 1) ? pl * (m * m / (rhoa * rhoa)) : pl / (rhoa * rhoa);
 }
 
@@ -1107,37 +1063,30 @@ __global__ __launch_bounds__(256) void k_ii_targets(Dev D, const float* __restri
 // stores u = d_ii p_l + sum_j d_ij p_j, the per-particle part of the
 // Jacobi update that neighbours read.
 struct OwnS {
-    float4 pa, dii;
-    float m, dt, pl;
+    float4 pa, dii;   // pa from the xk records the pass gathers (xyz = x during the loop)
+    float pl;
 };
-__device__ __forceinline__ OwnS own_s(const Dev& D, const Slot& s, int c) {
-    OwnS o{};
-    if (!s.live) return o;
-    // own position from the xk records the pass gathers (xyz = x during the
-    // loop), the phase from the count word: no read of x
-    o.pa = D.xk[s.i];
-    o.dii = D.f4a[s.i];
-    o.pl = D.kr[s.i];
-    o.dt = D.dt[s.scene];
-    o.m = D.mass[phase_of_cnt(c)];
-    return o;
-}
-__device__ __forceinline__ void sumdij_particle(const Dev& D, const Slot& s, const OwnS& o, int c, int nw,
-                                                const float4* wxk, const List16& L) {
+__device__ __forceinline__ OwnS own_s(const Dev& D, int i) { return OwnS{D.xk[i], D.f4a[i], D.kr[i]}; }
+template <int K>
+__device__ __forceinline__ void sumdij_particle(const Dev& D, const Slot& s, int h, const OwnS& o, int c, int nw,
+                                                const float4* wxk, const ListWords<K>* L) {
     if (!s.live) return;
     const float4 pa = o.pa;
     float sx = 0.f, sy = 0.f, sz = 0.f;
     auto fluid = [&](int, float4 pb) {
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
         float g = kernel_gradfac_sq(dot3f(dx, dy, dz, dx, dy, dz), D) * pb.w;
-        sx += dx * g; sy += dy * g; sz += dz * g;
+        return make_float4(dx, dy, dz, g);
     };
-    if (nw) {
-        each_in_win16(L, nf_of(c), [&](int k) { return wxk[k]; }, fluid);
-    } else {
-        each_fluid_lu<8>(D, s, nf_of(c), [&](int j) { return D.xk[j]; }, fluid);
+    auto add = [&](float4 t) { sx += t.x * t.w; sy += t.y * t.w; sz += t.z * t.w; };
+    bool win = false;
+    if constexpr (K > 1) {
+        win = nw != 0;
+        if (win) each_in_win<K>(*L, h, nf_of(c), [&](int k) { return wxk[k]; }, fluid, add);
     }
-    const float dt = o.dt, m = o.m;
+    if (!win) each_fluid<K, 8>(D, s, h, nf_of(c), [&](int j) { return D.xk[j]; }, fluid, add);
+    if (h != 0) return;
+    const float dt = D.dt[s.scene], m = mass_of(D, phase_of_cnt(c));   // (no read of x for the phase)
     // the records carry p/rho^2, or m^2 p/rho^2 with the number-density
     // force between phases (whose d_ij is dt^2 m_j^2 / (m_i rho_j^2) gradW)
     const float cf = (D.mpCons && D.nphases > 1) ? -dt * dt / m : -m * dt * dt;
@@ -1147,57 +1096,43 @@ __device__ __forceinline__ void sumdij_particle(const Dev& D, const Slot& s, con
 }
 
 template <bool WIN>
-__global__ __launch_bounds__(256, WIN ? 2 : 1) void k_ii_sumdij(Dev D) {
+__global__ __launch_bounds__(WIN ? 256 * WIN_LANES : 256, WIN ? 2 * WIN_LANES : 1) void k_ii_sumdij(Dev D) {
     loop_test(D);   // of the iteration before, on its pressure pass's partial sums
     if constexpr (WIN) {
         __shared__ float4 s_wxk[WIN_MAX];   // window records: xk of each neighbour
-        window_pair<WIN_SUMDIJ, false>(
-            D, [&](const Slot& s, int c) { return own_s(D, s, c); }, [&](int j) { return D.xk[j]; },
+        window_tile<WIN_LANES, WIN_SUMDIJ, false>(
+            D, [&](int i) { return own_s(D, i); }, [&](int j) { return D.xk[j]; },
             [&](int k, const float4& r) { s_wxk[k] = r; },
-            [&](const Slot& s, int c, int nw, const List16& L, const OwnS& o) {
-                sumdij_particle(D, s, o, c, nw, s_wxk, L);
+            [&](const Slot& s, int h, int c, int nw, const ListWords<WIN_LANES>& L, const OwnS& o) {
+                sumdij_particle<WIN_LANES>(D, s, h, o, c, nw, s_wxk, &L);
                 return 0.0;
             });
     } else {
-        Slot s = slot_nb(D, true);
+        OwnS o;
+        const Slot s = slot_nb<1>(D, true, [&](int i) { o = own_s(D, i); });
         if (!D.active[s.scene]) return;   // uniform per block
-        const int c = s.live ? D.cnt[s.i] : 0;
-        const OwnS o = own_s(D, s, c);
-        const List16 L{};
-        sumdij_particle(D, s, o, c, 0, nullptr, L);
+        sumdij_particle<1>(D, s, 0, o, s.c, 0, nullptr, nullptr);
     }
 }
 
 struct OwnP {
     float4 pa, ua, dia;
-    float m, rho0, rhoa, pla, dt, aii, radv, f2;
+    float rhoa, pla, aii, radv, f2;
 };
-__device__ __forceinline__ OwnP own_p(const Dev& D, const Slot& s) {
-    OwnP o{};
-    if (!s.live) return o;
-    const int i = s.i;
-    o.pa = D.x[i];
-    o.ua = D.f4b[i];
-    o.dia = D.f4a[i];
-    o.rhoa = D.rho[i];
-    o.pla = D.kr[i];
-    o.dt = D.dt[s.scene];
-    o.aii = D.alpha[i];
-    o.radv = D.kr0[i];
-    o.f2 = (D.mpCons && D.nphases > 1) ? D.f2[i] : 0.0f;
-    const int ph = phase_of(o.pa);
-    o.m = D.mass[ph];
-    o.rho0 = D.rho0[ph];
-    return o;
+__device__ __forceinline__ OwnP own_p(const Dev& D, int i) {
+    return OwnP{D.x[i],  D.f4b[i],   D.f4a[i],  D.rho[i],
+                D.kr[i], D.alpha[i], D.kr0[i], (D.mpCons && D.nphases > 1) ? D.f2[i] : 0.0f};
 }
-// one particle's Jacobi update; nw > 0: its fluid neighbours (x and u =
-// d_ii p_l + sum_j d_ij p_j) are in the window
-__device__ __forceinline__ double pressure_particle(const Dev& D, const Slot& s, const OwnP& o, int c, int nw,
-                                                    WinXV win, const List16& L) {
+// lane h of one particle's Jacobi update; nw > 0: its fluid neighbours (x and
+// u = d_ii p_l + sum_j d_ij p_j) are in the window
+template <int K>
+__device__ __forceinline__ double pressure_particle(const Dev& D, const Slot& s, int h, const OwnP& o, int c, int nw,
+                                                    WinXV win, const ListWords<K>* L) {
     if (!s.live) return 0.0;
     const int i = s.i;
     const float4 pa = o.pa, ua = o.ua, dia = o.dia;
-    const float m = o.m, rho0 = o.rho0, rhoa = o.rhoa, pla = o.pla, dt = o.dt;
+    const int ph = phase_of(pa);
+    const float m = mass_of(D, ph), rho0 = rho0_of(D, ph), rhoa = o.rhoa, pla = o.pla, dt = D.dt[s.scene];
     float cji = dt * dt * m / (rhoa * rhoa);
     // own sum_j d_ij p_j
     float sax = ua.x - dia.x * pla, say = ua.y - dia.y * pla, saz = ua.z - dia.z * pla;
@@ -1215,21 +1150,29 @@ __device__ __forceinline__ double pressure_particle(const Dev& D, const Slot& s,
         float tx = sax - ux + cj * gx * pla;
         float ty = say - uy + cj * gy * pla;
         float tz = saz - uz + cj * gz * pla;
-        ff += dot3f(tx, ty, tz, gx, gy, gz);
+        return dot3f(tx, ty, tz, gx, gy, gz);
     };
-    if (nw) {
-        each_in_win16(L, nf_of(c), [&](int k) { return RecW{win.xy[k], win.zv[k]}; },
-                      [&](int, RecW r) { fluid(r.a.x, r.a.y, r.b.x, r.b.y, r.b.z, r.b.w); });
-    } else {
-        each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.f4b[j]}; }, [&](int j, Rec2 rec) {
-            fluid(rec.a.x, rec.a.y, rec.a.z, rec.b.x, rec.b.y, rec.b.z);
-        });
+    auto add = [&](float t) { ff += t; };
+    bool win_on = false;
+    if constexpr (K > 1) {
+        win_on = nw != 0;
+        if (win_on)
+            each_in_win<K>(
+                *L, h, nf_of(c), [&](int k) { return RecW{win.xy[k], win.zv[k]}; },
+                [&](int, const RecW& r) { return fluid(r.a.x, r.a.y, r.b.x, r.b.y, r.b.z, r.b.w); }, add);
     }
-    each_boundary_lu<8>(D, s, nb_of(c), [&](int j) { return D.xb[j]; }, [&](int j, float4 pb) {
-        float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-        float g = kernel_gradfac_sq(dx * dx + dy * dy + dz * dz, D) * pb.w;
-        fb += (sax * dx + say * dy + saz * dz) * g;
-    });
+    if (!win_on)
+        each_fluid<K, 4>(
+            D, s, h, nf_of(c), [&](int j) { return Rec2{D.x[j], D.f4b[j]}; },
+            [&](int, const Rec2& r) { return fluid(r.a.x, r.a.y, r.a.z, r.b.x, r.b.y, r.b.z); }, add);
+    each_boundary<K, 8>(
+        D, s, h, nb_of(c), [&](int j) { return D.xb[j]; },
+        [&](int, float4 pb) {
+            float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
+            float g = kernel_gradfac_sq(dx * dx + dy * dy + dz * dz, D) * pb.w;
+            return make_float2(sax * dx + say * dy + saz * dz, g);
+        },
+        [&](float2 t) { fb += t.x * t.y; });
     float fin = m * ff + rho0 * fb;
     if (cons) fin += o.f2 * pla;
     const float aii = o.aii, radv = o.radv;
@@ -1242,6 +1185,7 @@ __device__ __forceinline__ double pressure_particle(const Dev& D, const Slot& s,
     }
     // the new p_l, published in place: this pass gathers x and
     // sum_j d_ij p_j of its neighbours, never their p_l
+    if (h != 0) return contrib;
     D.f1[i] = t;
     D.kr[i] = t;
     D.xk[i].w = cons ? t * (m * m / (rhoa * rhoa)) : t / (rhoa * rhoa);
@@ -1251,26 +1195,24 @@ __device__ __forceinline__ double pressure_particle(const Dev& D, const Slot& s,
 // relaxed Jacobi update (IISph_M.cpp:312-351) into f1; partial sum of the
 // relative density error of the particles that are not clamped.
 template <bool WIN>
-__global__ __launch_bounds__(256, WIN ? 2 : 1) void k_ii_pressure(Dev D) {
+__global__ __launch_bounds__(WIN ? 256 * WIN_LANES : 256, WIN ? 2 * WIN_LANES : 1) void k_ii_pressure(Dev D) {
     if constexpr (WIN) {
         WIN_XV_DECL(WIN_MAX)
-        window_pair<WIN_PRESSURE, true>(
-            D, [&](const Slot& s, int) { return own_p(D, s); }, [&](int j) { return load_xyz2(D.x, D.f4b, j); },
+        window_tile<WIN_LANES, WIN_PRESSURE, true>(
+            D, [&](int i) { return own_p(D, i); }, [&](int j) { return load_xyz2(D.x, D.f4b, j); },
             [&](int k, const Rec3x2& r) { store_xyz2(win, k, r); },
-            [&](const Slot& s, int c, int nw, const List16& L, const OwnP& o) {
-                return pressure_particle(D, s, o, c, nw, win, L);
+            [&](const Slot& s, int h, int c, int nw, const ListWords<WIN_LANES>& L, const OwnP& o) {
+                return pressure_particle<WIN_LANES>(D, s, h, o, c, nw, win, &L);
             });
     } else {
         __shared__ double lds[4];
-        Slot s = slot_nb(D, true);
+        OwnP o;
+        const Slot s = slot_nb<1>(D, true, [&](int i) { o = own_p(D, i); });
         if (!D.active[s.scene]) {   // uniform: a converged scene's tiles contribute nothing
             if (threadIdx.x == 0) D.partial[2 * s.tile] = 0.0;
             return;
         }
-        const int c = s.live ? D.cnt[s.i] : 0;
-        const OwnP o = own_p(D, s);
-        const List16 L{};
-        write_partial(D, s.tile, 0, pressure_particle(D, s, o, c, 0, WinXV{nullptr, nullptr}, L), lds);
+        write_partial(D, s.tile, 0, pressure_particle<1>(D, s, 0, o, s.c, 0, WinXV{nullptr, nullptr}, nullptr), lds);
     }
 }
 
@@ -1291,14 +1233,14 @@ __global__ __launch_bounds__(256) void k_ii_force(Dev D, int gate) {
     const int i = s.i;
     float4 pa = D.x[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], rho0 = D.rho0[ph], alpha = D.visc[ph];
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph), alpha = visc_of(D, ph);
     float rhoa = D.rho[i], pra = D.kr[i];
     float pa_r2 = pra / (rhoa * rhoa);
     const float Hcs2 = 2.0f * D.Hs * D.cs;
     const bool multi = D.nphases > 1;
     const bool cons = D.mpCons && multi;   // neighbour records carry m^2 p/rho^2
     float ax = 0.f, ay = 0.f, az = 0.f;
-    int c = D.cnt[i];
+    const int c = s.c;
     each_fluid_lu<8>(D, s, nf_of(c), [&](int j) { return D.xk[j]; }, [&](int j, float4 pb) {           // (x, p/rho^2)
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
         float r2 = dx * dx + dy * dy + dz * dz;
@@ -1361,17 +1303,17 @@ __global__ __launch_bounds__(256) void k_pci_rest_density(Dev D) {
 // pci_forceExceptPressure (PciSph.cpp:235-281, viscosity helpers 172-232):
 // a = g + viscosity, p = 0; first prediction x* = x + (v + a dt) dt
 __global__ __launch_bounds__(256) void k_pci_aext(Dev D) {
-    Slot s = slot_nb(D, false);
+    float4 pa, va;
+    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
     if (!s.live) return;
     const int i = s.i;
-    float4 pa = D.x[i], va = D.v[i];
     int ph = phase_of(pa);
-    float m = D.mass[ph], alpha = D.visc[ph], rho0 = D.rho0[ph];
+    float m = mass_of(D, ph), alpha = visc_of(D, ph), rho0 = rho0_of(D, ph);
     float rhoa = va.w;
     const float Hcs2 = 2.0f * D.Hs * D.cs;
     const bool multi = D.nphases > 1;
     float ax = D.gx, ay = D.gy, az = D.gz;
-    int c = D.cnt[i];
+    const int c = s.c;
     each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.v[j]}; }, [&](int j, Rec2 rec) {
         const float4 pb = rec.a, vb = rec.b;   // vb = (v, rho)
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
@@ -1415,17 +1357,17 @@ __global__ __launch_bounds__(256) void k_pci_aext(Dev D) {
 __global__ __launch_bounds__(256) void k_pci_density(Dev D) {
     __shared__ double lds[4];
     __shared__ float ldsf[4];
-    Slot s = slot_nb(D, true);
+    float4 xa;
+    const Slot s = slot_nb<1>(D, true, [&](int i) { xa = D.xk[i]; });
     double contrib = 0.0;
     float emax = 0.0f;
     if (s.live) {
         const int i = s.i;
-        const float4 xa = D.xk[i];
         int ph = phase_of(xa);
-        float m = D.mass[ph], rho0 = D.rho0[ph];
+        float m = mass_of(D, ph), rho0 = rho0_of(D, ph);
         Kahan rho;
         rho.init(m * D.W0);
-        int c = D.cnt[i];
+        const int c = s.c;
         each_fluid_lu<8>(D, s, nf_of(c), [&](int j) { return D.xk[j]; }, [&](int j, float4 pb) {
             float dx = xa.x - pb.x, dy = xa.y - pb.y, dz = xa.z - pb.z;
             float w = kernel_W(fast_sqrt(dx * dx + dy * dy + dz * dz), D);
@@ -1458,17 +1400,16 @@ __global__ __launch_bounds__(256) void k_pci_density(Dev D) {
 // a_p) dt) dt.
 __global__ __launch_bounds__(256) void k_pci_pressure(Dev D) {
     loop_test(D);   // on the density pass's partial sums
-    Slot s = slot_nb(D, true);
+    float4 pa, xa;
+    const Slot s = slot_nb<1>(D, true, [&](int i) { pa = D.vs[i], xa = D.x[i]; });
     if (!s.live) return;
     const int i = s.i;
-    const float4 pa = D.vs[i];
-    const float4 xa = D.x[i];
     int ph = phase_of(xa);
-    float m = D.mass[ph], rho0 = D.rho0[ph];
+    float m = mass_of(D, ph), rho0 = rho0_of(D, ph);
     const float qa = pa.w;
     const bool multi = D.nphases > 1;
     float ax = 0.f, ay = 0.f, az = 0.f;
-    int c = D.cnt[i];
+    const int c = s.c;
     each_fluid_lu<8>(D, s, nf_of(c), [&](int j) { return D.vs[j]; }, [&](int j, float4 pb) {
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
         float g = kernel_gradfac(fast_sqrt(dx * dx + dy * dy + dz * dz), D);
@@ -1582,20 +1523,21 @@ thread_local LaunchTiming g_launch_timing;
 // One block of 256 threads per tile; `lds` bytes of dynamic LDS that the
 // kernel does not use cap how many blocks share a CU (the gather builds of
 // the solver-loop passes run fastest below their register-limited occupancy)
-#define SPH_LAUNCH_GL(kern, blocks, lds, ...)                                                          \
+#define SPH_LAUNCH_GL(kern, blocks, threads, lds, ...)                                                          \
     do {                                                                                               \
         if ((blocks) > 0) {                                                                            \
             const LaunchTiming t_ = g_launch_timing;                                                   \
             if (t_.start) {                                                                            \
                 g_launch_timing = LaunchTiming{};                                                      \
-                hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(256), (lds), st, t_.start, t_.stop, 0, D, \
+                hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(threads), (lds), st, t_.start, t_.stop, 0, D, \
                                       ##__VA_ARGS__);                                                  \
             } else {                                                                                   \
-                hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), (lds), st, D, ##__VA_ARGS__);        \
+                hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), (lds), st, D, ##__VA_ARGS__);    \
             }                                                                                          \
         }                                                                                              \
     } while (0)
-#define SPH_LAUNCH_L(kern, lds, ...) SPH_LAUNCH_GL(kern, tiles_of(D), lds, ##__VA_ARGS__)
+#define SPH_LAUNCH_L(kern, lds, ...) SPH_LAUNCH_GL(kern, tiles_of(D), 256, lds, ##__VA_ARGS__)
+#define SPH_LAUNCH_WIN(kern, ...) SPH_LAUNCH_GL(kern, tiles_of(D), 256 * WIN_LANES, 0, ##__VA_ARGS__)
 #define SPH_LAUNCH(kern, ...) SPH_LAUNCH_L(kern, 0, ##__VA_ARGS__)
 
 void launch_wc_pressure(const Dev& D, hipStream_t st) { SPH_LAUNCH(k_wc_pressure); }
@@ -1616,21 +1558,21 @@ void launch_mlp_gather(const Dev& D, const float* feat, const float* tgt, float*
     if (n > 0)
         hipLaunchKernelGGL(k_mlp_gather, dim3((n + 255) / 256), dim3(256), 0, st, D, feat, tgt, bfeat, btgt, n, seed);
 }
-// Each window pass has two builds: with the LDS window (48-72 KB of LDS per
-// block, two tiles per block) and without (per-lane
+// Each window pass has two builds: with the LDS window (48-76 KB of LDS per
+// block, two lanes a particle) and without (per-lane
 // gathers only: no window LDS and fewer registers, so more waves per SIMD);
 // Dev::winMask picks per pass, and Dev::gatherLds caps the gather build's
 // blocks per CU.
 void launch_df_pass_density(const Dev& D, hipStream_t st) {
-    if (D.winMask & WIN_DENSITY) SPH_LAUNCH_GL(k_df_pass_density<true>, (tiles_of(D) + 1) / 2, 0);
+    if (D.winMask & WIN_DENSITY) SPH_LAUNCH_WIN(k_df_pass_density<true>);
     else SPH_LAUNCH_L(k_df_pass_density<false>, D.gatherLds[0]);
 }
 void launch_df_pass_divergence(const Dev& D, int projected, hipStream_t st) {
-    if (D.winMask & WIN_DIVERGENCE) SPH_LAUNCH_GL(k_df_pass_divergence<true>, (tiles_of(D) + 1) / 2, 0, projected);
+    if (D.winMask & WIN_DIVERGENCE) SPH_LAUNCH_WIN(k_df_pass_divergence<true>, projected);
     else SPH_LAUNCH_L(k_df_pass_divergence<false>, D.gatherLds[1], projected);
 }
 void launch_df_pass_velocity(const Dev& D, hipStream_t st) {
-    if (D.winMask & WIN_VELOCITY) SPH_LAUNCH_GL(k_df_pass_velocity<true>, (tiles_of(D) + 1) / 2, 0);
+    if (D.winMask & WIN_VELOCITY) SPH_LAUNCH_WIN(k_df_pass_velocity<true>);
     else SPH_LAUNCH_L(k_df_pass_velocity<false>, D.gatherLds[2]);
 }
 void launch_df_integrate(const Dev& D, hipStream_t st) { SPH_LAUNCH(k_df_integrate); }
@@ -1645,11 +1587,11 @@ void launch_ii_warm_apply(const Dev& D, const float* y, const float* feat, hipSt
 }
 void launch_ii_targets(const Dev& D, const float* feat, float* tgt, hipStream_t st) { SPH_LAUNCH(k_ii_targets, feat, tgt); }
 void launch_ii_sumdij(const Dev& D, hipStream_t st) {
-    if (D.winMask & WIN_SUMDIJ) SPH_LAUNCH_GL(k_ii_sumdij<true>, (tiles_of(D) + 1) / 2, 0);
+    if (D.winMask & WIN_SUMDIJ) SPH_LAUNCH_WIN(k_ii_sumdij<true>);
     else SPH_LAUNCH_L(k_ii_sumdij<false>, D.gatherLds[3]);
 }
 void launch_ii_pressure(const Dev& D, hipStream_t st) {
-    if (D.winMask & WIN_PRESSURE) SPH_LAUNCH_GL(k_ii_pressure<true>, (tiles_of(D) + 1) / 2, 0);
+    if (D.winMask & WIN_PRESSURE) SPH_LAUNCH_WIN(k_ii_pressure<true>);
     else SPH_LAUNCH_L(k_ii_pressure<false>, D.gatherLds[4]);
 }
 void launch_ii_force_integrate(const Dev& D, int gate, hipStream_t st) { SPH_LAUNCH(k_ii_force, gate); }

@@ -379,8 +379,43 @@ struct Kahan {
 
 // Deterministic FP64 block sum over 256 threads (4 waves): fixed shuffle tree
 // per wave, then waves in order.  Every thread of the block must call it.
+// v of lane l ^ X in a butterfly 32, 16, .., 1 over a wave: cross-row exchanges
+// and row rotations, which take a few cycles where a shuffle goes through the
+// LDS (64 a step).  X = 8, 4, 2, 1 read lane l + X of the row of 16, which
+// holds lane l ^ X's value once the steps above X are done.
+template <int X>
+__device__ __forceinline__ int butterfly(int v) {
+    if constexpr (X == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (threadIdx.x & 32) ? r[0] : r[1];
+    } else if constexpr (X == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (threadIdx.x & 16) ? r[0] : r[1];
+    } else {
+        return __builtin_amdgcn_mov_dpp(v, 0x120 + X, 0xf, 0xf, true);   // row_ror:X
+    }
+}
+template <int X>
+__device__ __forceinline__ double butterfly(double v) {
+    int w[2];
+    __builtin_memcpy(w, &v, 8);
+    w[0] = butterfly<X>(w[0]);
+    w[1] = butterfly<X>(w[1]);
+    __builtin_memcpy(&v, w, 8);
+    return v;
+}
+template <int X>
+__device__ __forceinline__ float butterfly(float v) {
+    return __int_as_float(butterfly<X>(__float_as_int(v)));
+}
+
 __device__ __forceinline__ double block_sum_256(double v, double* lds) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v += butterfly<32>(v);
+    v += butterfly<16>(v);
+    v += butterfly<8>(v);
+    v += butterfly<4>(v);
+    v += butterfly<2>(v);
+    v += butterfly<1>(v);
     if (lane_id() == 0) lds[threadIdx.x >> 6] = v;
     __syncthreads();
     double r = 0.0;
@@ -390,7 +425,12 @@ __device__ __forceinline__ double block_sum_256(double v, double* lds) {
 }
 
 __device__ __forceinline__ float block_max_256(float v, float* lds) {
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+    v = fmaxf(v, butterfly<32>(v));
+    v = fmaxf(v, butterfly<16>(v));
+    v = fmaxf(v, butterfly<8>(v));
+    v = fmaxf(v, butterfly<4>(v));
+    v = fmaxf(v, butterfly<2>(v));
+    v = fmaxf(v, butterfly<1>(v));
     if (lane_id() == 0) lds[threadIdx.x >> 6] = v;
     __syncthreads();
     float r = 0.0f;
