@@ -460,13 +460,12 @@ __global__ __launch_bounds__(256) void k_order_boundary(Dev D, const uint32_t* _
 // global memory directly (6 or 8 groups: LDS per block against blocks per
 // CU, chosen by the autotuner).  Both forms hold the same entries in the
 // same order.
-// Bound: on a large scene the candidate loop (about 216 candidates a
-// particle, 16 B of L1 return and fifteen VALU operations each); on a small
-// one the latency of a block's serial chain.  The loop's short form, the slot
+// Bound by the candidate loop (about 216 candidates a particle, 16 B of L1
+// return and fifteen VALU operations each); small scenes have a builder of
+// their own (k_neighbours_quarter).  The loop's short form, the slot
 // bounds from the rows' end lanes only and flushing without barriers took it
-// from 887 to 740 us at 4,000,752 particles, 234 to 176 us at 1,000,000, 100
-// to 77 us at 328,233 and 54 to 41 us at 1,728 (six groups).  Not kept: the
-// next group's loads issued before this group's tests (4 % slower at 4M), the
+// from 887 to 740 us at 4,000,752 particles, 234 to 176 us at 1,000,000 and
+// 100 to 77 us at 328,233 (six groups).  Not kept: the next group's loads issued before this group's tests (4 % slower at 4M), the
 // nine rows in one rolled loop (25 % slower).
 template <int NB_STAGE_GROUPS>
 __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
@@ -643,7 +642,7 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
             }
         }
     };
-    int nbn = 0, over = 0, zero = 0;
+    int nbn = 0, zero = 0;
     // Candidate loop of one kind (fluid or boundary), candidates four at a
     // time (four loads in flight, tested in order).  A candidate's entry is
     // stored in LDS at the next free entry before the test decides (a miss
@@ -653,8 +652,8 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
     // list width, the self index compared in the particle's own row only
     // (the one row run that holds it), and coincident pairs counted only when
     // the smallest of the four squared distances is zero.  Otherwise entries
-    // past the LDS stage go to global memory and entries past the list width
-    // are counted.  n: entries found.
+    // past the LDS stage go to global memory, those past the list width
+    // nowhere.  n: entries found.
     auto candidates = [&](auto packed_c, auto fluid_c, const int2* runs, const float4* __restrict__ xs, int cap,
                           int slot0, int4* list16, int* list32, int& n) {
         constexpr bool PK = decltype(packed_c)::value, FLUID = decltype(fluid_c)::value;
@@ -694,13 +693,9 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
                             if (PK) st16[(n << 8) + tid] = uint16_t(j + bias);
                             else st[(n << 8) + tid] = j;
                         }
-                        if (hit[k] && n >= STAGE) {
-                            if (n < cap) {
-                                if (PK) put16(list16, n, bias, j);
-                                else put(list32, n, j);
-                            } else {
-                                ++over;
-                            }
+                        if (hit[k] && n >= STAGE && n < cap) {
+                            if (PK) put16(list16, n, bias, j);
+                            else put(list32, n, j);
                         }
                         n += hit[k];
                     }
@@ -758,10 +753,251 @@ __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
     // stored fluid entries | fluid neighbours found << 8 | boundary << 16 | phase << 24
     if (i < D.npad) D.cnt[i] = cf | (act ? min(nf, 255) : 0) << 8 | (cb << 16) | ((act ? int(pa.w) : 0) << 24);
     if (!act) return;
-    int tm = nf + nbn - REF_NEIGHBOUR_CAP;
+    const int tm = nf + nbn - REF_NEIGHBOUR_CAP, over = max(nf - NBF_CAP, 0) + max(nbn - NBB_CAP, 0);
     if (tm > 0) atomicAdd(&D.counters[C_TOO_MANY], tm);
     if (over > 0) atomicAdd(&D.counters[C_LIST_OVF], over);
     if (zero > 0) atomicAdd(&D.counters[C_ZERO_DIS], zero);
+}
+
+// The list builder of scenes that leave the chip's CUs idle (launch_neighbours):
+// a block takes a quarter of a tile, 64 particles, and a wave one of their nine
+// row runs.  A tile's candidates (55,000 pairs) otherwise all pass through one
+// CU, whose arithmetic they keep busy for 20,000 cycles; a quarter's take a
+// fourth, and the chain of each thread is one row's.  Hits are bits of a mask,
+// so the rows' counts are known before anything is stored, and the entries go
+// to their places of the list in LDS, whose groups the waves then write out.
+// Rows in one loop and both kinds of neighbour in one copy of the code: on a
+// small scene a kernel's instructions are read from memory once a launch (the
+// 53 KB of k_neighbours<6> cost more than its loads).
+// The slot bounds come from the table's entries at the ends of the tile's rows,
+// so the table has to be filled (Dev::cellRuns).  Between two particles of a row
+// that are far apart they may take in a gap that k_neighbours leaves out; the
+// lists hold the same neighbours in the same order.
+// Bound by the pairs' arithmetic on the CUs that have a block, and under
+// 10,000 particles by the chain of its phases: 1,728 particles 34 -> 10.8 us,
+// 15,625 35 -> 11.8.
+constexpr int NBQ_ROWS = 9, NBQ_BATCH = 8;
+__global__ __launch_bounds__(64 * NBQ_ROWS) void k_neighbours_quarter(Dev D) {
+    __shared__ int sRow[256], sCx[256], sOrd[256];
+    __shared__ int sWave[4], sFirst[NB16_ROWS], sLast[NB16_ROWS];
+    __shared__ int sBase[2 * 32], sKey[32], sOverflow;
+    __shared__ int sWin[33];                  // as in k_neighbours
+    __shared__ int sCount[2][NBQ_ROWS][64];
+    __shared__ int sList[NBF_CAP + NBB_CAP][64];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = blockIdx.x >> 2, p = (int)(blockIdx.x & 3) * 64 + lane, i = tile * 256 + p;
+    const float4 pa = D.x[i];
+    const int valid = D.tileValid[tile];
+    const bool act = p < valid;
+    if (valid <= p - lane && p != lane) {     // uniform: none of the quarter (the first has the tile's table)
+        if (w == 0) D.cnt[i] = 0;
+        return;
+    }
+    const SceneGrid G = D.grids[D.tileScene[tile]];
+    // the tile's rows
+    if (tid < 256) {
+        int cx = 0, cy = 0, cz = 0;
+        if (tid < valid) cell_of(G, D.x[tile * 256 + tid], cx, cy, cz);
+        sRow[tid] = tid < valid ? cz * G.ny + cy : -1;
+        sCx[tid] = cx;
+    }
+    if (tid < NB16_ROWS) sFirst[tid] = sLast[tid] = -1;
+    if (tid == 0) sOverflow = 0;
+    __syncthreads();
+    const int row = tid < 256 ? sRow[tid] : -1;
+    const bool first = row >= 0 && (tid == 0 || sRow[tid - 1] != row);
+    const unsigned long long bal = __ballot(first);
+    if (w < 4 && lane == 0) sWave[w] = __popcll(bal);
+    __syncthreads();
+    const int rows = sWave[0] + sWave[1] + sWave[2] + sWave[3];
+    if (tid < 256) {
+        int ord = __popcll(bal & ((2ull << lane) - 1ull)) - 1;
+        for (int k = 0; k < w; ++k) ord += sWave[k];
+        sOrd[tid] = ord;
+        if (row >= 0 && ord < NB16_ROWS) {
+            if (first) sFirst[ord] = tid;
+            if (tid == 255 || sRow[tid + 1] != row) sLast[ord] = tid;
+        }
+    }
+    __syncthreads();
+    // row run r of the particles of a row: the key of its first cell, or -1
+    auto row_key = [&](int row, int r) {
+        const int z = row / G.ny + r / 3 - 1, y = row % G.ny + r % 3 - 1;
+        return z >= 0 && z < G.nz && y >= 0 && y < G.ny
+                   ? int(G.keyBase + (uint32_t)D.rowRank[G.rowBase + z * G.ny + y] * (uint32_t)G.nx)
+                   : -1;
+    };
+    // per slot: the tile's run, [start of the first particle's, end of the last's)
+    if (tid < 64) {
+        const int slot = lane & 31, o = slot / 9;
+        int base = INT_MAX, len = 0;
+        if (rows <= NB16_ROWS && o < rows) {
+            const int k = row_key(sRow[sFirst[o]], slot % 9);
+            if (lane < 32) sKey[slot] = k;
+            if (k >= 0) {
+                const int2* __restrict__ table = lane < 32 ? D.cellF : D.cellB;
+                const int s = table[k + max(sCx[sFirst[o]] - 1, 0)].x, e = table[k + min(sCx[sLast[o]] + 1, G.nx - 1)].y;
+                if (e > s) {
+                    base = s;
+                    len = e - s;
+                }
+            }
+        }
+        sBase[lane] = base;
+        if (len > (1 << NB16_OFF_BITS)) sOverflow = 1;
+        if (lane >= 32) len = 0;
+        int incl = len;
+        for (int off = 1; off < 32; off <<= 1) {
+            const int t = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += t;
+        }
+        if (lane < 32) sWin[lane] = (incl - len) - (lane << NB16_OFF_BITS);
+        if (lane == 31) sWin[32] = incl;
+    }
+    __syncthreads();
+    const bool packed = rows <= NB16_ROWS && sOverflow == 0;
+    const bool win = packed && sWin[32] <= WIN_MAX;
+    const int ord = sOrd[p], cx = sCx[p];
+    auto bias16 = [&](int slot) { return packed ? (slot << NB16_OFF_BITS) - sBase[slot] : 0; };
+    // the wave's run of each kind, and the hits of its first 64 candidates
+    const int key = act ? (rows <= NB16_ROWS ? sKey[ord * 9 + w] : row_key(sRow[p], w)) : -1;
+    int2 runs[2];
+#pragma unroll
+    for (int kind = 0; kind < 2; ++kind) {
+        const int2* __restrict__ table = kind ? D.cellB : D.cellF;
+        const int k = key >= 0 ? key + cx : 0;
+        runs[kind].x = table[key >= 0 && cx > 0 ? k - 1 : k].x;
+        runs[kind].y = table[key >= 0 && cx + 1 < G.nx ? k + 1 : k].y;
+        if (key < 0 || runs[kind].y < runs[kind].x) runs[kind].y = runs[kind].x;
+    }
+    unsigned long long mask[2];
+    int zero = 0;
+    const int self = w == 4 ? i : -1;         // the row run that holds the particle itself
+    // a longer run, candidate by candidate
+    auto walk = [&](int kind, int2 rr, auto&& each) {
+        const float4* __restrict__ xs = kind ? D.xb : D.x;
+#pragma unroll 1
+        for (int j = rr.x; j < rr.y; ++j) {
+            const float l2 = dis_square_exact(pa, xs[j]);
+            if (l2 < D.h2 && (kind || j != self)) each(j, l2);
+        }
+    };
+#pragma unroll 1
+    for (int kind = 0; kind < 2; ++kind) {
+        const int2 rr = kind ? runs[1] : runs[0];
+        const float4* __restrict__ xs = kind ? D.xb : D.x;
+        const int len = rr.y - rr.x;
+        unsigned long long m = 0, z = 0;
+        int n = 0;
+        if (len <= 64) {
+#pragma unroll 1
+            for (int k0 = 0; k0 < len; k0 += NBQ_BATCH) {
+                // (up to X_TAIL records past the run are read, and not used)
+                const float4* __restrict__ xg = xs + rr.x + k0;
+                float4 q[NBQ_BATCH];
+                unsigned mk = 0, zk = 0;
+#pragma unroll
+                for (int k = 0; k < NBQ_BATCH; ++k) q[k] = xg[k];
+#pragma unroll
+                for (int k = 0; k < NBQ_BATCH; ++k) {
+                    const float l2 = dis_square_exact(pa, q[k]);
+                    mk |= l2 < D.h2 ? 1u << k : 0u;
+                    zk |= l2 == 0.0f ? 1u << k : 0u;
+                }
+                m |= (unsigned long long)mk << k0;
+                z |= (unsigned long long)zk << k0;
+            }
+            unsigned long long in = len == 64 ? ~0ull : (1ull << len) - 1ull;
+            if (kind == 0 && self >= rr.x && self < rr.y) in &= ~(1ull << (self - rr.x));
+            m &= in;
+            n = __popcll(m);
+            zero += __popcll(z & m);
+        } else {
+            walk(kind, rr, [&](int, float l2) {
+                ++n;
+                zero += l2 == 0.0f;
+            });
+        }
+        if (kind) mask[1] = m;
+        else mask[0] = m;
+        sCount[kind][w][lane] = n;
+    }
+    __syncthreads();
+    // the rows in order: each wave's entries to their places
+    int found[2];
+#pragma unroll
+    for (int kind = 0; kind < 2; ++kind) {
+        int k = 0, total = 0;
+#pragma unroll
+        for (int r = 0; r < NBQ_ROWS; ++r) {
+            if (r == w) k = total;
+            total += sCount[kind][r][lane];
+        }
+        found[kind] = total;
+        const int cap = kind ? NBB_CAP : NBF_CAP, row0 = kind ? NBF_CAP : 0;
+        const int2 rr = runs[kind];
+        const int bias = rr.y > rr.x ? bias16(32 * kind + ord * 9 + w) : 0;
+        if (rr.y - rr.x <= 64) {
+#pragma unroll 1
+            for (unsigned long long m = mask[kind]; m; m &= m - 1) {
+                if (k < cap) sList[row0 + k][lane] = rr.x + __ffsll((long long)m) - 1 + bias;
+                ++k;
+            }
+        } else {
+            walk(kind, rr, [&](int j, float) {
+                if (k < cap) sList[row0 + k][lane] = j + bias;
+                ++k;
+            });
+        }
+    }
+    const int nf = found[0], nbn = found[1];
+    const int cf = act ? min(nf, NBF_CAP) : 0, cb = act ? min(nbn, NBB_CAP) : 0;
+    __syncthreads();
+    // groups of eight entries, padded to four: one packed group, or two of four
+#pragma unroll 1
+    for (int t = w; t < (NBF_CAP + NBB_CAP) / 8; t += NBQ_ROWS) {
+        const bool fluid = t < NBF_CAP / 8;
+        const int g = fluid ? t : t - NBF_CAP / 8, n = fluid ? cf : cb, padded = (n + 3) & ~3;
+        if (8 * g >= padded) continue;
+        // pads: the particle itself, or the far dummy particle
+        const int pad = fluid ? (packed ? bias16(ord * 9 + 4) : 0) + i : packed ? NB16_DUMMY << NB16_OFF_BITS : D.nb;
+        int e[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) e[q] = 8 * g + q < n ? sList[8 * t + q][lane] : pad;
+        if (packed) {
+            int v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = (e[2 * q] & 0xffff) | e[2 * q + 1] << 16;
+            (fluid ? D.nbF16 : D.nbB16)[(size_t)g * D.ncap + i] = make_int4(v[0], v[1], v[2], v[3]);
+            if (fluid && win) {
+                auto to_win = [&](unsigned x) { return (x + (unsigned)sWin[x >> NB16_OFF_BITS]) & 0xffffu; };
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    v[q] = int(to_win((unsigned)e[2 * q] & 0xffffu) | to_win((unsigned)e[2 * q + 1] & 0xffffu) << 16);
+                D.nbW16[(size_t)g * D.ncap + i] = make_int4(v[0], v[1], v[2], v[3]);
+            }
+        } else {
+            int4* const out = reinterpret_cast<int4*>(fluid ? D.nbF : D.nbB) + (size_t)(2 * g) * D.ncap + i;
+            out[0] = make_int4(e[0], e[1], e[2], e[3]);
+            if (8 * g + 4 < padded) out[D.ncap] = make_int4(e[4], e[5], e[6], e[7]);
+        }
+    }
+    if (p == lane && tid < NB16_TAB) {        // the first quarter: the tile's tables
+        const int slot = tid & 31;
+        int v;
+        if (tid == NB16_FLAG) v = packed ? 1 : 0;
+        else if (tid == 32 + NB16_DUMMY) v = D.nb - (NB16_DUMMY << NB16_OFF_BITS);
+        else v = sBase[tid] != INT_MAX ? sBase[tid] - (slot << NB16_OFF_BITS) : 0;
+        D.nbTab[(size_t)tile * NB16_TAB + tid] = v;
+        if (tid < 32) D.nbWin[(size_t)tile * 32 + tid] = packed ? sWin[tid] + (tid << NB16_OFF_BITS) : 0;
+    }
+    if (zero > 0) atomicAdd(&D.counters[C_ZERO_DIS], zero);
+    if (w != 0) return;
+    D.cnt[i] = act ? cf | min(nf, 255) << 8 | cb << 16 | int(pa.w) << 24 : 0;
+    if (!act) return;
+    const int tm = nf + nbn - REF_NEIGHBOUR_CAP, over = max(nf - NBF_CAP, 0) + max(nbn - NBB_CAP, 0);
+    if (tm > 0) atomicAdd(&D.counters[C_TOO_MANY], tm);
+    if (over > 0) atomicAdd(&D.counters[C_LIST_OVF], over);
 }
 
 // ---- boundary --------------------------------------------------------------
@@ -1123,6 +1359,10 @@ void launch_cell_build(const Dev& D, const uint32_t* keys, int n, int2* table, h
 
 void launch_neighbours_variant(const Dev& D, int groups, hipStream_t st) {
     const dim3 g(blocks_for(D.npad)), b(256);
+    if (D.cellRuns && D.npad / TILE <= QUARTER_TILES) {
+        if (D.npad > 0) hipLaunchKernelGGL(k_neighbours_quarter, dim3(4 * (D.npad / TILE)), dim3(64 * NBQ_ROWS), 0, st, D);
+        return;
+    }
     if (groups >= 8) hipLaunchKernelGGL(k_neighbours<8>, g, b, 0, st, D);
     else hipLaunchKernelGGL(k_neighbours<6>, g, b, 0, st, D);
 }

@@ -42,12 +42,20 @@ __shared__ int g_winoff[32];
 // pass starts with two dependent round trips to memory instead of five.  A
 // gated block whose scene has converged has no live particles and returns at
 // once: solver iterations launched past convergence cost little.
-template <int K = 1, class OWN>
+// T threads: 64 where a block takes a quarter of a tile (quarter_blocks).
+template <int K = 1, int T = TILE * K, class OWN>
 __device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated, OWN&& own, int blocks = 0) {
+    static_assert(T == TILE * K || (T == 64 && K == 1), "a tile, or a quarter with one lane a particle");
     Slot s;
-    s.tile = tile_of_block(D.tileMap, blocks ? blocks : (int)gridDim.x);
-    s.i = s.tile * TILE + (int)threadIdx.x / K;
     const int t = threadIdx.x;
+    int at = t / K;   // the particle in the tile
+    if constexpr (T == 64) {
+        s.tile = blockIdx.x >> 2;
+        at += (blockIdx.x & 3) * 64;
+    } else {
+        s.tile = tile_of_block(D.tileMap, blocks ? blocks : (int)gridDim.x);
+    }
+    s.i = s.tile * TILE + at;
     int tab = D.nbTab[(size_t)s.tile * NB16_TAB + (t & (NB16_TAB - 1))];
     int win = D.nbWin[(size_t)s.tile * 32 + (t & 31)];
     const int c = D.cnt[s.i];
@@ -55,13 +63,13 @@ __device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated, OWN&& own, int
     s.scene = D.tileScene[s.tile];
     const int valid = D.tileValid[s.tile];
     const bool on = !gated || D.active[s.scene] != 0;
-    s.live = on && (int)threadIdx.x / K < valid;
+    s.live = on && at < valid;
     s.packed = false;
     s.c = s.live ? c : 0;
     asm volatile("" : "+v"(tab), "+v"(win));   // (else the loads are moved behind the branch)
     if (!on) return s;   // uniform per block
     if (t < NB16_TAB) g_nbtab[t] = tab;
-    else if (t < NB16_TAB + 32) g_winoff[t - NB16_TAB] = win;
+    if (T == 64 ? t < 32 : t >= NB16_TAB && t < NB16_TAB + 32) g_winoff[t & 31] = win;
     __syncthreads();
     s.packed = __builtin_amdgcn_readfirstlane(g_nbtab[NB16_FLAG]) != 0;
     return s;

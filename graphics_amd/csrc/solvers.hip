@@ -344,9 +344,10 @@ __device__ __forceinline__ float density_change(const Dev& D, const Slot& s, int
 // ============================================================ WCSPH ======
 // WcSph::wc_computePressure (WcSph.cpp:99-153): rho (Kahan), Tait p >= 0.
 // Publishes the force pass's gather records: xk = (x, p/rho^2), v.w = rho.
-__global__ __launch_bounds__(256) void k_wc_pressure(Dev D) {
+template <int T>
+__global__ __launch_bounds__(T) void k_wc_pressure(Dev D) {
     float4 pa;
-    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i]; });
+    const Slot s = slot_nb<1, T>(D, false, [&](int i) { pa = D.x[i]; });
     if (!s.live) return;
     const int i = s.i;
     int ph = phase_of(pa);
@@ -363,9 +364,10 @@ __global__ __launch_bounds__(256) void k_wc_pressure(Dev D) {
 // WcSph::wc_computeForce (WcSph.cpp:156-312, 364-436) fused with the
 // Euler-Cromer update and domain removal of SphBase::updateFluids
 // (SphBase.cpp:377-402): writes x2/v2, the caller swaps buffers.
-__global__ __launch_bounds__(256) void k_wc_force(Dev D) {
+template <int T>
+__global__ __launch_bounds__(T) void k_wc_force(Dev D) {
     float4 pa, va;
-    const Slot s = slot_nb<1>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
+    const Slot s = slot_nb<1, T>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
     if (!s.live) return;
     const int i = s.i;
     int ph = phase_of(pa);
@@ -1540,8 +1542,18 @@ thread_local LaunchTiming g_launch_timing;
 #define SPH_LAUNCH_WIN(kern, ...) SPH_LAUNCH_GL(kern, tiles_of(D), 256 * WIN_LANES, 0, ##__VA_ARGS__)
 #define SPH_LAUNCH(kern, ...) SPH_LAUNCH_L(kern, 0, ##__VA_ARGS__)
 
-void launch_wc_pressure(const Dev& D, hipStream_t st) { SPH_LAUNCH(k_wc_pressure); }
-void launch_wc_force_integrate(const Dev& D, hipStream_t st) { SPH_LAUNCH(k_wc_force); }
+// A pass over few tiles runs with a block (one wave) for each quarter of a
+// tile: a gather takes its CU's L1 a cycle a lane, so a tile on one CU waits
+// 17,000 cycles for its pairs' records while most CUs are idle.
+bool quarter_blocks(const Dev& D) { return tiles_of(D) <= QUARTER_TILES; }
+#define SPH_LAUNCH_Q(kern, ...)                                                                  \
+    do {                                                                                         \
+        if (quarter_blocks(D)) SPH_LAUNCH_GL(kern<64>, 4 * tiles_of(D), 64, 0, ##__VA_ARGS__);   \
+        else SPH_LAUNCH(kern<256>, ##__VA_ARGS__);                                               \
+    } while (0)
+
+void launch_wc_pressure(const Dev& D, hipStream_t st) { SPH_LAUNCH_Q(k_wc_pressure); }
+void launch_wc_force_integrate(const Dev& D, hipStream_t st) { SPH_LAUNCH_Q(k_wc_force); }
 void launch_df_density_alpha(const Dev& D, hipStream_t st) { SPH_LAUNCH(k_df_density_alpha<false>, nullptr); }
 void launch_df_density_alpha_warm(const Dev& D, float* feat, hipStream_t st) {
     SPH_LAUNCH(k_df_density_alpha<true>, feat);

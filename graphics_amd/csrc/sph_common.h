@@ -482,10 +482,16 @@ constexpr float DUMMY_FAR = 1.0e15f;   // coordinate of the dummy boundary parti
 // Records of the LDS window of a packed tile at most (12 x 256): a larger
 // window is not staged and the tile's loops gather from memory.
 constexpr int WIN_MAX = 3072;
-// records past the end of a cell run that the list builder may read (its
-// candidate loads come four at a time); the position arrays are allocated
+// Up to this many tiles the list builder and some passes run with a block for
+// each quarter of a tile: there the CUs are not all busy, or take little more
+// than a tile each.  Builder times, quarters / tiles: 32 tiles 12.4 / 38.5 us,
+// 98 16.5 / 39.6, 188 23.2 / 38.6, 250 32 / 39, 313 34 / 41, 375 42 / 43, 1,283
+// 109 / 62.
+constexpr int QUARTER_TILES = 320;
+// records past the end of a cell run that the list builders may read (their
+// candidate loads come four or eight at a time); the position arrays are allocated
 // that much longer
-constexpr int X_TAIL = 3;
+constexpr int X_TAIL = 7;
 
 // ---------------------------------------------------------------------------
 // host-side launchers implemented in the .hip files
