@@ -465,8 +465,9 @@ __global__ __launch_bounds__(256) void k_order_boundary(Dev D, const uint32_t* _
 // their own (k_neighbours_quarter).  The loop's short form, the slot
 // bounds from the rows' end lanes only and flushing without barriers took it
 // from 887 to 740 us at 4,000,752 particles, 234 to 176 us at 1,000,000 and
-// 100 to 77 us at 328,233 (six groups).  Not kept: the next group's loads issued before this group's tests (4 % slower at 4M), the
-// nine rows in one rolled loop (25 % slower).
+// 100 to 77 us at 328,233 (six groups).  Not kept: the next group's loads
+// issued before this group's tests (4 % slower at 4M), the nine rows in one
+// rolled loop (25 % slower).
 template <int NB_STAGE_GROUPS>
 __global__ __launch_bounds__(256) void k_neighbours(Dev D) {
     __shared__ int4 stage[NB_STAGE_GROUPS][256];

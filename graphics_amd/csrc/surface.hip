@@ -4,21 +4,21 @@
 // marching_cubes.cpp:45-120) as HIP kernels:
 //
 //   1. particles binned by a radix sort into cells of h_field = 2 r_h;
-//   2. k_sf_aniso, one thread per particle: Yu & Turk's weighted mean x_bar
+//   2. k_sf_aniso, four lanes per particle: Yu & Turk's weighted mean x_bar
 //      (eq. 10, lambda = 1) and covariance (eq. 9) over the neighbours within
 //      h_field (weights 1 - (r/h_field)^3, eq. 11), symmetric eigen
 //      decomposition (cyclic Jacobi; equal to the SVD of the symmetric
 //      positive covariance), singular values clamped to sigma0 / k_r and
 //      scaled by k_s (eq. 15), G = U diag(1/sigma) U^T; fewer than N_e = 25
 //      neighbours: G = k_n (3 - 2 n / N_e) I at the particle;
-//   3. k_sf_field, one block per tile of 32 x 8 x 16 field nodes: det(G)
-//      W(|G (p - x_bar)|) of every particle whose ellipsoid's box reaches the
-//      tile, summed in LDS in particle order (float, as the reference's
+//   3. k_sf_field, one wave per block of 8 x 4 x 4 field nodes: det(G)
+//      W(|G (p - x_bar)|) of every particle whose ellipsoid reaches the block,
+//      summed in registers in particle order (float, as the reference's
 //      RE_TYPE); the few particles whose box reaches further than one cell
-//      from them are added by k_sf_splat_far (one block per particle, FP32
-//      atomics);
-//   4. marching cubes: a count pass per cube, an exclusive scan, an emit pass
-//      writing triangles in cube order (x fastest, then y, then z).
+//      from them, and all of them where the particles touch few nodes, are
+//      added by k_sf_splat (one block per particle, FP32 atomics);
+//   4. marching cubes: a count pass over units of nodes, an exclusive scan, a
+//      pass writing triangles in cube order (x fastest, then y, then z).
 #include "mc_table.h"
 #include "sph_common.h"
 #include "sphgpu.h"
@@ -62,7 +62,8 @@ struct SurfRec {          // per particle: ellipsoid centre, symmetric G, det(G)
 
 struct SurfBox {          // per particle: field nodes searched (lo..hi per axis)
     int lo[3], hi[3];
-    int empty, far;       // no node of the grid; reaches further than one cell (k_sf_splat_far)
+    short empty, far;     // no node of the grid; reaches further than one cell (k_sf_splat)
+    int cut;              // the box may leave out nodes within the support
 };
 
 __device__ __forceinline__ int cell_axis(float v, float mn, float inv, int n) {
@@ -174,6 +175,13 @@ __device__ __forceinline__ void each_near(const SurfParams& S, const float4* __r
         }
 }
 
+// Whether the nodes p - e .. p + e + 1 hold all within w nodes of a point whose
+// coordinate in nodes, cut towards zero, is p.  Above zero the next nodes outside are
+// at least e + 1 away (at w itself the kernel is zero), below one less.
+__device__ __forceinline__ bool holds(int e, float w, bool above) {
+    return float(e) >= w + 1.0f || (above && float(e + 1) >= w * 0.99999f);
+}
+
 // The nodes with |G d| <= rh lie in the ellipsoid's bounding box, whose
 // half-width along axis a is rh sqrt(sum_b (G^-1)_ab^2) (G symmetric); it is
 // searched instead of the cube of half-width ext (the largest stretch along
@@ -192,10 +200,13 @@ __device__ __forceinline__ SurfBox box_of(const SurfParams& S, const SurfRec& o,
     for (int a = 0; a < 3; ++a) {
         const long long p = int((xb[a] - S.fmin[a]) / S.cell);   // (an int even far outside the grid)
         int e = o.ext;
+        bool whole = false;
         if (dg > 0.0f) {
             const float w = S.rh * half[a] / dg / S.cell;    // half-width in nodes
             if (w < float(o.ext)) e = min(o.ext, int(w) + 2);
+            whole = holds(e, w, xb[a] >= S.fmin[a]);
         }
+        if (!whole) b.cut = 1;
         b.lo[a] = int(max(p - e, 0LL));
         b.hi[a] = int(min(p + e + 1, (long long)S.fnum[a] - 1));
         if (b.hi[a] < b.lo[a]) b.empty = 1;
@@ -301,6 +312,7 @@ __global__ __launch_bounds__(256) void k_sf_sphere(SurfParams S, const float4* _
     SurfBox b{};
     for (int a = 0; a < 3; ++a) {
         const long long c = int((xb[a] - S.fmin[a]) / S.cell);
+        if (!holds(S.hcells, S.rh / S.cell, xb[a] >= S.fmin[a])) b.cut = 1;
         b.lo[a] = int(max(c - S.hcells, 0LL));
         b.hi[a] = int(min(c + S.hcells + 1, (long long)S.fnum[a] - 1));
         if (b.hi[a] < b.lo[a]) b.empty = 1;
@@ -341,30 +353,37 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// Field nodes of one tile.  Each wave owns a quarter of its z layers in LDS: it
-// looks through the particles of the cells that can reach them, 64 at a time,
-// each lane setting up its own particle's box, and adds those that meet its
-// layers one after another, its lanes over the nodes of the common box.  One
-// wave alone writes a node, in particle order, so there are no atomics and the
-// sums are the same every run.  Bound by the arithmetic of the nodes (about 50
-// operations each; the boxes hold twice the nodes of the ellipsoids).  One
-// block per particle with FP32 atomics to memory took 5.6 ms for 120,000
-// particles and 22 million nodes, at the rate of the atomics (46 G/s); the
-// tiles take 2.2 ms.  Two nodes a lane at a time: 10 % slower.
-template <int FT_X, int FT_Y, int FT_Z>
-__global__ __launch_bounds__(256) void k_sf_field(SurfParams S, const SurfRec* __restrict__ rec,
-                                                  const SurfBox* __restrict__ box, const int2* __restrict__ ranges,
-                                                  int tx, int ty, float* __restrict__ field) {
-    constexpr int FT_SLAB = FT_X * FT_Y * (FT_Z / 4);   // nodes of a wave's layers
-    __shared__ float acc[4][FT_SLAB];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    float* const sum = acc[wave];
-    for (int k = lane; k < FT_SLAB; k += 64) sum[k] = 0.0f;
+// Field nodes of one block of 8 x 4 x 4 a wave (two nodes a lane), four blocks
+// along x a workgroup.  The wave looks through the particles of the cells that
+// can reach its nodes, 64 at a time: each lane takes one, sets up u = G (p -
+// x_bar), which is linear in the three node offsets, at the block's first node,
+// and drops it where its box misses the block or |u| at the block's centre
+// exceeds the support by more than |G| times the block's half diagonal.  The
+// particles left are taken one after another, their u, G and det read from
+// their lane into scalars, and added to the nodes in registers.  One wave alone
+// sums a node, in particle order, so there are no atomics and the sums are the
+// same every run.
+// Bound by the arithmetic: 0.92 G wave instructions, nine tenths of the time,
+// for 120,000 particles and 22 million nodes (1.69 ms).  Boxes of the particles
+// over tiles of nodes in LDS took 2.5 ms (index arithmetic for each node, and
+// a tile's edge cuts the boxes into parts that fill few lanes); one block per
+// particle with FP32 atomics to memory 5.6 ms, at the rate of the atomics (46
+// G/s).
+constexpr int FB_X = 8, FB_Y = 4, FB_Z = 4, FB_WAVES = 4;
+__global__ __launch_bounds__(64 * FB_WAVES) void k_sf_field(SurfParams S, const SurfRec* __restrict__ rec,
+                                                          const SurfBox* __restrict__ box,
+                                                          const int2* __restrict__ ranges, int tx, int ty,
+                                                          float* __restrict__ field) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int bx = blockIdx.x % tx, by = (blockIdx.x / tx) % ty, bz = blockIdx.x / (tx * ty);
     // the wave's nodes [n0, n1]
-    const int n0[3] = {bx * FT_X, by * FT_Y, bz * FT_Z + wave * (FT_Z / 4)};
-    const int n1[3] = {min(n0[0] + FT_X, S.fnum[0]) - 1, min(n0[1] + FT_Y, S.fnum[1]) - 1,
-                       min(n0[2] + FT_Z / 4, S.fnum[2]) - 1};
+    const int n0[3] = {(bx * FB_WAVES + wave) * FB_X, by * FB_Y, bz * FB_Z};
+    const int n1[3] = {min(n0[0] + FB_X, S.fnum[0]) - 1, min(n0[1] + FB_Y, S.fnum[1]) - 1,
+                       min(n0[2] + FB_Z, S.fnum[2]) - 1};
+    if (n1[0] < n0[0]) return;      // past the grid (no barrier follows)
+    const int ix = lane & 3, iy = (lane >> 2) & 3, iz = lane >> 4;
+    const float kx = float(ix), ky = float(iy), kz = float(iz);
+    float sum0 = 0.0f, sum1 = 0.0f;   // nodes ix and ix + 4
     // cells of the particles within one cell of the nodes along every axis
     // (a little more, for rounding); positions outside the cell grid are in
     // its border cells on both sides of the comparison
@@ -374,81 +393,90 @@ __global__ __launch_bounds__(256) void k_sf_field(SurfParams S, const SurfRec* _
         c0[a] = cell_axis(S.fmin[a] + float(n0[a]) * S.cell - reach, S.gmin[a], S.ginv, S.gnum[a]);
         c1[a] = cell_axis(S.fmin[a] + float(n1[a]) * S.cell + reach, S.gmin[a], S.ginv, S.gnum[a]);
     }
-    wave_order();
-    if (n1[2] < n0[2]) return;      // layers past the grid (no barrier follows)
-    for (int z = c0[2]; z <= c1[2]; ++z)
-        for (int y = c0[1]; y <= c1[1]; ++y) {
-            // the row's cells lie together
-            int s = INT_MAX, e = 0;
+    const float first[3] = {S.fmin[0] + n0[0] * S.cell, S.fmin[1] + n0[1] * S.cell, S.fmin[2] + n0[2] * S.cell};
+    const int ny = c1[1] - c0[1] + 1, rows = ny * (c1[2] - c0[2] + 1);
+    for (int r0 = 0; r0 < rows; r0 += 64) {
+        // a row of cells a lane: its particles lie together
+        int s = INT_MAX, e = 0;
+        if (r0 + lane < rows) {
+            const int z = c0[2] + (r0 + lane) / ny, y = c0[1] + (r0 + lane) % ny;
+            const int2* __restrict__ cells = ranges + (z * S.gnum[1] + y) * S.gnum[0];
             for (int x = c0[0]; x <= c1[0]; ++x) {
-                const int2 rg = ranges[(z * S.gnum[1] + y) * S.gnum[0] + x];
+                const int2 rg = cells[x];
                 if (rg.y > rg.x) {
                     s = min(s, rg.x);
                     e = max(e, rg.y);
                 }
             }
-            for (int j0 = s; j0 < e; j0 += 64) {
+        }
+        for (unsigned long long in = __ballot(e > s); in; in &= in - 1) {
+            const int row = __ffsll((long long)in) - 1;
+            const int js = __builtin_amdgcn_readlane(s, row), je = __builtin_amdgcn_readlane(e, row);
+            for (int j0 = js; j0 < je; j0 += 64) {
                 const int j = j0 + lane;
-                SurfBox b{};
                 bool meets = false;
-                if (j < e) {
+                SurfBox b{};
+                if (j < je) {
                     b = box[j];
                     meets = !b.far && !b.empty;
                     for (int a = 0; a < 3; ++a) meets = meets && b.lo[a] <= n1[a] && b.hi[a] >= n0[a];
                 }
-                unsigned long long m = __ballot(meets);
-                if (!m) continue;
-                // each lane: its own particle's box within the wave's nodes
-                // (first node and side lengths) and u = G (p - x_bar), which
-                // is linear in the three node offsets, at the first node
-                const SurfRec o = rec[meets ? j : s];
-                const int x0 = max(b.lo[0], n0[0]), y0 = max(b.lo[1], n0[1]), z0 = max(b.lo[2], n0[2]);
-                const int nx = min(b.hi[0], n1[0]) - x0 + 1, nxy = nx * (min(b.hi[1], n1[1]) - y0 + 1);
-                const float l_total = float(nxy * (min(b.hi[2], n1[2]) - z0 + 1));
-                const float l_fx = float(nx), l_fxy = float(nxy), l_rx = fast_rcp(l_fx), l_rxy = fast_rcp(l_fxy);
-                const float dx = S.fmin[0] + x0 * S.cell - o.x, dy = S.fmin[1] + y0 * S.cell - o.y,
-                            dz = S.fmin[2] + z0 * S.cell - o.z;
+                if (!__ballot(meets)) continue;
+                const SurfRec o = rec[meets ? j : js];
+                const float dx = first[0] - o.x, dy = first[1] - o.y, dz = first[2] - o.z;
                 const float l_ux = o.g00 * dx + o.g01 * dy + o.g02 * dz, l_uy = o.g01 * dx + o.g11 * dy + o.g12 * dz,
                             l_uz = o.g02 * dx + o.g12 * dy + o.g22 * dz;
-                const float l_at = float(((z0 - n0[2]) * FT_Y + y0 - n0[1]) * FT_X + x0 - n0[0]);
-                // then the wave takes them one after another, in order
-                for (; m; m &= m - 1) {
+                const float l00 = o.g00 * S.cell, l01 = o.g01 * S.cell, l02 = o.g02 * S.cell, l11 = o.g11 * S.cell,
+                            l12 = o.g12 * S.cell, l22 = o.g22 * S.cell;
+                // |G v| <= (largest absolute row sum) |v|; half diagonal
+                // sqrt(3.5^2 + 1.5^2 + 1.5^2) < 4.1 nodes
+                const float vx = l_ux + 3.5f * l00 + 1.5f * l01 + 1.5f * l02,
+                            vy = l_uy + 3.5f * l01 + 1.5f * l11 + 1.5f * l12,
+                            vz = l_uz + 3.5f * l02 + 1.5f * l12 + 1.5f * l22;
+                const float norm = fmaxf(fmaxf(fabsf(l00) + fabsf(l01) + fabsf(l02), fabsf(l01) + fabsf(l11) + fabsf(l12)),
+                                         fabsf(l02) + fabsf(l12) + fabsf(l22));
+                const float far = S.rh + 4.11f * norm;
+                meets = meets && vx * vx + vy * vy + vz * vz <= 1.001f * far * far;
+                const unsigned long long cut = __ballot(b.cut != 0);
+                for (unsigned long long m = __ballot(meets); m; m &= m - 1) {
                     const int p = __ffsll((long long)m) - 1;
-                    const float total = lane_value(l_total, p), fx = lane_value(l_fx, p), fxy = lane_value(l_fxy, p),
-                                rx = lane_value(l_rx, p), rxy = lane_value(l_rxy, p), ux = lane_value(l_ux, p),
-                                uy = lane_value(l_uy, p), uz = lane_value(l_uz, p), at0 = lane_value(l_at, p),
+                    const float a00 = lane_value(l00, p), a01 = lane_value(l01, p), a02 = lane_value(l02, p),
+                                a11 = lane_value(l11, p), a12 = lane_value(l12, p), a22 = lane_value(l22, p),
                                 det = lane_value(o.det, p);
-                    const float a00 = lane_value(o.g00, p) * S.cell, a01 = lane_value(o.g01, p) * S.cell,
-                                a02 = lane_value(o.g02, p) * S.cell, a11 = lane_value(o.g11, p) * S.cell,
-                                a12 = lane_value(o.g12, p) * S.cell, a22 = lane_value(o.g22, p) * S.cell;
-                    // node q of the box (x fastest) in whole floats: q / nx and
-                    // so on by reciprocals, (q + 0.5) / n being at least 0.5 /
-                    // 256 from a whole number and its rounding 1e-3 of that
-                    for (float q = float(lane); q < total; q += 64.0f) {
-                        const float kz = floorf((q + 0.5f) * rxy), u = q - kz * fxy;
-                        const float ky = floorf((u + 0.5f) * rx), kx = u - ky * fx;
-                        const float vx = ux + kx * a00 + ky * a01 + kz * a02;
-                        const float vy = uy + kx * a01 + ky * a11 + kz * a12;
-                        const float vz = uz + kx * a02 + ky * a12 + kz * a22;
-                        const float q2 = vx * vx + vy * vy + vz * vz;
-                        const int at = int(at0 + kx + ky * float(FT_X) + kz * float(FT_X * FT_Y));
-                        if (q2 <= S.rh2) sum[at] += det * ker_field(S, fast_sqrt(q2));
+                    float ux = kx * a00 + lane_value(l_ux, p), uy = kx * a01 + lane_value(l_uy, p),
+                          uz = kx * a02 + lane_value(l_uz, p);
+                    ux += ky * a01 + kz * a02;
+                    uy += ky * a11 + kz * a12;
+                    uz += ky * a12 + kz * a22;
+                    const float wx = ux + 4.0f * a00, wy = uy + 4.0f * a01, wz = uz + 4.0f * a02;
+                    const float q0 = ux * ux + uy * uy + uz * uz, q1 = wx * wx + wy * wy + wz * wz;
+                    bool in0 = q0 <= S.rh2, in1 = q1 <= S.rh2;
+                    if (cut >> p & 1) {   // uniform: only the nodes of the box
+                        bool yz = true;
+                        for (int a = 1; a < 3; ++a) {
+                            const int at = n0[a] + (a == 1 ? iy : iz);
+                            yz = yz && at >= __builtin_amdgcn_readlane(b.lo[a], p) && at <= __builtin_amdgcn_readlane(b.hi[a], p);
+                        }
+                        const int lo = __builtin_amdgcn_readlane(b.lo[0], p), hi = __builtin_amdgcn_readlane(b.hi[0], p);
+                        in0 = in0 && yz && n0[0] + ix >= lo && n0[0] + ix <= hi;
+                        in1 = in1 && yz && n0[0] + ix + 4 >= lo && n0[0] + ix + 4 <= hi;
                     }
-                    wave_order();
+                    if (in0) sum0 += det * ker_field(S, fast_sqrt(q0));
+                    if (in1) sum1 += det * ker_field(S, fast_sqrt(q1));
                 }
             }
         }
-    for (int k = lane; k < FT_SLAB; k += 64) {
-        const int ix = n0[0] + k % FT_X, iy = n0[1] + k / FT_X % FT_Y, iz = n0[2] + k / (FT_X * FT_Y);
-        if (ix <= n1[0] && iy <= n1[1] && iz <= n1[2])
-            field[((size_t)iz * S.fnum[1] + iy) * S.fnum[0] + ix] = sum[k];
     }
+    if (n0[1] + iy > n1[1] || n0[2] + iz > n1[2]) return;
+    float* const out = field + ((size_t)(n0[2] + iz) * S.fnum[1] + n0[1] + iy) * S.fnum[0] + n0[0];
+    if (n0[0] + ix <= n1[0]) out[ix] = sum0;
+    if (n0[0] + ix + 4 <= n1[0]) out[ix + 4] = sum1;
 }
 
 // One block per particle over the nodes of its box, added to the field with
 // atomics: of every particle (list null, after the field was cleared), or of
-// the listed far ones, whose box reaches past the cells a tile looks through,
-// after the tiles are written.
+// the listed far ones, whose box reaches past the cells a block looks through,
+// after the blocks are written.
 __global__ __launch_bounds__(256) void k_sf_splat(SurfParams S, const SurfRec* __restrict__ rec,
                                                   const SurfBox* __restrict__ box, const int* __restrict__ list,
                                                   const int* __restrict__ count, int n, float* __restrict__ field) {
@@ -710,26 +738,23 @@ int ensure_particles(sphgpu_surfacer* s, int n) {
     return 0;
 }
 
-enum { FIELD_SPLAT, FIELD_TILES, FIELD_SMALL_TILES };
-// Tiles where a kernel radius spans at least six nodes and the particles touch
-// many: below that the tiles' search through the particles takes longer than
-// the atomics.  Field calls of the anisotropic surfacer (MI355X, us: one block
-// per particle / tiles of 32 x 8 x 16 / of 16 x 8 x 8), n particles, r_h = c
-// nodes: 150,000, c 8: 7421 / 3520 / 3973; 60,000, c 8: 3394 / 2387 / 1981;
-// 60,000, c 6: 1534 / 1254 / 1134; 15,000, c 8: 942 / 1269 / 914; 15,000, c 6:
-// 595 / 1103 / 633; 150,000, c 4: 1940 / 2284 / 1947.  The smaller tiles while
-// there are under 4096 of the larger (16 for each of the 256 CUs).
-int field_mode(const sphgpu_surfacer* s, long long n) {
+// Blocks of nodes where the particles touch many nodes; where they touch few,
+// the blocks' search through the particles takes longer than the atomics.
+// Field calls (MI355X, us: one block per particle / blocks of nodes), n
+// particles, r_h = c nodes: anisotropic 150,000, c 8: 7968 / 3265; 60,000, c 8:
+// 3622 / 1964; 60,000, c 4: 1126 / 1049; 15,000, c 6: 657 / 648; 15,000, c 4:
+// 430 / 524; 4,000, c 8: 461 / 386; 4,000, c 6: 346 / 433; isotropic 60,000,
+// c 4: 607 / 599; 15,000, c 6: 307 / 255; 4,000, c 8: 167 / 129; 4,000, c 6:
+// 111 / 124.
+bool field_blocks(const sphgpu_surfacer* s, long long n) {
     const double c = s->S.hcells;
-    if (c < 6.0 || double(n) * c * c * c < 8.0e6) return FIELD_SPLAT;
-    const auto tiles = [s](int a, int t) { return (long long)((s->fnum[a] + t - 1) / t); };
-    return tiles(0, 32) * tiles(1, 8) * tiles(2, 16) < 4096 ? FIELD_SMALL_TILES : FIELD_TILES;
+    return c >= 4.0 && double(n) * c * c * c >= 2.0e6;
 }
 
-template <int X, int Y, int Z>
 void launch_field(sphgpu_surfacer* s) {
-    const int tx = (s->fnum[0] + X - 1) / X, ty = (s->fnum[1] + Y - 1) / Y, tz = (s->fnum[2] + Z - 1) / Z;
-    hipLaunchKernelGGL((k_sf_field<X, Y, Z>), dim3(unsigned(tx) * ty * tz), dim3(256), 0, s->st, s->S,
+    const int tx = (s->fnum[0] + FB_X * FB_WAVES - 1) / (FB_X * FB_WAVES), ty = (s->fnum[1] + FB_Y - 1) / FB_Y,
+              tz = (s->fnum[2] + FB_Z - 1) / FB_Z;
+    hipLaunchKernelGGL(k_sf_field, dim3(unsigned(tx) * ty * tz), dim3(64 * FB_WAVES), 0, s->st, s->S,
                        (const SurfRec*)s->rec, (const SurfBox*)s->box, (const int2*)s->ranges, tx, ty, s->field);
 }
 
@@ -769,15 +794,13 @@ int field_of(sphgpu_surfacer* s, long long n, const float* xyz, bool aniso) {
             hipLaunchKernelGGL(k_sf_sphere, dim3(blocks), dim3(256), 0, s->st, s->S, (const float4*)s->xs, int(n),
                                s->rec, s->box, s->far, nfar);
     }
-    const int mode = field_mode(s, n);
-    if (mode == FIELD_SPLAT) {
+    if (!field_blocks(s, n)) {
         SCHECK(s, hipMemsetAsync(s->field, 0, sizeof(float) * s->nfield, s->st));
         if (n > 0)
             hipLaunchKernelGGL(k_sf_splat, dim3(unsigned(n)), dim3(256), 0, s->st, s->S, (const SurfRec*)s->rec,
                                (const SurfBox*)s->box, (const int*)nullptr, (const int*)nullptr, int(n), s->field);
     } else {
-        if (mode == FIELD_TILES) launch_field<32, 8, 16>(s);
-        else launch_field<16, 8, 8>(s);
+        launch_field(s);
         if (n > 0)
             hipLaunchKernelGGL(k_sf_splat, dim3(unsigned(std::min<long long>(n, 1024))), dim3(256), 0, s->st, s->S,
                                (const SurfRec*)s->rec, (const SurfBox*)s->box, (const int*)s->far, (const int*)nfar, 0,
