@@ -4,10 +4,102 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
+#include <new>
 #include <system_error>
 #include <thread>
+#include <vector>
 
 namespace sphgpu {
+
+namespace {
+struct Stage {
+    int device = 0;
+    char* mem = nullptr;
+    size_t cap = 0;
+    hipEvent_t done[HostRing::kSlots] = {};
+};
+struct Stages {
+    std::mutex lock;
+    std::vector<Stage*> idle;
+    int users = 0;
+};
+// (never destroyed: an object of static duration may release its ring late)
+Stages& stages() {
+    alignas(Stages) static char place[sizeof(Stages)];
+    static Stages* s = new (place) Stages;
+    return *s;
+}
+constexpr size_t kMaxIdle = 2;
+
+void destroy(Stage* s) {
+    if (s->mem) (void)hipHostFree(s->mem);
+    for (hipEvent_t e : s->done)
+        if (e) (void)hipEventDestroy(e);
+    delete s;
+}
+
+// a stage of `bytes`, at most all slots, for transfers on st; nullptr and `err`
+// if there is none to be had
+Stage* borrow(size_t bytes, hipStream_t st, bool& counted, hipError_t& err) {
+    hipDevice_t device = 0;
+    if ((err = hipStreamGetDevice(st, &device)) != hipSuccess) return nullptr;
+    Stage* s = nullptr;
+    Stages& all = stages();
+    {
+        std::lock_guard<std::mutex> l(all.lock);
+        if (!counted) ++all.users;
+        counted = true;
+        for (Stage* o : all.idle)
+            if (o->device == device && (!s || o->cap > s->cap)) s = o;
+        if (s) all.idle.erase(std::find(all.idle.begin(), all.idle.end(), s));
+    }
+    if (!s) {
+        s = new (std::nothrow) Stage;
+        if (!s) {
+            err = hipErrorOutOfMemory;
+            return nullptr;
+        }
+        s->device = device;
+        int current = 0;
+        err = hipGetDevice(&current);
+        if (err == hipSuccess && current != device) err = hipSetDevice(device);   // (an event is its device's)
+        for (hipEvent_t& e : s->done)
+            if (err == hipSuccess) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+        if (current != device) (void)hipSetDevice(current);
+    }
+    const size_t want = std::min((bytes + HostRing::kChunk - 1) / HostRing::kChunk, size_t(HostRing::kSlots)) * HostRing::kChunk;
+    if (err == hipSuccess && s->cap < want) {
+        if (s->mem) (void)hipHostFree(s->mem);
+        s->mem = nullptr;
+        s->cap = 0;
+        void* p = nullptr;
+        if ((err = hipHostMalloc(&p, want)) == hipSuccess) {
+            s->mem = static_cast<char*>(p);
+            s->cap = want;
+        }
+    }
+    if (err == hipSuccess) return s;
+    destroy(s);
+    return nullptr;
+}
+
+void give_back(Stage* s) {
+    Stages& all = stages();
+    {
+        std::lock_guard<std::mutex> l(all.lock);
+        const size_t same = std::count_if(all.idle.begin(), all.idle.end(), [s](Stage* o) { return o->device == s->device; });
+        if (all.users > 0 && same < kMaxIdle) {
+            try {
+                all.idle.push_back(s);
+                return;
+            } catch (const std::bad_alloc&) {
+            }
+        }
+    }
+    destroy(s);
+}
+}  // namespace
 
 hipError_t HostRing::drain(hipStream_t st) {
     if (!used) return hipSuccess;
@@ -16,7 +108,7 @@ hipError_t HostRing::drain(hipStream_t st) {
 }
 
 hipError_t HostRing::reserve(size_t bytes, hipStream_t st) {
-    const size_t want = std::min((bytes + 0xFFFF) & ~size_t(0xFFFF), kSlots * kChunk);
+    const size_t want = std::min((bytes + 0xFFFF) & ~size_t(0xFFFF), kOwn);
     if (want <= cap) return hipSuccess;
     if (hipError_t e = drain(st); e != hipSuccess) return e;
     if (mem) (void)hipHostFree(mem);
@@ -26,20 +118,22 @@ hipError_t HostRing::reserve(size_t bytes, hipStream_t st) {
     if (hipError_t e = hipHostMalloc(&p, want); e != hipSuccess) return e;
     mem = static_cast<char*>(p);
     cap = want;
-    for (hipEvent_t& e : done)
-        if (!e)
-            if (hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming); r != hipSuccess) return r;
     return hipSuccess;
 }
 
 void HostRing::release() {
     if (mem) (void)hipHostFree(mem);
-    for (hipEvent_t& e : done) {
-        if (e) (void)hipEventDestroy(e);
-        e = nullptr;
-    }
     mem = nullptr;
     cap = used = 0;
+    if (!borrowed) return;
+    borrowed = false;
+    std::vector<Stage*> last;
+    Stages& all = stages();
+    {
+        std::lock_guard<std::mutex> l(all.lock);
+        if (--all.users == 0) last.swap(all.idle);
+    }
+    for (Stage* s : last) destroy(s);
 }
 
 namespace {
@@ -66,19 +160,27 @@ int helpers(size_t bytes, size_t from, int most, int chunks) {
 
 hipError_t HostRing::to_device(void* dst, const void* src, size_t bytes, hipStream_t st) {
     if (bytes == 0) return hipSuccess;
-    if (bytes <= kChunk) {
+    if (bytes <= kUpOwnBytes) {
         // small ones one after another into the ring, until it is full
-        if (hipError_t e = reserve(std::max(used + bytes, size_t(1) << 20), st); e != hipSuccess) return e;
-        if (used + bytes > cap)
+        if (used + bytes > cap) {
             if (hipError_t e = drain(st); e != hipSuccess) return e;
+            if (hipError_t e = reserve(2 * bytes, st); e != hipSuccess) return e;
+        }
         char* at = mem + used;
         std::memcpy(at, src, bytes);
         used += (bytes + 255) & ~size_t(255);
         return hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, st);
     }
-    if (hipError_t e = reserve(bytes, st); e != hipSuccess) return e;
-    if (hipError_t e = drain(st); e != hipSuccess) return e;
-    const int n = int((bytes + kChunk - 1) / kChunk), slots = std::min<int>(int(cap / kChunk), n);
+    if (bytes < kUpSlotsBytes) {
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
+        return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    }
+    hipError_t got = hipSuccess;
+    Stage* const stage = borrow(bytes, st, borrowed, got);
+    if (!stage) return got;
+    char* const mem = stage->mem;
+    hipEvent_t* const done = stage->done;
+    const int n = int((bytes + kChunk - 1) / kChunk), slots = std::min<int>(int(stage->cap / kChunk), n);
     std::atomic<int> next{0}, err{int(hipSuccess)};
     std::atomic<int> queued[kSlots];   // the chunk last queued from each slot
     for (auto& q : queued) q.store(-1);
@@ -105,23 +207,36 @@ hipError_t HostRing::to_device(void* dst, const void* src, size_t bytes, hipStre
             queued[s].store(c);
         }
     };
-    used = cap;
-    share(helpers(bytes, kUpThreadedBytes, kUpThreads, n), work);
-    return hipError_t(err.load());
+    share(helpers(bytes, 0, kUpThreads, n), work);
+    const hipError_t e = hipStreamSynchronize(st);   // (the stage is another transfer's next)
+    give_back(stage);
+    return err.load() != int(hipSuccess) ? hipError_t(err.load()) : e;
 }
 
 hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream_t st) {
     if (bytes == 0) return hipStreamSynchronize(st);
-    if (hipError_t e = reserve(bytes, st); e != hipSuccess) return e;
-    used = 0;   // (this transfer follows the queued ones on st, and ends with a wait)
-    if (bytes <= kChunk) {
-        hipError_t e = hipMemcpyAsync(mem, src, bytes, hipMemcpyDeviceToHost, st);
+    auto through = [&](char* at) {
+        hipError_t e = hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e == hipSuccess) std::memcpy(dst, mem, bytes);
+        if (e == hipSuccess) std::memcpy(dst, at, bytes);
+        return e;
+    };
+    if (bytes <= kDownOwnBytes) {
+        if (hipError_t e = reserve(bytes, st); e != hipSuccess) return e;
+        used = 0;   // (this transfer follows the queued ones on st, and ends with a wait)
+        return through(mem);
+    }
+    hipError_t got = hipSuccess;
+    Stage* const stage = borrow(bytes, st, borrowed, got);
+    if (!stage) return got;
+    if (bytes <= kChunk) {
+        const hipError_t e = through(stage->mem);
+        give_back(stage);
         return e;
     }
-    const int n = int((bytes + kChunk - 1) / kChunk), slots = std::min<int>(int(cap / kChunk), n);
-    // slots >= 1: more than one chunk is asked for, so at least one is pinned
+    char* const mem = stage->mem;
+    hipEvent_t* const done = stage->done;
+    const int n = int((bytes + kChunk - 1) / kChunk), slots = std::min<int>(int(stage->cap / kChunk), n);
     std::atomic<int> next{0}, err{int(hipSuccess)};
     std::atomic<int> queued[kSlots];   // the chunk last queued into each slot
     for (auto& q : queued) q.store(-1);
@@ -152,7 +267,8 @@ hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream
         }
     };
     share(helpers(bytes, kThreadedBytes, kMaxThreads, n), work);
-    const hipError_t e = hipStreamSynchronize(st);   // (after an error: no DMA may still write the ring)
+    const hipError_t e = hipStreamSynchronize(st);   // (after an error: no DMA may still write the stage)
+    give_back(stage);
     return err.load() != int(hipSuccess) ? hipError_t(err.load()) : e;
 }
 

@@ -18,31 +18,41 @@ namespace sphgpu {
 // 188 KB 85 -> 16 us, 1.4 MB 139 -> 78 us, 12 MB 777 -> 411 us, 48 MB 4.85 ->
 // 1.44 ms; chunks of 1 and 4 MB were 25 and 4 % slower at 48 MB, eight
 // threads no faster than four.
-// To the device: hipMemcpy from a pageable buffer took 33 us for 64 KB, 47 to
-// 210 for 512 KB and 1.29 ms for 38 MB; through the ring 10, 21 and 0.97 (two
-// threads; one 1.30).
+// To the device the runtime's own copy from a pageable buffer is as fast
+// between 0.5 MB (31 us against 38) and 13 MB (383 / 406); below it costs a
+// call that waits (64 KB 33 -> 10 us), and 38 MB took 1.24 ms against 1.05
+// through the slots (two threads).
+//
+// The host's first touch of new pinned memory costs 0.4 ms a MB, several times
+// the transfer.  So each object owns 1 MB at most, for small transfers,
+// and larger ones borrow a stage of up to 16 MB that the process's objects
+// share: one transfer at a time has it, idle ones are kept (two at most, per
+// device) while an object that has borrowed one lives.
 struct HostRing {
     static constexpr int kSlots = 8;
+    static constexpr size_t kOwn = size_t(1) << 20;
+    static constexpr size_t kDownOwnBytes = size_t(64) << 10;   // to the host: up to this through the own bytes
     static constexpr size_t kChunk = size_t(2) << 20;
     static constexpr size_t kThreadedBytes = 2 * kChunk;
     static constexpr int kMaxThreads = 4;
-    static constexpr size_t kUpThreadedBytes = 4 * kChunk;
+    static constexpr size_t kUpOwnBytes = size_t(512) << 10;    // to the device: up to this through the own bytes,
+    static constexpr size_t kUpSlotsBytes = size_t(32) << 20;   // from this on through the slots
     static constexpr int kUpThreads = 2;
-
-    char* mem = nullptr;
-    size_t cap = 0;                    // bytes pinned, at most kSlots * kChunk
-    hipEvent_t done[kSlots] = {};
 
     // device -> host; waits for everything queued on st before it, and
     // returns with `dst` complete
     hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t st);
-    // host -> device, queued on st; `src` may be changed once it returns.
-    // Every transfer of a ring goes through one stream.
+    // host -> device, queued on st (one past kUpOwnBytes has arrived on return); `src`
+    // may be changed once it returns.  Every transfer of a ring goes through
+    // one stream.
     hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t st);
     void release();
 
 private:
+    char* mem = nullptr;               // the object's own pinned bytes
+    size_t cap = 0;                    // at most kOwn
     size_t used = 0;                   // bytes from `mem` on that queued transfers to the device may still read
+    bool borrowed = false;             // counted among the users of the shared stages
     hipError_t reserve(size_t bytes, hipStream_t st);
     hipError_t drain(hipStream_t st);  // waits for them
 };
