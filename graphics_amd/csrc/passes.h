@@ -42,14 +42,14 @@ __shared__ int g_winoff[32];
 // pass starts with two dependent round trips to memory instead of five.  A
 // gated block whose scene has converged has no live particles and returns at
 // once: solver iterations launched past convergence cost little.
-// T threads: 64 where a block takes a quarter of a tile (quarter_blocks).
-template <int K = 1, int T = TILE * K, class OWN>
+// QUARTER: a block takes a quarter of a tile (quarter_blocks).
+template <int K = 1, bool QUARTER = false, class OWN>
 __device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated, OWN&& own, int blocks = 0) {
-    static_assert(T == TILE * K || (T == 64 && K == 1), "a tile, or a quarter with one lane a particle");
+    static_assert(!QUARTER || 64 * K >= NB16_TAB + 32, "a thread for each word of the tables");
     Slot s;
     const int t = threadIdx.x;
     int at = t / K;   // the particle in the tile
-    if constexpr (T == 64) {
+    if constexpr (QUARTER) {
         s.tile = blockIdx.x >> 2;
         at += (blockIdx.x & 3) * 64;
     } else {
@@ -69,7 +69,7 @@ __device__ __forceinline__ Slot slot_nb(const Dev& D, bool gated, OWN&& own, int
     asm volatile("" : "+v"(tab), "+v"(win));   // (else the loads are moved behind the branch)
     if (!on) return s;   // uniform per block
     if (t < NB16_TAB) g_nbtab[t] = tab;
-    if (T == 64 ? t < 32 : t >= NB16_TAB && t < NB16_TAB + 32) g_winoff[t & 31] = win;
+    else if (t < NB16_TAB + 32) g_winoff[t - NB16_TAB] = win;
     __syncthreads();
     s.packed = __builtin_amdgcn_readfirstlane(g_nbtab[NB16_FLAG]) != 0;
     return s;
@@ -199,7 +199,9 @@ __device__ __forceinline__ void each_boundary_lu(const Dev& D, const Slot& s, in
 // list entries lane h gathers and evaluates entries h * 8/K .. + 8/K - 1 (term),
 // then lane 0 adds the terms of the eight in list order (add), taking the
 // others' with a DPP quad permute, so its sums, the particle's, have the same
-// bits as those of one lane a particle (the other lanes' sums are not used).
+// bits as those of one lane a particle (the other lanes' sums are not used),
+// as long as a term is rounded before it is added: a product that one lane fuses
+// into its sum differs in the last place.
 template <int K>
 struct Lanes {
     static_assert(K == 2 || K == 4, "two or four lanes a particle");

@@ -283,19 +283,28 @@ __global__ __launch_bounds__(256) void k_stats_reduce(Dev D, const double* part,
 // density m W(0) + sum_f m W + sum_b rho0 V_b W, Kahan-compensated
 // (WcSph.cpp:121-138, DFSPH.cpp:132-169, IISph_M.cpp:101-112); coincident
 // pairs contribute W(0), the padding (self) entries nothing.
-__device__ __forceinline__ float density_sum(const Dev& D, const Slot& s, float4 pa, float m, float rho0, int c) {
+template <int K = 1>
+__device__ __forceinline__ float density_sum(const Dev& D, const Slot& s, float4 pa, float m, float rho0, int c,
+                                             int h = 0) {
     const int i = s.i;
     Kahan rho;
     rho.init(m * D.W0);
-    each_fluid_lu<8>(D, s, nf_of(c), [&](int j) { return D.x[j]; }, [&](int j, float4 pb) {
-        float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-        float w = kernel_W(fast_sqrt(dx * dx + dy * dy + dz * dz), D);
-        rho.add(j != i ? m * w : 0.0f);
-    });
-    each_boundary_lu<8>(D, s, nb_of(c), [&](int j) { return D.xb[j]; }, [&](int j, float4 pb) {
-        float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-        rho.add(rho0 * pb.w * kernel_W(fast_sqrt(dx * dx + dy * dy + dz * dz), D));
-    });
+    auto add = [&](float t) { rho.add(t); };
+    each_fluid<K, 8>(
+        D, s, h, nf_of(c), [&](int j) { return D.x[j]; },
+        [&](int j, float4 pb) {
+            float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
+            float w = kernel_W(fast_sqrt(dx * dx + dy * dy + dz * dz), D);
+            return j != i ? m * w : 0.0f;
+        },
+        add);
+    each_boundary<K, 8>(
+        D, s, h, nb_of(c), [&](int j) { return D.xb[j]; },
+        [&](int, float4 pb) {
+            float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
+            return rho0 * pb.w * kernel_W(fast_sqrt(dx * dx + dy * dy + dz * dz), D);
+        },
+        add);
     return rho.s;
 }
 
@@ -344,15 +353,17 @@ __device__ __forceinline__ float density_change(const Dev& D, const Slot& s, int
 // ============================================================ WCSPH ======
 // WcSph::wc_computePressure (WcSph.cpp:99-153): rho (Kahan), Tait p >= 0.
 // Publishes the force pass's gather records: xk = (x, p/rho^2), v.w = rho.
-template <int T>
-__global__ __launch_bounds__(T) void k_wc_pressure(Dev D) {
+// K lanes a particle, in blocks of a quarter of a tile where K > 1
+template <int K>
+__global__ __launch_bounds__(256) void k_wc_pressure(Dev D) {
     float4 pa;
-    const Slot s = slot_nb<1, T>(D, false, [&](int i) { pa = D.x[i]; });
+    const Slot s = slot_nb<K, (K > 1)>(D, false, [&](int i) { pa = D.x[i]; });
     if (!s.live) return;
-    const int i = s.i;
+    const int i = s.i, h = threadIdx.x % K;
     int ph = phase_of(pa);
     float m = mass_of(D, ph), rho0 = rho0_of(D, ph);
-    float density = density_sum(D, s, pa, m, rho0, s.c);
+    float density = density_sum<K>(D, s, pa, m, rho0, s.c, h);
+    if (h != 0) return;
     float p = D.tait_B[ph] * (powf(density / rho0, D.gamma) - 1.0f);
     p = p < 0.0f ? 0.0f : p;
     D.rho[i] = density;
@@ -364,12 +375,12 @@ __global__ __launch_bounds__(T) void k_wc_pressure(Dev D) {
 // WcSph::wc_computeForce (WcSph.cpp:156-312, 364-436) fused with the
 // Euler-Cromer update and domain removal of SphBase::updateFluids
 // (SphBase.cpp:377-402): writes x2/v2, the caller swaps buffers.
-template <int T>
-__global__ __launch_bounds__(T) void k_wc_force(Dev D) {
+template <int K>
+__global__ __launch_bounds__(256) void k_wc_force(Dev D) {
     float4 pa, va;
-    const Slot s = slot_nb<1, T>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
+    const Slot s = slot_nb<K, (K > 1)>(D, false, [&](int i) { pa = D.x[i], va = D.v[i]; });
     if (!s.live) return;
-    const int i = s.i;
+    const int i = s.i, h = threadIdx.x % K;
     int ph = phase_of(pa);
     float m = mass_of(D, ph), rho0 = rho0_of(D, ph), alpha = visc_of(D, ph);
     float rhoa = va.w, pra = D.f1[i];
@@ -378,7 +389,9 @@ __global__ __launch_bounds__(T) void k_wc_force(Dev D) {
     const bool multi = D.nphases > 1;
     float ax = D.gx, ay = D.gy, az = D.gz;
     const int c = s.c;
-    each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.xk[j], D.v[j]}; }, [&](int j, Rec2 rec) {
+    // (x_ab, acceleration factor): the pair's term is their product
+    auto add = [&](float4 t) { ax += t.x * t.w; ay += t.y * t.w; az += t.z * t.w; };
+    each_fluid<K, 4>(D, s, h, nf_of(c), [&](int j) { return Rec2{D.xk[j], D.v[j]}; }, [&](int j, const Rec2& rec) {
         const float4 pb = rec.a, vb = rec.b;   // (x, p/rho^2), (v, rho)
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
         float r2 = dx * dx + dy * dy + dz * dz;
@@ -398,9 +411,9 @@ __global__ __launch_bounds__(T) void k_wc_force(Dev D) {
             float pi = pro < 0.0f ? -nu * pro * fast_rcp(r2 + D.visc_eps) : 0.0f;
             acce += g * (-0.5f * (m + mb) * pi);
         }
-        ax += dx * acce; ay += dy * acce; az += dz * acce;
-    });
-    each_boundary_lu<4>(D, s, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; }, [&](int j, Rec2 rec) {
+        return make_float4(dx, dy, dz, acce);
+    }, add);
+    each_boundary<K, 4>(D, s, h, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; }, [&](int, const Rec2& rec) {
         const float4 pb = rec.a, vb = rec.b;
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
         float r2 = dx * dx + dy * dy + dz * dz;
@@ -410,8 +423,9 @@ __global__ __launch_bounds__(T) void k_wc_force(Dev D) {
         float nu = D.solid_visc * Hcs2 / (rhoa * 2.0f);
         float pi = pro < 0.0f ? -nu * pro * fast_rcp(r2 + D.visc_eps) : 0.0f;
         acce += g * (-rho0 * pb.w * pi);
-        ax += dx * acce; ay += dy * acce; az += dz * acce;
-    });
+        return make_float4(dx, dy, dz, acce);
+    }, add);
+    if (h != 0) return;
     float dt = D.dt[s.scene];
     D.f4a[i] = make_float4(ax, ay, az, 0.0f);
     float4 vn = make_float4(va.x + ax * dt, va.y + ay * dt, va.z + az * dt, 0.0f);
@@ -1542,14 +1556,19 @@ thread_local LaunchTiming g_launch_timing;
 #define SPH_LAUNCH_WIN(kern, ...) SPH_LAUNCH_GL(kern, tiles_of(D), 256 * WIN_LANES, 0, ##__VA_ARGS__)
 #define SPH_LAUNCH(kern, ...) SPH_LAUNCH_L(kern, 0, ##__VA_ARGS__)
 
-// A pass over few tiles runs with a block (one wave) for each quarter of a
-// tile: a gather takes its CU's L1 a cycle a lane, so a tile on one CU waits
-// 17,000 cycles for its pairs' records while most CUs are idle.
+// A pass over few tiles runs with a block for each quarter of a tile and two
+// lanes a particle: the CUs are not all busy, a gather takes its CU's L1 a
+// cycle a lane (17,000 cycles for a tile's pairs), and a lane's chain of pairs
+// is what a wave that has its SIMD to itself takes.  The line is the list
+// builder's.  WCSPH steps, tiles / quarters with one lane / with two: 1,728
+// particles 51 / 47.1 / 42.9 us, 15,625 57 / 49.1 / 45.5, 64,000 85 / 85.6 /
+// 82.3; four lanes 46, 69 and 104.
+constexpr int QUARTER_LANES = 2;
 bool quarter_blocks(const Dev& D) { return tiles_of(D) <= QUARTER_TILES; }
-#define SPH_LAUNCH_Q(kern, ...)                                                                  \
-    do {                                                                                         \
-        if (quarter_blocks(D)) SPH_LAUNCH_GL(kern<64>, 4 * tiles_of(D), 64, 0, ##__VA_ARGS__);   \
-        else SPH_LAUNCH(kern<256>, ##__VA_ARGS__);                                               \
+#define SPH_LAUNCH_Q(kern)                                                           \
+    do {                                                                             \
+        if (quarter_blocks(D)) SPH_LAUNCH_GL(kern<QUARTER_LANES>, 4 * tiles_of(D), 64 * QUARTER_LANES, 0); \
+        else SPH_LAUNCH(kern<1>);                                                    \
     } while (0)
 
 void launch_wc_pressure(const Dev& D, hipStream_t st) { SPH_LAUNCH_Q(k_wc_pressure); }
