@@ -258,19 +258,26 @@ __device__ __forceinline__ void kappa_boundary(const Dev& D, int b, int mode) {
     D.bk[b] = kr;
 }
 
+// Lanes a particle of the iterations' passes (each_fluid): with one, a wave
+// waits for one batch of records after another.  A step of four iterations
+// each, one lane / two: 8,000 particles 307 / 288 us, 88,704 448 / 418, 378,000
+// 765 / 719, 864,000 1483 / 1374; the same bits.
+constexpr int K = 2;
+
 // fluid stiffness (mode 0 density, IISph.cpp:910-965; mode 1 divergence,
 // 1120-1165) -> xk = (x, kappa/rho); partial sums of the loop's error:
 // (rho_adv - rest)/rest (IISph.cpp:956-957), or Drho/Dt dt (1204-1207).
 // Blocks past the tiles take the boundary particles (neither reads what the
 // other writes).
-__global__ __launch_bounds__(256) void k_idf_kappa(Dev D, int mode, int tiles) {
+__global__ __launch_bounds__(256 * K) void k_idf_kappa(Dev D, int mode, int tiles) {
     if ((int)blockIdx.x >= tiles) {
-        kappa_boundary(D, ((int)blockIdx.x - tiles) * 256 + threadIdx.x, mode);
+        kappa_boundary(D, ((int)blockIdx.x - tiles) * 256 * K + threadIdx.x, mode);
         return;
     }
-    __shared__ double lds[4];
+    __shared__ double lds[4 * K], part[TILE];
+    const int h = threadIdx.x % K;
     float4 pa, va;
-    const Slot s = slot_nb<1>(D, true, [&](int i) { pa = D.x[i], va = D.vs[i]; }, tiles);
+    const Slot s = slot_nb<K>(D, true, [&](int i) { pa = D.x[i], va = D.vs[i]; }, tiles);
     if (!D.active[s.scene]) {   // uniform: a converged scene's tiles contribute nothing
         if (threadIdx.x == 0) D.partial[2 * s.tile] = 0.0;
         return;
@@ -283,16 +290,18 @@ __global__ __launch_bounds__(256) void k_idf_kappa(Dev D, int mode, int tiles) {
         const int c = s.c;
         const bool adjust = mode == 0 && D.adjustDensity;
         float sf = 0.0f, sb = 0.0f;
-        each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return Rec2{D.x[j], D.vs[j]}; }, [&](int, Rec2 rec) {
+        // (weight g, v_ab.x_ab): the pair's term is their product
+        each_fluid<K, 4>(D, s, h, nf_of(c), [&](int j) { return Rec2{D.x[j], D.vs[j]}; }, [&](int, const Rec2& rec) {
             const float4 u = rec.b;
             const Pair p = pair_of(D, pa, rec.a);
-            sf += (adjust ? ma : u.w) * p.g * dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz);
-        });
-        each_boundary_lu<4>(D, s, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; }, [&](int, Rec2 rec) {
+            return make_float2((adjust ? ma : u.w) * p.g,
+                               dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz));
+        }, [&](float2 t) { sf += t.x * t.y; });
+        each_boundary<K, 4>(D, s, h, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; }, [&](int, const Rec2& rec) {
             const float4 pb = rec.a, u = rec.b;
             const Pair p = pair_of(D, pa, pb);
-            sb += pb.w * p.g * dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz);
-        });
+            return make_float2(pb.w * p.g, dot3f(va.x - u.x, va.y - u.y, va.z - u.z, p.dx, p.dy, p.dz));
+        }, [&](float2 t) { sb += t.x * t.y; });
         const float dt = D.dt[s.scene], rho = D.rho[i];
         float kr;
         if (mode == 0) {
@@ -306,33 +315,34 @@ __global__ __launch_bounds__(256) void k_idf_kappa(Dev D, int mode, int tiles) {
             kr = dd * D.alpha[i] / dt / rho;
             contrib = (double)dd * (double)dt;
         }
-        D.xk[i] = make_float4(pa.x, pa.y, pa.z, kr);
+        if (h == 0) D.xk[i] = make_float4(pa.x, pa.y, pa.z, kr);
     }
-    write_partial(D, s.tile, 0, contrib, lds);
+    const double sum = tile_sum<K>(contrib, part, lds);
+    if (threadIdx.x == 0) D.partial[2 * s.tile] = sum;
 }
 
 // velocity pass of both loops (IISph.cpp:966-1001, 1166-1206):
 // v_adv -= dt (sum_f m_b (k_a/rho_a + k_b/rho_b) gradW
 //              + sum_b boundaryDensity V_b (k_a/rho_a + k_b/rho_b) gradW)
-__global__ __launch_bounds__(256) void k_idf_velocity(Dev D) {
+__global__ __launch_bounds__(256 * K) void k_idf_velocity(Dev D) {
     loop_test(D);   // on the stiffness pass's partial sums
     float4 pa;
-    const Slot s = slot_nb<1>(D, true, [&](int i) { pa = D.xk[i]; });
+    const Slot s = slot_nb<K>(D, true, [&](int i) { pa = D.xk[i]; });
     if (!s.live) return;
-    const int i = s.i;
+    const int i = s.i, h = threadIdx.x % K;
     const float ka = pa.w;
     const int c = s.c;
     float fx = 0.f, fy = 0.f, fz = 0.f, bx = 0.f, by = 0.f, bz = 0.f;
-    each_fluid_lu<4>(D, s, nf_of(c), [&](int j) { return RecM{D.xk[j], D.pm[j]}; }, [&](int, RecM rec) {
+    // (x_ab, factor): the pair's term is their product
+    each_fluid<K, 4>(D, s, h, nf_of(c), [&](int j) { return RecM{D.xk[j], D.pm[j]}; }, [&](int, const RecM& rec) {
         const Pair p = pair_of(D, pa, rec.x);
-        const float w = p.g * rec.m * (ka + rec.x.w);
-        fx += p.dx * w; fy += p.dy * w; fz += p.dz * w;
-    });
-    each_boundary_lu<4>(D, s, nb_of(c), [&](int j) { return RecM{D.xb[j], D.bk[j]}; }, [&](int, RecM rec) {
+        return make_float4(p.dx, p.dy, p.dz, p.g * rec.m * (ka + rec.x.w));
+    }, [&](float4 t) { fx += t.x * t.w; fy += t.y * t.w; fz += t.z * t.w; });
+    each_boundary<K, 4>(D, s, h, nb_of(c), [&](int j) { return RecM{D.xb[j], D.bk[j]}; }, [&](int, const RecM& rec) {
         const Pair p = pair_of(D, pa, rec.x);
-        const float w = p.g * rec.x.w * (ka + rec.m);
-        bx += p.dx * w; by += p.dy * w; bz += p.dz * w;
-    });
+        return make_float4(p.dx, p.dy, p.dz, p.g * rec.x.w * (ka + rec.m));
+    }, [&](float4 t) { bx += t.x * t.w; by += t.y * t.w; bz += t.z * t.w; });
+    if (h != 0) return;
     const float dt = D.dt[s.scene], cb = dt * D.boundaryDensity;
     float4 v = D.vs[i];
     v.x -= dt * fx + cb * bx;
@@ -360,12 +370,12 @@ void launch_idf_vadv(const Dev& D, int mode, hipStream_t st) {
 }
 
 void launch_idf_kappa(const Dev& D, int mode, hipStream_t st) {
-    const int t = tiles_of(D), g = t + bblocks(D);
-    if (g > 0) hipLaunchKernelGGL(k_idf_kappa, dim3(g), dim3(256), 0, st, D, mode, t);
+    const int t = tiles_of(D), g = t + (D.nb + 256 * K - 1) / (256 * K);
+    if (g > 0) hipLaunchKernelGGL(k_idf_kappa, dim3(g), dim3(256 * K), 0, st, D, mode, t);
 }
 
 void launch_idf_velocity(const Dev& D, hipStream_t st) {
-    if (tiles_of(D) > 0) hipLaunchKernelGGL(k_idf_velocity, dim3(tiles_of(D)), dim3(256), 0, st, D);
+    if (tiles_of(D) > 0) hipLaunchKernelGGL(k_idf_velocity, dim3(tiles_of(D)), dim3(256 * K), 0, st, D);
 }
 
 }  // namespace sphgpu
