@@ -68,7 +68,12 @@ Stage* borrow(size_t bytes, hipStream_t st, bool& counted, hipError_t& err) {
             if (err == hipSuccess) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
         if (current != device) (void)hipSetDevice(current);
     }
-    const size_t want = std::min((bytes + HostRing::kChunk - 1) / HostRing::kChunk, size_t(HostRing::kSlots)) * HostRing::kChunk;
+    // up to a chunk the next power of two: a process that reads 100 KB does not
+    // touch 2 MB for it, and one that reads more each time touches twice that at most
+    // (the first reading of a small mesh 1.64 -> 1.29 ms)
+    size_t want = std::min((bytes + HostRing::kChunk - 1) / HostRing::kChunk, size_t(HostRing::kSlots)) * HostRing::kChunk;
+    if (bytes <= HostRing::kChunk)
+        for (want = 2 * HostRing::kDownOwnBytes; want < bytes;) want *= 2;
     if (err == hipSuccess && s->cap < want) {
         if (s->mem) (void)hipHostFree(s->mem);
         s->mem = nullptr;

@@ -25,7 +25,8 @@ namespace sphgpu {
 //
 // The host's first touch of new pinned memory costs 0.4 ms a MB, several times
 // the transfer.  So each object owns 1 MB at most, for small transfers,
-// and larger ones borrow a stage of up to 16 MB that the process's objects
+// and larger ones borrow a stage (the next power of two up to 2 MB, then whole
+// chunks up to 16 MB) that the process's objects
 // share: one transfer at a time has it, idle ones are kept (two at most, per
 // device) while an object that has borrowed one lives.
 struct HostRing {
