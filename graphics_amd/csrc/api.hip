@@ -315,7 +315,9 @@ int loop_cap(const sphgpu_handle* h, int which) {
 // (DFSPH, PCISPH, IISPH_DF) or in the next iteration's first pass (IISPH,
 // whose partial sums come from its second; the last iteration of a batch is
 // tested by a kernel of its own).  A separate test costs 4.7 us an
-// iteration, 6 % of one at 300,000 particles.
+// iteration, 6 % of one at 300,000 particles.  A handle with fewer tiles than
+// scenes (some, or all, still without fluid) has no block for every scene's
+// test: there each iteration is followed by that kernel.
 void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bool lastOfBatch) {
     const sphgpu_params& P = h->P;
     h->curIter = it;
@@ -328,6 +330,7 @@ void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bo
     const int mode = P.solver == SPHGPU_DFSPH && !div ? 0 : P.solver == SPHGPU_PCISPH ? 2 : 1;
     const float tol = div ? P.divergence_tol : P.density_tol;
     const int minIt = div ? P.min_iter_div : P.min_iter_density, cap = loop_cap(h, which);
+    const bool fused = D.npad / TILE >= D.nscenes;
     auto with_test = [&](Dev q) {
         q.redMode = mode;
         q.redTol = tol;
@@ -336,8 +339,6 @@ void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bo
         return q;
     };
     if (P.solver == SPHGPU_DFSPH) {
-        // (a separate reduction kernel when a scene has no tile to host its test)
-        const bool fused = D.npad / TILE >= D.nscenes;
         if (!div) {
             ProfScope ps(h, "df_pass_density", nf_live(h) * 36.0);
             launch_df_pass_density(D, h->st);
@@ -357,14 +358,12 @@ void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bo
             ProfScope ps(h, !div ? "idf_kappa_density" : "idf_kappa_divergence", nf_live(h) * 36.0);
             launch_idf_kappa(D, which, h->st);
         }
-        const bool fused = D.npad / TILE >= D.nscenes;
         {
             ProfScope ps(h, "idf_velocity", nf_live(h) * 44.0);
             launch_idf_velocity(fused ? with_test(D) : D, h->st);
         }
         if (!fused) launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
     } else if (P.solver == SPHGPU_PCISPH) {
-        const bool fused = D.npad / TILE >= D.nscenes;
         {
             ProfScope ps(h, "pci_density", nf_live(h) * 44.0);
             launch_pci_density(D, h->st);
@@ -381,7 +380,7 @@ void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bo
             // too many for a scene that has just converged, whose result
             // (f4b) nothing reads
             Dev q = D;
-            if (!firstOfBatch) {
+            if (fused && !firstOfBatch) {
                 q = with_test(D);
                 q.active = buf[(it + 1) & 1];
                 q.activeNext = buf[it & 1];
@@ -393,7 +392,7 @@ void launch_iteration(sphgpu_handle* h, int which, int it, bool firstOfBatch, bo
             ProfScope ps(h, "ii_pressure", nf_live(h) * 56.0);
             launch_ii_pressure(D, h->st);
         }
-        if (lastOfBatch) launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
+        if (!fused || lastOfBatch) launch_scene_reduce(D, mode, tol, minIt, cap, h->st);
     }
 }
 

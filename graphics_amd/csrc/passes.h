@@ -453,11 +453,11 @@ __device__ __forceinline__ void scene_reduce_block(const Dev& D, int sc, int mod
     }
 }
 
-// the loop's convergence test in front of a pass (scene b on blocks b, b + gridDim, ...)
+// the loop's convergence test in front of a pass, scene b on block b: a pass that
+// holds it has a block for every scene
 __device__ __forceinline__ void loop_test(const Dev& D) {
-    if (D.redMode >= 0)
-        for (int sc = blockIdx.x; sc < D.nscenes; sc += gridDim.x)
-            scene_reduce_block(D, sc, D.redMode, D.redTol, D.redMinIt, D.redCap, D.activeNext);
+    if (D.redMode >= 0 && (int)blockIdx.x < D.nscenes)
+        scene_reduce_block(D, blockIdx.x, D.redMode, D.redTol, D.redMinIt, D.redCap, D.activeNext);
 }
 
 }  // namespace
