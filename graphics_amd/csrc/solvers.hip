@@ -294,7 +294,7 @@ __device__ __forceinline__ float density_sum(const Dev& D, const Slot& s, float4
         D, s, h, nf_of(c), [&](int j) { return D.x[j]; },
         [&](int j, float4 pb) {
             float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-            float w = kernel_W(fast_sqrt(dx * dx + dy * dy + dz * dz), D);
+            float w = kernel_W(fast_sqrt(dot3y(dx, dy, dz, dx, dy, dz)), D);
             return j != i ? m * w : 0.0f;
         },
         add);
@@ -302,7 +302,7 @@ __device__ __forceinline__ float density_sum(const Dev& D, const Slot& s, float4
         D, s, h, nb_of(c), [&](int j) { return D.xb[j]; },
         [&](int, float4 pb) {
             float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-            return rho0 * pb.w * kernel_W(fast_sqrt(dx * dx + dy * dy + dz * dz), D);
+            return rho0 * pb.w * kernel_W(fast_sqrt(dot3y(dx, dy, dz, dx, dy, dz)), D);
         },
         add);
     return rho.s;
@@ -389,14 +389,21 @@ __global__ __launch_bounds__(256) void k_wc_force(Dev D) {
     const bool multi = D.nphases > 1;
     float ax = D.gx, ay = D.gy, az = D.gz;
     const int c = s.c;
-    // (x_ab, acceleration factor): the pair's term is their product
-    auto add = [&](float4 t) { ax += t.x * t.w; ay += t.y * t.w; az += t.z * t.w; };
+    // (x_ab, acceleration factor): the pair's term is their product.  The terms
+    // are written with their fused operations: the compiler would choose others
+    // for another K, and a scene's bits would depend on the handle's tiles.
+    auto add = [&](float4 t) {
+        ax = __builtin_fmaf(t.x, t.w, ax);
+        ay = __builtin_fmaf(t.y, t.w, ay);
+        az = __builtin_fmaf(t.z, t.w, az);
+    };
     each_fluid<K, 4>(D, s, h, nf_of(c), [&](int j) { return Rec2{D.xk[j], D.v[j]}; }, [&](int j, const Rec2& rec) {
+#pragma clang fp contract(off)
         const float4 pb = rec.a, vb = rec.b;   // (x, p/rho^2), (v, rho)
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-        float r2 = dx * dx + dy * dy + dz * dz;
+        float r2 = dot3y(dx, dy, dz, dx, dy, dz);
         float g = kernel_gradfac(fast_sqrt(r2), D);
-        float pro = (va.x - vb.x) * dx + (va.y - vb.y) * dy + (va.z - vb.z) * dz;
+        float pro = dot3y(va.x - vb.x, va.y - vb.y, va.z - vb.z, dx, dy, dz);
         int phb = multi ? phase_of(D.x[j]) : ph;
         float acce;
         if (phb == ph) {
@@ -406,23 +413,24 @@ __global__ __launch_bounds__(256) void k_wc_force(Dev D) {
         } else {                                      /* SP08 multiphase, WcSph.cpp:220-260 */
             float mb = D.mass[phb], al = 0.5f * (alpha + D.visc[phb]);
             // p/delta^2 with delta = rho/m: p m^2 / rho^2
-            acce = g * (-1.0f / m * (pa_r2 * m * m + pb.w * mb * mb));
+            float pp = -1.0f / m * __builtin_fmaf(mb, pb.w * mb, pa_r2 * m * m);
             float nu = al * Hcs2 / (rhoa + vb.w);
             float pi = pro < 0.0f ? -nu * pro * fast_rcp(r2 + D.visc_eps) : 0.0f;
-            acce += g * (-0.5f * (m + mb) * pi);
+            acce = __builtin_fmaf(g, pp, g * (-0.5f * (m + mb) * pi));
         }
         return make_float4(dx, dy, dz, acce);
     }, add);
     each_boundary<K, 4>(D, s, h, nb_of(c), [&](int j) { return Rec2{D.xb[j], D.vb[j]}; }, [&](int, const Rec2& rec) {
+#pragma clang fp contract(off)
         const float4 pb = rec.a, vb = rec.b;
         float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
-        float r2 = dx * dx + dy * dy + dz * dz;
+        float r2 = dot3y(dx, dy, dz, dx, dy, dz);
         float g = kernel_gradfac(fast_sqrt(r2), D);
         float acce = pra > 0.0f ? g * (-rho0 * pb.w * (pa_r2 * 2.0f)) : 0.0f;
-        float pro = (va.x - vb.x) * dx + (va.y - vb.y) * dy + (va.z - vb.z) * dz;
+        float pro = dot3y(va.x - vb.x, va.y - vb.y, va.z - vb.z, dx, dy, dz);
         float nu = D.solid_visc * Hcs2 / (rhoa * 2.0f);
         float pi = pro < 0.0f ? -nu * pro * fast_rcp(r2 + D.visc_eps) : 0.0f;
-        acce += g * (-rho0 * pb.w * pi);
+        acce = __builtin_fmaf(g, -rho0 * pb.w * pi, acce);
         return make_float4(dx, dy, dz, acce);
     }, add);
     if (h != 0) return;
@@ -1559,8 +1567,9 @@ thread_local LaunchTiming g_launch_timing;
 // A pass over few tiles runs with a block for each quarter of a tile and two
 // lanes a particle: the CUs are not all busy, a gather takes its CU's L1 a
 // cycle a lane (17,000 cycles for a tile's pairs), and a lane's chain of pairs
-// is what a wave that has its SIMD to itself takes.  The line is the list
-// builder's.  WCSPH steps, tiles / quarters with one lane / with two: 1,728
+// is what a wave that has its SIMD to itself takes.  Both builds give the same
+// bits, so a scene's results do not depend on the tiles beside it.  The line is
+// the list builder's.  WCSPH steps, tiles / quarters with one lane / with two: 1,728
 // particles 51 / 47.1 / 42.9 us, 15,625 57 / 49.1 / 45.5, 64,000 85 / 85.6 /
 // 82.3; four lanes 46, 69 and 104.
 constexpr int QUARTER_LANES = 2;

@@ -309,10 +309,11 @@ __device__ __forceinline__ uint32_t morton2(uint32_t a, uint32_t b) {
 }
 
 // cubic spline W(r), SphBase.h:855-871, with q = r/h.
+// (one rounding order, in every kernel: see dot3f)
 __device__ __forceinline__ float kernel_W(float r, const Dev& D) {
     float q = r * D.inv_kh;
-    float qm2 = 2.0f - q;
-    float w1 = D.sigma * (1.0f - 1.5f * q * q + 0.75f * q * q * q);
+    float qm2 = __builtin_fmaf(-r, D.inv_kh, 2.0f);
+    float w1 = D.sigma * __builtin_fmaf(q, 0.75f * q * q, __builtin_fmaf(q, -1.5f * q, 1.0f));
     float w2 = D.sigma * (0.25f * qm2 * qm2 * qm2);
     float w = q <= 1.0f ? w1 : w2;
     return q <= 2.0f ? w : 0.0f;
@@ -330,8 +331,8 @@ __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcp
 // At r = 0 the q <= 1 branch is selected (finite).
 __device__ __forceinline__ float kernel_gradfac(float r, const Dev& D) {
     float q = r * D.inv_kh;
-    float qm2 = 2.0f - q;
-    float g1 = -(D.sigma_h * D.inv_kh) * (3.0f - 2.25f * q);
+    float qm2 = __builtin_fmaf(-r, D.inv_kh, 2.0f);
+    float g1 = -(D.sigma_h * D.inv_kh) * __builtin_fmaf(q, -2.25f, 3.0f);
     float g2 = -0.75f * D.sigma_h * qm2 * qm2 * fast_rcp(r);
     float g = q <= 1.0f ? g1 : g2;
     return q <= 2.0f ? g : 0.0f;
@@ -362,6 +363,11 @@ __device__ __forceinline__ float kernel_gradfac_sq(float r2, const Dev& D) {
 // must round identically.
 __device__ __forceinline__ float dot3f(float ax, float ay, float az, float bx, float by, float bz) {
     return __builtin_fmaf(az, bz, __builtin_fmaf(ay, by, __fmul_rn(ax, bx)));
+}
+// the same, the product of y first: the order the WCSPH passes always had with
+// one lane a particle
+__device__ __forceinline__ float dot3y(float ax, float ay, float az, float bx, float by, float bz) {
+    return __builtin_fmaf(az, bz, __builtin_fmaf(ax, bx, __fmul_rn(ay, by)));
 }
 
 // Kahan-compensated FP32 accumulator.
