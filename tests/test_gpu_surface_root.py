@@ -1,0 +1,39 @@
+"""The surfacer's spline takes a correctly rounded distance, in both forms of the
+field kernel.  All coordinates are dyadic, so that squared distances are exact
+and, near the edge of the support where the spline is k (r_h - r)^3, the value's
+error is that of r: half a last place of r, three times over r_h - r."""
+import numpy as np
+import pytest
+
+from graphics_amd import sphgpu as sg
+
+pytestmark = pytest.mark.gpu
+
+RH, RP, CELL = 0.5, 0.25, 2.0 ** -7
+
+
+@pytest.mark.parametrize("n", [4, 8])   # 64 nodes a radius: one block a particle, blocks of nodes
+def test_distance_is_correctly_rounded(gpu, n):
+    print(f"[surface root] n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    corners = np.array([(i, j, k) for k in (0, 1) for j in (0, 1) for i in (0, 1)][:n], np.float64)
+    # (no two supports meet)
+    x = 0.125 + corners + (2 * corners - 1) * rng.integers(0, 6, (n, 3)) * 2.0 ** -10
+    s = sg.Surfacer((0.0,) * 3, (1.25,) * 3, RP, RH, CELL)
+    s.isotro(x.astype(np.float32))
+    f = s.field().astype(np.float64)
+    at = [s.grid_min[a] + np.arange(s.grid_num[a]) * CELL for a in range(3)]
+    seen = 0
+    for p in x:
+        d2 = ((at[2] - p[2]) ** 2)[:, None, None] + ((at[1] - p[1]) ** 2)[None, :, None] + ((at[0] - p[0]) ** 2)[None, None, :]
+        edge = RH - np.sqrt(d2)
+        pick = (edge >= 2.0 ** -12) & (edge <= 2.0 ** -7)
+        d = edge[pick]
+        want = 16.0 / (np.pi * RH ** 6) * RP ** 3 * d ** 3
+        # r in [1/4, 1/2): half a last place is 2^-26; the constant and three products round too
+        bound = 3.0 * 2.0 ** -26 / d * (1.0 + 2.0 ** -10) + 5.0 * 2.0 ** -24
+        err = np.abs(f[pick] - want) / want
+        seen += d.size
+        assert np.all(err <= bound), (np.count_nonzero(err > bound), d.size)
+    assert seen > 100000
+
