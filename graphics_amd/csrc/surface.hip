@@ -705,6 +705,12 @@ __global__ __launch_bounds__(256) void k_mc_emit(McGrid G, const float* __restri
 
 }  // namespace
 
+struct SurfRecs {          // records in cell order and the particle of each
+    SurfRec* rec = nullptr;
+    uint32_t* vals = nullptr;
+    int cap = 0;
+};
+
 struct sphgpu_surfacer {
     SurfParams S{};
     double fmin[3], cell;
@@ -715,9 +721,9 @@ struct sphgpu_surfacer {
     int cap = 0;
     float* x = nullptr;            // positions as given
     float4* xs = nullptr;          // by cell
-    uint32_t *keys = nullptr, *vals = nullptr;
+    uint32_t* keys = nullptr;
     int2* ranges = nullptr;
-    SurfRec* rec = nullptr;
+    SurfRecs spheres, ellipsoids;  // (apart: the last aniso call's stay for surfacer_particles)
     SurfBox* box = nullptr;
     int* far = nullptr;            // far particles' indices, then their number at [cap]
     HostRing ring;                 // staging of transfers
@@ -728,7 +734,7 @@ struct sphgpu_surfacer {
     uint32_t* mcTmp = nullptr;
     float* mcOut = nullptr;        // triangles
     long long mcOutCap = 0;
-    int nrec = 0;
+    int nrec = 0;                  // particles of the ellipsoids
     std::string err;
 };
 
@@ -752,22 +758,35 @@ int sfail(sphgpu_surfacer* s, int code, const char* fmt, ...) {
 
 int ensure_particles(sphgpu_surfacer* s, int n) {
     if (s->cap > 0 && n <= s->cap) return 0;
-    (void)hipFree(s->x); (void)hipFree(s->xs); (void)hipFree(s->keys); (void)hipFree(s->vals);
-    (void)hipFree(s->rec); (void)hipFree(s->box); (void)hipFree(s->far); (void)hipFree(s->sortMem);
+    (void)hipFree(s->x); (void)hipFree(s->xs); (void)hipFree(s->keys);
+    (void)hipFree(s->box); (void)hipFree(s->far); (void)hipFree(s->sortMem);
     s->cap = 0;
     s->box = nullptr; s->far = nullptr;
-    s->x = nullptr; s->xs = nullptr; s->keys = s->vals = nullptr; s->rec = nullptr; s->sortMem = nullptr;
+    s->x = nullptr; s->xs = nullptr; s->keys = nullptr; s->sortMem = nullptr;
     const int cap = std::max(n, 1024);
     SCHECK(s, hipMalloc(&s->x, 3 * sizeof(float) * cap));
     SCHECK(s, hipMalloc(&s->xs, sizeof(float4) * cap));
     SCHECK(s, hipMalloc(&s->keys, sizeof(uint32_t) * cap));
-    SCHECK(s, hipMalloc(&s->vals, sizeof(uint32_t) * cap));
-    SCHECK(s, hipMalloc(&s->rec, sizeof(SurfRec) * cap));
     SCHECK(s, hipMalloc(&s->box, sizeof(SurfBox) * cap));
     SCHECK(s, hipMalloc(&s->far, sizeof(int) * (size_t(cap) + 1)));
     SCHECK(s, hipMalloc(&s->sortMem, sort_scratch_bytes(cap)));
     sort_scratch_bind(s->sort, s->sortMem, cap);
     s->cap = cap;
+    return 0;
+}
+
+void free_records(SurfRecs& r) {
+    (void)hipFree(r.rec); (void)hipFree(r.vals);
+    r = SurfRecs{};
+}
+
+int ensure_records(sphgpu_surfacer* s, SurfRecs& r, int n) {
+    if (r.cap > 0 && n <= r.cap) return 0;
+    free_records(r);
+    const int cap = std::max(n, 1024);
+    SCHECK(s, hipMalloc(&r.rec, sizeof(SurfRec) * cap));
+    SCHECK(s, hipMalloc(&r.vals, sizeof(uint32_t) * cap));
+    r.cap = cap;
     return 0;
 }
 
@@ -784,11 +803,11 @@ bool field_blocks(const sphgpu_surfacer* s, long long n) {
     return c >= 4.0 && double(n) * c * c * c >= 2.0e6 && s->S.rh >= 0x1p-30f;
 }
 
-void launch_field(sphgpu_surfacer* s) {
+void launch_field(sphgpu_surfacer* s, const SurfRecs& r) {
     const int tx = (s->fnum[0] + FB_X * FB_WAVES - 1) / (FB_X * FB_WAVES), ty = (s->fnum[1] + FB_Y - 1) / FB_Y,
               tz = (s->fnum[2] + FB_Z - 1) / FB_Z;
     hipLaunchKernelGGL(k_sf_field, dim3(unsigned(tx) * ty * tz), dim3(64 * FB_WAVES), 0, s->st, s->S,
-                       (const SurfRec*)s->rec, (const SurfBox*)s->box, (const int2*)s->ranges, tx, ty, s->field);
+                       (const SurfRec*)r.rec, (const SurfBox*)s->box, (const int2*)s->ranges, tx, ty, s->field);
 }
 
 // the field of n particles: binned, ellipsoids (aniso) or spheres, tiles
@@ -806,7 +825,8 @@ int field_of(sphgpu_surfacer* s, long long n, const float* xyz, bool aniso) {
         i = end;
     }
     SCHECK(s, s->ring.to_device(s->x, xyz, 3 * sizeof(float) * size_t(n), s->st));
-    s->nrec = int(n);
+    // (an isotropic call of as many particles leaves the last aniso call's records)
+    if (aniso || n != s->nrec) s->nrec = 0;
     const int blocks = int((n + 255) / 256);
     const bool inBlocks = field_blocks(s, n);
     if (!inBlocks) SCHECK(s, hipMemsetAsync(s->field, 0, sizeof(float) * s->nfield, s->st));
@@ -818,38 +838,41 @@ int field_of(sphgpu_surfacer* s, long long n, const float* xyz, bool aniso) {
         SCHECK(s, hipStreamSynchronize(s->st));
         return 0;
     }
+    SurfRecs& recs = aniso ? s->ellipsoids : s->spheres;
+    if (int rc = ensure_records(s, recs, int(n))) return rc;
     int* const nfar = s->far + s->cap;
     SCHECK(s, hipMemsetAsync(nfar, 0, sizeof(int), s->st));
     if (n > 0) {
         hipLaunchKernelGGL(k_sf_keys, dim3(blocks), dim3(256), 0, s->st, s->S, (const float*)s->x, int(n), s->keys,
-                           s->vals);
-        radix_sort_pairs(s->keys, s->vals, int(n), s->keyBits, s->sort, s->st);
+                           recs.vals);
+        radix_sort_pairs(s->keys, recs.vals, int(n), s->keyBits, s->sort, s->st);
         hipLaunchKernelGGL(k_sf_gather, dim3(blocks), dim3(256), 0, s->st, (const float*)s->x,
-                           (const uint32_t*)s->vals, int(n), s->xs);
+                           (const uint32_t*)recs.vals, int(n), s->xs);
     }
     hipLaunchKernelGGL(k_sf_fill_i2, dim3(int((s->ncells + 255) / 256)), dim3(256), 0, s->st, s->ranges, int(s->ncells));
     if (n > 0) {
         hipLaunchKernelGGL(k_sf_ranges, dim3(blocks), dim3(256), 0, s->st, (const uint32_t*)s->keys, int(n), s->ranges);
         if (aniso)
             hipLaunchKernelGGL(k_sf_aniso, dim3(unsigned((4 * n + 255) / 256)), dim3(256), 0, s->st, s->S,
-                               (const float4*)s->xs, (const int2*)s->ranges, int(n), s->rec, s->box, s->far, nfar);
+                               (const float4*)s->xs, (const int2*)s->ranges, int(n), recs.rec, s->box, s->far, nfar);
         else
             hipLaunchKernelGGL(k_sf_sphere, dim3(blocks), dim3(256), 0, s->st, s->S, (const float4*)s->xs, int(n),
-                               s->rec, s->box, s->far, nfar);
+                               recs.rec, s->box, s->far, nfar);
     }
     if (!inBlocks) {
         if (n > 0)
-            hipLaunchKernelGGL(k_sf_splat, dim3(unsigned(n)), dim3(256), 0, s->st, s->S, (const SurfRec*)s->rec,
+            hipLaunchKernelGGL(k_sf_splat, dim3(unsigned(n)), dim3(256), 0, s->st, s->S, (const SurfRec*)recs.rec,
                                (const SurfBox*)s->box, (const int*)nullptr, (const int*)nullptr, int(n), s->field);
     } else {
-        launch_field(s);
+        launch_field(s, recs);
         if (n > 0)
             hipLaunchKernelGGL(k_sf_splat, dim3(unsigned(std::min<long long>(n, 1024))), dim3(256), 0, s->st, s->S,
-                               (const SurfRec*)s->rec, (const SurfBox*)s->box, (const int*)s->far, (const int*)nfar, 0,
+                               (const SurfRec*)recs.rec, (const SurfBox*)s->box, (const int*)s->far, (const int*)nfar, 0,
                                s->field);
     }
     SCHECK(s, hipGetLastError());
     SCHECK(s, hipStreamSynchronize(s->st));
+    if (aniso) s->nrec = int(n);
     return 0;
 }
 
@@ -945,7 +968,9 @@ void sphgpu_surfacer_destroy(sphgpu_surfacer* s) {
     if (!s) return;
     if (s->st) (void)hipStreamSynchronize(s->st);
     (void)hipFree(s->field); (void)hipFree(s->ranges); (void)hipFree(s->x); (void)hipFree(s->xs);
-    (void)hipFree(s->keys); (void)hipFree(s->vals); (void)hipFree(s->rec); (void)hipFree(s->box); (void)hipFree(s->far); (void)hipFree(s->sortMem);
+    (void)hipFree(s->keys); (void)hipFree(s->box); (void)hipFree(s->far); (void)hipFree(s->sortMem);
+    free_records(s->spheres);
+    free_records(s->ellipsoids);
     s->ring.release();
     (void)hipFree(s->mcCount); (void)hipFree(s->mcTmp); (void)hipFree(s->mcOut);
     if (s->st) (void)hipStreamDestroy(s->st);
@@ -983,8 +1008,8 @@ int sphgpu_surfacer_particles(sphgpu_surfacer* s, float* xbar, float* G, float* 
     std::vector<SurfRec> r(size_t(std::max(n, 0)));
     std::vector<uint32_t> order(size_t(std::max(n, 0)));
     if (n > 0) {
-        SCHECK(s, hipMemcpyAsync(r.data(), s->rec, sizeof(SurfRec) * n, hipMemcpyDeviceToHost, s->st));
-        SCHECK(s, hipMemcpyAsync(order.data(), s->vals, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s->st));
+        SCHECK(s, hipMemcpyAsync(r.data(), s->ellipsoids.rec, sizeof(SurfRec) * n, hipMemcpyDeviceToHost, s->st));
+        SCHECK(s, hipMemcpyAsync(order.data(), s->ellipsoids.vals, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s->st));
     }
     SCHECK(s, hipStreamSynchronize(s->st));
     for (int k = 0; k < n; ++k) {

@@ -317,7 +317,9 @@ int sphgpu_surfacer_grid(const sphgpu_surfacer* s, double grid_min[3], int grid_
 int sphgpu_surfacer_aniso(sphgpu_surfacer* s, long long n, const float* xyz);
 int sphgpu_surfacer_isotro(sphgpu_surfacer* s, long long n, const float* xyz);
 /* After sphgpu_surfacer_aniso, per particle in input order (each optional):
- * ellipsoid centre x_bar (3), G row-major (9), det G, neighbours within 2 r_h. */
+ * ellipsoid centre x_bar (3), G row-major (9), det G, neighbours within 2 r_h.
+ * They stay over a sphgpu_surfacer_isotro of as many particles; after one of
+ * another number there are none, and nothing is written. */
 int sphgpu_surfacer_particles(sphgpu_surfacer* s, float* xbar, float* G, float* det, int* neighbours);
 /* The node field (get_field), x fastest: grid_num[0] * grid_num[1] * grid_num[2]
  * floats; set_field replaces it (marching cubes on a caller's field). */
