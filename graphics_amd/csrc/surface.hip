@@ -797,17 +797,27 @@ int ensure_records(sphgpu_surfacer* s, SurfRecs& r, int n) {
 // 3622 / 1964; 60,000, c 4: 1126 / 1049; 15,000, c 6: 657 / 648; 15,000, c 4:
 // 430 / 524; 4,000, c 8: 461 / 386; 4,000, c 6: 346 / 433; isotropic 60,000,
 // c 4: 607 / 599; 15,000, c 6: 307 / 255; 4,000, c 8: 167 / 129; 4,000, c 6:
-// 111 / 124.  (A radius under 2^-30: see root.)
+// 111 / 124.  (A radius under 2^-30: see root.  A thin grid of nearly 2^31 nodes
+// can have more blocks than a launch of 2^32 threads holds.)
+struct FieldGrid {
+    long long x, y, z;
+    long long blocks() const { return x * y * z; }
+};
+FieldGrid field_grid(const sphgpu_surfacer* s) {
+    return {(s->fnum[0] + FB_X * FB_WAVES - 1) / (FB_X * FB_WAVES), (s->fnum[1] + FB_Y - 1) / FB_Y,
+            (s->fnum[2] + FB_Z - 1) / FB_Z};
+}
 bool field_blocks(const sphgpu_surfacer* s, long long n) {
     const double c = s->S.hcells;
-    return c >= 4.0 && double(n) * c * c * c >= 2.0e6 && s->S.rh >= 0x1p-30f;
+    return c >= 4.0 && double(n) * c * c * c >= 2.0e6 && s->S.rh >= 0x1p-30f &&
+           field_grid(s).blocks() < (1LL << 32) / (64 * FB_WAVES);
 }
 
 void launch_field(sphgpu_surfacer* s, const SurfRecs& r) {
-    const int tx = (s->fnum[0] + FB_X * FB_WAVES - 1) / (FB_X * FB_WAVES), ty = (s->fnum[1] + FB_Y - 1) / FB_Y,
-              tz = (s->fnum[2] + FB_Z - 1) / FB_Z;
-    hipLaunchKernelGGL(k_sf_field, dim3(unsigned(tx) * ty * tz), dim3(64 * FB_WAVES), 0, s->st, s->S,
-                       (const SurfRec*)r.rec, (const SurfBox*)s->box, (const int2*)s->ranges, tx, ty, s->field);
+    const FieldGrid g = field_grid(s);
+    hipLaunchKernelGGL(k_sf_field, dim3(unsigned(g.blocks())), dim3(64 * FB_WAVES), 0, s->st, s->S,
+                       (const SurfRec*)r.rec, (const SurfBox*)s->box, (const int2*)s->ranges, int(g.x), int(g.y),
+                       s->field);
 }
 
 // the field of n particles: binned, ellipsoids (aniso) or spheres, tiles

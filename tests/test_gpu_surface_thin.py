@@ -1,0 +1,38 @@
+"""A field on a thin grid of nearly 2^31 nodes, whose blocks of nodes would be more
+than one launch holds: the call runs, and the field holds the particles' sum."""
+import numpy as np
+import pytest
+
+from graphics_amd import sphgpu as sg
+
+pytestmark = pytest.mark.gpu
+
+
+def test_thin_grid_of_many_blocks(gpu):
+    print("[thin]", flush=True)
+    rh, cell, n = 0.02, 0.005, 32000          # 4 nodes a radius, 2.05 million touched nodes
+    side = (16600 - 6.5) * cell
+    s = sg.Surfacer((0.0,) * 3, (0.5 * cell, side, side), 0.01, rh, cell)
+    assert s.grid_num == (7, 16600, 16600)
+    blocks = -(-s.grid_num[1] // 4) * -(-s.grid_num[2] // 4)
+    assert blocks * 256 >= 1 << 32
+    rng = np.random.default_rng(0)
+    x = np.zeros((n, 3), np.float32)
+    x[:, 1:] = rng.uniform(0.0, 0.25, (n, 2))
+    x[-1, 1:] = side                          # the far corner
+    s.isotro(x)
+    f = s.field()
+    near = f[:80, :80]
+    want = np.zeros(near.shape)
+    at = [s.grid_min[a] + np.arange(near.shape[2 - a]) * cell for a in range(3)]
+    for p in x[:-1].astype(np.float64):
+        lo = [max(int((p[a] - s.grid_min[a]) / cell) - 5, 0) for a in range(3)]
+        d = [at[a][lo[a]:lo[a] + 12] - p[a] for a in range(3)]
+        r = np.sqrt((d[2] ** 2)[:, None, None] + (d[1] ** 2)[None, :, None] + (d[0] ** 2)[None, None, :]) / rh
+        w = np.where(r < 0.5, 8 * (1 - 6 * r ** 2 + 6 * r ** 3), np.where(r < 1.0, 16 * (1 - r) ** 3, 0.0))
+        want[lo[2]:lo[2] + 12, lo[1]:lo[1] + 12, lo[0]:lo[0] + 12] += w
+    want *= 0.01 ** 3 / (np.pi * rh ** 3)
+    # (coordinates up to 0.3 rounded at 3e-8, the spline's slope at most 3 of its peak a radius)
+    assert np.abs(near - want).max() <= 2e-5 * want.max()
+    assert f[-40:, -40:].max() > 0 and not f[400:420, 400:420].any()
+    s.close()
