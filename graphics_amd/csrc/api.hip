@@ -1893,7 +1893,7 @@ int read_in_order(sphgpu_handle* h, void* out, const void* dev, size_t bytes,
     if (h->D.npad == 0) return 0;
     if (h->nLive == h->nextId) {
         pass(nullptr);
-        HIPCHECK(h, h->ring.to_host(out, dev, bytes * (size_t)h->nextId, h->st));
+        HIPCHECK(h, h->ring.to_host(out, dev, bytes * (size_t)h->nextId, h->st, h->hRemoved));
         HIPCHECK(h, hipGetLastError());
         if (*h->hRemoved == 0) return 0;
     }

@@ -218,12 +218,14 @@ hipError_t HostRing::to_device(void* dst, const void* src, size_t bytes, hipStre
     return err.load() != int(hipSuccess) ? hipError_t(err.load()) : e;
 }
 
-hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream_t st) {
+hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream_t st, const int* veto) {
     if (bytes == 0) return hipStreamSynchronize(st);
+    // (asked for after the first bytes have arrived: the word was set before them)
+    auto wanted = [veto] { return !veto || __atomic_load_n(veto, __ATOMIC_ACQUIRE) == 0; };
     auto through = [&](char* at) {
         hipError_t e = hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e == hipSuccess) std::memcpy(dst, at, bytes);
+        if (e == hipSuccess && wanted()) std::memcpy(dst, at, bytes);
         return e;
     };
     if (bytes <= kDownOwnBytes) {
@@ -264,7 +266,7 @@ hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream
         for (int c; (c = next.fetch_add(1)) < n;) {
             const int s = c % slots;
             while (queued[s].load() != c) std::this_thread::yield();
-            if (err.load() == int(hipSuccess) && note(hipEventSynchronize(done[s]))) {
+            if (err.load() == int(hipSuccess) && note(hipEventSynchronize(done[s])) && wanted()) {
                 const size_t b = size_t(c) * kChunk;
                 std::memcpy(static_cast<char*>(dst) + b, mem + size_t(s) * kChunk, std::min(kChunk, bytes - b));
             }

@@ -41,8 +41,9 @@ struct HostRing {
     static constexpr int kUpThreads = 2;
 
     // device -> host; waits for everything queued on st before it, and
-    // returns with `dst` complete
-    hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t st);
+    // returns with `dst` complete.  veto: a pinned word that work queued before
+    // the call sets; `dst` is left as it was where it is not zero
+    hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t st, const int* veto = nullptr);
     // host -> device, queued on st (one past kUpOwnBytes has arrived on return); `src`
     // may be changed once it returns.  Every transfer of a ring goes through
     // one stream.
