@@ -220,9 +220,9 @@ __device__ __forceinline__ SurfBox box_of(const SurfParams& S, const SurfRec& o,
 // particles are two waves a SIMD, which wait for one load after another (774
 // us; 334 with four).
 __global__ __launch_bounds__(256) void k_sf_aniso(SurfParams S, const float4* __restrict__ xs,
-                                                  const int2* __restrict__ ranges, int n, SurfRec* rec, SurfBox* box,
-                                                  int* far, int* nfar) {
-    const int r0 = (blockIdx.x * 256 + threadIdx.x) >> 2, lane = threadIdx.x & 3;
+                                                  const int2* __restrict__ ranges, int first, int n, SurfRec* rec,
+                                                  SurfBox* box, int* far, int* nfar) {
+    const int r0 = first + int((blockIdx.x * 256 + threadIdx.x) >> 2), lane = threadIdx.x & 3;
     const int r = min(r0, n - 1);   // (every lane takes part in the sums)
     const float4 pi = xs[r];
     // pass 1: weighted mean (relative to the particle), neighbour count
@@ -519,13 +519,15 @@ __global__ __launch_bounds__(256) void k_sf_splat(SurfParams S, const SurfRec* _
 // The same for spheres, straight from the caller's positions: binning them costs
 // more than the splat of few nodes.  Isotropic calls with their field read, MI355X:
 // 4,000 particles at 4 nodes a radius 136 -> 81 us, 15,000 290 -> 229.
-__global__ __launch_bounds__(256) void k_sf_splat_spheres(SurfParams S, const float* __restrict__ x,
+__global__ __launch_bounds__(256) void k_sf_splat_spheres(SurfParams S, const float* __restrict__ x, int n,
                                                           float* __restrict__ field) {
-    const size_t q = 3 * (size_t)blockIdx.x;
-    SurfRec o;
-    SurfBox b;
-    sphere_of(S, make_float4(x[q], x[q + 1], x[q + 2], 0.0f), o, b);
-    splat(S, o, b, field);
+    for (int p = blockIdx.x; p < n; p += gridDim.x) {
+        const size_t q = 3 * (size_t)p;
+        SurfRec o;
+        SurfBox b;
+        sphere_of(S, make_float4(x[q], x[q + 1], x[q + 2], 0.0f), o, b);
+        splat(S, o, b, field);
+    }
 }
 
 struct McTable {
@@ -798,7 +800,8 @@ int ensure_records(sphgpu_surfacer* s, SurfRecs& r, int n) {
 // 430 / 524; 4,000, c 8: 461 / 386; 4,000, c 6: 346 / 433; isotropic 60,000,
 // c 4: 607 / 599; 15,000, c 6: 307 / 255; 4,000, c 8: 167 / 129; 4,000, c 6:
 // 111 / 124.  (A radius under 2^-30: see root.  A thin grid of nearly 2^31 nodes
-// can have more blocks than a launch of 2^32 threads holds.)
+// can have more blocks than a launch holds.)
+constexpr long long MAX_THREADS = 1LL << 31;   // of a launch (one of 2^32 is cut to its low 32 bits)
 struct FieldGrid {
     long long x, y, z;
     long long blocks() const { return x * y * z; }
@@ -810,7 +813,7 @@ FieldGrid field_grid(const sphgpu_surfacer* s) {
 bool field_blocks(const sphgpu_surfacer* s, long long n) {
     const double c = s->S.hcells;
     return c >= 4.0 && double(n) * c * c * c >= 2.0e6 && s->S.rh >= 0x1p-30f &&
-           field_grid(s).blocks() < (1LL << 32) / (64 * FB_WAVES);
+           field_grid(s).blocks() <= MAX_THREADS / (64 * FB_WAVES);
 }
 
 void launch_field(sphgpu_surfacer* s, const SurfRecs& r) {
@@ -839,10 +842,12 @@ int field_of(sphgpu_surfacer* s, long long n, const float* xyz, bool aniso) {
     if (aniso || n != s->nrec) s->nrec = 0;
     const int blocks = int((n + 255) / 256);
     const bool inBlocks = field_blocks(s, n);
+    // (a launch of 2^32 threads or more is cut: blocks take several particles from there)
+    const dim3 splatGrid(unsigned(std::min<long long>(n, MAX_THREADS / 256)));
     if (!inBlocks) SCHECK(s, hipMemsetAsync(s->field, 0, sizeof(float) * s->nfield, s->st));
     if (!inBlocks && !aniso) {
         if (n > 0)
-            hipLaunchKernelGGL(k_sf_splat_spheres, dim3(unsigned(n)), dim3(256), 0, s->st, s->S, (const float*)s->x,
+            hipLaunchKernelGGL(k_sf_splat_spheres, splatGrid, dim3(256), 0, s->st, s->S, (const float*)s->x, int(n),
                                s->field);
         SCHECK(s, hipGetLastError());
         SCHECK(s, hipStreamSynchronize(s->st));
@@ -863,15 +868,17 @@ int field_of(sphgpu_surfacer* s, long long n, const float* xyz, bool aniso) {
     if (n > 0) {
         hipLaunchKernelGGL(k_sf_ranges, dim3(blocks), dim3(256), 0, s->st, (const uint32_t*)s->keys, int(n), s->ranges);
         if (aniso)
-            hipLaunchKernelGGL(k_sf_aniso, dim3(unsigned((4 * n + 255) / 256)), dim3(256), 0, s->st, s->S,
-                               (const float4*)s->xs, (const int2*)s->ranges, int(n), recs.rec, s->box, s->far, nfar);
+            for (long long i = 0; i < n; i += MAX_THREADS / 4)
+                hipLaunchKernelGGL(k_sf_aniso, dim3(unsigned((4 * std::min(n - i, MAX_THREADS / 4) + 255) / 256)),
+                                   dim3(256), 0, s->st, s->S, (const float4*)s->xs, (const int2*)s->ranges, int(i),
+                                   int(n), recs.rec, s->box, s->far, nfar);
         else
             hipLaunchKernelGGL(k_sf_sphere, dim3(blocks), dim3(256), 0, s->st, s->S, (const float4*)s->xs, int(n),
                                recs.rec, s->box, s->far, nfar);
     }
     if (!inBlocks) {
         if (n > 0)
-            hipLaunchKernelGGL(k_sf_splat, dim3(unsigned(n)), dim3(256), 0, s->st, s->S, (const SurfRec*)recs.rec,
+            hipLaunchKernelGGL(k_sf_splat, splatGrid, dim3(256), 0, s->st, s->S, (const SurfRec*)recs.rec,
                                (const SurfBox*)s->box, (const int*)nullptr, (const int*)nullptr, int(n), s->field);
     } else {
         launch_field(s, recs);
