@@ -23,6 +23,7 @@ struct Stages {
     std::mutex lock;
     std::vector<Stage*> idle;
     int users = 0;
+    double rent = 0.0;   // us that plain copies since the last new stage took longer than through one
 };
 // (never destroyed: an object of static duration may release its ring late)
 Stages& stages() {
@@ -39,11 +40,27 @@ void destroy(Stage* s) {
     delete s;
 }
 
-// a stage of `bytes`, at most all slots, for transfers on st; nullptr and `err`
-// if there is none to be had
-Stage* borrow(size_t bytes, hipStream_t st, bool& counted, hipError_t& err) {
+// us that a stage of `bytes` costs when it is new (its allocation and the host's first
+// touch: 0.38 a KB, or next to nothing where the process gets memory that it had
+// before; half of it), and that a transfer to the host through one saves
+double price(size_t bytes) { return 25.0 + 0.19 / 1024.0 * double(bytes); }
+double saving(size_t bytes) {
+    const double kb = double(bytes) / 1024.0;
+    return bytes <= (size_t(512) << 10) ? 0.36 * kb : bytes <= HostRing::kChunk ? 15.0
+           : bytes < (size_t(32) << 20) ? 0.03 * kb : 0.07 * kb;
+}
+
+// a stage for a transfer of `bytes` on st; nullptr where none is idle and the
+// transfers so far (this one saves `saves` us) have not paid for a new one, or there
+// is none to be had
+Stage* borrow(size_t bytes, double saves, hipStream_t st, bool& counted) {
     hipDevice_t device = 0;
-    if ((err = hipStreamGetDevice(st, &device)) != hipSuccess) return nullptr;
+    if (hipStreamGetDevice(st, &device) != hipSuccess) return nullptr;
+    // up to a chunk the next power of two: a process that reads 100 KB does not
+    // touch 2 MB for it, and one that reads more each time touches twice that at most
+    size_t want = std::min((bytes + HostRing::kChunk - 1) / HostRing::kChunk, size_t(HostRing::kSlots)) * HostRing::kChunk;
+    if (bytes <= HostRing::kChunk)
+        for (want = 2 * HostRing::kDownOwnBytes; want < bytes;) want *= 2;
     Stage* s = nullptr;
     Stages& all = stages();
     {
@@ -52,14 +69,22 @@ Stage* borrow(size_t bytes, hipStream_t st, bool& counted, hipError_t& err) {
         counted = true;
         for (Stage* o : all.idle)
             if (o->device == device && (!s || o->cap > s->cap)) s = o;
+        if (!s || s->cap < want) {
+            all.rent += saves;
+            if (all.rent >= price(want)) {
+                all.rent = 0.0;
+            } else if (s && s->cap >= 2 * HostRing::kChunk) {
+                want = s->cap;         // (two chunks in turn will do)
+            } else {
+                return nullptr;
+            }
+        }
         if (s) all.idle.erase(std::find(all.idle.begin(), all.idle.end(), s));
     }
+    hipError_t err = hipSuccess;
     if (!s) {
         s = new (std::nothrow) Stage;
-        if (!s) {
-            err = hipErrorOutOfMemory;
-            return nullptr;
-        }
+        if (!s) return nullptr;
         s->device = device;
         int current = 0;
         err = hipGetDevice(&current);
@@ -68,12 +93,6 @@ Stage* borrow(size_t bytes, hipStream_t st, bool& counted, hipError_t& err) {
             if (err == hipSuccess) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
         if (current != device) (void)hipSetDevice(current);
     }
-    // up to a chunk the next power of two: a process that reads 100 KB does not
-    // touch 2 MB for it, and one that reads more each time touches twice that at most
-    // (the first reading of a small mesh 1.64 -> 1.29 ms)
-    size_t want = std::min((bytes + HostRing::kChunk - 1) / HostRing::kChunk, size_t(HostRing::kSlots)) * HostRing::kChunk;
-    if (bytes <= HostRing::kChunk)
-        for (want = 2 * HostRing::kDownOwnBytes; want < bytes;) want *= 2;
     if (err == hipSuccess && s->cap < want) {
         if (s->mem) (void)hipHostFree(s->mem);
         s->mem = nullptr;
@@ -85,6 +104,7 @@ Stage* borrow(size_t bytes, hipStream_t st, bool& counted, hipError_t& err) {
         }
     }
     if (err == hipSuccess) return s;
+    (void)hipGetLastError();           // (the transfer goes without)
     destroy(s);
     return nullptr;
 }
@@ -112,18 +132,21 @@ hipError_t HostRing::drain(hipStream_t st) {
     return hipStreamSynchronize(st);
 }
 
-hipError_t HostRing::reserve(size_t bytes, hipStream_t st) {
+bool HostRing::reserve(size_t bytes, hipStream_t st) {
     const size_t want = std::min((bytes + 0xFFFF) & ~size_t(0xFFFF), kOwn);
-    if (want <= cap) return hipSuccess;
-    if (hipError_t e = drain(st); e != hipSuccess) return e;
+    if (want <= cap) return true;
+    if (drain(st) != hipSuccess) return false;
     if (mem) (void)hipHostFree(mem);
     mem = nullptr;
     cap = 0;
     void* p = nullptr;
-    if (hipError_t e = hipHostMalloc(&p, want); e != hipSuccess) return e;
+    if (hipHostMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();       // (the transfer goes without)
+        return false;
+    }
     mem = static_cast<char*>(p);
     cap = want;
-    return hipSuccess;
+    return true;
 }
 
 void HostRing::release() {
@@ -136,7 +159,10 @@ void HostRing::release() {
     Stages& all = stages();
     {
         std::lock_guard<std::mutex> l(all.lock);
-        if (--all.users == 0) last.swap(all.idle);
+        if (--all.users == 0) {
+            last.swap(all.idle);
+            all.rent = 0.0;
+        }
     }
     for (Stage* s : last) destroy(s);
 }
@@ -165,24 +191,28 @@ int helpers(size_t bytes, size_t from, int most, int chunks) {
 
 hipError_t HostRing::to_device(void* dst, const void* src, size_t bytes, hipStream_t st) {
     if (bytes == 0) return hipSuccess;
+    auto plain = [&] {
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
+        return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    };
     if (bytes <= kUpOwnBytes) {
         // small ones one after another into the ring, until it is full
         if (used + bytes > cap) {
             if (hipError_t e = drain(st); e != hipSuccess) return e;
-            if (hipError_t e = reserve(2 * bytes, st); e != hipSuccess) return e;
+            if (bytes > cap && bytes > kUpAtOnceBytes && !upBefore) {
+                upBefore = true;
+                return plain();
+            }
+            if (!reserve(2 * bytes, st)) return plain();
         }
         char* at = mem + used;
         std::memcpy(at, src, bytes);
         used += (bytes + 255) & ~size_t(255);
         return hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, st);
     }
-    if (bytes < kUpSlotsBytes) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st);
-        return e == hipSuccess ? hipStreamSynchronize(st) : e;
-    }
-    hipError_t got = hipSuccess;
-    Stage* const stage = borrow(bytes, st, borrowed, got);
-    if (!stage) return got;
+    if (bytes < kUpSlotsBytes) return plain();
+    Stage* const stage = borrow(bytes, 0.005 / 1024.0 * double(bytes), st, borrowed);
+    if (!stage) return plain();
     char* const mem = stage->mem;
     hipEvent_t* const done = stage->done;
     const int n = int((bytes + kChunk - 1) / kChunk), slots = std::min<int>(int(stage->cap / kChunk), n);
@@ -222,6 +252,12 @@ hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream
     if (bytes == 0) return hipStreamSynchronize(st);
     // (asked for after the first bytes have arrived: the word was set before them)
     auto wanted = [veto] { return !veto || __atomic_load_n(veto, __ATOMIC_ACQUIRE) == 0; };
+    auto plain = [&] {
+        hipError_t e = veto ? hipStreamSynchronize(st) : hipSuccess;
+        if (e != hipSuccess || !wanted()) return e;
+        e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
+        return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    };
     auto through = [&](char* at) {
         hipError_t e = hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -229,13 +265,16 @@ hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream
         return e;
     };
     if (bytes <= kDownOwnBytes) {
-        if (hipError_t e = reserve(bytes, st); e != hipSuccess) return e;
+        if (bytes > cap && !downBefore) {
+            downBefore = true;
+            return plain();
+        }
+        if (!reserve(bytes, st)) return plain();
         used = 0;   // (this transfer follows the queued ones on st, and ends with a wait)
         return through(mem);
     }
-    hipError_t got = hipSuccess;
-    Stage* const stage = borrow(bytes, st, borrowed, got);
-    if (!stage) return got;
+    Stage* const stage = borrow(bytes, saving(bytes), st, borrowed);
+    if (!stage) return plain();
     if (bytes <= kChunk) {
         const hipError_t e = through(stage->mem);
         give_back(stage);

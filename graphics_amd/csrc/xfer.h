@@ -24,11 +24,17 @@ namespace sphgpu {
 // through the slots (two threads).
 //
 // The host's first touch of new pinned memory costs 0.4 ms a MB, several times
-// the transfer.  So each object owns 1 MB at most, for small transfers,
-// and larger ones borrow a stage (the next power of two up to 2 MB, then whole
-// chunks up to 16 MB) that the process's objects
-// share: one transfer at a time has it, idle ones are kept (two at most, per
-// device) while an object that has borrowed one lives.
+// the transfer.  So each object owns 1 MB at most, for small transfers, from its
+// second one on (the first upload of up to 64 KB), and larger ones borrow a stage
+// (the next power of two up to 2 MB, then whole chunks up to 16 MB) that the
+// process's objects share: one transfer at a time has it, idle ones are kept (two at
+// most, per device) while an object that has asked for one lives.  A stage is made, or grows, once the plain copies made
+// instead have cost what it does: at the first or second transfer of 64 to 512 KB
+// (256 KB plain 111 us, through a stage 20), after some thirty of 1 to 2 MB (126 / 110
+// at 2 MB), seven of 4 to 16 MB (470 / 270 at 8 MB), at the first of 48 MB.  (The first
+// mesh of a new surfacer, MI355X, pinned at once / plain: 40^3 nodes 137 / 101 us, 200 x
+// 150 x 160 2.6 / 1.25 ms, 241 x 173 x 229 5.3 / 2.3 ms.)  Where no pinned memory is to be
+// had, the copy is a plain one.
 struct HostRing {
     static constexpr int kSlots = 8;
     static constexpr size_t kOwn = size_t(1) << 20;
@@ -37,6 +43,7 @@ struct HostRing {
     static constexpr size_t kThreadedBytes = 2 * kChunk;
     static constexpr int kMaxThreads = 4;
     static constexpr size_t kUpOwnBytes = size_t(512) << 10;    // to the device: up to this through the own bytes,
+    static constexpr size_t kUpAtOnceBytes = size_t(64) << 10;  // the first one past this without own bytes is a plain copy
     static constexpr size_t kUpSlotsBytes = size_t(32) << 20;   // from this on through the slots
     static constexpr int kUpThreads = 2;
 
@@ -55,7 +62,8 @@ private:
     size_t cap = 0;                    // at most kOwn
     size_t used = 0;                   // bytes from `mem` on that queued transfers to the device may still read
     bool borrowed = false;             // counted among the users of the shared stages
-    hipError_t reserve(size_t bytes, hipStream_t st);
+    bool upBefore = false, downBefore = false;   // a small transfer was made without own bytes
+    bool reserve(size_t bytes, hipStream_t st);
     hipError_t drain(hipStream_t st);  // waits for them
 };
 
