@@ -793,14 +793,15 @@ int ensure_records(sphgpu_surfacer* s, SurfRecs& r, int n) {
 }
 
 // Blocks of nodes where the particles touch many nodes; where they touch few,
-// the blocks' search through the particles takes longer than the atomics.
-// Field calls (MI355X, us: one block per particle / blocks of nodes), n
-// particles, r_h = c nodes: anisotropic 150,000, c 8: 7968 / 3265; 60,000, c 8:
-// 3622 / 1964; 60,000, c 4: 1126 / 1049; 15,000, c 6: 657 / 648; 15,000, c 4:
-// 430 / 524; 4,000, c 8: 461 / 386; 4,000, c 6: 346 / 433; isotropic 60,000,
-// c 4: 607 / 599; 15,000, c 6: 307 / 255; 4,000, c 8: 167 / 129; 4,000, c 6:
-// 111 / 124.  (A radius under 2^-30: see root.  A thin grid of nearly 2^31 nodes
-// can have more blocks than a launch holds.)
+// the search through the particles takes longer than the atomics, and for spheres
+// the binning too, which they need for it alone.  Field calls (MI355X, us: one
+// block per particle / blocks of nodes), n particles, r_h = c nodes: anisotropic
+// 60,000, c 8: 3201 / 1698; 60,000, c 4: 896 / 772; 15,000, c 6: 570 / 576; 30,000, c 4:
+// 668 / 539; 4,000, c 8: 446 / 411; 8,000, c 6: 465 / 444; 15,000, c 4: 419 / 443; 4,000,
+// c 6: 335 / 403; isotropic 15,000, c 8: 380 / 236; 30,000, c 6: 337 / 257; 8,000, c 8:
+// 210 / 187; 60,000, c 4: 530 / 601; 15,000, c 6: 177 / 200; 4,000, c 8: 115 / 145.  (A
+// radius under 2^-30: see root.  A thin grid of nearly 2^31 nodes can have more
+// blocks than a launch holds.)
 constexpr long long MAX_THREADS = 1LL << 31;   // of a launch (one of 2^32 is cut to its low 32 bits)
 struct FieldGrid {
     long long x, y, z;
@@ -810,9 +811,9 @@ FieldGrid field_grid(const sphgpu_surfacer* s) {
     return {(s->fnum[0] + FB_X * FB_WAVES - 1) / (FB_X * FB_WAVES), (s->fnum[1] + FB_Y - 1) / FB_Y,
             (s->fnum[2] + FB_Z - 1) / FB_Z};
 }
-bool field_blocks(const sphgpu_surfacer* s, long long n) {
+bool field_blocks(const sphgpu_surfacer* s, long long n, bool aniso) {
     const double c = s->S.hcells;
-    return c >= 4.0 && double(n) * c * c * c >= 2.0e6 && s->S.rh >= 0x1p-30f &&
+    return c >= 4.0 && double(n) * c * c * c >= (aniso ? 2.0e6 : 4.0e6) && s->S.rh >= 0x1p-30f &&
            field_grid(s).blocks() <= MAX_THREADS / (64 * FB_WAVES);
 }
 
@@ -841,7 +842,7 @@ int field_of(sphgpu_surfacer* s, long long n, const float* xyz, bool aniso) {
     // (an isotropic call of as many particles leaves the last aniso call's records)
     if (aniso || n != s->nrec) s->nrec = 0;
     const int blocks = int((n + 255) / 256);
-    const bool inBlocks = field_blocks(s, n);
+    const bool inBlocks = field_blocks(s, n, aniso);
     // (a launch of 2^32 threads or more is cut: blocks take several particles from there)
     const dim3 splatGrid(unsigned(std::min<long long>(n, MAX_THREADS / 256)));
     if (!inBlocks) SCHECK(s, hipMemsetAsync(s->field, 0, sizeof(float) * s->nfield, s->st));

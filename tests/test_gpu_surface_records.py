@@ -9,7 +9,7 @@ from graphics_amd import sphgpu as sg
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,fine", [(900, 4), (1500, 2), (4000, 4), (40000, 2)])   # few nodes, and (the last two) blocks of nodes
+@pytest.mark.parametrize("n,fine", [(900, 4), (1500, 2), (8000, 4), (64000, 2)])   # few nodes, and (the last two) blocks of nodes
 def test_ellipsoids_stay_over_an_isotropic_field(gpu, n, fine):
     print(f"[records] n={n} fine={fine}", flush=True)
     rng = np.random.default_rng(n)

@@ -12,14 +12,14 @@ pytestmark = pytest.mark.gpu
 RH, RP, CELL = 0.5, 0.25, 2.0 ** -7
 
 
-@pytest.mark.parametrize("n", [4, 8])   # 64 nodes a radius: one block a particle, blocks of nodes
+@pytest.mark.parametrize("n", [8, 18])   # 64 nodes a radius: one block a particle, blocks of nodes
 def test_distance_is_correctly_rounded(gpu, n):
     print(f"[surface root] n={n}", flush=True)
     rng = np.random.default_rng(n)
-    corners = np.array([(i, j, k) for k in (0, 1) for j in (0, 1) for i in (0, 1)][:n], np.float64)
+    corners = np.array([(i, j, k) for k in (0, 1, 2) for j in (0, 1, 2) for i in (0, 1)][:n], np.float64)
     # (no two supports meet)
-    x = 0.125 + corners + (2 * corners - 1) * rng.integers(0, 6, (n, 3)) * 2.0 ** -10
-    s = sg.Surfacer((0.0,) * 3, (1.25,) * 3, RP, RH, CELL)
+    x = 0.125 + corners * (1.0 + 2.0 ** -6) + rng.integers(0, 8, (n, 3)) * 2.0 ** -10
+    s = sg.Surfacer((0.0,) * 3, (1.3125, 2.3125, 2.3125), RP, RH, CELL)
     s.isotro(x.astype(np.float32))
     f = s.field().astype(np.float64)
     at = [s.grid_min[a] + np.arange(s.grid_num[a]) * CELL for a in range(3)]
@@ -35,5 +35,5 @@ def test_distance_is_correctly_rounded(gpu, n):
         err = np.abs(f[pick] - want) / want
         seen += d.size
         assert np.all(err <= bound), (np.count_nonzero(err > bound), d.size)
-    assert seen > 100000
+    assert seen > 300000
 

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 def test_thin_grid_of_many_blocks(gpu):
     print("[thin]", flush=True)
-    rh, cell, n = 0.02, 0.005, 32000          # 4 nodes a radius, 2.05 million touched nodes
+    rh, cell, n = 0.02, 0.005, 63000          # 4 nodes a radius, 4.03 million touched nodes
     side = (16600 - 6.5) * cell
     s = sg.Surfacer((0.0,) * 3, (0.5 * cell, side, side), 0.01, rh, cell)
     assert s.grid_num == (7, 16600, 16600)
