@@ -327,7 +327,7 @@ __device__ __forceinline__ void layout_block(const Dev& D, uint32_t total, int* 
 // the table is written, and the counts cleared for the next search, key by
 // lane, so both stores are whole lines (eight keys a thread straight from
 // registers took 70 us for 5.3 million keys, this way 18).
-template <bool FLUID, int W>
+template <int W>
 __device__ __forceinline__ uint32_t scan_counts(uint32_t* __restrict__ c, int n, int per, uint32_t first,
                                                 uint32_t* lds) {
     const int t0 = (int)threadIdx.x * per, t1 = min(t0 + per, n);
@@ -360,8 +360,7 @@ __device__ __forceinline__ void write_runs(const Dev& D, uint32_t k0, const uint
     }
 }
 
-// a grid of at most SEARCH_KEYS_ONE keys: scan, layout and cell table in one block
-template <bool FLUID>
+// several scenes on at most SEARCH_KEYS_ONE keys: scan, layout and cell table in one block
 __global__ __launch_bounds__(SCAN1_THREADS) void k_search_one(Dev D, int2* __restrict__ table, int* __restrict__ out) {
     constexpr int W = SCAN1_THREADS / 64;
     __shared__ uint32_t lds[W];
@@ -369,15 +368,13 @@ __global__ __launch_bounds__(SCAN1_THREADS) void k_search_one(Dev D, int2* __res
     const int n = (int)D.totalKeys, per = ((n + SCAN1_THREADS - 1) / SCAN1_THREADS) | 1;
     for (int k = threadIdx.x; k < n; k += SCAN1_THREADS) c[k] = D.cellCnt[k];
     __syncthreads();
-    const uint32_t total = scan_counts<FLUID, W>(c, n, per, 0, lds);
-    if (FLUID) {
-        layout_block(D, total, out, lds);
-        __syncthreads();
-    }
-    write_runs<FLUID, W>(D, 0, c, n, table);
+    const uint32_t total = scan_counts<W>(c, n, per, 0, lds);
+    layout_block(D, total, out, lds);
+    __syncthreads();
+    write_runs<true, W>(D, 0, c, n, table);
 }
 
-// The same for one scene by several blocks: each adds up the counts before its
+// The same for one scene, and for the boundary, by several blocks: each adds up the counts before its
 // part for itself (the counts are in the cache, and a block that waited for the
 // others' sums would take another launch); k_place clears the counts.  For
 // 28,000 keys one block takes 11 us, mostly to write the table; parts of 2,048
@@ -399,7 +396,7 @@ __global__ __launch_bounds__(SCAN1_THREADS) void k_search_part(Dev D, int2* __re
         for (int q = 0; q < 8; ++q) s += v[q];
     }
     block_scan<W>(s, lds, &before);   // (its barriers also complete the staging of c)
-    const uint32_t own = scan_counts<FLUID, W>(c, n, (SEARCH_PART / SCAN1_THREADS) | 1, before, lds);
+    const uint32_t own = scan_counts<W>(c, n, (SEARCH_PART / SCAN1_THREADS) | 1, before, lds);
     write_runs<FLUID, W, false>(D, (uint32_t)k0, c, n, table);
     if (FLUID && blockIdx.x == gridDim.x - 1) layout_block(D, before + own, out, lds);
 }
@@ -432,7 +429,7 @@ __global__ __launch_bounds__(256) void k_cell_runs(Dev D, int2* __restrict__ tab
         if (k < n) c[k] = D.cellCnt[k0 + k];
     }
     __syncthreads();
-    scan_counts<FLUID, 4>(c, n, SEARCH_KEYS / 256, D.cellSums[blockIdx.x], lds);
+    scan_counts<4>(c, n, SEARCH_KEYS / 256, D.cellSums[blockIdx.x], lds);
     write_runs<FLUID, 4>(D, k0, c, n, table);
 }
 
@@ -1331,9 +1328,11 @@ void scan_cells(const Dev& D, int2* table, int* layoutOut, hipStream_t st) {
         hipLaunchKernelGGL(k_search_part<FLUID>, dim3(parts), dim3(SCAN1_THREADS), 0, st, D, table, layoutOut);
         return;
     }
-    if (D.totalKeys <= (uint32_t)SEARCH_KEYS_ONE) {
-        hipLaunchKernelGGL(k_search_one<FLUID>, dim3(1), dim3(SCAN1_THREADS), 0, st, D, table, layoutOut);
-        return;
+    if constexpr (FLUID) {
+        if (D.totalKeys <= (uint32_t)SEARCH_KEYS_ONE) {
+            hipLaunchKernelGGL(k_search_one, dim3(1), dim3(SCAN1_THREADS), 0, st, D, table, layoutOut);
+            return;
+        }
     }
     const int blocks = int((D.totalKeys + SEARCH_KEYS - 1) / SEARCH_KEYS);
     hipLaunchKernelGGL(k_cell_sums, dim3(blocks), dim3(256), 0, st, D);

@@ -491,7 +491,7 @@ double mlp_loss_sum(const double* part, int n) {
 
 // ---- gradient on caller-provided device buffers, scratch in a static array
 // Every buffer mlp_grad needs beyond its inputs and outputs (weight
-// fragments, activations, their gradients, loss and gradient partials) lives
+// fragments, loss and gradient partials) lives
 // in one file-scope device array, so the entry point allocates nothing.
 // Each GPU holds its own copy until the process ends; host code reaches it
 // only through the address hipGetSymbolAddress returns on that device.
@@ -667,8 +667,7 @@ extern "C" int sphgpu_mlp_gradient_device(const float* params, long long n, cons
     m.cap = MLP_DEV_MAX;
     const int k = int(n);
     // every scratch word the kernels read is written earlier in this call:
-    // fragments by the pack, activations and gradients for samples < n, loss
-    // partials per block, gradient partials per slice
+    // fragments by the pack, loss and gradient partials per slice
     mlp_pack(m, st);
     mlp_grad(m, feat, target, k, st);
     hipLaunchKernelGGL(k_mlp_loss_final, dim3(1), dim3(64), 0, st, (const double*)m.lossPart, mlp_slices(k), k,

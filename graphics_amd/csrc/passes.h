@@ -194,31 +194,31 @@ __device__ __forceinline__ void each_boundary_lu(const Dev& D, const Slot& s, in
     else each_in_list_lu(D.nbB, D.ncap, s.i, nb, nt, load, use);
 }
 
-// ---- K lanes a particle ---------------------------------------------------
-// K = 2 or 4 neighbouring lanes of a wave share a particle: of every eight
-// list entries lane h gathers and evaluates entries h * 8/K .. + 8/K - 1 (term),
-// then lane 0 adds the terms of the eight in list order (add), taking the
-// others' with a DPP quad permute, so its sums, the particle's, have the same
-// bits as those of one lane a particle (the other lanes' sums are not used),
-// as long as a term is rounded before it is added: a product that one lane fuses
-// into its sum differs in the last place.
+// ---- two lanes a particle ---------------------------------------------------
+// K = 2 neighbouring lanes of a wave share a particle: of every eight list
+// entries lane h gathers and evaluates entries 4 h .. 4 h + 3 (term), then lane 0
+// adds the terms of the eight in list order (add), taking the other's with a DPP
+// quad permute, so its sums, the particle's, have the same bits as those of one
+// lane a particle (the other lane's sums are not used), as long as a term is
+// rounded before it is added: a product that one lane fuses into its sum differs in
+// the last place, so such a term is a pair of factors that `add` multiplies.  (Four
+// lanes were slower everywhere but on the smallest scenes.)
 template <int K>
 struct Lanes {
-    static_assert(K == 2 || K == 4, "two or four lanes a particle");
+    static_assert(K == 2, "two lanes a particle");
     static constexpr int E = 8 / K;   // entries of a group a lane owns
 };
-// v of lane O of the particle's K
+// v of lane O of the particle's
 template <int K, int O, class T>
 __device__ __forceinline__ T lane_term(const T& v) {
     if constexpr (O == 0) {
         return v;   // (lane 0's sum is the particle's)
     } else {
-        constexpr int ctrl = K == 2 ? 0xF5 : O * 0x55;
         constexpr int N = sizeof(T) / 4;
         int w[N];
         __builtin_memcpy(w, &v, sizeof(T));
 #pragma unroll
-        for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_mov_dpp(w[k], ctrl, 0xf, 0xf, true);
+        for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_mov_dpp(w[k], 0xF5, 0xf, 0xf, true);
         T r;
         __builtin_memcpy(&r, w, sizeof(T));
         return r;
@@ -240,25 +240,18 @@ __device__ __forceinline__ void add_group(const T (&t)[Lanes<K>::E], bool second
     }
 }
 
-// a lane's 8/K packed entries of a group: 4/K words
+// a lane's four packed entries of a group: two words
 template <int K>
 struct Words {
     unsigned w[4 / K];
 };
 template <int K>
 __device__ __forceinline__ Words<K> ld_words(const int4* group, int h, bool nt) {
-    Words<K> r;
-    const unsigned* p = reinterpret_cast<const unsigned*>(group) + h * (4 / K);
-    if constexpr (K == 2) {
-        typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
-        const v2u_t* q = reinterpret_cast<const v2u_t*>(p);
-        const v2u_t v = nt ? __builtin_nontemporal_load(q) : *q;
-        r.w[0] = v.x;
-        r.w[1] = v.y;
-    } else {
-        r.w[0] = nt ? __builtin_nontemporal_load(p) : *p;
-    }
-    return r;
+    static_assert(K == 2, "two lanes a particle");
+    typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
+    const v2u_t* q = reinterpret_cast<const v2u_t*>(group) + h;
+    const v2u_t v = nt ? __builtin_nontemporal_load(q) : *q;
+    return Words<K>{{v.x, v.y}};
 }
 // entry e of the words
 template <int K>
@@ -298,8 +291,8 @@ __device__ __forceinline__ void each_in_list16_lanes(const int4* __restrict__ li
     }
 }
 
-// the same for 32-bit lists (groups of four, all listed or padding): lane h
-// owns entries h * 4/K .. of each group
+// the same for 32-bit lists (groups of four, all listed or padding): lane h owns
+// every second group
 template <int K, class LD, class TM, class AD>
 __device__ __forceinline__ void each_in_list_lanes(const int* __restrict__ list, int ncap, int i, int h, int n,
                                                    bool nt, LD&& load, TM&& term, AD&& add) {
@@ -316,7 +309,7 @@ __device__ __forceinline__ void each_in_list_lanes(const int* __restrict__ list,
         int j[E];
 #pragma unroll
         for (int k = 0; k < E; ++k) {
-            j[k] = K == 2 ? w[k] : ((h & 1) ? w[2 + k] : w[k]);
+            j[k] = w[k];
             r[k] = load(j[k]);
         }
         decltype(term(0, r[0])) t[E];

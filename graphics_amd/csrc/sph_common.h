@@ -105,7 +105,7 @@ struct Dev {
     int* id;           // original id, -1 for padding / removed
     float* ksum;       // DFSPH accumulated kappa*dt^2; IISPH pressure (warm start)
     float* kvsum;      // DFSPH accumulated kappaV*dt
-    uint32_t* key;     // cell key of each slot (KEY_INVALID for padding)
+    uint32_t* key;     // radix search: cell key of each slot (KEY_INVALID for padding)
     // alternate buffers (reorder / integration targets)
     float4* x2;
     float4* v2;
@@ -383,8 +383,6 @@ struct Kahan {
     }
 };
 
-// Deterministic FP64 block sum over 256 threads (4 waves): fixed shuffle tree
-// per wave, then waves in order.  Every thread of the block must call it.
 // v of lane l ^ X in a butterfly 32, 16, .., 1 over a wave: cross-row exchanges
 // and row rotations, which take a few cycles where a shuffle goes through the
 // LDS (64 a step).  X = 8, 4, 2, 1 read lane l + X of the row of 16, which
@@ -415,6 +413,8 @@ __device__ __forceinline__ float butterfly(float v) {
     return __int_as_float(butterfly<X>(__float_as_int(v)));
 }
 
+// Deterministic FP64 block sum over 256 threads (4 waves): fixed shuffle tree
+// per wave, then waves in order.  Every thread of the block must call it.
 __device__ __forceinline__ double block_sum_256(double v, double* lds) {
     v += butterfly<32>(v);
     v += butterfly<16>(v);
@@ -532,7 +532,8 @@ void exclusive_scan_u32(uint32_t* data, int n, uint32_t* tmp, hipStream_t st);
 // Counting search (Dev::cellRuns): particles counted per cell key, the counts
 // scanned into the cell table, and each cell's particles put in slot order.
 constexpr int SEARCH_KEYS = 9 * 256;       // keys per block of the scan (nine a thread: odd)
-constexpr int SEARCH_KEYS_ONE = 32768;     // grids up to this are scanned by one block
+constexpr int SEARCH_KEYS_ONE = 32768;     // grids up to this take one launch: parts of one scene or the
+                                           // boundary, one block for several scenes
 constexpr int SEARCH_CELLS_MIN = 12000000; // largest grid: SEARCH_CELLS_MIN cells and
 constexpr int SEARCH_CELLS_PER = 8;        // SEARCH_CELLS_PER per particle slot
 void launch_search_fluid(const Dev& D, uint32_t* keys, uint32_t* arrival, uint32_t* order, int* layoutOut,

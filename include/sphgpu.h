@@ -428,8 +428,8 @@ int  sphgpu_mlp_train(sphgpu_mlp* m, long long n, const float* feat, const float
  * (a hipStream_t; NULL = the default stream) and the call returns without
  * waiting.  No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight training
- * loops).  Its scratch (weight fragments, activations, partial sums; 8.2
- * MB) is one static array per GPU, held until the process ends, so
+ * loops).  Its scratch (weight fragments, partial sums; 3.5 MB) is one
+ * static array per GPU, held until the process ends, so
  * n <= SPHGPU_MLP_DEVICE_MAX (else SPHGPU_E_CAPACITY), and calls that
  * overlap on one GPU (on different streams, or from different threads)
  * race on it; calls on one stream run one after another.  Same kernels and
