@@ -145,7 +145,7 @@ struct Rec3x2 {
 // A window of the size a tile needs (2,400 records on a dam) leaves room for
 // two blocks a CU (pass A), so the passes wait on memory unless each block
 // holds many waves: with two lanes a particle there are 16 on a CU, and the
-// arithmetic takes two thirds of the time.  Two tiles a block with one lane a
+// VALU is busy three quarters of the time.  Two tiles a block with one lane a
 // particle, the second tile's window requested during the first's loops (8
 // waves a CU), took 290 / 292 us for the divergence / density pass of 4M
 // particles, 80 / 84 of 1M and 21 / 21 of 117k; two lanes take 248 / 256,

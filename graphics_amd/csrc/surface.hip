@@ -363,8 +363,9 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 // mantissa of even and odd binades: the same for every float from 2^-102 up.  Below
 // 2^-100 the root of 2^-100: for the radii that come here (field_blocks) the spline
 // is its value at 0 to the last place at both.  The hardware's own root is one
-// place off in 15 cases of 100.  120,000 particles and 22 million nodes, the
-// whole call: with the hardware's root 4.97 ms, sqrtf 5.30, this 4.95.
+// place off in 15 cases of 100.  120,000 particles and 22 million nodes: the kernel
+// with the hardware's root 1.72 ms, with this 1.83; the whole call 4.97 and 5.0, with
+// sqrtf 5.30.
 __device__ __forceinline__ float root(float x) {
     x = fmaxf(x, 0x1p-100f);
     const float y = __builtin_amdgcn_rsqf(x), g = x * y;
@@ -381,8 +382,8 @@ __device__ __forceinline__ float root(float x) {
 // their lane into scalars, and added to the nodes in registers.  One wave alone
 // sums a node, in particle order, so there are no atomics and the sums are the
 // same every run.
-// Bound by the arithmetic: 0.92 G wave instructions, nine tenths of the time,
-// for 120,000 particles and 22 million nodes (1.69 ms).  Boxes of the particles
+// Bound by the arithmetic: 1.04 G wave instructions, nine tenths of the time,
+// for 120,000 particles and 22 million nodes (1.83 ms).  Boxes of the particles
 // over tiles of nodes in LDS took 2.5 ms (index arithmetic for each node, and
 // a tile's edge cuts the boxes into parts that fill few lanes); one block per
 // particle with FP32 atomics to memory 5.6 ms, at the rate of the atomics (46
