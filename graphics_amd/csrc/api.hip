@@ -1865,8 +1865,8 @@ int live_slots(sphgpu_handle* h, std::vector<std::pair<int, int>>& out) {
 }  // namespace
 
 namespace {
-// ranks of the live ids (general readback: particles were removed); *live = their number
-int live_ranks(sphgpu_handle* h, long long* live) {
+// queues the ranks of the live ids (general readback: particles were removed)
+int live_ranks(sphgpu_handle* h) {
     const long long words = h->nextId + 1;
     if (h->idRankCap < words) {
         hipFree(h->idRank);
@@ -1877,29 +1877,33 @@ int live_ranks(sphgpu_handle* h, long long* live) {
         h->idRankCap = cap;
     }
     launch_live_ranks(h->D, h->idRank, int(h->nextId), h->idRank + h->idRankCap, h->st);
-    uint32_t n = 0;
-    HIPCHECK(h, hipMemcpyAsync(&n, h->idRank + h->nextId, sizeof(n), hipMemcpyDeviceToHost, h->st));
-    HIPCHECK(h, hipStreamSynchronize(h->st));
-    *live = n;
     return 0;
 }
 
-// `pass(rank, removed)` queues the kernel that writes n values of `bytes`
-// each, in id order, to the device buffer `dev`; copied to `out`.  While every
-// id ever given is live (the host's count says so, and the device counts no
-// removal since) a value's place is its id; otherwise it is the rank of the id.
+// `pass(rank)` queues the kernel that writes a value of `bytes` for each live
+// particle, in id order, to the device buffer `dev`, and the device's count of
+// removals since the host's; copied to `out`.  While every id ever given is live a
+// value's place is its id; otherwise it is the rank of the id.  The host's count of
+// the live ones holds unless particles were removed that no statistics have
+// reported: the transfer asks for those before it writes, so nothing past the live
+// particles' values is written to `out`, and it is made again then.
 int read_in_order(sphgpu_handle* h, void* out, const void* dev, size_t bytes,
                   const std::function<void(const uint32_t*)>& pass) {
     if (h->D.npad == 0) return 0;
-    if (h->nLive == h->nextId) {
-        pass(nullptr);
-        HIPCHECK(h, h->ring.to_host(out, dev, bytes * (size_t)h->nextId, h->st, h->hRemoved));
-        HIPCHECK(h, hipGetLastError());
-        if (*h->hRemoved == 0) return 0;
+    const bool all = h->nLive == h->nextId;
+    if (!all)
+        if (int rc = live_ranks(h)) return rc;
+    pass(all ? nullptr : h->idRank);
+    HIPCHECK(h, h->ring.to_host(out, dev, bytes * (size_t)h->nLive, h->st, h->hRemoved));
+    HIPCHECK(h, hipGetLastError());
+    if (*h->hRemoved == 0) return 0;
+    if (all) {
+        if (int rc = live_ranks(h)) return rc;
+        pass(h->idRank);
     }
-    long long live = 0;
-    if (int rc = live_ranks(h, &live)) return rc;
-    pass(h->idRank);
+    uint32_t live = 0;
+    HIPCHECK(h, hipMemcpyAsync(&live, h->idRank + h->nextId, sizeof(live), hipMemcpyDeviceToHost, h->st));
+    HIPCHECK(h, hipStreamSynchronize(h->st));
     HIPCHECK(h, h->ring.to_host(out, dev, bytes * (size_t)live, h->st));
     HIPCHECK(h, hipGetLastError());
     return 0;
@@ -1950,13 +1954,9 @@ int sphgpu_get_fluid_ids(sphgpu_handle* h, long long* out) {
             return SPHGPU_OK;
         }
     }
-    long long live = 0;
-    if (int rc = live_ranks(h, &live)) return rc;
     long long* dev = reinterpret_cast<long long*>(D.x2);
-    launch_ids_by_rank(D, h->idRank, dev, h->hRemoved, h->st);
-    HIPCHECK(h, h->ring.to_host(out, dev, sizeof(long long) * (size_t)live, h->st));
-    HIPCHECK(h, hipGetLastError());
-    return SPHGPU_OK;
+    return read_in_order(h, out, dev, sizeof(long long),
+                         [&](const uint32_t* rank) { launch_ids_by_rank(D, rank, dev, h->hRemoved, h->st); });
 }
 
 // ---- frame output ---------------------------------------------------------

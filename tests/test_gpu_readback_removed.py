@@ -13,34 +13,56 @@ pytestmark = pytest.mark.gpu
 S = 0.02
 
 
+def _read(sim, n):
+    """Fields and ids in buffers of n particles, with what was not written left as it was."""
+    fp, lp = C.POINTER(C.c_float), C.POINTER(C.c_longlong)
+    got = {}
+    for field, comp in ((sg.F_POS, 3), (sg.F_VEL, 3), (sg.F_RHO, 1)):
+        a = np.full((n, comp), -7.25, np.float32)
+        assert sim.lib.sphgpu_get_fluid(sim.h, field, a.ctypes.data_as(fp)) == 0
+        got[field] = a
+    ids = np.full(n, -3, np.int64)
+    assert sim.lib.sphgpu_get_fluid_ids(sim.h, ids.ctypes.data_as(lp)) == 0
+    return got, ids
+
+
 @pytest.mark.parametrize("n", [(10, 10, 10), (40, 39, 38), (80, 80, 70)])
 def test_nothing_past_the_live_particles(gpu, n):
     print(f"[removed] {n}", flush=True)
     g = np.stack(np.meshgrid(*(np.arange(k) for k in n), indexing="ij"), -1).reshape(-1, 3)
     x = ((g + 1.0) * S).astype(np.float32)
     v = np.zeros_like(x)
-    out = np.flatnonzero(g[:, 1] == n[1] - 1)[::3]
-    v[out] = (0.0, 300.0, 0.0)                       # past the roof in the first step
+    roof = np.flatnonzero(g[:, 1] == n[1] - 1)
+    first, later = roof[::3], roof[1::3]
+    v[first] = (0.0, 300.0, 0.0)                     # past the roof, 3 S above, in the first step
+    v[later] = (0.0, 25.0, 0.0)                      # and in the third (60 mm at 25 mm a step)
     top = tuple((k + 3) * S for k in n)
     sim = sg.Simulation(sg.default_params(solver=sg.WCSPH, spacing_r=S, smooth_radius_h=2 * S, dt=1e-3,
                                           space_min=(-0.05,) * 3, space_max=top))
     sim.add_phase(1000.0, 0.01)
     sim.add_fluid(x, v)
     sim.init()
+
+    def check(gone):
+        size = sim.num_fluid()
+        got, ids = _read(sim, size)
+        keep = np.setdiff1d(np.arange(len(x)), gone)
+        assert np.array_equal(ids[:len(keep)], keep)
+        assert np.all(ids[len(keep):] == -3)
+        for a in got.values():
+            assert np.all(a[len(keep):] == -7.25)
+            assert not np.any(a[:len(keep)] == -7.25)
+        still = np.isin(keep, roof, invert=True)
+        assert np.abs(got[sg.F_POS][:len(keep)][still] - x[keep][still]).max() < S
+        return size
+
     sim.step(stats=False)
-    live = len(x) - len(out)
-    assert sim.num_fluid() == len(x)                 # (not reported yet)
-    lib, fp = sim.lib, C.POINTER(C.c_float)
-    got = {}
-    for field, comp in ((sg.F_POS, 3), (sg.F_VEL, 3), (sg.F_RHO, 1)):
-        a = np.full(len(x) * comp, -7.25, np.float32)
-        assert lib.sphgpu_get_fluid(sim.h, field, a.ctypes.data_as(fp)) == 0
-        assert np.all(a[live * comp:] == -7.25), np.count_nonzero(a[live * comp:] != -7.25)
-        got[field] = a[:live * comp]
-    ids = np.full(len(x), -3, np.int64)
-    assert lib.sphgpu_get_fluid_ids(sim.h, ids.ctypes.data_as(C.POINTER(C.c_longlong))) == 0
-    assert np.all(ids[live:] == -3)
-    assert np.array_equal(ids[:live], np.setdiff1d(np.arange(len(x)), out))
-    keep = np.setdiff1d(np.arange(len(x)), out)
-    assert np.abs(got[sg.F_POS].reshape(-1, 3) - x[keep]).max() < 0.5 * S
+    assert check(first) == len(x)                    # (not reported yet)
+    sim.step()
+    assert check(first) == len(x) - len(first)       # reported: read by rank
+    sim.step(stats=False)
+    sim.step(stats=False)
+    assert check(np.concatenate([first, later])) == len(x) - len(first)   # and more that are not
+    sim.step()
+    assert check(np.concatenate([first, later])) == len(x) - len(first) - len(later)
     sim.close()
