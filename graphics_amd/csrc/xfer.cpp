@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <mutex>
 #include <new>
@@ -42,17 +43,29 @@ void destroy(Stage* s) {
 
 // us that a stage of `bytes` costs when it is new (its allocation and the host's first
 // touch: 0.38 a KB, or next to nothing where the process gets memory that it had
-// before; half of it), and that a transfer to the host through one saves
+// before; half of it), and that a transfer through one takes
 double price(size_t bytes) { return 25.0 + 0.19 / 1024.0 * double(bytes); }
-double saving(size_t bytes) {
-    const double kb = double(bytes) / 1024.0;
-    return bytes <= (size_t(512) << 10) ? 0.36 * kb : bytes <= HostRing::kChunk ? 15.0
-           : bytes < (size_t(32) << 20) ? 0.03 * kb : 0.07 * kb;
+double staged(size_t bytes, bool up) {
+    return 10.0 + (up ? 0.027 : bytes <= HostRing::kChunk ? 0.05 : 0.033) / 1024.0 * double(bytes);
 }
 
-// a stage for a transfer of `bytes` on st; nullptr where none is idle and the
-// transfers so far (this one saves `saves` us) have not paid for a new one, or there
-// is none to be had
+// a plain copy of a transfer that a stage would take: what it takes longer counts
+// towards a stage
+template <class F>
+hipError_t rented(size_t bytes, bool up, hipStream_t st, F&& copy) {
+    if (const hipError_t e = hipStreamSynchronize(st); e != hipSuccess) return e;   // (not the wait for other work)
+    const auto from = std::chrono::steady_clock::now();
+    const hipError_t e = copy();
+    const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - from).count();
+    Stages& all = stages();
+    std::lock_guard<std::mutex> l(all.lock);
+    all.rent += std::max(0.0, us - staged(bytes, up));
+    return e;
+}
+
+// a stage for a transfer of `bytes` on st; nullptr where none is idle and the plain
+// copies so far, with what this one would (`saves`), have not cost what a new one
+// does, or there is none to be had
 Stage* borrow(size_t bytes, double saves, hipStream_t st, bool& counted) {
     hipDevice_t device = 0;
     if (hipStreamGetDevice(st, &device) != hipSuccess) return nullptr;
@@ -70,8 +83,7 @@ Stage* borrow(size_t bytes, double saves, hipStream_t st, bool& counted) {
         for (Stage* o : all.idle)
             if (o->device == device && (!s || o->cap > s->cap)) s = o;
         if (!s || s->cap < want) {
-            all.rent += saves;
-            if (all.rent >= price(want)) {
+            if (all.rent + saves >= price(want)) {
                 all.rent = 0.0;
             } else if (s && s->cap >= 2 * HostRing::kChunk) {
                 want = s->cap;         // (two chunks in turn will do)
@@ -211,8 +223,8 @@ hipError_t HostRing::to_device(void* dst, const void* src, size_t bytes, hipStre
         return hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, st);
     }
     if (bytes < kUpSlotsBytes) return plain();
-    Stage* const stage = borrow(bytes, 0.005 / 1024.0 * double(bytes), st, borrowed);
-    if (!stage) return plain();
+    Stage* const stage = borrow(bytes, 0.0, st, borrowed);
+    if (!stage) return rented(bytes, true, st, plain);
     char* const mem = stage->mem;
     hipEvent_t* const done = stage->done;
     const int n = int((bytes + kChunk - 1) / kChunk), slots = std::min<int>(int(stage->cap / kChunk), n);
@@ -259,7 +271,11 @@ hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream
         return e == hipSuccess ? hipStreamSynchronize(st) : e;
     };
     auto through = [&](char* at) {
-        hipError_t e = hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, st);
+        hipError_t e = launch_copy_out(at, src, bytes, st);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            e = hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, st);
+        }
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e == hipSuccess && wanted()) std::memcpy(dst, at, bytes);
         return e;
@@ -273,8 +289,10 @@ hipError_t HostRing::to_host(void* dst, const void* src, size_t bytes, hipStream
         used = 0;   // (this transfer follows the queued ones on st, and ends with a wait)
         return through(mem);
     }
-    Stage* const stage = borrow(bytes, saving(bytes), st, borrowed);
-    if (!stage) return plain();
+    // (a plain copy of 32 MB or more is bound by the destination's page faults on one
+    // thread: a stage pays at the first)
+    Stage* const stage = borrow(bytes, bytes < kUpSlotsBytes ? 0.0 : 0.07 / 1024.0 * double(bytes), st, borrowed);
+    if (!stage) return rented(bytes, false, st, plain);
     if (bytes <= kChunk) {
         const hipError_t e = through(stage->mem);
         give_back(stage);

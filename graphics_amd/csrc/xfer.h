@@ -28,13 +28,21 @@ namespace sphgpu {
 // second one on (the first upload of up to 64 KB), and larger ones borrow a stage
 // (the next power of two up to 2 MB, then whole chunks up to 16 MB) that the
 // process's objects share: one transfer at a time has it, idle ones are kept (two at
-// most, per device) while an object that has asked for one lives.  A stage is made, or grows, once the plain copies made
-// instead have cost what it does: at the first or second transfer of 64 to 512 KB
-// (256 KB plain 111 us, through a stage 20), after some thirty of 1 to 2 MB (126 / 110
-// at 2 MB), seven of 4 to 16 MB (470 / 270 at 8 MB), at the first of 48 MB.  (The first
-// mesh of a new surfacer, MI355X, pinned at once / plain: 40^3 nodes 137 / 101 us, 200 x
-// 150 x 160 2.6 / 1.25 ms, 241 x 173 x 229 5.3 / 2.3 ms.)  Where no pinned memory is to be
-// had, the copy is a plain one.
+// most, per device) while an object that has asked for one lives.  A stage is made,
+// or grows, once the plain copies made instead have cost what it does: they take 32
+// or 134 us for 256 KB, 75 or 420 for 1 MB, as the runtime's engine for the stream
+// goes (through a stage 20 and 60), 470 for 8 MB (270), 4.9 ms for 48 MB (1.4).  (The
+// first mesh of a new surfacer, MI355X, pinned at once / plain: 40^3 nodes 137 / 101
+// us, 200 x 150 x 160 2.6 / 1.25 ms, 241 x 173 x 229 5.3 / 2.3 ms.)  Where no pinned
+// memory is to be had, the copy is a plain one.
+//
+// To the host, transfers of up to a chunk are a kernel's stores to the pinned
+// bytes: 15 us for 20 KB, 33 for 1 MB and 52 for 2 MB with the wait, where the
+// runtime's copy takes 20, 39 and 57, and 60 to 130 for 20 KB in some handles' streams.
+// (readback.hip; where the launch is refused, as on a stream of another device than
+// the caller's or for odd addresses, the runtime's copy does it)
+hipError_t launch_copy_out(void* pinned, const void* src, size_t bytes, hipStream_t st);
+
 struct HostRing {
     static constexpr int kSlots = 8;
     static constexpr size_t kOwn = size_t(1) << 20;
