@@ -14,7 +14,7 @@ namespace sphgpu {
 // finished ones out.  The host copy of a large transfer is bound by the
 // destination's page faults on one thread (3.4 of 3.7 ms at 48 MB), so above
 // kThreadedBytes the chunks are shared by up to four threads that end before
-// the call returns.  Measured (MI355X, fresh destination): 20 KB 16 -> 9 us,
+// the call returns.  Measured (MI355X, fresh destination, engine alone): 20 KB 16 -> 9 us,
 // 188 KB 85 -> 16 us, 1.4 MB 139 -> 78 us, 12 MB 777 -> 411 us, 48 MB 4.85 ->
 // 1.44 ms; chunks of 1 and 4 MB were 25 and 4 % slower at 48 MB, eight
 // threads no faster than four.
@@ -37,7 +37,7 @@ namespace sphgpu {
 // memory is to be had, the copy is a plain one.
 //
 // To the host, transfers of up to a chunk are a kernel's stores to the pinned
-// bytes: 15 us for 20 KB, 33 for 1 MB and 52 for 2 MB with the wait, where the
+// bytes: 15 us for 20 KB, 33 for 1 MB and 52 for 2 MB with a kernel before and the wait, where the
 // runtime's copy takes 20, 39 and 57, and 60 to 130 for 20 KB in some handles' streams.
 // (readback.hip; where the launch is refused, as on a stream of another device than
 // the caller's or for odd addresses, the runtime's copy does it)
